@@ -340,31 +340,41 @@ static void fill_seg(Seg<T>& s, const Op* op, int64_t off, int nblocks, int nr, 
     s.part = part;
 }
 
-// Block maps of a launch over segments of nb[g] blocks each (entries: segment
-// | block within it << kSegBits), one after the other: segment by segment,
-// which the vector kernels run (a workgroup's rows stream from one region of
+// Block maps of a launch over segments of nb[g] row blocks and ng[g] gather
+// workgroups each (entries: segment | block within it << kSegBits), one after
+// the other: segment by segment over the row blocks, which the vector kernels run (a workgroup's rows stream from one region of
 // each vector), then round-robin (block b of every segment, then block b +
 // 1), which the E gathers run: segments that share an operator (the groups of
 // a streamed solve) gather through each tile together, its metadata read
 // into an L2 once for all of them rather than once per segment.
-static std::vector<int> block_map(const std::vector<int>& nb) {
+static std::vector<int> block_map(const std::vector<int>& nb, const std::vector<int>& ng) {
     if (nb.size() > (size_t)kMaxSegs) throw ArgError("too many segments in one launch");
     int most = 0;
     size_t total = 0;
-    for (int v : nb) {
-        most = std::max(most, v);
-        total += (size_t)v;
+    for (size_t g = 0; g < nb.size(); ++g) {
+        most = std::max(most, std::max(nb[g], ng[g]));
+        total += (size_t)nb[g] + (size_t)ng[g];
     }
     if (most > (1 << (31 - kSegBits))) throw ArgError("operator too large for one launch's block map");
     std::vector<int> m;
-    m.reserve(2 * total);
+    m.reserve(total);
     for (size_t g = 0; g < nb.size(); ++g)   // segment by segment: the vector kernels
         for (int b = 0; b < nb[g]; ++b) m.push_back((int)g | (b << kSegBits));
     for (int b = 0; b < most; ++b)           // round-robin: the gathers
-        for (size_t g = 0; g < nb.size(); ++g)
-            if (b < nb[g]) m.push_back((int)g | (b << kSegBits));
+        for (size_t g = 0; g < ng.size(); ++g)
+            if (b < ng[g]) m.push_back((int)g | (b << kSegBits));
     return m;
 }
+
+// Fewest shared-stencil tiles of the operators of a launch (0: some have none).
+template <typename It, typename F>
+static int fewest_tiles(It b, It e, F&& op_of) {
+    int grp = b == e ? 0 : INT_MAX;
+    for (; b != e; ++b) grp = std::min(grp, op_of(*b)->ngt);
+    return grp;
+}
+
+static int row_blocks(const Op* op) { return (int)((op->D + kBlock - 1) / kBlock); }
 
 // The launches of a run of iterations between two host checks (16 of a
 // streamed solve, 4 at a time of a batch solve's chunks) captured once into a
@@ -418,25 +428,26 @@ struct BatchBytes {
         return r256(tables) + r256(vec64) + (vec32 ? r256(vec32) : 0) + r256(pack);
     }
 };
-static BatchBytes batch_bytes(int G, int blocks, int64_t total, int NR, bool refine) {
+static BatchBytes batch_bytes(int G, int blocks, int gblocks, int64_t total, int NR, bool refine) {
     auto r256 = [](size_t n) { return (n + 255) & ~size_t(255); };
     BatchBytes b;
-    b.tables = r256(sizeof(Seg<double>) * G) + r256(sizeof(Seg<float>) * G) + r256(sizeof(int) * 2 * (size_t)blocks) +
+    b.tables = r256(sizeof(Seg<double>) * G) + r256(sizeof(Seg<float>) * G) + r256(sizeof(int) * ((size_t)blocks + gblocks)) +
                r256(sizeof(KState) * (size_t)G * kMaxNR) + r256(sizeof(double) * 2 * NR * (size_t)blocks) + 256;
     b.vec64 = sizeof(double) * (size_t)total * (refine ? 5 : 11) + 1024;
     b.vec32 = refine ? sizeof(float) * (size_t)total * 10 + 1024 : 0;
     b.pack = sizeof(PackEntry) * (size_t)G * NR + sizeof(int) * (size_t)blocks * NR + 512;
     return b;
 }
-// One operator of D rows with NR right-hand sides.
-static BatchBytes batch_bytes1(int64_t D, int NR, bool refine) {
-    return batch_bytes(1, (int)((D + kBlock - 1) / kBlock), (D * NR + 63) & ~int64_t(63), NR, refine);
+// One operator with NR right-hand sides.
+static BatchBytes batch_bytes1(const Op* op, int NR, bool refine) {
+    const int nb = row_blocks(op);
+    return batch_bytes(1, nb, std::max(nb, op->ngt), (op->D * NR + 63) & ~int64_t(63), NR, refine);
 }
 
-// Grow the context's workspaces to what a batch of one operator of D rows
-// with NR right-hand sides needs, so that such a batch allocates nothing.
-static void reserve_batch_workspaces(Ctx* ctx, int64_t D, int NR, bool refine) {
-    const BatchBytes b = batch_bytes1(D, NR, refine);
+// Grow the context's workspaces to what a batch of one operator with NR
+// right-hand sides needs, so that such a batch allocates nothing.
+static void reserve_batch_workspaces(Ctx* ctx, const Op* op, int NR, bool refine) {
+    const BatchBytes b = batch_bytes1(op, NR, refine);
     ctx->workspace("tables", b.tables);
     ctx->workspace("vec64", b.vec64);
     if (refine) ctx->workspace("vec32", b.vec32);
@@ -452,26 +463,26 @@ static void run_batch(Ctx* ctx, const std::vector<Group>& groups, const std::vec
     if (ctx->arena) {
         // no-alloc solve: every workspace of this batch is carved from the
         // scratch (an earlier batch of the same call, e.g. the FP64 re-solve's
-        // first attempt, has already written its results out); shared-stencil
-        // tiles are used only if an earlier call built them
+        // first attempt, has already written its results out)
         ctx->arena->used = 0;
-    } else if (!ctx->no_builds) {
-        std::vector<Op*> ops;
-        for (auto& g : groups) ops.push_back(g.op);
-        ensure_group_tiles_for(ops, refine ? 4 : 8, NR);   // before the views are taken
     }
+    grp_refresh_override();
+    const int grp = fewest_tiles(groups.begin(), groups.end(), [](const Group& g) { return g.op; });
+    const bool by_tile = refine ? grp_gather<float, NR>(grp) : grp_gather<double, NR>(grp);
     // layout
     std::vector<int64_t> off(G);
-    std::vector<int> b0(G), nb(G);
+    std::vector<int> b0(G), nb(G), ng(G);
     int64_t total = 0;
-    int blocks = 0;
+    int blocks = 0, gblocks = 0;
     for (int g = 0; g < G; ++g) {
         off[g] = total;
         total += groups[g].op->D * NR;
         total = (total + 63) & ~int64_t(63);
         b0[g] = blocks;
-        nb[g] = (int)((groups[g].op->D + kBlock - 1) / kBlock);
+        nb[g] = row_blocks(groups[g].op);
+        ng[g] = grp_blocks(by_tile, groups[g].op->ngt, nb[g]);
         blocks += nb[g];
+        gblocks += ng[g];
     }
     // device tables: segments (one per precision), block map, states, partials.
     // The FP64 and FP32 segments of a group share one state record per rhs.
@@ -479,7 +490,7 @@ static void run_batch(Ctx* ctx, const std::vector<Group>& groups, const std::vec
     if (nstate > Ctx::kHostStates) throw ArgError("batch too large");
     const size_t part_stride = 2 * NR;
     auto r256 = [](size_t n) { return (n + 255) & ~size_t(255); };
-    const BatchBytes bb = batch_bytes(G, blocks, total, NR, refine);
+    const BatchBytes bb = batch_bytes(G, blocks, gblocks, total, NR, refine);
     const size_t bytes_tables = bb.tables;
     char* tb = reinterpret_cast<char*>(ctx->workspace("tables", bytes_tables));
     char* const tb_end = tb + bytes_tables;
@@ -491,7 +502,7 @@ static void run_batch(Ctx* ctx, const std::vector<Group>& groups, const std::vec
     };
     auto* segs64 = reinterpret_cast<Seg<double>*>(carve(sizeof(Seg<double>) * G));
     auto* segs32 = reinterpret_cast<Seg<float>*>(carve(sizeof(Seg<float>) * G));
-    int* bseg = reinterpret_cast<int*>(carve(sizeof(int) * 2 * (size_t)blocks));   // two block maps
+    int* bseg = reinterpret_cast<int*>(carve(sizeof(int) * ((size_t)blocks + gblocks)));   // two block maps
     KState* sts = reinterpret_cast<KState*>(carve(sizeof(KState) * nstate));
     double* part = reinterpret_cast<double*>(carve(sizeof(double) * part_stride * blocks));
 
@@ -504,7 +515,7 @@ static void run_batch(Ctx* ctx, const std::vector<Group>& groups, const std::vec
         h64[g].m = h32[g].m = groups[g].m;
         h64[g].n = h32[g].n = groups[g].n;
     }
-    const std::vector<int> hb = block_map(nb);
+    const std::vector<int> hb = block_map(nb, ng);
     HIPCHK(hipMemcpyAsync(segs64, h64.data(), sizeof(Seg<double>) * G, hipMemcpyHostToDevice, st));
     if (refine) HIPCHK(hipMemcpyAsync(segs32, h32.data(), sizeof(Seg<float>) * G, hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(bseg, hb.data(), sizeof(int) * hb.size(), hipMemcpyHostToDevice, st));
@@ -554,10 +565,8 @@ static void run_batch(Ctx* ctx, const std::vector<Group>& groups, const std::vec
     int sweeps = 0;
     for (auto& g : groups)
         if (g.op->precond == CPM_PRECOND_JACOBI) sweeps = std::max(sweeps, g.op->precond_iters);
-    int grp = groups.empty() ? 0 : INT_MAX;
-    for (auto& g : groups) grp = std::min(grp, g.op->ngt);
-    const LaunchCfg<double> c64{segs64, bseg, blocks, G, st, sweeps, grp};
-    const LaunchCfg<float> c32{segs32, bseg, blocks, G, st, sweeps, grp};
+    const LaunchCfg<double> c64{segs64, bseg, blocks, gblocks, G, st, sweeps, grp};
+    const LaunchCfg<float> c32{segs32, bseg, blocks, gblocks, G, st, sweeps, grp};
     KState* hs = ctx->host_states;
     const double delta = o.update_delta > 0 ? std::min(o.update_delta, 0.999) : kDefaultUpdateDelta;
     launch_reset_states(sts, nstate, o.tol * o.tol, o.max_iters, delta * delta, st);
@@ -655,19 +664,21 @@ static void run_stream(Ctx* ctx, Op* op, const std::vector<const double*>& rhs, 
     const int blocks = G * nb;
     const int nstate = G * kMaxNR;
     if (nstate > Ctx::kHostStates) throw ArgError("too many lanes");
-    ensure_group_tiles_for({op}, o.precision == CPM_FP32_REFINE ? 4 : 8, NR);
+    grp_refresh_override();
+    const int ng = grp_blocks(grp_gather<float, NR>(op->ngt), op->ngt, nb);
+    const int gblocks = G * ng;
     const int64_t seg_total = (D * NR + 63) & ~int64_t(63);   // vector entries of one segment
     const int64_t total = seg_total * G;
     auto r256 = [](size_t k) { return (k + 255) & ~size_t(255); };
     const size_t part_stride = 2 * NR;
-    const size_t bytes = r256(sizeof(Seg<double>) * G) + r256(sizeof(Seg<float>) * G) + 3 * r256(sizeof(int) * blocks) +
+    const size_t bytes = r256(sizeof(Seg<double>) * G) + r256(sizeof(Seg<float>) * G) + r256(sizeof(int) * ((size_t)blocks + gblocks)) + r256(sizeof(int) * blocks) +
                          r256(sizeof(KState) * nstate) + r256(sizeof(double) * part_stride * blocks) +
                          r256(sizeof(PackEntry) * 4) + 256;
     char* tb = reinterpret_cast<char*>(ctx->workspace("stream_tables", bytes));
     auto carve = [&](size_t k) { char* p = tb; tb += r256(k); return p; };
     auto* seg64 = reinterpret_cast<Seg<double>*>(carve(sizeof(Seg<double>) * G));
     auto* seg32 = reinterpret_cast<Seg<float>*>(carve(sizeof(Seg<float>) * G));
-    int* bseg = reinterpret_cast<int*>(carve(sizeof(int) * 2 * (size_t)blocks));   // two block maps
+    int* bseg = reinterpret_cast<int*>(carve(sizeof(int) * ((size_t)blocks + gblocks)));   // two block maps
     int* bzero = reinterpret_cast<int*>(carve(sizeof(int) * blocks));   // all zero: one pack entry
     KState* sts = reinterpret_cast<KState*>(carve(sizeof(KState) * nstate));
     double* part = reinterpret_cast<double*>(carve(sizeof(double) * part_stride * blocks));
@@ -681,7 +692,7 @@ static void run_stream(Ctx* ctx, Op* op, const std::vector<const double*>& rhs, 
         fill_seg(h64[g], op, g * seg_total, nb, nr0[g], sts + g * kMaxNR, part + part_stride * g * nb);
         fill_seg(h32[g], op, g * seg_total, nb, nr0[g], sts + g * kMaxNR, part + part_stride * g * nb);
     }
-    const std::vector<int> hb = block_map(std::vector<int>((size_t)G, nb));
+    const std::vector<int> hb = block_map(std::vector<int>((size_t)G, nb), std::vector<int>((size_t)G, ng));
     HIPCHK(hipMemcpyAsync(seg64, h64.data(), sizeof(Seg<double>) * G, hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(seg32, h32.data(), sizeof(Seg<float>) * G, hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(bseg, hb.data(), sizeof(int) * hb.size(), hipMemcpyHostToDevice, st));
@@ -739,7 +750,7 @@ static void run_stream(Ctx* ctx, Op* op, const std::vector<const double*>& rhs, 
         }
     HIPCHK(hipMemcpyAsync(sts, hst.data(), sizeof(KState) * nstate, hipMemcpyHostToDevice, st));
     int sweeps = op->precond == CPM_PRECOND_JACOBI ? op->precond_iters : 0;
-    const LaunchCfg<float> c32{seg32, bseg, blocks, G, st, sweeps, op->ngt};
+    const LaunchCfg<float> c32{seg32, bseg, blocks, gblocks, G, st, sweeps, op->ngt};
     const MixVec mv{V64.x, V64.r, V64.b, V64.tmp};
     KState* hs = ctx->host_states;
     int done = 0;
@@ -971,7 +982,8 @@ void multiply(Op* op, const double* dx, double* dy, double m, double n) {
     HIPCHK(hipMemcpyAsync(dbseg, hb.data(), sizeof(int) * nblocks, hipMemcpyHostToDevice, st));
     double* w = ctx->workspace("mul_tmp", sizeof(double) * op->D * 3);
     double *xi = w, *yi = w + op->D, *tmp = w + 2 * op->D;
-    LaunchCfg<double> c{dseg, dbseg, nblocks, 1, st, 0, op->ngt};
+    grp_refresh_override();
+    LaunchCfg<double> c{dseg, dbseg, nblocks, grp_blocks(grp_gather<double, 1>(op->ngt), op->ngt, nblocks), 1, st, 0, op->ngt};
     if (op->perm.p) {   // caller order -> internal order and back
         hipLaunchKernelGGL(k_pack, dim3(nblocks), dim3(256), 0, st, dpe, dbseg, xi, (float*)nullptr, 1);
         Launch<double, 1>::apply(c, xi, tmp, yi);
@@ -984,17 +996,18 @@ void multiply(Op* op, const double* dx, double* dy, double m, double n) {
 
 template <typename T, int NR>
 static void profile_egather_t(Op* op, int G, int reps, double* avg_ms, double* bytes) {
-    ensure_group_tiles_for({op}, sizeof(T), NR);
+    grp_refresh_override();
     Ctx* ctx = op->ctx;
     const hipStream_t st = ctx->stream;
     const int nblocks = (int)((op->D + kBlock - 1) / kBlock);
     const int64_t seg_total = (op->D * NR + 63) & ~int64_t(63);
     std::vector<Seg<T>> h(G);
-    std::vector<int> hb((size_t)G * nblocks);
+    const int ng = grp_blocks(grp_gather<T, NR>(op->ngt), op->ngt, nblocks);
     for (int g = 0; g < G; ++g) {   // G copies of the operator in one launch, as streamed solves of 16, 32 lanes
         fill_seg(h[g], op, g * seg_total, nblocks, NR, nullptr, nullptr);
     }
-    hb = block_map(std::vector<int>((size_t)G, nblocks));   // both maps (the gather runs the second)
+    const std::vector<int> hb =   // both maps (the gather runs the second)
+        block_map(std::vector<int>((size_t)G, nblocks), std::vector<int>((size_t)G, ng));
     const size_t seg_bytes = (sizeof(Seg<T>) * G + 255) & ~size_t(255);
     char* tb = reinterpret_cast<char*>(ctx->workspace("prof_tables", seg_bytes + sizeof(int) * hb.size()));
     auto* dseg = reinterpret_cast<Seg<T>*>(tb);
@@ -1008,7 +1021,7 @@ static void profile_egather_t(Op* op, int G, int reps, double* avg_ms, double* b
     T* xs = reinterpret_cast<T*>(ctx->workspace("prof_x", vec_bytes * nbuf));
     T* ys = reinterpret_cast<T*>(ctx->workspace("prof_y", vec_bytes * nbuf));
     HIPCHK(hipMemsetAsync(xs, 0, vec_bytes * nbuf, st));
-    LaunchCfg<T> c{dseg, dbseg, nblocks * G, G, st, 0, op->ngt};
+    LaunchCfg<T> c{dseg, dbseg, nblocks * G, ng * G, G, st, 0, op->ngt};
     auto buf = [&](T* b, int r) { return b + (size_t)(r % nbuf) * seg_total * G; };
     // the gather the iterations launch: of P^-1 x unless Jacobi sweeps follow the first
     const bool fly = !(op->precond == CPM_PRECOND_JACOBI && op->precond_iters > 1);
@@ -1036,7 +1049,7 @@ static void profile_egather_t(Op* op, int G, int reps, double* avg_ms, double* b
     // extra entry; LDS tiles also read their lists, 4 bytes per row)
     double opb;
     const double sT = sizeof(T);
-    if (op->fmt == OP_TP && op->ngt > 0 && grp_gather(sizeof(T), NR, op->ngt) && GrpTile<T, NR>::kRows > 0) {
+    if (grp_gather<T, NR>(op->ngt)) {
         // shared-stencil tiles: per plain item 16 int16 positions and its
         // slot offset, per plain row 12 weights and its row index; exception
         // rows as in the row tiles plus slot offset and row index; identity
@@ -1130,7 +1143,7 @@ static PackEntry pack_out(double* dst) { PackEntry e{}; e.dst = dst; return e; }
 // apply kernel with tmp = x, the identity rows from the held Lfull rows.
 static void explicit_diffusion(Op* op, const StepTables& t, int k, double c, const double* x, double* z) {
     const hipStream_t st = op->ctx->stream;
-    LaunchCfg<double> cfg{t.seg + k, t.bseg, t.nblocks, 1, st, 0};
+    LaunchCfg<double> cfg{t.seg + k, t.bseg, t.nblocks, t.nblocks, 1, st, 0};
     launch_lfinish_plain<double>(cfg, x, x, z);
     if (op->nh > 0)
         hipLaunchKernelGGL(k_held_apply, dim3((unsigned)((op->nh + 255) / 256)), dim3(256), 0, st, op->nh, op->hw,
@@ -1139,7 +1152,8 @@ static void explicit_diffusion(Op* op, const StepTables& t, int k, double c, con
 }
 
 static void extension(Op* op, const StepTables& t, const double* z, double* y) {
-    LaunchCfg<double> cfg{t.seg, t.bseg, t.nblocks, 1, op->ctx->stream, 0};
+    LaunchCfg<double> cfg{t.seg, t.bseg, t.nblocks, grp_blocks(grp_gather<double, 1>(op->ngt), op->ngt, t.nblocks), 1,
+                          op->ctx->stream, 0, op->ngt};
     launch_egather<double, 1>(cfg, z, y);
 }
 
@@ -1337,7 +1351,7 @@ struct Server : ServerBase {
     RangePool ranges;   // vector ranges of the pools
     std::vector<Req> reqs;
     bool dirty = true;
-    int nblocks = 0;
+    int nblocks = 0, gblocks = 0, grp = 0;
     Seg<float>* d_segs = nullptr;
     int* d_bseg = nullptr;
     double* d_part = nullptr;
@@ -1384,12 +1398,15 @@ struct Server : ServerBase {
     // partial sums, one pack entry and an all-zero block map for packing.
     // Growing them reallocates (and marks the segment table for rebuilding).
     void ensure_tables() {
-        int blocks = 0;
-        for (auto& q : reqs) blocks += (int)((q.op->D + kBlock - 1) / kBlock);
+        int blocks = 0, gblocks = 0;
+        for (auto& q : reqs) {
+            blocks += row_blocks(q.op);
+            gblocks += std::max(row_blocks(q.op), q.op->ngt);
+        }
         const int zn = (int)((cap + kBlock - 1) / kBlock);   // no request has more blocks
         auto r256 = [](size_t k) { return (k + 255) & ~size_t(255); };
         const size_t sseg = r256(sizeof(Seg<float>) * std::max<size_t>(reqs.size(), 1));
-        const size_t smap = r256(sizeof(int) * 2 * std::max(blocks, 1));   // two block maps
+        const size_t smap = r256(sizeof(int) * (size_t)std::max(blocks + gblocks, 1));   // two block maps
         const size_t spart = r256(sizeof(double) * 2 * NR * std::max(blocks, 1));
         const size_t spack = r256(sizeof(PackEntry));
         const size_t szero = r256(sizeof(int) * zn);
@@ -1426,13 +1443,12 @@ struct Server : ServerBase {
         if (len > cap) throw ArgError("request larger than the server pool");
         // the FP64 re-solve of this request's lanes (when their refinement stalls) runs in the
         // context's workspaces: grow them now, so that retiring the request allocates nothing
-        reserve_batch_workspaces(ctx, op->D, NR, false);
+        reserve_batch_workspaces(ctx, op, NR, false);
         if (fp64_routing() && prefer_fp64(ctx, op)) {
             // the operator (or its family) stalled in FP32 before: the request is solved in FP64
             // from zero now, as the re-solve of a stalled request is, without FP32 iterations
             Done d{tag, std::vector<cpm_solve_info>((size_t)nrhs)};
             for (auto& inf : d.infos) inf.status = ST_FALLBACK;
-            NoBuilds nb(ctx);
             fp64_fallback(ctx, std::vector<Op*>((size_t)nrhs, op), std::vector<const double*>(rhs, rhs + nrhs),
                           std::vector<double*>(xs, xs + nrhs), o, d.infos, nullptr);
             done.push_back(std::move(d));
@@ -1477,23 +1493,24 @@ struct Server : ServerBase {
 
     void rebuild() {
         ensure_tables();
-        {
-            std::vector<Op*> ops;
-            for (const Req& q : reqs) ops.push_back(q.op);
-            ensure_group_tiles_for(ops, 4, NR);
-        }
+        grp_refresh_override();
+        grp = fewest_tiles(reqs.begin(), reqs.end(), [](const Req& q) { return q.op; });
+        const bool by_tile = grp_gather<float, NR>(grp);
         std::vector<Seg<float>> h(reqs.size());
-        std::vector<int> nbs;
+        std::vector<int> nbs, ngs;
         int b0 = 0;
+        gblocks = 0;
         for (size_t g = 0; g < reqs.size(); ++g) {
             const Req& q = reqs[g];
             const int nb = (int)((q.op->D + kBlock - 1) / kBlock);
             fill_seg(h[g], q.op, q.off, nb, q.nr, states.template as<KState>() + (size_t)q.slot * kMaxNR,
                      d_part + (size_t)2 * NR * b0);
             nbs.push_back(nb);
+            ngs.push_back(grp_blocks(by_tile, q.op->ngt, nb));
             b0 += nb;
+            gblocks += ngs.back();
         }
-        const std::vector<int> map = block_map(nbs);
+        const std::vector<int> map = block_map(nbs, ngs);
         nblocks = b0;
         const hipStream_t st = ctx->stream;
         HIPCHK(hipMemcpyAsync(d_segs, h.data(), sizeof(Seg<float>) * h.size(), hipMemcpyHostToDevice, st));
@@ -1508,9 +1525,7 @@ struct Server : ServerBase {
         const hipStream_t st = ctx->stream;
         const Vecs<float> V32{nullptr, v32(0), v32(1), v32(2), v32(3), v32(4), v32(5), v32(6), v32(7), v32(8), v32(9)};
         const MixVec mv{v64(1), v64(2), v64(0), v64(4)};
-        int grp = INT_MAX;
-        for (const Req& q : reqs) grp = std::min(grp, q.op->ngt);
-        const LaunchCfg<float> c{d_segs, d_bseg, nblocks, (int)reqs.size(), st, 0, grp};
+        const LaunchCfg<float> c{d_segs, d_bseg, nblocks, gblocks, (int)reqs.size(), st, 0, grp};
         Vecs<float> w = V32;
         for (int i = 0; i < iters; ++i) Launch<float, NR>::iteration(c, w, true, mv);
         HIPCHK(hipGetLastError());
@@ -1544,7 +1559,7 @@ struct Server : ServerBase {
             }
             try {
                 for (int k = 0; k < q.nr; ++k) lane_pack(q, k, v64(1), 0);
-                NoBuilds nb(ctx);   // the re-solve uses the workspaces reserved at submission
+                // the re-solve uses the workspaces reserved at submission
                 const std::vector<Op*> ops((size_t)q.nr, q.op);
                 fp64_fallback(ctx, ops, q.rhs, q.xs, o, d.infos, nullptr);
                 record_fp32(ctx, ops, d.infos);
@@ -1588,7 +1603,7 @@ struct Server64 : ServerBase {
     RangePool ranges;
     std::vector<Req> reqs;
     bool dirty = true;
-    int nblocks = 0;
+    int nblocks = 0, gblocks = 0, grp = 0;
     Seg<double>* d_segs = nullptr;
     int* d_bseg = nullptr;
     double* d_part = nullptr;
@@ -1639,11 +1654,14 @@ struct Server64 : ServerBase {
         HIPCHK(hipStreamSynchronize(st));   // the entry is rewritten by the next call
     }
     void ensure_tables() {
-        int blocks = 0;
-        for (auto& q : reqs) blocks += (int)((q.op->D + kBlock - 1) / kBlock);
+        int blocks = 0, gblocks = 0;
+        for (auto& q : reqs) {
+            blocks += row_blocks(q.op);
+            gblocks += std::max(row_blocks(q.op), q.op->ngt);
+        }
         auto r256 = [](size_t k) { return (k + 255) & ~size_t(255); };
         const size_t sseg = r256(sizeof(Seg<double>) * std::max<size_t>(reqs.size(), 1));
-        const size_t smap = r256(sizeof(int) * 2 * std::max(blocks, 1));   // two block maps
+        const size_t smap = r256(sizeof(int) * (size_t)std::max(blocks + gblocks, 1));   // two block maps
         const size_t spart = r256(sizeof(double) * 2 * NR * std::max(blocks, 1));
         const size_t need = sseg + smap + spart;
         if (need > tables_bytes) {
@@ -1664,7 +1682,6 @@ struct Server64 : ServerBase {
         if (op->precond == CPM_PRECOND_JACOBI) throw ArgError("served operators use the diagonal or no preconditioner");
         const int64_t len = (op->D * NR + 63) & ~int64_t(63);
         if (len > cap) throw ArgError("request larger than the server pool");
-        ensure_group_tiles_for({op}, 8, NR);   // before its view is taken
         int64_t off;
         if (free_slots.empty() || !ranges.take(len, off)) return false;   // wait for memory
         Req q{tag, op, nrhs, off, len, free_slots.back(), {}};
@@ -1688,7 +1705,7 @@ struct Server64 : ServerBase {
         Seg<double> h{};
         fill_seg(h, op, off, nb, nrhs, sts, i_part());
         HIPCHK(hipMemcpyAsync(i_seg(), &h, sizeof(h), hipMemcpyHostToDevice, st));
-        const LaunchCfg<double> c1{i_seg(), nullptr, nb, 1, st, 0, op->ngt};
+        const LaunchCfg<double> c1{i_seg(), nullptr, nb, nb, 1, st, 0, 0};   // no gather
         Launch<double, NR>::init(c1, v64(0), v64(1), v64(2), v64(3), v64(4), v64(5));
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(st));
@@ -1699,18 +1716,24 @@ struct Server64 : ServerBase {
 
     void rebuild() {
         ensure_tables();
+        grp_refresh_override();
+        grp = fewest_tiles(reqs.begin(), reqs.end(), [](const Req& q) { return q.op; });
+        const bool by_tile = grp_gather<double, NR>(grp);
         std::vector<Seg<double>> h(reqs.size());
-        std::vector<int> nbs;
+        std::vector<int> nbs, ngs;
         int b0 = 0;
+        gblocks = 0;
         for (size_t g = 0; g < reqs.size(); ++g) {
             const Req& q = reqs[g];
             const int nb = (int)((q.op->D + kBlock - 1) / kBlock);
             fill_seg(h[g], q.op, q.off, nb, q.nr, states.template as<KState>() + (size_t)q.slot * kMaxNR,
                      d_part + (size_t)2 * NR * b0);
             nbs.push_back(nb);
+            ngs.push_back(grp_blocks(by_tile, q.op->ngt, nb));
             b0 += nb;
+            gblocks += ngs.back();
         }
-        const std::vector<int> map = block_map(nbs);
+        const std::vector<int> map = block_map(nbs, ngs);
         nblocks = b0;
         const hipStream_t st = ctx->stream;
         HIPCHK(hipMemcpyAsync(d_segs, h.data(), sizeof(Seg<double>) * h.size(), hipMemcpyHostToDevice, st));
@@ -1724,9 +1747,7 @@ struct Server64 : ServerBase {
         if (dirty) rebuild();
         const hipStream_t st = ctx->stream;
         Vecs<double> V{v64(0), v64(1), v64(2), v64(3), v64(4), v64(5), v64(6), v64(7), v64(8), v64(9), v64(10)};
-        int grp = INT_MAX;
-        for (const Req& q : reqs) grp = std::min(grp, q.op->ngt);
-        const LaunchCfg<double> c{d_segs, d_bseg, nblocks, (int)reqs.size(), st, 0, grp};
+        const LaunchCfg<double> c{d_segs, d_bseg, nblocks, gblocks, (int)reqs.size(), st, 0, grp};
         for (int i = 0; i < iters; ++i) Launch<double, NR>::iteration(c, V, false, MixVec{});
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(ctx->host_states, states.template as<KState>(), sizeof(KState) * (size_t)slots * kMaxNR,
@@ -1904,18 +1925,14 @@ int cpm_op_format(const cpm_op* op) { return op ? O(op)->fmt : -1; }
 
 int cpm_op_gather_kind(const cpm_op* op, int precision, int nrhs) {
     if (!op || (nrhs != 1 && nrhs != 2 && nrhs != 4 && nrhs != 8)) return -1;
-    Op* o = const_cast<Op*>(O(op));   // the lazy tile build does not change what the operator computes
+    const Op* o = O(op);
     const bool f32 = precision == CPM_FP32_REFINE;
-    try {
-        ensure_group_tiles_for({o}, f32 ? 4 : 8, nrhs);
-    } catch (...) {
-        return -1;
-    }
-    const bool fits = f32 ? (nrhs == 1 ? GrpTile<float, 1>::kRows : nrhs == 2 ? GrpTile<float, 2>::kRows
-                             : nrhs == 4 ? GrpTile<float, 4>::kRows : GrpTile<float, 8>::kRows) > 0
-                          : (nrhs == 1 ? GrpTile<double, 1>::kRows : nrhs == 2 ? GrpTile<double, 2>::kRows
-                             : nrhs == 4 ? GrpTile<double, 4>::kRows : GrpTile<double, 8>::kRows) > 0;
-    if (o->fmt == OP_TP && o->ngt > 0 && fits && grp_gather(f32 ? 4 : 8, nrhs, o->ngt)) return 2;
+    grp_refresh_override();
+    const bool grp = f32 ? (nrhs == 1 ? grp_gather<float, 1>(o->ngt) : nrhs == 2 ? grp_gather<float, 2>(o->ngt)
+                            : nrhs == 4 ? grp_gather<float, 4>(o->ngt) : grp_gather<float, 8>(o->ngt))
+                         : (nrhs == 1 ? grp_gather<double, 1>(o->ngt) : nrhs == 2 ? grp_gather<double, 2>(o->ngt)
+                            : nrhs == 4 ? grp_gather<double, 4>(o->ngt) : grp_gather<double, 8>(o->ngt));
+    if (grp) return 2;
     const int bytes = (f32 ? 4 : 8) * nrhs;
     if (o->fmt == OP_TP && o->tln.p && kLdsRows * bytes <= kLdsBytes) return 1;
     return 0;
@@ -1924,8 +1941,12 @@ int cpm_op_gather_kind(const cpm_op* op, int precision, int nrhs) {
 int cpm_op_tile_stats(const cpm_op* op, int64_t* out) {
     return guard([&] {
         if (!op || !out) throw ArgError("null operator or output");
-        Op* o = const_cast<Op*>(O(op));   // the lazy tile build does not change what the operator computes
-        op_ensure_group_tiles(*o);
+        Op* o = const_cast<Op*>(O(op));
+        if (o->ngt > 0) {   // row tiles beside them only for this report: no launch of the operator reads them
+            const int64_t before = (int64_t)o->device_bytes();
+            op_ensure_row_tiles(*o);
+            o->ctx->op_bytes += (int64_t)o->device_bytes() - before;
+        }
         int64_t row_tiles = 0;
         if (o->tln.p) {
             std::vector<int> tln(o->tln.bytes / 4);
@@ -2061,7 +2082,7 @@ int cpm_solve_device_noalloc(cpm_op* op, const double* d_rhs, double* d_x, const
         Ctx* cx = o->ctx;
         const cpm_solve_opts so = resolve_opts(opts);
         if (so.precision != CPM_FP64 && so.precision != CPM_FP32_REFINE) throw ArgError("unknown precision");
-        const size_t need = std::max(batch_bytes1(o->D, 1, false).arena(), batch_bytes1(o->D, 1, true).arena());
+        const size_t need = std::max(batch_bytes1(o, 1, false).arena(), batch_bytes1(o, 1, true).arena());
         if (need > (size_t)CPM_NOALLOC_SCRATCH_BYTES)
             throw ArgError("operator of " + std::to_string(o->D) + " rows needs " + std::to_string(need) +
                            " bytes of workspace; the no-alloc scratch holds " +

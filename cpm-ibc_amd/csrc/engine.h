@@ -99,7 +99,7 @@ constexpr int kExcPos = 72;      // positions per exception record (64 slots, ex
 #define CPMGPU_GROUP_WAVES_WIDE 2
 #endif
 #ifndef CPMGPU_GROUP_LDS_ROWS
-#define CPMGPU_GROUP_LDS_ROWS 1280
+#define CPMGPU_GROUP_LDS_ROWS 1024
 #endif
 constexpr int kGrpRows = CPMGPU_GROUP_ROWS;   // rows per shared-stencil item
 static_assert(kGrpRows >= 1 && kGrpRows <= 8, "an identity item's rows fit the 8 words of its line positions");
@@ -112,10 +112,6 @@ struct GrpTile {
     static constexpr int kRows = (kGrpLdsRows * NR * (int)sizeof(T) <= kGrpLdsBytes) ? kGrpLdsRows : 0;
 };
 constexpr int kGrpKindShift = 28;             // item kind above the slot offset in gofs
-#ifndef CPMGPU_GROUP_MIN_TILES
-#define CPMGPU_GROUP_MIN_TILES 256
-#endif
-constexpr int kGrpMinTiles = CPMGPU_GROUP_MIN_TILES;   // fewer shared-stencil tiles: row tiles only
 constexpr int kGrpOfsMask = (1 << kGrpKindShift) - 1;
 
 // One instance group of a batched launch: an operator, NR right-hand sides

@@ -8,20 +8,25 @@ template <typename T>
 struct LaunchCfg {
     const Seg<T>* segs;    // device segment table
     const int* bseg;       // device block maps (segment | block << kSegBits), nblocks entries segment by
-                           // segment, then nblocks round-robin over the segments (the E gathers')
+                           // segment, then gblocks round-robin over the segments (the E gathers')
     int nblocks;
+    int gblocks;           // workgroups of an E gather (grp_blocks)
     int nseg;
     hipStream_t stream;
     int jacobi_sweeps;     // largest precond_iters over Jacobi-preconditioned segments (0: none)
     int grp = 0;           // fewest shared-stencil tiles of the segments' operators (0: some have none)
 };
 
-// Whether E gathers of T x nr values use shared-stencil tiles when every
-// operator of the launch has at least ntiles of them.
-bool grp_gather(int tsize, int nr, int ntiles);
-// Whether a launch of T x nr values builds its operators' shared-stencil tiles
-// (other shapes use them only where an earlier launch built them).
-bool grp_build(int tsize, int nr);
+// Whether the E gathers of a launch use shared-stencil tiles: values whose
+// rows fit the tiles' LDS, every operator with tiles (ntiles: the fewest).
+template <typename T, int NR>
+bool grp_gather(int ntiles);
+// Workgroups that the E gathers of such a launch (grp) take for an operator
+// of ntiles tiles and nblocks row blocks; other launches gather by row blocks
+// (the refinement lanes' FP64 gathers by tiles in both).
+inline int grp_blocks(bool grp, int ntiles, int nblocks) {
+    return grp ? ntiles : ntiles > nblocks ? ntiles : nblocks;
+}
 // Re-read the CPMGPU_GROUP_GATHER override (once per launch sequence).
 void grp_refresh_override();
 

@@ -157,9 +157,11 @@ __device__ void block_partials(const double (&v)[NV][NR], double* part, int lb, 
     }
 }
 
-constexpr int kXcdRun = CPMGPU_XCD_RUN;
+constexpr int kXcdRun = CPMGPU_XCD_RUN;        // vector kernels
+constexpr int kGatherRun = CPMGPU_GATHER_RUN;  // E gathers
+constexpr int kLfinishRun = CPMGPU_LFINISH_RUN;
 
-template <typename T>
+template <int kXcdRun, typename T>
 __device__ __forceinline__ const Seg<T>& seg_of(const Seg<T>* __restrict__ segs, const int* __restrict__ bseg, int& lb, int64_t& row) {
     // Workgroups are dispatched to the 8 XCDs round-robin (workgroup b to XCD
     // b mod 8).  Renumber them so that each XCD takes runs of kXcdRun
@@ -814,7 +816,7 @@ __global__ __launch_bounds__(kBlock) void k_init(const Seg<T>* __restrict__ segs
                                                  T* r0, T* p, T* v) {
     int lb;
     int64_t row;
-    const Seg<T>& sg = seg_of(segs, bseg, lb, row);
+    const Seg<T>& sg = seg_of<kXcdRun>(segs, bseg, lb, row);
     double pv[1][NR];
 #pragma unroll
     for (int k = 0; k < NR; ++k) pv[0][k] = 0.0;
@@ -840,7 +842,7 @@ __global__ __launch_bounds__(kBlock) void k_pupdate(const Seg<T>* __restrict__ s
                                                     const T* r, T* y, T* x, MixVec mv, int fly) {
     int lb;
     int64_t row;
-    const Seg<T>& sg = seg_of(segs, bseg, lb, row);
+    const Seg<T>& sg = seg_of<kXcdRun>(segs, bseg, lb, row);
     const auto L = lane_stat<NR>(sg);
     if (row >= sg.op.D || !seg_any(L, M_STAGE1)) return;
     const size_t i = (size_t)(sg.off + row * NR);
@@ -886,7 +888,8 @@ __global__ __launch_bounds__(kBlock) void k_egather(const Seg<T>* __restrict__ s
     const LdsRows<V> lrows{lx, LR > 0 ? LR : 1};
     int lb;
     int64_t row;
-    const Seg<T>& sg = seg_of(segs, bseg, lb, row);
+    const Seg<T>& sg = seg_of<kGatherRun>(segs, bseg, lb, row);
+    if (lb >= sg.nblocks) return;   // a launch with more tiles (k_egather_upd's) than row blocks
     const auto L = lane_stat<NR>(sg, lanes != 0);
     if (lanes && !seg_any(L, lanes)) return;               // uniform per workgroup
     const bool main = !lanes || seg_any(L, lanes & ~M_UPDATE);
@@ -955,7 +958,7 @@ __global__ __launch_bounds__(kBlock) void k_egather_upd(const Seg<float>* __rest
     const LdsRows<double> lrows{lx, LR};
     int lb;
     int64_t row;
-    const Seg<float>& sg = seg_of(segs, bseg, lb, row);
+    const Seg<float>& sg = seg_of<kGatherRun>(segs, bseg, lb, row);
     const auto L = lane_stat<NR>(sg);
     if (!seg_any(L, M_UPDATE)) return;   // uniform per workgroup
     if (sg.op64.ngt > 0) {
@@ -977,8 +980,7 @@ __global__ __launch_bounds__(kBlock) void k_egather_upd(const Seg<float>* __rest
 }
 
 // E x for launches whose every segment has shared-stencil tiles: block lb of
-// a segment takes its tile lb (blocks past the last tile have nothing to
-// do).  40 KB of LDS and at most 128 VGPRs, so four
+// a segment takes its tile lb.  32 KB of LDS and at most 128 VGPRs, so four
 // workgroups share a CU (a direct-read path for other segments, even out of
 // line, made the FP32 x 8 kernel spill).
 // FLY: x is p (or s) and the launch gathers y = P^-1 p (z = P^-1 s).
@@ -992,7 +994,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
     const LdsRows<V> lrows{lx, LR};
     int lb;
     int64_t row;
-    const Seg<T>& sg = seg_of(segs, bseg, lb, row);
+    const Seg<T>& sg = seg_of<kGatherRun>(segs, bseg, lb, row);
     const auto L = lane_stat<NR>(sg, lanes != 0);
     if (lanes && !seg_any(L, lanes)) return;               // uniform per workgroup
     const bool main = !lanes || seg_any(L, lanes & ~M_UPDATE);
@@ -1009,7 +1011,7 @@ __global__ __launch_bounds__(kBlock) void k_lfinish(const Seg<T>* __restrict__ s
                                                     unsigned lanes, MixVec mv, int fly) {
     int lb;
     int64_t row;
-    const Seg<T>& sg = seg_of(segs, bseg, lb, row);
+    const Seg<T>& sg = seg_of<kLfinishRun>(segs, bseg, lb, row);
     const auto L = lane_stat<NR>(sg, lanes != 0);
     if (lanes && !seg_any(L, lanes)) return;   // uniform per segment
     constexpr int NV = RED == 2 ? 2 : 1;
@@ -1080,7 +1082,7 @@ __global__ __launch_bounds__(kBlock) void k_supdate(const Seg<T>* __restrict__ s
                                                     T* r0, T* p, MixVec mv, int fly) {
     int lb;
     int64_t row;
-    const Seg<T>& sg = seg_of(segs, bseg, lb, row);
+    const Seg<T>& sg = seg_of<kXcdRun>(segs, bseg, lb, row);
     const auto L = lane_stat<NR>(sg);
     if (row >= sg.op.D || !seg_any(L, M_STAGE2)) return;
     const size_t i = (size_t)(sg.off + row * NR);
@@ -1123,7 +1125,7 @@ __global__ __launch_bounds__(kBlock) void k_jacobi(const Seg<T>* __restrict__ se
                                                    const T* x, const T* ay, T* y, int sweep) {
     int lb;
     int64_t row;
-    const Seg<T>& sg = seg_of(segs, bseg, lb, row);
+    const Seg<T>& sg = seg_of<kXcdRun>(segs, bseg, lb, row);
     const auto L = lane_stat<NR>(sg);
     if (sg.precond != 2 || sweep >= sg.precond_iters) return;
     if (row >= sg.op.D - sg.op.nD || !seg_any(L, M_RUN)) return;
@@ -1144,7 +1146,7 @@ __global__ __launch_bounds__(kBlock) void k_xrupdate(const Seg<T>* __restrict__ 
                                                      const T* z, T* r, const T* s, const T* t, const T* r0, int fly) {
     int lb;
     int64_t row;
-    const Seg<T>& sg = seg_of(segs, bseg, lb, row);
+    const Seg<T>& sg = seg_of<kXcdRun>(segs, bseg, lb, row);
     const auto L = lane_stat<NR>(sg);
     if (!seg_any(L, M_RUN)) return;
     double pv[2][NR];
@@ -1195,7 +1197,7 @@ __global__ __launch_bounds__(kBlock) void k_restart(const Seg<T>* __restrict__ s
                                                     const T* ax, T* r, T* r0) {
     int lb;
     int64_t row;
-    const Seg<T>& sg = seg_of(segs, bseg, lb, row);
+    const Seg<T>& sg = seg_of<kXcdRun>(segs, bseg, lb, row);
     const auto L = lane_stat<NR>(sg);
     if (!seg_any(L, M_RESTART)) return;
     double pv[1][NR];
@@ -1228,7 +1230,7 @@ __global__ __launch_bounds__(kBlock) void k_mx_start(const Seg<double>* __restri
                                                      double* x, double* r) {
     int lb;
     int64_t row;
-    const Seg<double>& sg = seg_of(segs, bseg, lb, row);
+    const Seg<double>& sg = seg_of<kXcdRun>(segs, bseg, lb, row);
     double pv[1][NR];
 #pragma unroll
     for (int k = 0; k < NR; ++k) pv[0][k] = 0.0;
@@ -1252,7 +1254,7 @@ __global__ __launch_bounds__(kBlock) void k_mx_down(const Seg<double>* __restric
                                                     float* r, float* r0, float* p, float* v, float* x) {
     int lb;
     int64_t row;
-    const Seg<double>& sg = seg_of(segs, bseg, lb, row);
+    const Seg<double>& sg = seg_of<kXcdRun>(segs, bseg, lb, row);
     const auto L = lane_stat<NR>(sg);
     if (!seg_any(L, M_RESCALE)) return;
     double pv[1][NR];
@@ -1446,14 +1448,14 @@ void launch_reset_states(KState* st, int n, double tol2, int max_it, double delt
     hipLaunchKernelGGL(kern, dim3(c.nblocks), dim3(kBlock), 0, c.stream, c.segs, c.nseg == 1 ? nullptr : c.bseg, __VA_ARGS__)
 // The E gathers run the round-robin block map.
 #define LAUNCH_GATHER(kern, ...)                                                                         \
-    hipLaunchKernelGGL(kern, dim3(c.nblocks), dim3(kBlock), 0, c.stream, c.segs,                        \
+    hipLaunchKernelGGL(kern, dim3(c.gblocks), dim3(kBlock), 0, c.stream, c.segs,                        \
                        c.nseg == 1 ? nullptr : c.bseg + c.nblocks, __VA_ARGS__)
 // E gather of launch c; FL: form P^-1 of the gathered vector (only with
 // shared-stencil tiles, grp_launch).
 #define EGATHER(FL, ...)                                                     \
     do {                                                                     \
         if constexpr (GrpTile<T, NR>::kRows > 0) {                           \
-            if (c.grp > 0 && grp_gather(sizeof(T), NR, c.grp)) {             \
+            if (grp_launch<T, NR>(c)) {                                      \
                 if (FL) LAUNCH_GATHER((k_egather_grp<T, NR, GrpWaves<T, NR>::kWaves, true>), __VA_ARGS__); \
                 else LAUNCH_GATHER((k_egather_grp<T, NR, GrpWaves<T, NR>::kWaves, false>), __VA_ARGS__); \
                 break;                                                       \
@@ -1470,16 +1472,11 @@ struct GrpWaves {
     static constexpr int kWaves = (sizeof(T) == 4 && NR != 4) ? 4 : CPMGPU_GROUP_WAVES_WIDE;
 };
 
-// Value shapes whose E gathers use shared-stencil tiles when every operator
-// of the launch has at least ntiles of them: by default FP32 x 8, x 2 and
-// FP64 x 4 from kGrpMinTiles tiles, FP32 x 1 from 768, where they were
-// measured faster than row tiles (tubes of 42 k to 406 k rows).
-// CPMGPU_GROUP_GATHER=all uses them for every shape whose tile fits the LDS,
-// =none for none.
+// CPMGPU_GROUP_GATHER=none: no launch gathers through shared-stencil tiles.
 // The override is read from the environment once per solve, tile build or
 // query (grp_refresh_override, called where a launch sequence starts), not
 // per launch: a solve makes thousands of launches.
-static std::atomic<int> g_grp_override{-2};   // -2 unread, -1 none, 0 "none", 1 "all"
+static std::atomic<int> g_grp_override{-2};   // -2 unread, -1 no override, 0 "none"
 // y = P^-1 p and z = P^-1 s formed where they are read (launches that allow
 // it, Launch::iteration); CPMGPU_PRECOND_FLY=0 stores them instead.
 static std::atomic<int> g_fly_override{-1};   // -1 none, 0 off
@@ -1488,39 +1485,21 @@ static bool precond_fly() { return g_fly_override.load(std::memory_order_relaxed
 void grp_refresh_override() {
     const char* e = std::getenv("CPMGPU_GROUP_GATHER");
     const std::string v = e ? e : "";
-    g_grp_override.store(v == "all" ? 1 : v == "none" ? 0 : -1, std::memory_order_relaxed);
+    g_grp_override.store(v == "none" ? 0 : -1, std::memory_order_relaxed);
     const char* fe = std::getenv("CPMGPU_PRECOND_FLY");
     g_fly_override.store(fe && std::string(fe) == "0" ? 0 : -1, std::memory_order_relaxed);
 }
 
-bool grp_gather(int tsize, int nr, int ntiles) {
-    (void)tsize;
+template <typename T, int NR>
+bool grp_gather(int ntiles) {
     if (g_grp_override.load(std::memory_order_relaxed) == -2) grp_refresh_override();
-    const int ov = g_grp_override.load(std::memory_order_relaxed);
-    if (ov >= 0) return ov == 1;
-    // every shape whose rows fit the tiles' LDS is faster through them where the
-    // operator has them (torus-knot system, one / eight groups per launch: FP64 x
-    // 1 20.0 / 87.0 -> 16.9 / 69.8 us, FP64 x 2 23.6 / 99.8 -> 19.6 / 90.9 us,
-    // FP32 x 4 21.3 / 92.1 -> 17.7 / 72.2 us); one right-hand side: row tiles
-    // were faster up to ~600 tiles
-    return ntiles >= (nr == 1 ? 768 : kGrpMinTiles);
-}
-
-bool grp_build(int tsize, int nr) {
-    if (g_grp_override.load(std::memory_order_relaxed) == -2) grp_refresh_override();
-    const int ov = g_grp_override.load(std::memory_order_relaxed);
-    if (ov >= 0) return ov == 1;
-    // the shapes of the solves that repeat on one operator: FP32 x 1, 2, 8 (FP32+refine
-    // batches and streams) and FP64 x 4 (FP64 batches); an operator served at FP32 x 4
-    // is solved once and would not win back the build (0.14 s at 1.27 M rows)
-    return (tsize == 4 && nr != 4) || (tsize == 8 && nr == 4);
+    return GrpTile<T, NR>::kRows > 0 && ntiles > 0 && g_grp_override.load(std::memory_order_relaxed) != 0;
 }
 
 // Whether the E gathers of launch c use shared-stencil tiles (EGATHER's choice).
 template <typename T, int NR>
 static bool grp_launch(const LaunchCfg<T>& c) {
-    if constexpr (GrpTile<T, NR>::kRows > 0) return c.grp > 0 && grp_gather(sizeof(T), NR, c.grp);
-    return false;
+    return grp_gather<T, NR>(c.grp);
 }
 
 template <typename T, int NR>
@@ -1546,7 +1525,7 @@ void Launch<T, NR>::iteration(const LaunchCfg<T>& c, Vecs<T>& w, bool mixed, con
     if constexpr (std::is_same<T, float>::value) {
         if (mixed) {   // FP32 lanes in the gather, refinement lanes' FP64 gathers in a launch of their own
             EGATHER(fly, yp, w.tmp, M_RUN, mv);
-            LAUNCH((k_egather_upd<NR>), mv);   // few groups refine at once: their blocks together
+            LAUNCH_GATHER((k_egather_upd<NR>), mv);
         } else {
             EGATHER(fly, yp, w.tmp, M_STAGE1, mv);
         }
@@ -1607,7 +1586,7 @@ void MixedLaunch<NR>::down(const LaunchCfg<double>& c, const double* r64, Vecs<f
     FIN(double, NR, FIN_MX_INIT);
 }
 
-#define CPM_INST(T, NR) template struct Launch<T, NR>; template void launch_egather<T, NR>(const LaunchCfg<T>&, const T*, T*, bool);
+#define CPM_INST(T, NR) template struct Launch<T, NR>; template bool grp_gather<T, NR>(int); template void launch_egather<T, NR>(const LaunchCfg<T>&, const T*, T*, bool);
 CPM_INST(double, 1) CPM_INST(double, 2) CPM_INST(double, 4) CPM_INST(double, 8)
 CPM_INST(float, 1) CPM_INST(float, 2) CPM_INST(float, 4) CPM_INST(float, 8)
 template struct MixedLaunch<1>;

@@ -36,7 +36,6 @@ struct Ctx {
     std::map<void*, int64_t> user_bytes;
     int64_t op_bytes = 0;
     Arena* arena = nullptr;   // set: workspace() carves from it and never allocates
-    bool no_builds = false;   // set: solves build no shared-stencil tiles (they would allocate)
     // FP32+refine history of tensor-product operators by family (the same m, n, L_off and L_ii:
     // one equation on one grid spacing), which FP64 routing consults for an operator with no
     // history of its own (a served request's operator is built for it and solved once)
@@ -44,16 +43,6 @@ struct Ctx {
     explicit Ctx(int dev);
     ~Ctx();
     double* workspace(const char* name, size_t bytes);
-};
-
-// Solves on the context build no tiles while this object lives.
-struct NoBuilds {
-    Ctx* c;
-    bool old;
-    explicit NoBuilds(Ctx* c_) : c(c_), old(c_->no_builds) { c->no_builds = true; }
-    ~NoBuilds() { c->no_builds = old; }
-    NoBuilds(const NoBuilds&) = delete;
-    NoBuilds& operator=(const NoBuilds&) = delete;
 };
 
 // Operator in device memory, in one of two execution formats (see OpView):
@@ -78,7 +67,6 @@ struct Op {
     Buffer gofs, grow, gpl, gw64, gw32, gln, glr, glx;   // shared-stencil tiles (OP_TP)
     int ngt = 0, nitem = 0;
     int64_t nslot = 0;
-    bool grp_mode = false, grp_tried = false;   // shared-stencil tiles wanted / build attempted
     // gathered (non-identity) rows: [0] plain and [1] exception rows of LDS
     // tiles, [2] plain and [3] exception rows read directly; rows in all lists;
     // kind-0 items of shared-stencil tiles
@@ -102,12 +90,8 @@ struct Op {
     size_t device_bytes() const;
 };
 
-// Builds a tensor-product operator's shared-stencil tiles on the first call
-// (when its build asked for them); later calls return at once.
-void op_ensure_group_tiles(Op& op);
-// The same for every operator of a launch of T x nr values, if that shape
-// uses shared-stencil tiles.
-void ensure_group_tiles_for(const std::vector<Op*>& ops, int tsize, int nr);
+// Builds a tensor-product operator's row tiles if it has none.
+void op_ensure_row_tiles(Op& op);
 
 // Batched BiCGStab over instances (ops[i], rhs[i] -> xs[i], caller-order
 // device vectors); mn, when given, overrides each instance's (m, n).

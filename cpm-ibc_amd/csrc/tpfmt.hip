@@ -18,6 +18,7 @@
 // (w_z w_y) w_x, the order of Interpolation.cpp:95-107.  Otherwise the caller
 // keeps the ELL format.
 #include <hip/hip_runtime.h>
+#include <hipcub/hipcub.hpp>
 
 #include <algorithm>
 #include <atomic>
@@ -247,9 +248,8 @@ static void ensure_lex(Tube& t, Ctx* ctx) {
 }
 
 // CPMGPU_LDS_TILES selects the LDS tiles built with tensor-product
-// operators: unset or "1", row tiles and shared-stencil tiles (these unless
-// they would need more workgroups than the operator has row blocks); "rows",
-// row tiles only; "0", none (every gather reads x directly).
+// operators: unset or "1", shared-stencil tiles; "rows", row tiles; "0", none
+// (every gather reads x directly).
 static int lds_tile_mode() {
     const char* e = std::getenv("CPMGPU_LDS_TILES");
     if (!e) return 2;
@@ -316,220 +316,435 @@ static void parallel_for(int64_t n, Body&& body) {
     for (auto& x : th) x.join();
 }
 
-// Shared-stencil tiles.  Plain rows are sorted by their stencil block (the
-// first column of line (0, 0)) and rows with the same block are cut into
-// items of up to kGrpRows rows; exception rows are single items placed by
-// their smallest column, identity rows are items of up to kGrpRows rows at
-// the end.  Tiles take items in that order while the tile's list of distinct
-// x rows stays within kGrpLdsRows and its items within kBlock; inside a tile,
-// plain items come first, by row count (larger first), then exception rows,
-// then identity rows, so that a wave's threads take one code path and their
-// loops over the rows of an item end together (which item a thread takes
-// changes no row's arithmetic).  Returns false (nothing built) if the tiles
-// would outnumber the operator's row blocks, which size every launch, or
-// number fewer than kGrpMinTiles.
-static bool build_group_tiles(Op& op, const HostTp& h, const Buffer& tpw64, const Buffer& tpw32) {
-    const int64_t D = h.D;
-    // CPMGPU_GROUP_ITEMS: fewer items per tile (more, smaller tiles); read once per process
-    static const int max_items = [] {
-        const char* e = std::getenv("CPMGPU_GROUP_ITEMS");
-        return e ? std::max(1, std::min(kBlock, std::atoi(e))) : kBlock;
-    }();
-    const int64_t nblocks = (D + kBlock - 1) / kBlock;
-    if (D >= (int64_t)kGrpOfsMask || nblocks < kGrpMinTiles) return false;
-    struct Item {
-        int r0, n, kind;   // rows trow[r0 .. r0 + n)
-    };
-    // non-identity rows by key with a counting sort (rows in increasing order
-    // within a key, plain rows before exception rows): a plain row's key is its
-    // stencil block (the first column of line (0, 0)), an exception row's its
-    // smallest column; every key is a column, below D
-    std::vector<int> key((size_t)D, -1), cnt((size_t)D + 1, 0), pcnt((size_t)D, 0), ident;
-    int64_t nplain = 0, nexcr = 0;
-    for (int64_t r = 0; r < D; ++r) {
-        int k;
-        if (h.flag[(size_t)r] & ROW_IDENTITY) {
-            ident.push_back((int)r);
-            continue;
-        } else if (h.exc[(size_t)r] >= 0) {
-            k = INT32_MAX;
-            h.columns(r, [&](int c) { k = std::min(k, c); });
-            ++nexcr;
-        } else {
-            k = h.tpc[(size_t)r];
-            if (k >= 0 && k < D) ++pcnt[(size_t)k];
-            ++nplain;
-        }
-        if (k < 0 || k >= D) throw std::logic_error("shared-stencil tiles: a row's key is out of range");
-        key[(size_t)r] = k;
-        ++cnt[(size_t)k + 1];
-    }
-    for (int64_t k = 0; k < D; ++k) cnt[(size_t)k + 1] += cnt[(size_t)k];
-    std::vector<int> trow((size_t)D), fill(cnt.begin(), cnt.end() - 1);
-    for (int pass = 0; pass < 2; ++pass)   // plain rows, then exception rows
-        for (int64_t r = 0; r < D; ++r) {
-            const int k = key[(size_t)r];
-            if (k >= 0 && (h.exc[(size_t)r] >= 0) == (pass == 1)) trow[(size_t)fill[(size_t)k]++] = (int)r;
-        }
-    std::vector<Item> items;
-    items.reserve((size_t)(nplain / kGrpRows + nexcr + (int64_t)ident.size() / kGrpRows + 2));
-    int64_t items0 = 0;
-    for (int64_t k = 0; k < D; ++k) {
-        const int a = cnt[(size_t)k], b = cnt[(size_t)k + 1], pe = a + pcnt[(size_t)k];
-        for (int c = a; c < pe; c += kGrpRows) {
-            items.push_back({c, std::min(kGrpRows, pe - c), 0});
-            ++items0;
-        }
-        for (int c = pe; c < b; ++c) items.push_back({c, 1, 1});
-    }
-    trow.resize((size_t)cnt[(size_t)D]);
-    for (size_t c = 0; c < ident.size(); c += kGrpRows) {
-        const int n = (int)std::min<size_t>(kGrpRows, ident.size() - c);
-        items.push_back({(int)trow.size(), n, 2});
-        for (int g = 0; g < n; ++g) trow.push_back(ident[c + g]);
-    }
-    const int64_t nitem = (int64_t)items.size();
-    // greedy tiles over contiguous item ranges, one host thread each (a range
-    // ends its last tile early); stamp[c] = tile whose list holds column c
-    const int nparts = (int)std::max<int64_t>(
-        1, std::min<int64_t>({16, nitem / 4096 + 1, (int64_t)std::max(1u, std::thread::hardware_concurrency())}));
-    std::vector<std::vector<int>> starts((size_t)nparts);
-    parallel_for(nparts, [&](int64_t part) {
-        const int64_t i0 = nitem * part / nparts, i1 = nitem * (part + 1) / nparts;
-        std::vector<int> stamp((size_t)D, -1), fresh;
-        std::vector<int>& first = starts[(size_t)part];
-        if (i1 > i0) first.push_back((int)i0);
-        int tile = 0, list = 0, nin = 0;
-        for (int64_t i = i0; i < i1;) {
-            const Item& it = items[(size_t)i];
-            fresh.clear();
-            if (it.kind != 2)
-                h.columns(trow[(size_t)it.r0], [&](int c) {
-                    if (stamp[(size_t)c] != tile) {
-                        stamp[(size_t)c] = tile;
-                        fresh.push_back(c);
-                    }
-                });
-            if (nin > 0 && (list + (int)fresh.size() > kGrpLdsRows || nin + 1 > max_items)) {
-                for (int c : fresh) stamp[(size_t)c] = -1;
-                first.push_back((int)i);
-                ++tile;
-                list = 0;
-                nin = 0;
-                continue;   // the item again, in a new tile
-            }
-            list += (int)fresh.size();
-            ++nin;
-            ++i;
-        }
-    });
-    std::vector<int> first;
-    for (const auto& v : starts) first.insert(first.end(), v.begin(), v.end());
-    if (first.empty()) first.push_back(0);
-    first.push_back((int)nitem);
-    const int64_t ngt = (int64_t)first.size() - 1;
-    // with fewer tiles the row tiles' 2.3 times as many workgroups fill the
-    // GPU better (measured on spheres of 41,870 and 65,294 rows)
-    if (ngt > nblocks || ngt < kGrpMinTiles) return false;
-    // per tile: items by row count, the sorted list, positions
-    std::vector<std::vector<int>> lists((size_t)ngt);
-    std::vector<int> order((size_t)nitem);
-    const int64_t nip = ngt * kBlock;   // item places: tile t owns t kBlock .. (t + 1) kBlock - 1
-    std::vector<int> gpl((size_t)8 * nip, 0);
-    std::vector<int16_t> tlx((size_t)std::max<int64_t>(h.ne, 1) * kExcPos, -1);
-    std::atomic<int> bad{0};
-    parallel_for(ngt, [&](int64_t t) {
-        const int i0 = first[(size_t)t], i1 = first[(size_t)t + 1];
-        for (int i = i0; i < i1; ++i) order[(size_t)i] = i;
-        auto rank = [&](int u) {   // plain items by row count, then exception rows, then identity rows
-            const Item& it = items[(size_t)u];
-            return it.kind == 0 ? kGrpRows - it.n : kGrpRows + it.kind;
-        };
-        std::stable_sort(order.begin() + i0, order.begin() + i1, [&](int u, int v) { return rank(u) < rank(v); });
-        std::vector<int>& u = lists[(size_t)t];
-        for (int i = i0; i < i1; ++i)
-            if (items[(size_t)i].kind != 2) h.columns(trow[(size_t)items[(size_t)i].r0], [&](int c) { u.push_back(c); });
-        std::sort(u.begin(), u.end());
-        u.erase(std::unique(u.begin(), u.end()), u.end());
-        if ((int64_t)u.size() > kGrpLdsRows || i1 - i0 > kBlock) bad = 1;
-        auto pos = [&](int c) { return (int16_t)(std::lower_bound(u.begin(), u.end(), c) - u.begin()); };
-        for (int q = i0; q < i1 && q - i0 < kBlock; ++q) {
-            const Item& it = items[(size_t)order[(size_t)q]];
-            const int r = trow[(size_t)it.r0];
-            const size_t qp = (size_t)t * kBlock + (size_t)(q - i0);   // the item's place
-            if (it.kind == 0) {
-                for (int l = 0; l < 16; ++l) {
-                    const int16_t p = pos(h.tpc[(size_t)l * D + r]);
-                    if (p < 0 || p + 3 >= (int)u.size()) bad = 1;
-                    gpl[(size_t)(l >> 1) * nip + qp] |= (int)((unsigned)(uint16_t)p << (16 * (l & 1)));
-                }
-            } else if (it.kind == 1) {
-                const int e = h.exc[(size_t)r];
-                for (int s = 0; s < 64; ++s) tlx[(size_t)e * kExcPos + s] = pos(h.ecx[(size_t)e * 64 + s]);
-                if (h.xcol[(size_t)e] >= 0) tlx[(size_t)e * kExcPos + 64] = pos(h.xcol[(size_t)e]);
-                gpl[qp] = e;   // read with the line positions, a step before the record
+// ---------------------------------------------------------------- shared-stencil tiles
+// Built on the device.  Rows are sorted by the place of their stencil block
+// (the first node of line (0, 0)) along a Hilbert curve through the grid, so
+// that consecutive rows read a compact patch of x rows; identity rows come
+// last.  Plain rows of one block are cut into items of up to kGrpRows rows,
+// exception rows are single items beside the plain rows of their block, and
+// identity rows are items of up to kGrpRows rows.  A tile is a run of items
+// whose list of distinct x rows fits kGrpLdsRows.
+//
+// In the lexicographic order of the blocks a tile of 256 items is a strip one
+// grid column wide; along the curve it is a patch, whose stencils overlap in
+// both directions of the surface: 2.47 -> 1.53 list rows per row on the
+// h = 0.02 torus (Morton order: 1.54).
+
+constexpr uint32_t kIdentKey = 0xffffffffu;
+constexpr int kMinTileItems = 8;
+static_assert(kMinTileItems * 65 <= kGrpLdsRows, "the lists of this few items always fit");
+static_assert((kGrpLdsRows & (kGrpLdsRows - 1)) == 0, "the lists are sorted by a bitonic network");
+constexpr int kHash = 4 * 1024;        // open-addressing table of a tile's x rows (LDS)
+
+// Position of (x, y, z), each below 2^10, along the Hilbert curve of the 2^10
+// cube (Skilling, "Programming the Hilbert curve", AIP Conf. Proc. 707, 2004:
+// the axes' Gray-code transform, then their bits interleaved).
+__host__ __device__ inline uint32_t hilbert_index(uint32_t x, uint32_t y, uint32_t z) {
+    uint32_t v[3] = {x, y, z};
+    for (uint32_t q = 1u << 9; q > 1; q >>= 1) {
+        const uint32_t low = q - 1;
+        for (int i = 0; i < 3; ++i) {
+            if (v[i] & q) {
+                v[0] ^= low;
             } else {
-                for (int g = 0; g < kGrpRows; ++g)   // the rows (kind 2 reads their x values after the barrier)
-                    gpl[(size_t)g * nip + qp] = g < it.n ? trow[(size_t)it.r0 + g] : -1;
+                const uint32_t t = (v[0] ^ v[i]) & low;
+                v[0] ^= t;
+                v[i] ^= t;
             }
+        }
+    }
+    v[1] ^= v[0];
+    v[2] ^= v[1];
+    uint32_t t = 0;
+    for (uint32_t q = 1u << 9; q > 1; q >>= 1)
+        if (v[2] & q) t ^= q - 1;
+    uint32_t h = 0;
+    for (int b = 9; b >= 0; --b)
+        for (int i = 0; i < 3; ++i) h = (h << 1) | (((v[i] ^ t) >> b) & 1u);
+    return h;
+}
+
+// Sort key of each row: twice the curve position of its block, plus one for
+// exception rows; identity rows sort last.
+__global__ void k_grp_keys(int64_t D, const uint8_t* flag, const int* tpc, const int* exc, const int32_t* lex,
+                           const int64_t* rec, int64_t N1d, uint32_t* key, int* row) {
+    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (r >= D) return;
+    row[r] = (int)r;
+    if (flag[r] & ROW_IDENTITY) { key[r] = kIdentKey; return; }
+    const int64_t l = rec[lex[tpc[r]]];   // line (0, 0) starts at a tube node
+    const uint32_t z = (uint32_t)(l % N1d), y = (uint32_t)((l / N1d) % N1d), x = (uint32_t)(l / (N1d * N1d));
+    key[r] = 2u * hilbert_index(x, y, z) + (exc[r] >= 0 ? 1u : 0u);
+}
+
+// First position of each run of equal keys (0 elsewhere), for a maximum scan.
+__global__ void k_grp_heads(int64_t D, const uint32_t* key, int* head) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < D) head[i] = (i == 0 || key[i] != key[i - 1]) ? (int)i : 0;
+}
+
+__device__ __forceinline__ bool grp_exc_key(uint32_t k) { return k != kIdentKey && (k & 1u); }
+
+// 1 where an item starts.
+__global__ void k_grp_starts(int64_t D, const uint32_t* key, const int* head, int* start) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < D) start[i] = grp_exc_key(key[i]) || ((int)i - head[i]) % kGrpRows == 0;
+}
+
+// pos: exclusive sums of start; ifirst[item] = its first sorted row, ifirst[nitem] = D;
+// counts: items, plain items, exception rows, identity rows, identity items.
+__global__ void k_grp_items(int64_t D, const uint32_t* key, const int* start, const int* pos, int* ifirst, int* counts) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const bool in = i < D;
+    const bool st = in && start[i];
+    const bool id = in && key[i] == kIdentKey, ex = in && grp_exc_key(key[i]);
+    if (st) ifirst[pos[i]] = (int)i;
+    if (in && i == D - 1) {
+        const int n = pos[i] + start[i];
+        ifirst[n] = (int)D;
+        counts[0] = n;
+    }
+    const unsigned long long p = __ballot(st && !id && !ex), e = __ballot(ex), d = __ballot(id), di = __ballot(id && st);
+    if ((threadIdx.x & 63) == 0) {
+        if (p) atomicAdd(&counts[1], __popcll(p));
+        if (e) atomicAdd(&counts[2], __popcll(e));
+        if (d) atomicAdd(&counts[3], __popcll(d));
+        if (di) atomicAdd(&counts[4], __popcll(di));
+    }
+}
+
+struct GrpSrc {
+    int64_t D;
+    int nitem;
+    const uint32_t* key;    // sorted
+    const int* row;         // rows in sorted order
+    const int* ifirst;      // [nitem + 1]
+    const uint8_t* flag;
+    const int* tpc;
+    const int* exc;
+    const int* ecx;
+    const int* xcol;
+};
+
+// f(c) for the x rows that thread t's share of items [i0, i1) reads: 16
+// threads an item, one stencil line each.
+template <typename F>
+__device__ __forceinline__ void grp_columns(const GrpSrc& s, int i0, int i1, F&& f) {
+    for (int u = (int)threadIdx.x; u < (i1 - i0) * 16; u += (int)blockDim.x) {
+        const int p = s.ifirst[i0 + (u >> 4)], l = u & 15;
+        const uint32_t k = s.key[p];
+        if (k == kIdentKey) continue;
+        const int64_t r = s.row[p];
+        if (grp_exc_key(k)) {
+            const int e = s.exc[r];
+            for (int q = 0; q < 4; ++q) f(s.ecx[(int64_t)e * 64 + 4 * l + q]);
+            if (l == 0 && s.xcol[e] >= 0) f(s.xcol[e]);
+        } else {
+            const int c = s.tpc[(int64_t)l * s.D + r];
+            for (int q = 0; q < 4; ++q) f(c + q);
+        }
+    }
+}
+
+// Distinct x rows of items [i0, i1) into the hash table `tab` (all -1 outside
+// the entries); returns their number, or more than kGrpLdsRows when they do
+// not fit (the table is then incomplete).  Threads stop inserting past the
+// limit, so at most kGrpLdsRows + blockDim entries are ever taken.
+__device__ int grp_collect(const GrpSrc& s, int i0, int i1, int* tab, int* count) {
+    for (int k = (int)threadIdx.x; k < kHash; k += (int)blockDim.x) tab[k] = -1;
+    if (threadIdx.x == 0) *count = 0;
+    __syncthreads();
+    grp_columns(s, i0, i1, [&](int c) {
+        if (*(volatile int*)count > kGrpLdsRows) return;
+        unsigned h = ((unsigned)c * 2654435761u) >> 20;
+        for (;;) {
+            const int old = atomicCAS(&tab[h & (kHash - 1)], -1, c);
+            if (old == c) return;
+            if (old == -1) { atomicAdd(count, 1); return; }
+            ++h;
         }
     });
-    if (bad) throw std::logic_error("shared-stencil tiles: a list or position is out of range");
-    // slots in final item order, item places padded to kBlock per tile with
-    // empty items (kind 3, no slot)
-    std::vector<int> gofs((size_t)nip + 1), grow;
-    grow.reserve((size_t)D);
-    for (int64_t t = 0; t < ngt; ++t) {
-        const int i0 = first[(size_t)t], i1 = first[(size_t)t + 1];
-        for (int j = 0; j < kBlock; ++j) {
-            const size_t qp = (size_t)t * kBlock + (size_t)j;
-            if (j >= i1 - i0) {
-                gofs[qp] = (int)grow.size() | (3 << kGrpKindShift);
-                continue;
-            }
-            const Item& it = items[(size_t)order[(size_t)(i0 + j)]];
-            gofs[qp] = (int)grow.size() | (it.kind << kGrpKindShift);
-            for (int g = 0; g < it.n; ++g) grow.push_back(trow[(size_t)it.r0 + g]);
+    __syncthreads();
+    const int n = *count;
+    __syncthreads();
+    return n;
+}
+static_assert(kGrpLdsRows + 2 * kBlock < kHash, "the table always keeps empty entries, so every probe ends");
+
+// One workgroup per run of `m` items: the number of equal parts (1, 2, 4 ..)
+// the run is cut into so that every part's list fits.
+__global__ __launch_bounds__(kBlock) void k_grp_count(GrpSrc s, int m, int* parts) {
+    __shared__ int tab[kHash];
+    __shared__ int count;
+    const int i0 = (int)blockIdx.x * m, i1 = min(s.nitem, i0 + m);
+    int sz = m;
+    for (int a = i0; a < i1;) {
+        const int n = grp_collect(s, a, min(i1, a + sz), tab, &count);
+        if (n > kGrpLdsRows && sz > kMinTileItems) {   // start over with parts of half the size
+            sz >>= 1;
+            a = i0;
+            continue;
         }
+        a += sz;
     }
-    gofs[(size_t)nip] = (int)grow.size();
-    if ((int64_t)grow.size() != D) throw std::logic_error("shared-stencil tiles: not every row has a slot");
-    // lists at kGrpLdsRows places per tile, the unused places repeating the
-    // last entry (the gather reads every place without a branch); an entry is
-    // the x row with the row's class in bit 30 (the gather's kListPlainBit)
-    std::vector<int> tln((size_t)ngt), tlr((size_t)ngt * kGrpLdsRows, 0);
-    op.grp_list = 0;
-    for (int64_t t = 0; t < ngt; ++t) {
-        const std::vector<int>& u = lists[(size_t)t];
-        tln[(size_t)t] = (int)u.size();
-        int* dst = tlr.data() + (size_t)t * kGrpLdsRows;
-        // bit 30: the row's P^-1 leaves it as it is (identity or no-diagonal row)
-        for (size_t k = 0; k < u.size(); ++k)
-            dst[k] = u[k] | ((h.flag[(size_t)u[k]] & (ROW_IDENTITY | ROW_NODIAG)) ? 1 << 30 : 0);
-        std::fill(dst + u.size(), dst + kGrpLdsRows, u.empty() ? 0 : dst[u.size() - 1]);
-        op.grp_list += tln[(size_t)t];
+    if (threadIdx.x == 0) parts[blockIdx.x] = m / sz;
+}
+
+struct GrpOut {
+    int64_t nip;            // item places
+    int* gofs;
+    int* grow;
+    int* gpl;
+    int* gln;
+    int* glr;
+    int16_t* glx;
+    int* total_list;        // rows in all lists
+    int* err;
+};
+
+// One workgroup per run: the tiles of its parts (first[run] is the first).
+// A tile's items are placed by kind and row count (plain items with more rows
+// first, then exception rows, then identity rows), so that a wave's threads
+// take one path of the gather and end together; which thread takes an item
+// changes no row's arithmetic.
+__global__ __launch_bounds__(kBlock) void k_grp_tiles(GrpSrc s, GrpOut o, int m, const int* first, int nruns, int ntiles) {
+    __shared__ int tab[kHash];
+    __shared__ int list[kGrpLdsRows];
+    __shared__ int count, used;
+    __shared__ int place[kBlock];      // item at a place
+    __shared__ int rows[kBlock];       // its rows, then their exclusive sums
+    __shared__ int ccount[4][kGrpRows + 3];
+    const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int i0 = (int)blockIdx.x * m, i1 = min(s.nitem, i0 + m);
+    const int t0 = first[blockIdx.x], t1 = (int)blockIdx.x + 1 < nruns ? first[blockIdx.x + 1] : ntiles;
+    const int sz = m / (t1 - t0);
+    for (int tile = t0; tile < t1; ++tile) {
+        const int a = min(i1, i0 + (tile - t0) * sz), b = min(i1, a + sz), ni = b - a;
+        const int nu = grp_collect(s, a, b, tab, &count);
+        if (nu > kGrpLdsRows) {   // uniform (the parts were cut so that none is)
+            if (t == 0) atomicOr(o.err, 1);
+            return;
+        }
+        // the table's entries, sorted (unused places sort last)
+        if (t == 0) used = 0;
+        for (int k = t; k < kGrpLdsRows; k += kBlock) list[k] = INT_MAX;
+        __syncthreads();
+        for (int k = t; k < kHash; k += kBlock)
+            if (tab[k] >= 0) list[atomicAdd(&used, 1)] = tab[k];
+        __syncthreads();
+        for (int w = 2; w <= kGrpLdsRows; w <<= 1)
+            for (int h = w >> 1; h > 0; h >>= 1) {
+                for (int k = t; k < kGrpLdsRows / 2; k += kBlock) {
+                    const int p = 2 * k - (k & (h - 1)), q = p + h;
+                    const int u = list[p], v = list[q];
+                    if ((u > v) == ((p & w) == 0)) {
+                        list[p] = v;
+                        list[q] = u;
+                    }
+                }
+                __syncthreads();
+            }
+        auto pos = [&](int c) {   // index of c in the list
+            int lo = 0, hi = nu;
+            while (lo < hi) {
+                const int mid = (lo + hi) >> 1;
+                if (list[mid] < c) lo = mid + 1;
+                else hi = mid;
+            }
+            if (lo >= nu || list[lo] != c) atomicOr(o.err, 2);
+            return lo;
+        };
+        // list entries, the unused places repeating the last (the gather reads every place without
+        // a branch); bit 30: P^-1 leaves the row as it is (identity or no-diagonal row)
+        for (int k = t; k < kGrpLdsRows; k += kBlock) {
+            int c = nu > 0 ? list[min(k, nu - 1)] : 0;
+            if (nu > 0 && (s.flag[c] & (ROW_IDENTITY | ROW_NODIAG))) c |= 1 << 30;
+            o.glr[(int64_t)tile * kGrpLdsRows + k] = c;
+        }
+        if (t == 0) {
+            o.gln[tile] = nu;
+            atomicAdd(o.total_list, nu);
+        }
+        // places: a stable counting sort of the items by class
+        int cls = -1, n = 0, p0 = 0;
+        if (t < ni) {
+            p0 = s.ifirst[a + t];
+            n = s.ifirst[a + t + 1] - p0;
+            const uint32_t k = s.key[p0];
+            cls = k == kIdentKey ? kGrpRows + 1 : (k & 1u) ? kGrpRows : kGrpRows - n;
+        }
+        int before = 0;
+        for (int c = 0; c < kGrpRows + 2; ++c) {
+            const unsigned long long same = __ballot(cls == c);
+            if (cls == c) before = __popcll(same & ((1ull << lane) - 1ull));
+            if (lane == 0) ccount[wave][c] = __popcll(same);
+        }
+        rows[t] = 0;
+        __syncthreads();
+        if (t < ni) {
+            for (int c = 0; c < cls; ++c)
+                for (int w = 0; w < 4; ++w) before += ccount[w][c];
+            for (int w = 0; w < wave; ++w) before += ccount[w][cls];
+            place[before] = t;
+            rows[before] = n;
+        }
+        __syncthreads();
+        int sum = rows[t];   // inclusive sums
+        for (int d = 1; d < kBlock; d <<= 1) {
+            const int add = t >= d ? rows[t - d] : 0;
+            __syncthreads();
+            sum += add;
+            rows[t] = sum;
+            __syncthreads();
+        }
+        // the items in place order: slots, rows, positions
+        const int64_t qp = (int64_t)tile * kBlock + t;
+        const int base = s.ifirst[a];
+        int word[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        if (t < ni) {
+            const int it = a + place[t];
+            const int q0 = s.ifirst[it], cnt = s.ifirst[it + 1] - q0;
+            const int slot = base + rows[t] - cnt;
+            const uint32_t k = s.key[q0];
+            const int kind = k == kIdentKey ? 2 : (k & 1u) ? 1 : 0;
+            o.gofs[qp] = slot | (kind << kGrpKindShift);
+            const int64_t r = s.row[q0];
+            for (int g = 0; g < cnt; ++g) o.grow[slot + g] = s.row[q0 + g];
+            if (kind == 0) {
+#pragma unroll
+                for (int l = 0; l < 16; ++l) {
+                    const int p = pos(s.tpc[(int64_t)l * s.D + r]);
+                    if (p + 3 >= nu) atomicOr(o.err, 4);
+                    word[l >> 1] |= (int)((unsigned)p << (16 * (l & 1)));
+                }
+            } else if (kind == 1) {
+                const int e = s.exc[r];
+                for (int q = 0; q < 64; ++q) o.glx[(int64_t)e * kExcPos + q] = (int16_t)pos(s.ecx[(int64_t)e * 64 + q]);
+                const int xc = s.xcol[e];
+                o.glx[(int64_t)e * kExcPos + 64] = xc >= 0 ? (int16_t)pos(xc) : (int16_t)-1;
+                for (int q = 65; q < kExcPos; ++q) o.glx[(int64_t)e * kExcPos + q] = -1;
+                word[0] = e;   // read with the line positions, a step before the record
+            } else {
+#pragma unroll
+                for (int g = 0; g < kGrpRows; ++g) word[g] = g < cnt ? s.row[q0 + g] : -1;
+            }
+        } else {
+            o.gofs[qp] = s.ifirst[b] | (3 << kGrpKindShift);   // an empty place
+        }
+#pragma unroll
+        for (int h = 0; h < 8; ++h) o.gpl[(int64_t)h * o.nip + qp] = word[h];
+        __syncthreads();
     }
-    op.grp_items = nitem;
-    op.grp_items0 = items0;
-    op.grp_rows0 = nplain;
-    op.grp_exc = nexcr;
-    op.grp_ident = (int64_t)ident.size();
-    op.grp_ident_items = ((int64_t)ident.size() + kGrpRows - 1) / kGrpRows;
-    upload(op.gln, tln.data(), tln.size() * 4);
-    upload(op.glr, tlr.data(), tlr.size() * 4);
-    upload(op.glx, tlx.data(), tlx.size() * 2);
-    upload(op.gofs, gofs.data(), gofs.size() * 4);
-    upload(op.grow, grow.data(), grow.size() * 4);
-    upload(op.gpl, gpl.data(), gpl.size() * 4);
-    op.gw64 = Buffer((size_t)12 * D * 8);
-    op.gw32 = Buffer((size_t)12 * D * 4);
+    if (t1 == ntiles && t == 0) o.gofs[o.nip] = (int)s.D;
+}
+
+// Exclusive sums of the runs' parts (one workgroup; a few thousand runs at most per million rows).
+__global__ void k_grp_first(const int* parts, int n, int* first, int* total) {
+    __shared__ int sums[256];
+    const int t = (int)threadIdx.x, per = (n + 255) / 256, b = min(n, t * per), e = min(n, b + per);
+    int s = 0;
+    for (int k = b; k < e; ++k) s += parts[k];
+    sums[t] = s;
+    __syncthreads();
+    for (int d = 1; d < 256; d <<= 1) {
+        const int add = t >= d ? sums[t - d] : 0;
+        __syncthreads();
+        sums[t] += add;
+        __syncthreads();
+    }
+    int run = sums[t] - s;
+    for (int k = b; k < e; ++k) {
+        first[k] = run;
+        run += parts[k];
+    }
+    if (t == 255) *total = sums[255];
+}
+
+// Items per tile: 256 (one per thread of a gather workgroup) where that
+// leaves a workgroup or more for each of the 256 CUs, fewer for smaller
+// operators.
+static int group_tile_items(int nitem) {
+    // CPMGPU_GROUP_ITEMS: items per tile, rounded down to a power of two (measurements); read once per process
+    static const int forced = [] {
+        const char* e = std::getenv("CPMGPU_GROUP_ITEMS");
+        int m = kBlock;
+        while (e && m > kMinTileItems && m > std::atoi(e)) m >>= 1;
+        return e ? m : 0;
+    }();
+    if (forced) return forced;
+    int m = kBlock;
+    while (m > 32 && nitem < m * 512) m >>= 1;
+    return m;
+}
+
+// Returns false (nothing built) for operators whose slots exceed gofs's bits.
+static bool build_group_tiles(Op& op, const Tube& tube) {
+    const int64_t D = op.D;
+    if (D >= (int64_t)kGrpOfsMask) return false;
     const hipStream_t st = op.ctx->stream;
-    hipLaunchKernelGGL(k_slot_weights<double>, dim3(nblk(D)), dim3(256), 0, st, tpw64.as<double>(), D,
-                       op.grow.as<int>(), D, op.gw64.as<double>());
-    hipLaunchKernelGGL(k_slot_weights<float>, dim3(nblk(D)), dim3(256), 0, st, tpw32.as<float>(), D,
-                       op.grow.as<int>(), D, op.gw32.as<float>());
+    const dim3 gb(nblk(D)), tb(256);
+    Buffer key((size_t)D * 8), row((size_t)D * 8), head((size_t)D * 4), start((size_t)D * 4), pos((size_t)D * 4),
+        ifirst((size_t)(D + 1) * 4), small(256);
+    uint32_t *k0 = key.as<uint32_t>(), *k1 = k0 + D;
+    int *r0 = row.as<int>(), *r1 = r0 + D;
+    int* counts = small.as<int>();   // [0..4] items by kind, [5] list rows, [6] errors, [7] tiles
+    HIPCHK(hipMemsetAsync(small.p, 0, 256, st));
+    hipLaunchKernelGGL(k_grp_keys, gb, tb, 0, st, D, op.flag.as<uint8_t>(), op.tpc.as<int>(), op.exc.as<int>(),
+                       tube.lex.as<int32_t>(), tube.rec.as<int64_t>(), tube.N1d, k0, r0);
+    size_t sort_bytes = 0, max_bytes = 0, sum_bytes = 0;
+    HIPCHK(hipcub::DeviceRadixSort::SortPairs(nullptr, sort_bytes, k0, k1, r0, r1, (int)D, 0, 32, st));
+    HIPCHK(hipcub::DeviceScan::InclusiveScan(nullptr, max_bytes, head.as<int>(), head.as<int>(), hipcub::Max(), (int)D, st));
+    HIPCHK(hipcub::DeviceScan::ExclusiveSum(nullptr, sum_bytes, start.as<int>(), pos.as<int>(), (int)D, st));
+    Buffer tmp(std::max({sort_bytes, max_bytes, sum_bytes, (size_t)256}));
+    HIPCHK(hipcub::DeviceRadixSort::SortPairs(tmp.p, sort_bytes, k0, k1, r0, r1, (int)D, 0, 32, st));
+    hipLaunchKernelGGL(k_grp_heads, gb, tb, 0, st, D, k1, pos.as<int>());
+    HIPCHK(hipcub::DeviceScan::InclusiveScan(tmp.p, max_bytes, pos.as<int>(), head.as<int>(), hipcub::Max(), (int)D, st));
+    hipLaunchKernelGGL(k_grp_starts, gb, tb, 0, st, D, k1, head.as<int>(), start.as<int>());
+    HIPCHK(hipcub::DeviceScan::ExclusiveSum(tmp.p, sum_bytes, start.as<int>(), pos.as<int>(), (int)D, st));
+    hipLaunchKernelGGL(k_grp_items, gb, tb, 0, st, D, k1, start.as<int>(), pos.as<int>(), ifirst.as<int>(), counts);
     HIPCHK(hipGetLastError());
+    int h[8] = {0};
+    HIPCHK(hipMemcpyAsync(h, counts, 32, hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
+    const int nitem = h[0];
+    const int m = group_tile_items(nitem);
+    const int nruns = (nitem + m - 1) / m;
+    GrpSrc src{D, nitem, k1, r1, ifirst.as<int>(), op.flag.as<uint8_t>(), op.tpc.as<int>(), op.exc.as<int>(),
+               op.ecx.as<int>(), op.xcol.as<int>()};
+    // start and pos are free again: parts of each run, first tile of each run
+    hipLaunchKernelGGL(k_grp_count, dim3((unsigned)nruns), dim3(kBlock), 0, st, src, m, start.as<int>());
+    hipLaunchKernelGGL(k_grp_first, dim3(1), dim3(256), 0, st, start.as<int>(), nruns, pos.as<int>(), counts + 7);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(h, counts, 32, hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+    const int64_t ngt = h[7], nip = ngt * kBlock;
+    Buffer gofs((size_t)(nip + 1) * 4), grow((size_t)D * 4), gpl((size_t)8 * nip * 4), gln((size_t)ngt * 4),
+        glr((size_t)ngt * kGrpLdsRows * 4), glx((size_t)std::max<int64_t>(op.nexc, 1) * kExcPos * 2),
+        gw64((size_t)12 * D * 8), gw32((size_t)12 * D * 4);
+    GrpOut out{nip, gofs.as<int>(), grow.as<int>(), gpl.as<int>(), gln.as<int>(), glr.as<int>(), glx.as<int16_t>(),
+               counts + 5, counts + 6};
+    hipLaunchKernelGGL(k_grp_tiles, dim3((unsigned)nruns), dim3(kBlock), 0, st, src, out, m, pos.as<int>(), nruns, (int)ngt);
+    hipLaunchKernelGGL(k_slot_weights<double>, gb, tb, 0, st, op.tpw64.as<double>(), D, grow.as<int>(), D, gw64.as<double>());
+    hipLaunchKernelGGL(k_slot_weights<float>, gb, tb, 0, st, op.tpw32.as<float>(), D, grow.as<int>(), D, gw32.as<float>());
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(h, counts, 32, hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+    if (h[6]) throw std::logic_error("shared-stencil tiles: a list or position is out of range");
+    op.gofs = std::move(gofs);
+    op.grow = std::move(grow);
+    op.gpl = std::move(gpl);
+    op.gln = std::move(gln);
+    op.glr = std::move(glr);
+    op.glx = std::move(glx);
+    op.gw64 = std::move(gw64);
+    op.gw32 = std::move(gw32);
+    op.grp_items = nitem;
+    op.grp_items0 = h[1];
+    op.grp_exc = h[2];
+    op.grp_ident = h[3];
+    op.grp_ident_items = h[4];
+    op.grp_rows0 = D - h[2] - h[3];
+    op.grp_list = h[5];
     op.ngt = (int)ngt;
     op.nitem = (int)nip;
     op.nslot = D;
@@ -673,11 +888,6 @@ bool op_build_tp(Op& op, Tube& t, const TpSource& src) {
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(st));
 
-    if (const int mode = lds_tile_mode()) {
-        const HostTp h(D, ne, tpc, exc, ecx, xcol, flag);
-        build_lds_tiles(op, h);
-        op.grp_mode = mode == 2;   // shared-stencil tiles: on first use (op_ensure_group_tiles)
-    }
     op.fmt = OP_TP;
     op.ew = kS * kS * kS;
     op.lw = 6;
@@ -703,20 +913,14 @@ bool op_build_tp(Op& op, Tube& t, const TpSource& src) {
     op.lval32 = Buffer();
     op.ldiag64 = Buffer();
     op.ldiag32 = Buffer();
+    const int mode = lds_tile_mode();
+    if (mode > 0 && !(mode == 2 && build_group_tiles(op, t))) op_ensure_row_tiles(op);
     return true;
 }
 
-void op_ensure_group_tiles(Op& op) {
-    if (op.grp_tried || !op.grp_mode || op.fmt != OP_TP) return;
-    op.grp_tried = true;
-    const HostTp h(op.D, op.nexc, op.tpc, op.exc, op.ecx, op.xcol, op.flag);
-    build_group_tiles(op, h, op.tpw64, op.tpw32);
-}
-
-void ensure_group_tiles_for(const std::vector<Op*>& ops, int tsize, int nr) {
-    grp_refresh_override();
-    if (!grp_build(tsize, nr)) return;
-    for (Op* o : ops) op_ensure_group_tiles(*o);
+void op_ensure_row_tiles(Op& op) {
+    if (op.fmt != OP_TP || op.tln.p) return;
+    build_lds_tiles(op, HostTp(op.D, op.nexc, op.tpc, op.exc, op.ecx, op.xcol, op.flag));
 }
 
 }  // namespace cpmgpu

@@ -32,6 +32,12 @@
 #ifndef CPMGPU_XCD_RUN
 #define CPMGPU_XCD_RUN 16
 #endif
+#ifndef CPMGPU_GATHER_RUN
+#define CPMGPU_GATHER_RUN 16
+#endif
+#ifndef CPMGPU_LFINISH_RUN
+#define CPMGPU_LFINISH_RUN 16
+#endif
 #ifndef CPMGPU_LDS_ROWS
 #define CPMGPU_LDS_ROWS 2560
 #endif
@@ -39,5 +45,5 @@
 #define CPMGPU_GROUP_ROWS 2
 #endif
 #ifndef CPMGPU_GROUP_LDS_ROWS
-#define CPMGPU_GROUP_LDS_ROWS 1280
+#define CPMGPU_GROUP_LDS_ROWS 1024
 #endif
