@@ -321,7 +321,7 @@ struct Group {
 };
 
 template <typename T>
-static void fill_seg(Seg<T>& s, const Op* op, int64_t off, int nblocks, int nr, KState* st, double* part) {
+static void fill_seg(Seg<T>& s, const Op* op, int64_t off, int nblocks, int nr, KState* st, double* part, int64_t sst = 0) {
     s.op = op->view<T>();
     s.op64 = op->view<double>();
     s.m = op->m;
@@ -337,6 +337,7 @@ static void fill_seg(Seg<T>& s, const Op* op, int64_t off, int nblocks, int nr, 
     s.dinv = (T)(1.0f / (m32 + (float)op->ldu * n32));
     s.tinv = (T)(1.0f / (float)(op->m - op->n));
     s.st = st;
+    s.sst = sst;
     s.part = part;
 }
 
@@ -346,14 +347,17 @@ static void fill_seg(Seg<T>& s, const Op* op, int64_t off, int nblocks, int nr, 
 // each vector), then round-robin (block b of every segment, then block b +
 // 1), which the E gathers run: segments that share an operator (the groups of
 // a streamed solve) gather through each tile together, its metadata read
-// into an L2 once for all of them rather than once per segment.
+// into an L2 once for all of them rather than once per segment.  The
+// refinement lanes' FP64 gathers take the gather workgroups segment by
+// segment: few segments refine at once, and their workgroups belong together
+// (round-robin 43 us against 29 us a launch, 8 groups of 405,928 rows).
 static std::vector<int> block_map(const std::vector<int>& nb, const std::vector<int>& ng) {
     if (nb.size() > (size_t)kMaxSegs) throw ArgError("too many segments in one launch");
     int most = 0;
     size_t total = 0;
     for (size_t g = 0; g < nb.size(); ++g) {
         most = std::max(most, std::max(nb[g], ng[g]));
-        total += (size_t)nb[g] + (size_t)ng[g];
+        total += (size_t)nb[g] + 2 * (size_t)ng[g];
     }
     if (most > (1 << (31 - kSegBits))) throw ArgError("operator too large for one launch's block map");
     std::vector<int> m;
@@ -363,6 +367,8 @@ static std::vector<int> block_map(const std::vector<int>& nb, const std::vector<
     for (int b = 0; b < most; ++b)           // round-robin: the gathers
         for (size_t g = 0; g < ng.size(); ++g)
             if (b < ng[g]) m.push_back((int)g | (b << kSegBits));
+    for (size_t g = 0; g < ng.size(); ++g)   // segment by segment: the refinement lanes' gathers
+        for (int b = 0; b < ng[g]; ++b) m.push_back((int)g | (b << kSegBits));
     return m;
 }
 
@@ -428,11 +434,23 @@ struct BatchBytes {
         return r256(tables) + r256(vec64) + (vec32 ? r256(vec32) : 0) + r256(pack);
     }
 };
-static BatchBytes batch_bytes(int G, int blocks, int gblocks, int64_t total, int NR, bool refine) {
+// Whether a launch folds its finalisers into the kernels that need them
+// (krylov.hip): every workgroup then sums its segment's partials, most a
+// segment's row blocks.
+static bool fold_fins(int most, int NR) { return most * NR <= 1024; }
+// Whether its iterations run fused as well (krylov.hip).
+static bool fuse_iterations(bool fold, int NR) { return fold && NR == 1; }
+
+// Bytes of a launch's block maps (block_map); a launch of one segment has none.
+static size_t map_bytes(int G, int blocks, int gblocks) {
+    return G == 1 ? 0 : sizeof(int) * ((size_t)blocks + 2 * (size_t)gblocks);
+}
+
+static BatchBytes batch_bytes(int G, int blocks, int gblocks, int64_t total, int NR, bool refine, bool fold) {
     auto r256 = [](size_t n) { return (n + 255) & ~size_t(255); };
     BatchBytes b;
-    b.tables = r256(sizeof(Seg<double>) * G) + r256(sizeof(Seg<float>) * G) + r256(sizeof(int) * ((size_t)blocks + gblocks)) +
-               r256(sizeof(KState) * (size_t)G * kMaxNR) + r256(sizeof(double) * 2 * NR * (size_t)blocks) + 256;
+    b.tables = r256(sizeof(Seg<double>) * G) + r256(sizeof(Seg<float>) * G) + r256(map_bytes(G, blocks, gblocks)) +
+               r256(sizeof(KState) * (size_t)G * kMaxNR * (fold ? 3 : 1)) + r256(sizeof(double) * (fold ? 4 : 2) * NR * (size_t)blocks) + 256;
     b.vec64 = sizeof(double) * (size_t)total * (refine ? 5 : 11) + 1024;
     b.vec32 = refine ? sizeof(float) * (size_t)total * 10 + 1024 : 0;
     b.pack = sizeof(PackEntry) * (size_t)G * NR + sizeof(int) * (size_t)blocks * NR + 512;
@@ -441,7 +459,7 @@ static BatchBytes batch_bytes(int G, int blocks, int gblocks, int64_t total, int
 // One operator with NR right-hand sides.
 static BatchBytes batch_bytes1(const Op* op, int NR, bool refine) {
     const int nb = row_blocks(op);
-    return batch_bytes(1, nb, std::max(nb, op->ngt), (op->D * NR + 63) & ~int64_t(63), NR, refine);
+    return batch_bytes(1, nb, std::max(nb, op->ngt), (op->D * NR + 63) & ~int64_t(63), NR, refine, fold_fins(nb, NR));
 }
 
 // Grow the context's workspaces to what a batch of one operator with NR
@@ -473,7 +491,7 @@ static void run_batch(Ctx* ctx, const std::vector<Group>& groups, const std::vec
     std::vector<int64_t> off(G);
     std::vector<int> b0(G), nb(G), ng(G);
     int64_t total = 0;
-    int blocks = 0, gblocks = 0;
+    int blocks = 0, gblocks = 0, most = 0;
     for (int g = 0; g < G; ++g) {
         off[g] = total;
         total += groups[g].op->D * NR;
@@ -483,14 +501,16 @@ static void run_batch(Ctx* ctx, const std::vector<Group>& groups, const std::vec
         ng[g] = grp_blocks(by_tile, groups[g].op->ngt, nb[g]);
         blocks += nb[g];
         gblocks += ng[g];
+        most = std::max(most, nb[g]);
     }
+    const bool fold = fold_fins(most, NR), fuse = fuse_iterations(fold, NR);
     // device tables: segments (one per precision), block map, states, partials.
     // The FP64 and FP32 segments of a group share one state record per rhs.
     const int nstate = G * kMaxNR;
     if (nstate > Ctx::kHostStates) throw ArgError("batch too large");
-    const size_t part_stride = 2 * NR;
+    const size_t part_stride = (fold ? 4 : 2) * NR;
     auto r256 = [](size_t n) { return (n + 255) & ~size_t(255); };
-    const BatchBytes bb = batch_bytes(G, blocks, gblocks, total, NR, refine);
+    const BatchBytes bb = batch_bytes(G, blocks, gblocks, total, NR, refine, fold);
     const size_t bytes_tables = bb.tables;
     char* tb = reinterpret_cast<char*>(ctx->workspace("tables", bytes_tables));
     char* const tb_end = tb + bytes_tables;
@@ -502,23 +522,24 @@ static void run_batch(Ctx* ctx, const std::vector<Group>& groups, const std::vec
     };
     auto* segs64 = reinterpret_cast<Seg<double>*>(carve(sizeof(Seg<double>) * G));
     auto* segs32 = reinterpret_cast<Seg<float>*>(carve(sizeof(Seg<float>) * G));
-    int* bseg = reinterpret_cast<int*>(carve(sizeof(int) * ((size_t)blocks + gblocks)));   // two block maps
-    KState* sts = reinterpret_cast<KState*>(carve(sizeof(KState) * nstate));
+    int* bseg = reinterpret_cast<int*>(carve(map_bytes(G, blocks, gblocks)));   // block maps
+    KState* sts = reinterpret_cast<KState*>(carve(sizeof(KState) * nstate * (fold ? 3 : 1)));
+    const int64_t sst = fold ? nstate : 0;
     double* part = reinterpret_cast<double*>(carve(sizeof(double) * part_stride * blocks));
 
     std::vector<Seg<double>> h64(G);
     std::vector<Seg<float>> h32(G);
     for (int g = 0; g < G; ++g) {
         const int nr = (int)groups[g].inst.size();
-        fill_seg(h64[g], groups[g].op, off[g], nb[g], nr, sts + g * kMaxNR, part + part_stride * b0[g]);
-        fill_seg(h32[g], groups[g].op, off[g], nb[g], nr, sts + g * kMaxNR, part + part_stride * b0[g]);
+        fill_seg(h64[g], groups[g].op, off[g], nb[g], nr, sts + g * kMaxNR, part + part_stride * b0[g], sst);
+        fill_seg(h32[g], groups[g].op, off[g], nb[g], nr, sts + g * kMaxNR, part + part_stride * b0[g], sst);
         h64[g].m = h32[g].m = groups[g].m;
         h64[g].n = h32[g].n = groups[g].n;
     }
-    const std::vector<int> hb = block_map(nb, ng);
+    const std::vector<int> hb = G > 1 ? block_map(nb, ng) : std::vector<int>();
     HIPCHK(hipMemcpyAsync(segs64, h64.data(), sizeof(Seg<double>) * G, hipMemcpyHostToDevice, st));
     if (refine) HIPCHK(hipMemcpyAsync(segs32, h32.data(), sizeof(Seg<float>) * G, hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(bseg, hb.data(), sizeof(int) * hb.size(), hipMemcpyHostToDevice, st));
+    if (G > 1) HIPCHK(hipMemcpyAsync(bseg, hb.data(), sizeof(int) * hb.size(), hipMemcpyHostToDevice, st));
 
     // workspace vectors, each `total` entries: FP64 b x r r0 p v s t y z tmp;
     // mixed: FP64 b x r t tmp and FP32 x r r0 p v s t y z tmp.
@@ -565,14 +586,14 @@ static void run_batch(Ctx* ctx, const std::vector<Group>& groups, const std::vec
     int sweeps = 0;
     for (auto& g : groups)
         if (g.op->precond == CPM_PRECOND_JACOBI) sweeps = std::max(sweeps, g.op->precond_iters);
-    const LaunchCfg<double> c64{segs64, bseg, blocks, gblocks, G, st, sweeps, grp};
-    const LaunchCfg<float> c32{segs32, bseg, blocks, gblocks, G, st, sweeps, grp};
-    KState* hs = ctx->host_states;
+    const LaunchCfg<double> c64{segs64, h64.data(), bseg, blocks, gblocks, G, st, sweeps, fold, fuse, grp};
+    const LaunchCfg<float> c32{segs32, h32.data(), bseg, blocks, gblocks, G, st, sweeps, fold, fuse, grp};
     const double delta = o.update_delta > 0 ? std::min(o.update_delta, 0.999) : kDefaultUpdateDelta;
     launch_reset_states(sts, nstate, o.tol * o.tol, o.max_iters, delta * delta, st);
 
     // Iterations are queued in growing chunks; every kernel skips instances
     // that have stopped, so the host only looks at the states between chunks.
+    KState* hs = ctx->host_states;
     auto poll = [&](bool& run, bool& restart) {
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(hs, sts, sizeof(KState) * nstate, hipMemcpyDeviceToHost, st));
@@ -593,42 +614,28 @@ static void run_batch(Ctx* ctx, const std::vector<Group>& groups, const std::vec
     // (never inside the allocation-free entry point: instantiating a graph allocates)
     const bool graph = !ctx->arena && use_graph(refine && G == 1);
     IterGraph ig;
-    if (!refine) {
-        Launch<double, NR>::init(c64, V64.b, V64.x, V64.r, V64.r0, V64.p, V64.v);
-        auto four = [&] {
-            for (int c = 0; c < 4; ++c) Launch<double, NR>::iteration(c64, V64, false, MixVec{});
-        };
-        for (;;) {
-            for (int c = 0; c < chunk; c += 4) {
-                if (graph) ig.run(st, four);
-                else four();
-            }
-            poll(run, restart);
-            if (restart) {   // rare: handled between chunks, the other instances wait
-                Launch<double, NR>::restart(c64, V64);
-                continue;
-            }
-            if (!run) break;
-            chunk = std::min(chunk * 2, 64);
-        }
+    const MixVec mv{V64.x, V64.r, V64.b, V64.tmp};
+    auto iterations = [&](int n) {
+        if (refine) Launch<float, NR>::iterations(c32, V32, true, mv, n);
+        else Launch<double, NR>::iterations(c64, V64, false, MixVec{}, n);
+    };
+    if (refine) {
+        MixedLaunch<NR>::start(c64, V64.b, V64.x, V64.r);
+        MixedLaunch<NR>::down(c64, V64.r, V32);
     } else {
-        double* x64 = V64.x;
-        double* r64 = V64.r;
-        MixedLaunch<NR>::start(c64, V64.b, x64, r64);
-        MixedLaunch<NR>::down(c64, r64, V32);
-        const MixVec mv{x64, r64, V64.b, V64.tmp};
-        auto four = [&] {
-            for (int c = 0; c < 4; ++c) Launch<float, NR>::iteration(c32, V32, true, mv);
-        };
-        for (;;) {
-            for (int c = 0; c < chunk; c += 4) {
-                if (graph) ig.run(st, four);
-                else four();
-            }
-            poll(run, restart);
-            if (!run) break;
-            chunk = std::min(chunk * 2, 64);
+        Launch<double, NR>::init(c64, V64.b, V64.x, V64.r, V64.r0, V64.p, V64.v);
+    }
+    for (;;) {
+        if (graph)
+            for (int c = 0; c < chunk; c += 4) ig.run(st, [&] { iterations(4); });
+        else iterations(chunk);
+        poll(run, restart);
+        if (restart) {   // rare: handled between chunks, the other instances wait
+            Launch<double, NR>::restart(c64, V64);
+            continue;
         }
+        if (!run) break;
+        chunk = std::min(chunk * 2, 64);
     }
     hipLaunchKernelGGL(k_pack, dim3((unsigned)pb.size()), dim3(256), 0, st, dpe, dpb, V64.x, (float*)nullptr, 0);
     HIPCHK(hipGetLastError());
@@ -664,23 +671,25 @@ static void run_stream(Ctx* ctx, Op* op, const std::vector<const double*>& rhs, 
     const int blocks = G * nb;
     const int nstate = G * kMaxNR;
     if (nstate > Ctx::kHostStates) throw ArgError("too many lanes");
+    const bool fold = fold_fins(nb, NR), fuse = fuse_iterations(fold, NR);
+    const int64_t sst = fold ? nstate : 0;
     grp_refresh_override();
     const int ng = grp_blocks(grp_gather<float, NR>(op->ngt), op->ngt, nb);
     const int gblocks = G * ng;
     const int64_t seg_total = (D * NR + 63) & ~int64_t(63);   // vector entries of one segment
     const int64_t total = seg_total * G;
     auto r256 = [](size_t k) { return (k + 255) & ~size_t(255); };
-    const size_t part_stride = 2 * NR;
-    const size_t bytes = r256(sizeof(Seg<double>) * G) + r256(sizeof(Seg<float>) * G) + r256(sizeof(int) * ((size_t)blocks + gblocks)) + r256(sizeof(int) * blocks) +
-                         r256(sizeof(KState) * nstate) + r256(sizeof(double) * part_stride * blocks) +
+    const size_t part_stride = (fold ? 4 : 2) * NR;
+    const size_t bytes = r256(sizeof(Seg<double>) * G) + r256(sizeof(Seg<float>) * G) + r256(map_bytes(G, blocks, gblocks)) + r256(sizeof(int) * blocks) +
+                         r256(sizeof(KState) * nstate * (fold ? 3 : 1)) + r256(sizeof(double) * part_stride * blocks) +
                          r256(sizeof(PackEntry) * 4) + 256;
     char* tb = reinterpret_cast<char*>(ctx->workspace("stream_tables", bytes));
     auto carve = [&](size_t k) { char* p = tb; tb += r256(k); return p; };
     auto* seg64 = reinterpret_cast<Seg<double>*>(carve(sizeof(Seg<double>) * G));
     auto* seg32 = reinterpret_cast<Seg<float>*>(carve(sizeof(Seg<float>) * G));
-    int* bseg = reinterpret_cast<int*>(carve(sizeof(int) * ((size_t)blocks + gblocks)));   // two block maps
+    int* bseg = reinterpret_cast<int*>(carve(map_bytes(G, blocks, gblocks)));   // block maps
     int* bzero = reinterpret_cast<int*>(carve(sizeof(int) * blocks));   // all zero: one pack entry
-    KState* sts = reinterpret_cast<KState*>(carve(sizeof(KState) * nstate));
+    KState* sts = reinterpret_cast<KState*>(carve(sizeof(KState) * nstate * (fold ? 3 : 1)));
     double* part = reinterpret_cast<double*>(carve(sizeof(double) * part_stride * blocks));
     PackEntry* dpe = reinterpret_cast<PackEntry*>(carve(sizeof(PackEntry) * 4));
     std::vector<int> nr0(G);
@@ -689,13 +698,14 @@ static void run_stream(Ctx* ctx, Op* op, const std::vector<const double*>& rhs, 
     std::vector<int> hz(blocks, 0);
     for (int g = 0; g < G; ++g) {
         nr0[g] = std::min(NR, n - g * NR);
-        fill_seg(h64[g], op, g * seg_total, nb, nr0[g], sts + g * kMaxNR, part + part_stride * g * nb);
-        fill_seg(h32[g], op, g * seg_total, nb, nr0[g], sts + g * kMaxNR, part + part_stride * g * nb);
+        fill_seg(h64[g], op, g * seg_total, nb, nr0[g], sts + g * kMaxNR, part + part_stride * g * nb, sst);
+        fill_seg(h32[g], op, g * seg_total, nb, nr0[g], sts + g * kMaxNR, part + part_stride * g * nb, sst);
     }
-    const std::vector<int> hb = block_map(std::vector<int>((size_t)G, nb), std::vector<int>((size_t)G, ng));
+    const std::vector<int> hb =
+        G > 1 ? block_map(std::vector<int>((size_t)G, nb), std::vector<int>((size_t)G, ng)) : std::vector<int>();
     HIPCHK(hipMemcpyAsync(seg64, h64.data(), sizeof(Seg<double>) * G, hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(seg32, h32.data(), sizeof(Seg<float>) * G, hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(bseg, hb.data(), sizeof(int) * hb.size(), hipMemcpyHostToDevice, st));
+    if (G > 1) HIPCHK(hipMemcpyAsync(bseg, hb.data(), sizeof(int) * hb.size(), hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(bzero, hz.data(), sizeof(int) * blocks, hipMemcpyHostToDevice, st));
     Vecs<double> V64{};
     Vecs<float> V32{};
@@ -750,14 +760,14 @@ static void run_stream(Ctx* ctx, Op* op, const std::vector<const double*>& rhs, 
         }
     HIPCHK(hipMemcpyAsync(sts, hst.data(), sizeof(KState) * nstate, hipMemcpyHostToDevice, st));
     int sweeps = op->precond == CPM_PRECOND_JACOBI ? op->precond_iters : 0;
-    const LaunchCfg<float> c32{seg32, bseg, blocks, gblocks, G, st, sweeps, op->ngt};
+    const LaunchCfg<float> c32{seg32, h32.data(), bseg, blocks, gblocks, G, st, sweeps, fold, fuse, op->ngt};
     const MixVec mv{V64.x, V64.r, V64.b, V64.tmp};
     KState* hs = ctx->host_states;
     int done = 0;
     const bool graph = use_graph();
     IterGraph ig;
     auto iterations = [&] {
-        for (int c = 0; c < 16; ++c) Launch<float, NR>::iteration(c32, V32, true, mv);
+        Launch<float, NR>::iterations(c32, V32, true, mv, 16);
     };
     while (done < n) {
         if (graph) ig.run(st, iterations);
@@ -983,7 +993,7 @@ void multiply(Op* op, const double* dx, double* dy, double m, double n) {
     double* w = ctx->workspace("mul_tmp", sizeof(double) * op->D * 3);
     double *xi = w, *yi = w + op->D, *tmp = w + 2 * op->D;
     grp_refresh_override();
-    LaunchCfg<double> c{dseg, dbseg, nblocks, grp_blocks(grp_gather<double, 1>(op->ngt), op->ngt, nblocks), 1, st, 0, op->ngt};
+    LaunchCfg<double> c{dseg, &h, dbseg, nblocks, grp_blocks(grp_gather<double, 1>(op->ngt), op->ngt, nblocks), 1, st, 0, false, false, op->ngt};
     if (op->perm.p) {   // caller order -> internal order and back
         hipLaunchKernelGGL(k_pack, dim3(nblocks), dim3(256), 0, st, dpe, dbseg, xi, (float*)nullptr, 1);
         Launch<double, 1>::apply(c, xi, tmp, yi);
@@ -1021,7 +1031,7 @@ static void profile_egather_t(Op* op, int G, int reps, double* avg_ms, double* b
     T* xs = reinterpret_cast<T*>(ctx->workspace("prof_x", vec_bytes * nbuf));
     T* ys = reinterpret_cast<T*>(ctx->workspace("prof_y", vec_bytes * nbuf));
     HIPCHK(hipMemsetAsync(xs, 0, vec_bytes * nbuf, st));
-    LaunchCfg<T> c{dseg, dbseg, nblocks * G, ng * G, G, st, 0, op->ngt};
+    LaunchCfg<T> c{dseg, h.data(), dbseg, nblocks * G, ng * G, G, st, 0, false, false, op->ngt};
     auto buf = [&](T* b, int r) { return b + (size_t)(r % nbuf) * seg_total * G; };
     // the gather the iterations launch: of P^-1 x unless Jacobi sweeps follow the first
     const bool fly = !(op->precond == CPM_PRECOND_JACOBI && op->precond_iters > 1);
@@ -1143,7 +1153,7 @@ static PackEntry pack_out(double* dst) { PackEntry e{}; e.dst = dst; return e; }
 // apply kernel with tmp = x, the identity rows from the held Lfull rows.
 static void explicit_diffusion(Op* op, const StepTables& t, int k, double c, const double* x, double* z) {
     const hipStream_t st = op->ctx->stream;
-    LaunchCfg<double> cfg{t.seg + k, t.bseg, t.nblocks, t.nblocks, 1, st, 0};
+    LaunchCfg<double> cfg{t.seg + k, nullptr, t.bseg, t.nblocks, t.nblocks, 1, st, 0};
     launch_lfinish_plain<double>(cfg, x, x, z);
     if (op->nh > 0)
         hipLaunchKernelGGL(k_held_apply, dim3((unsigned)((op->nh + 255) / 256)), dim3(256), 0, st, op->nh, op->hw,
@@ -1152,8 +1162,8 @@ static void explicit_diffusion(Op* op, const StepTables& t, int k, double c, con
 }
 
 static void extension(Op* op, const StepTables& t, const double* z, double* y) {
-    LaunchCfg<double> cfg{t.seg, t.bseg, t.nblocks, grp_blocks(grp_gather<double, 1>(op->ngt), op->ngt, t.nblocks), 1,
-                          op->ctx->stream, 0, op->ngt};
+    LaunchCfg<double> cfg{t.seg, nullptr, t.bseg, t.nblocks, grp_blocks(grp_gather<double, 1>(op->ngt), op->ngt, t.nblocks), 1,
+                          op->ctx->stream, 0, false, false, op->ngt};
     launch_egather<double, 1>(cfg, z, y);
 }
 
@@ -1406,7 +1416,7 @@ struct Server : ServerBase {
         const int zn = (int)((cap + kBlock - 1) / kBlock);   // no request has more blocks
         auto r256 = [](size_t k) { return (k + 255) & ~size_t(255); };
         const size_t sseg = r256(sizeof(Seg<float>) * std::max<size_t>(reqs.size(), 1));
-        const size_t smap = r256(sizeof(int) * (size_t)std::max(blocks + gblocks, 1));   // two block maps
+        const size_t smap = r256(sizeof(int) * (size_t)std::max(blocks + 2 * gblocks, 1));   // block maps
         const size_t spart = r256(sizeof(double) * 2 * NR * std::max(blocks, 1));
         const size_t spack = r256(sizeof(PackEntry));
         const size_t szero = r256(sizeof(int) * zn);
@@ -1525,9 +1535,9 @@ struct Server : ServerBase {
         const hipStream_t st = ctx->stream;
         const Vecs<float> V32{nullptr, v32(0), v32(1), v32(2), v32(3), v32(4), v32(5), v32(6), v32(7), v32(8), v32(9)};
         const MixVec mv{v64(1), v64(2), v64(0), v64(4)};
-        const LaunchCfg<float> c{d_segs, d_bseg, nblocks, gblocks, (int)reqs.size(), st, 0, grp};
+        const LaunchCfg<float> c{d_segs, nullptr, d_bseg, nblocks, gblocks, (int)reqs.size(), st, 0, false, false, grp};
         Vecs<float> w = V32;
-        for (int i = 0; i < iters; ++i) Launch<float, NR>::iteration(c, w, true, mv);
+        Launch<float, NR>::iterations(c, w, true, mv, iters);
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(ctx->host_states, states.template as<KState>(), sizeof(KState) * (size_t)slots * kMaxNR,
                               hipMemcpyDeviceToHost, st));
@@ -1661,7 +1671,7 @@ struct Server64 : ServerBase {
         }
         auto r256 = [](size_t k) { return (k + 255) & ~size_t(255); };
         const size_t sseg = r256(sizeof(Seg<double>) * std::max<size_t>(reqs.size(), 1));
-        const size_t smap = r256(sizeof(int) * (size_t)std::max(blocks + gblocks, 1));   // two block maps
+        const size_t smap = r256(sizeof(int) * (size_t)std::max(blocks + 2 * gblocks, 1));   // block maps
         const size_t spart = r256(sizeof(double) * 2 * NR * std::max(blocks, 1));
         const size_t need = sseg + smap + spart;
         if (need > tables_bytes) {
@@ -1705,7 +1715,7 @@ struct Server64 : ServerBase {
         Seg<double> h{};
         fill_seg(h, op, off, nb, nrhs, sts, i_part());
         HIPCHK(hipMemcpyAsync(i_seg(), &h, sizeof(h), hipMemcpyHostToDevice, st));
-        const LaunchCfg<double> c1{i_seg(), nullptr, nb, nb, 1, st, 0, 0};   // no gather
+        const LaunchCfg<double> c1{i_seg(), &h, nullptr, nb, nb, 1, st, 0, false, false, 0};   // no gather
         Launch<double, NR>::init(c1, v64(0), v64(1), v64(2), v64(3), v64(4), v64(5));
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(st));
@@ -1747,8 +1757,8 @@ struct Server64 : ServerBase {
         if (dirty) rebuild();
         const hipStream_t st = ctx->stream;
         Vecs<double> V{v64(0), v64(1), v64(2), v64(3), v64(4), v64(5), v64(6), v64(7), v64(8), v64(9), v64(10)};
-        const LaunchCfg<double> c{d_segs, d_bseg, nblocks, gblocks, (int)reqs.size(), st, 0, grp};
-        for (int i = 0; i < iters; ++i) Launch<double, NR>::iteration(c, V, false, MixVec{});
+        const LaunchCfg<double> c{d_segs, nullptr, d_bseg, nblocks, gblocks, (int)reqs.size(), st, 0, false, false, grp};
+        Launch<double, NR>::iterations(c, V, false, MixVec{}, iters);
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(ctx->host_states, states.template as<KState>(), sizeof(KState) * (size_t)slots * kMaxNR,
                               hipMemcpyDeviceToHost, st));

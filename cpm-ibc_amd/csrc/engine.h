@@ -127,8 +127,10 @@ struct Seg {
     int precond;         // CPM_PRECOND_*
     int precond_iters;   // Jacobi sweeps
     T dinv, tinv;        // FP32: 1 / (m + ldu n) (tensor-product format) and 1 / (m - n), for P^-1
-    KState* st;          // nr states
-    double* part;        // [2 * NR][nblocks] partial sums of the last reducing kernel
+    KState* st;          // nr states (kMaxNR places); with folded finalisers, three copies sst apart
+    int64_t sst;         // (after the loop test, after alpha, after omega), 0: one copy
+    double* part;        // [2 * NR][nblocks] partial sums of the last reducing kernel; with folded
+                         // finalisers [4 * NR][nblocks], xrupdate's in the second half
 };
 
 void hip_check(hipError_t e, const char* what);

@@ -4,16 +4,29 @@
 
 namespace cpmgpu {
 
+// The segments of a fused kernel: the table and a block map, or the only
+// segment by value.
+template <typename T>
+struct SegArg {
+    const Seg<T>* segs;
+    const int* bseg;
+    Seg<T> one;
+};
+
 template <typename T>
 struct LaunchCfg {
     const Seg<T>* segs;    // device segment table
+    const Seg<T>* first;   // its first entry on the host
     const int* bseg;       // device block maps (segment | block << kSegBits), nblocks entries segment by
-                           // segment, then gblocks round-robin over the segments (the E gathers')
+                           // segment, gblocks round-robin over the segments (the E gathers'), gblocks
+                           // segment by segment (the refinement lanes' gathers'); not read where nseg = 1
     int nblocks;
     int gblocks;           // workgroups of an E gather (grp_blocks)
     int nseg;
     hipStream_t stream;
     int jacobi_sweeps;     // largest precond_iters over Jacobi-preconditioned segments (0: none)
+    bool fold = false;     // the finalisers run inside the kernels that need them (Seg::sst set)
+    bool fuse = false;     // ... and pupdate and supdate inside the gathers and lfinish, where those allow it
     int grp = 0;           // fewest shared-stencil tiles of the segments' operators (0: some have none)
 };
 
@@ -49,9 +62,11 @@ struct MixVec {
 template <typename T, int NR>
 struct Launch {
     static void init(const LaunchCfg<T>& c, const T* b, T* x, T* r, T* r0, T* p, T* v);
-    // mixed: FP32 recurrence whose lanes take FP64 refinement steps in place
+    // n iterations; mixed: FP32 recurrence whose lanes take FP64 refinement steps in place
     // (mv holds the FP64 vectors); otherwise the reference's FP64 loop
-    static void iteration(const LaunchCfg<T>& c, Vecs<T>& w, bool mixed, const MixVec& mv);
+    static void iterations(const LaunchCfg<T>& c, Vecs<T>& w, bool mixed, const MixVec& mv, int n);
+    template <bool FOLD>
+    static void iteration(const LaunchCfg<T>& c, Vecs<T>& w, bool mixed, const MixVec& mv, bool first);
     static void restart(const LaunchCfg<T>& c, Vecs<T>& w);
     // y = A x; lanes = status mask restricting the work to instances with such a lane (0: all)
     static void apply(const LaunchCfg<T>& c, const T* x, T* tmp, T* y, unsigned lanes = 0);

@@ -157,11 +157,9 @@ __device__ void block_partials(const double (&v)[NV][NR], double* part, int lb, 
     }
 }
 
-constexpr int kXcdRun = CPMGPU_XCD_RUN;        // vector kernels
-constexpr int kGatherRun = CPMGPU_GATHER_RUN;  // E gathers
-constexpr int kLfinishRun = CPMGPU_LFINISH_RUN;
+constexpr int kXcdRun = CPMGPU_XCD_RUN;
 
-template <int kXcdRun, typename T>
+template <typename T>
 __device__ __forceinline__ const Seg<T>& seg_of(const Seg<T>* __restrict__ segs, const int* __restrict__ bseg, int& lb, int64_t& row) {
     // Workgroups are dispatched to the 8 XCDs round-robin (workgroup b to XCD
     // b mod 8).  Renumber them so that each XCD takes runs of kXcdRun
@@ -186,6 +184,14 @@ __device__ __forceinline__ const Seg<T>& seg_of(const Seg<T>* __restrict__ segs,
     lb = e >> kSegBits;
     row = (int64_t)lb * kBlock + threadIdx.x;
     return segs[e & (kMaxSegs - 1)];
+}
+// ... of a kernel that takes the only segment as an argument where the launch
+// has one (ONE): the fields come with the kernel's arguments, one dependent
+// load less than through the table.
+template <bool ONE, typename T>
+__device__ __forceinline__ const Seg<T>& seg_of(const SegArg<T>& a, int& lb, int64_t& row) {
+    const Seg<T>& t = seg_of(a.segs, ONE ? nullptr : a.bseg, lb, row);
+    return ONE ? a.one : t;
 }
 
 // Lane masks: bit s set = act on lanes whose status is s.
@@ -236,10 +242,11 @@ struct LaneStat {
     }
 };
 template <int NR, typename T>
-__device__ __forceinline__ LaneStat<NR> lane_stat(const Seg<T>& sg, bool valid = true) {
+__device__ __forceinline__ LaneStat<NR> lane_stat(const Seg<T>& sg, bool valid = true, int copy = 0) {
     LaneStat<NR> L;
+    const KState* st = sg.st + (int64_t)copy * sg.sst;
 #pragma unroll
-    for (int k = 0; k < NR; ++k) L.s[k] = valid ? ldg(&sg.st[k].status) : 0;
+    for (int k = 0; k < NR; ++k) L.s[k] = valid ? ldg(&st[k].status) : 0;
     L.nr = valid ? sg.nr : 0;
     return L;
 }
@@ -635,23 +642,100 @@ __device__ __forceinline__ void lds_fill_rows(const FillIdx<LR>& f, const T* xb,
     __syncthreads();
 }
 
-// One shared-stencil tile of E x: thread t takes the item at place
-// tile kBlock + t.
-// Tile `tile` of op: ob[row] = (E x)_row from xb (both with NR values per
-// row).  FLY: xb holds p (or s) and the tile gathers y = P^-1 p (z = P^-1 s)
-// with the preconditioner of segment *pre, formed as the rows go into LDS.
-template <typename T, int NR, int LR, bool FLY, typename V>
-__device__ __forceinline__ void egather_grp_tile(const OpView<T>& op, const Seg<T>* pre, int tile, const T* xb, T* ob,
-                                                 const LdsRows<V>& lrows) {
+// Where a tile's x rows come from: load(row) issues a row's loads, value()
+// forms the gathered row from them (ident: an identity or no-diagonal row).
+// SrcPlain: x itself, or with FLY P^-1 x (x is p or s of an iteration that
+// forms y and z where it reads them) with the preconditioner of segment *sg.
+template <typename T, int NR, bool FLY>
+struct SrcPlain {
+    typedef typename VT<T, NR>::type V;
+    typedef V Raw;
+    const Seg<T>* sg;
+    const T* x;
+    __device__ __forceinline__ Raw load(int64_t row) const { return vload<T, NR>(x + (size_t)row * NR); }
+    __device__ __forceinline__ V value(const Raw& v, int64_t row, bool ident) const {
+        if constexpr (FLY) return precond_row<T, NR, true>(*sg, row, ident ? ROW_IDENTITY : 0, v);
+        else return v;
+    }
+};
+// P^-1 of the direction that pupdate would store: p = (p - w v) beta + r on
+// the running lanes (the same operations, so the same bits).
+template <typename T, int NR>
+struct SrcP {
+    typedef typename VT<T, NR>::type V;
+    struct Raw { V p, v, r; };
+    const Seg<T>* sg;
+    const T *p, *v, *r;
+    T beta[NR], w[NR];
+    unsigned run;
+    __device__ __forceinline__ Raw load(int64_t row) const {
+        const size_t i = (size_t)row * NR;
+        return Raw{vload<T, NR>(p + i), vload<T, NR>(v + i), vload<T, NR>(r + i)};
+    }
+    __device__ __forceinline__ V direction(const Raw& q) const {
+        V pv = q.p;
+#pragma unroll
+        for (int k = 0; k < NR; ++k) {
+            const T pk = (-w[k] * lane(q.v, k) + lane(q.p, k)) * beta[k] + lane(q.r, k);
+            if ((run >> k) & 1u) setlane(pv, k, pk);
+        }
+        return pv;
+    }
+    __device__ __forceinline__ V value(const Raw& q, int64_t row, bool ident) const {
+        return precond_row<T, NR, true>(*sg, row, ident ? ROW_IDENTITY : 0, direction(q));
+    }
+};
+// P^-1 of the residual that supdate would store: s = r - alpha v.
+template <typename T, int NR>
+struct SrcS {
+    typedef typename VT<T, NR>::type V;
+    struct Raw { V r, v; };
+    const Seg<T>* sg;
+    const T *r, *v;
+    T alpha[NR];
+    __device__ __forceinline__ Raw load(int64_t row) const {
+        const size_t i = (size_t)row * NR;
+        return Raw{vload<T, NR>(r + i), vload<T, NR>(v + i)};
+    }
+    __device__ __forceinline__ V residual(const Raw& q) const {
+        V sv;
+#pragma unroll
+        for (int k = 0; k < NR; ++k) setlane(sv, k, -alpha[k] * lane(q.v, k) + lane(q.r, k));
+        return sv;
+    }
+    __device__ __forceinline__ V value(const Raw& q, int64_t row, bool ident) const {
+        return precond_row<T, NR, true>(*sg, row, ident ? ROW_IDENTITY : 0, residual(q));
+    }
+};
+// A refinement lane's FP64 solution as pupdate would store it: x64 + x32 / scale.
+template <int NR>
+struct SrcX64 {
+    typedef double V;
+    struct Raw { double x; float d; };
+    const double* x;
+    const float* x32;
+    double scale;
+    __device__ __forceinline__ Raw load(int64_t row) const { return Raw{ldg(x + row), ldg(x32 + (size_t)row * NR)}; }
+    __device__ __forceinline__ V value(const Raw& q, int64_t, bool) const { return q.x + (double)q.d / scale; }
+};
+
+// One shared-stencil tile of E x, ob[row] = (E x)_row with x from src: thread
+// t takes the item at place tile kBlock + t.  mid(src), called once the loads
+// are under way, completes src (the scalars its values need) and says whether
+// to go on (the same on every thread).
+template <typename T, int NR, int LR, typename V, typename Src, typename Mid>
+__device__ __forceinline__ void egather_grp_tile(const OpView<T>& op, int tile, Src& src, T* ob, const LdsRows<V>& lrows,
+                                                 Mid&& mid) {
     // Loads in two rounds, each issued as soon as the previous one's values
     // are in: the list entries (first: the x rows wait on them), the item's
     // offsets and line words, all at fixed places of the tile; then the x
     // rows and the item's data.
-    static_assert(FillIdx<LR>::KF * kBlock == LR && LR == kGrpLdsRows, "a tile's list places are read whole");
-    FillIdx<LR> f;
-    f.nu = ldg(&op.gln[tile]);
+    constexpr int KF = FillIdx<LR>::KF;
+    static_assert(KF * kBlock == LR && LR == kGrpLdsRows, "a tile's list places are read whole");
+    int e[KF];
+    const int nu = ldg(&op.gln[tile]);
 #pragma unroll
-    for (int k = 0; k < FillIdx<LR>::KF; ++k) f.src[k] = ldg(&op.glr[(size_t)tile * LR + threadIdx.x + k * kBlock]);
+    for (int k = 0; k < KF; ++k) e[k] = ldg(&op.glr[(size_t)tile * LR + threadIdx.x + k * kBlock]);
     const int64_t NI = op.nitem;
     const int item = tile * kBlock + (int)threadIdx.x;
     const int a = ldg(&op.gofs[item]), b = ldg(&op.gofs[item + 1]);
@@ -672,15 +756,22 @@ __device__ __forceinline__ void egather_grp_tile(const OpView<T>& op, const Seg<
     ExcRow mx;
     T xval = (T)0;
     if (kind == 1) {   // issued before the weights: they need only the line words
-        const int e = m.pp[0];
-        exc_row_load(op.glx, e, mx);
-        xval = ldg(&op.xval[e]);
+        const int x = m.pp[0];
+        exc_row_load(op.glx, x, mx);
+        xval = ldg(&op.xval[x]);
     }
     grp_item_load(op, s0, m);   // kinds 0 and 1 (kind 1: slot s0's row and weights)
-    lds_fill_rows<T, NR, LR>(f, xb, lrows, [&](const V& v, int e) {
-        if constexpr (FLY) return precond_row<T, NR, true>(*pre, e & kListRowMask, (e >> kListPlainBit) & 1 ? ROW_IDENTITY : 0, v);
-        else return v;
-    });
+    typename Src::Raw buf[KF];
+#pragma unroll
+    for (int k = 0; k < KF; ++k)
+        if ((int)threadIdx.x + k * kBlock < nu) buf[k] = src.load(e[k] & kListRowMask);
+    if (!mid(src)) return;
+#pragma unroll
+    for (int k = 0; k < KF; ++k) {
+        const int u = (int)threadIdx.x + k * kBlock;
+        if (u < nu) lrows.store(u, src.value(buf[k], e[k] & kListRowMask, (e[k] >> kListPlainBit) & 1));
+    }
+    __syncthreads();
     if (kind == 0) {
         V acc[kGrpRows];
 #pragma unroll
@@ -698,9 +789,8 @@ __device__ __forceinline__ void egather_grp_tile(const OpView<T>& op, const Seg<
         for (int g = 0; g < kGrpRows; ++g)
             if (g < n) {
                 const int64_t r = m.pp[g];
-                V v = vload<T, NR>(xb + (size_t)r * NR);
-                if constexpr (FLY) v = precond_row<T, NR, true>(*pre, r, ldg(&op.flag[r]), v);
-                vstore<T, NR>(ob + (size_t)r * NR, v);
+                vstore<T, NR>(ob + (size_t)r * NR,
+                              src.value(src.load(r), r, ldg(&op.flag[r]) & (ROW_IDENTITY | ROW_NODIAG)));
             }
     }
 }
@@ -810,483 +900,6 @@ __device__ __forceinline__ typename VT<T, W>::type arow_tp(const Seg<T>& sg, int
     return res;
 }
 
-// ---------------------------------------------------------------- vector kernels
-template <typename T, int NR>
-__global__ __launch_bounds__(kBlock) void k_init(const Seg<T>* __restrict__ segs, const int* __restrict__ bseg, const T* b, T* x, T* r,
-                                                 T* r0, T* p, T* v) {
-    int lb;
-    int64_t row;
-    const Seg<T>& sg = seg_of<kXcdRun>(segs, bseg, lb, row);
-    double pv[1][NR];
-#pragma unroll
-    for (int k = 0; k < NR; ++k) pv[0][k] = 0.0;
-    if (row < sg.op.D) {
-        const size_t i = (size_t)(sg.off + row * NR);
-        auto bv = vload<T, NR>(b + i);
-        typename VT<T, NR>::type zero = (typename VT<T, NR>::type)(T)0;
-        vstore<T, NR>(r + i, bv);
-        vstore<T, NR>(r0 + i, bv);
-        vstore<T, NR>(x + i, zero);
-        vstore<T, NR>(p + i, zero);
-        vstore<T, NR>(v + i, zero);
-#pragma unroll
-        for (int k = 0; k < NR; ++k) pv[0][k] = (double)lane(bv, k) * (double)lane(bv, k);
-    }
-    block_partials<1, NR>(pv, sg.part, lb, sg.nblocks);
-}
-
-// RUN lanes: p = (p - w v) beta + r ; y = P^-1 p (fly: y is formed where it is read).
-// UPDATE lanes (mixed): x64 += x32 / scale ; x32 = 0.
-template <typename T, int NR>
-__global__ __launch_bounds__(kBlock) void k_pupdate(const Seg<T>* __restrict__ segs, const int* __restrict__ bseg, T* p, const T* v,
-                                                    const T* r, T* y, T* x, MixVec mv, int fly) {
-    int lb;
-    int64_t row;
-    const Seg<T>& sg = seg_of<kXcdRun>(segs, bseg, lb, row);
-    const auto L = lane_stat<NR>(sg);
-    if (row >= sg.op.D || !seg_any(L, M_STAGE1)) return;
-    const size_t i = (size_t)(sg.off + row * NR);
-    if (seg_any(L, M_RUN)) {
-        const uint8_t f = ldg(&sg.op.flag[row]);
-        auto pv = vload<T, NR>(p + i);
-        auto vv = vload<T, NR>(v + i);
-        auto rv = vload<T, NR>(r + i);
-        const unsigned run = L.of(M_RUN);
-#pragma unroll
-        for (int k = 0; k < NR; ++k) {   // a group owns kMaxNR states: every lane's load is valid
-            const T beta = (T)ldg(&sg.st[k].beta), w = (T)ldg(&sg.st[k].omega);
-            const T pk = (-w * lane(vv, k) + lane(pv, k)) * beta + lane(rv, k);   // p.Copy(-w,v,p); p*=beta; p+=r
-            if ((run >> k) & 1u) setlane(pv, k, pk);
-        }
-        vstore<T, NR>(p + i, pv);
-        if (!fly) vstore<T, NR>(y + i, prow_apply<T, NR>(prow_of(sg, row, f), prow_div(sg), pv));
-    }
-    if (std::is_same<T, float>::value && seg_any(L, M_UPDATE)) {
-        auto xv = vload<T, NR>(x + i);
-#pragma unroll
-        for (int k = 0; k < NR; ++k)
-            if (lane_in(L, k, M_UPDATE)) {
-                double* xd = mv.x64 + lm_at(sg, k, row);
-                stg(xd, ldg(xd) + (double)lane(xv, k) / ldg(&sg.st[k].scale));
-                setlane(xv, k, (T)0);
-            }
-        vstore<T, NR>(x + i, xv);
-    }
-}
-
-// tmp = E x.  Rows are independent; a thread owns one row and all NR rhs.
-// UPDATE lanes (mixed, first gather of the iteration): tmp64 = E64 x64.
-// E x for the instance segments.  Tiles with an LDS list copy their x rows
-// into LDS once and gather every stencil line from there; the other tiles
-// (lists longer than the LDS, or operators without tiles) read x directly.
-template <typename T, int NR>
-__global__ __launch_bounds__(kBlock) void k_egather(const Seg<T>* __restrict__ segs, const int* __restrict__ bseg, const T* x, T* out,
-                                                    unsigned lanes, MixVec mv) {
-    typedef typename VT<T, NR>::type V;
-    constexpr int LR = LdsTile<T, NR>::kRows;
-    __shared__ V lx[LR > 0 ? LR : 1];
-    const LdsRows<V> lrows{lx, LR > 0 ? LR : 1};
-    int lb;
-    int64_t row;
-    const Seg<T>& sg = seg_of<kGatherRun>(segs, bseg, lb, row);
-    if (lb >= sg.nblocks) return;   // a launch with more tiles (k_egather_upd's) than row blocks
-    const auto L = lane_stat<NR>(sg, lanes != 0);
-    if (lanes && !seg_any(L, lanes)) return;               // uniform per workgroup
-    const bool main = !lanes || seg_any(L, lanes & ~M_UPDATE);
-    const size_t i = (size_t)(sg.off + row * NR);
-    const T* xb = x + sg.off;
-    const int nu = (LR > 0 && main && sg.op.fmt == OP_TP && sg.op.tln) ? ldg(&sg.op.tln[lb]) : -1;
-    if (nu >= 0 && nu <= LR) {
-        // Loads in two rounds, each issued as soon as the previous one's
-        // values are in: the tile's list entries with the row's flag,
-        // exception record and weights (rows past the end read the last
-        // row's, unused), all unconditional; then the listed x rows with the
-        // row's LDS positions (a plain row's 16 line positions, or a moved
-        // row's exception record and extra value, in one register array) or
-        // an identity row's own x.  Then the LDS copy, the barrier and every
-        // stencil line from LDS.
-        FillIdx<LR> f;
-        lds_fill_index<LR>(sg.op.tlr + ldg(&sg.op.tlo[lb]), nu, f);
-        const bool act = row < sg.op.D;
-        const int64_t rr = act ? row : sg.op.D - 1;
-        const int64_t D = sg.op.D;
-        const int e = ldg(&sg.op.exc[rr]);
-        const uint8_t fl = ldg(&sg.op.flag[rr]);
-        TpRow<T> m;
-#pragma unroll
-        for (int q = 0; q < 12; ++q) m.w[q] = ldg(&sg.op.tpw[q * D + rr]);
-        const int kind = act ? ((fl & ROW_IDENTITY) ? 2 : (e < 0 ? 0 : 1)) : 3;
-        ExcRow mx;   // kind 0: words 0..15 are the line positions; kind 1: the exception record
-        T xval = (T)0;
-        V xi = (V)(T)0;
-        if (kind == 0) {
-#pragma unroll
-            for (int l = 0; l < 16; ++l) mx.pk[l] = ldg(&sg.op.tpl[l * D + row]);
-        } else if (kind == 1) {   // rows an interior boundary moved
-            exc_row_load(sg.op.tlx, e, mx);
-            xval = ldg(&sg.op.xval[e]);
-        } else if (kind == 2) {
-            xi = vload<T, NR>(xb + (size_t)row * NR);
-        }
-        lds_fill_rows<T, NR, LR>(f, xb, lrows, [](const V& v, int) { return v; });
-        if (act) {
-            V acc = (V)(T)0;
-#pragma unroll
-            for (int l = 0; l < 16; ++l) m.p[l] = mx.pk[l];
-            if (kind == 2) acc = xi;
-            else if (kind == 0) egather_tp_lds<T, V, NR>(m, lrows, acc);
-            else egather_grp_exc<T, V>(m.w, xval, mx, lrows, acc);
-            vstore<T, NR>(out + i, acc);
-        }
-    } else if (main && row < sg.op.D) {
-        vstore<T, NR>(out + i, erow<T, NR>(sg.op, row, xb, NR));
-    }
-}
-
-// FP64 gathers of the refinement lanes of FP32 segments: tmp64 = E64 x64 for
-// every lane in an UPDATE status (a launch of its own beside the FP32
-// gather, which then carries only FP32 work).  A lane's FP64 vectors are a
-// run of D values, the one-right-hand-side layout, so block lb gathers tile
-// lb of the operator's shared-stencil tiles for each such lane in turn;
-// operators without tiles read x64 directly, a row per thread.
-template <int NR>
-__global__ __launch_bounds__(kBlock) void k_egather_upd(const Seg<float>* __restrict__ segs, const int* __restrict__ bseg,
-                                                        MixVec mv) {
-    constexpr int LR = GrpTile<double, 1>::kRows;
-    static_assert(LR > 0, "FP64 shared-stencil tiles fit the LDS");
-    __shared__ double lx[LR];
-    const LdsRows<double> lrows{lx, LR};
-    int lb;
-    int64_t row;
-    const Seg<float>& sg = seg_of<kGatherRun>(segs, bseg, lb, row);
-    const auto L = lane_stat<NR>(sg);
-    if (!seg_any(L, M_UPDATE)) return;   // uniform per workgroup
-    if (sg.op64.ngt > 0) {
-        if (lb >= sg.op64.ngt) return;
-        bool first = true;
-        for (int k = 0; k < sg.nr; ++k)
-            if (lane_in(L, k, M_UPDATE)) {
-                if (!first) __syncthreads();   // the previous lane's LDS reads are done
-                first = false;
-                egather_grp_tile<double, 1, LR, false>(sg.op64, (const Seg<double>*)nullptr, lb, mv.x64 + lm_at(sg, k, 0),
-                                                       mv.tmp64 + lm_at(sg, k, 0), lrows);
-            }
-        return;
-    }
-    if (row >= sg.op.D) return;
-    for (int k = 0; k < sg.nr; ++k)
-        if (lane_in(L, k, M_UPDATE))
-            stg(&mv.tmp64[lm_at(sg, k, row)], erow<double, 1>(sg.op64, row, mv.x64 + lm_at(sg, k, 0), 1));
-}
-
-// E x for launches whose every segment has shared-stencil tiles: block lb of
-// a segment takes its tile lb.  32 KB of LDS and at most 128 VGPRs, so four
-// workgroups share a CU (a direct-read path for other segments, even out of
-// line, made the FP32 x 8 kernel spill).
-// FLY: x is p (or s) and the launch gathers y = P^-1 p (z = P^-1 s).
-template <typename T, int NR, int WPE, bool FLY>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) void k_egather_grp(
-    const Seg<T>* __restrict__ segs, const int* __restrict__ bseg, const T* x, T* out, unsigned lanes, MixVec mv) {
-    typedef typename VT<T, NR>::type V;
-    constexpr int LR = GrpTile<T, NR>::kRows;
-    static_assert(LR > 0, "shared-stencil tiles do not fit this value size");
-    __shared__ V lx[LR];
-    const LdsRows<V> lrows{lx, LR};
-    int lb;
-    int64_t row;
-    const Seg<T>& sg = seg_of<kGatherRun>(segs, bseg, lb, row);
-    const auto L = lane_stat<NR>(sg, lanes != 0);
-    if (lanes && !seg_any(L, lanes)) return;               // uniform per workgroup
-    const bool main = !lanes || seg_any(L, lanes & ~M_UPDATE);
-    if (main && lb < sg.op.ngt) egather_grp_tile<T, NR, LR, FLY>(sg.op, &sg, lb, x + sg.off, out + sg.off, lrows);
-}
-
-// out = A x from tmp = E x.  RED = 0: no reduction; 1: partial (other, out);
-// 2: partials (out, out), (out, other).
-// Mixed, RED = 1: UPDATE lanes r64 = b - A64 x64, partial (r64, r64).
-// Mixed, RED = 2: RESCALE lanes partial (r32, r32) (rv32 = r32).
-template <typename T, int NR, int RED>
-__global__ __launch_bounds__(kBlock) void k_lfinish(const Seg<T>* __restrict__ segs, const int* __restrict__ bseg, const T* x,
-                                                    const T* tmp, T* out, const T* other, const T* rv32,
-                                                    unsigned lanes, MixVec mv, int fly) {
-    int lb;
-    int64_t row;
-    const Seg<T>& sg = seg_of<kLfinishRun>(segs, bseg, lb, row);
-    const auto L = lane_stat<NR>(sg, lanes != 0);
-    if (lanes && !seg_any(L, lanes)) return;   // uniform per segment
-    constexpr int NV = RED == 2 ? 2 : 1;
-    double pv[NV][NR];
-#pragma unroll
-    for (int a = 0; a < NV; ++a)
-#pragma unroll
-        for (int k = 0; k < NR; ++k) pv[a][k] = 0.0;
-    if (row < sg.op.D) {
-        const size_t i = (size_t)(sg.off + row * NR);
-        if (!lanes || seg_any(L, lanes & ~(M_UPDATE | M_RESCALE))) {
-            typename VT<T, NR>::type res, ov;
-            if (sg.op.fmt == OP_TP) {   // every load that waits on no other in one round
-                TpLRow<T, NR> a;
-                arow_tp_load<T, NR>(sg.op, row, x + i, a);
-                if (RED > 0) ov = vload<T, NR>(other + i);
-                res = arow_tp<T, NR>(sg, row, a, tmp + sg.off, NR, fly);   // fly: x is p or s
-            } else {
-                auto xv = vload<T, NR>(x + i);
-                if (RED > 0) ov = vload<T, NR>(other + i);
-                if (fly) xv = precond_row<T, NR>(sg, row, ldg(&sg.op.flag[row]), xv);
-                res = arow<T, NR>(sg.op, sg.m, sg.n, row, xv, tmp + sg.off, NR);
-            }
-            vstore<T, NR>(out + i, res);
-            if (RED > 0) {
-#pragma unroll
-                for (int k = 0; k < NR; ++k) {
-                    const double rk = (double)lane(res, k);
-                    if (RED == 1) {
-                        pv[0][k] = (double)lane(ov, k) * rk;
-                    } else {
-                        pv[0][k] = rk * rk;
-                        pv[NV - 1][k] = rk * (double)lane(ov, k);
-                    }
-                }
-            }
-        }
-        if (std::is_same<T, float>::value && RED == 1 && seg_any(L, M_UPDATE)) {
-#pragma unroll
-            for (int k = 0; k < NR; ++k)   // constant indices keep pv in registers
-                if (k < sg.nr && lane_in(L, k, M_UPDATE)) {
-                    const size_t j = lm_at(sg, k, row);
-                    const double ax =
-                        arow<double, 1>(sg.op64, sg.m, sg.n, row, ldg(&mv.x64[j]), mv.tmp64 + lm_at(sg, k, 0), 1);
-                    const double rk = ldg(&mv.b64[j]) - ax;
-                    stg(&mv.r64[j], rk);
-                    pv[0][k] = rk * rk;
-                }
-        }
-        if (std::is_same<T, float>::value && RED == 2 && seg_any(L, M_RESCALE)) {
-            auto rr = vload<T, NR>(rv32 + i);
-#pragma unroll
-            for (int k = 0; k < NR; ++k)
-                if (lane_in(L, k, M_RESCALE)) {
-                    const double rk = (double)lane(rr, k);
-                    pv[0][k] = rk * rk;
-                    pv[NV - 1][k] = 0.0;
-                }
-        }
-    }
-    if (RED > 0) block_partials<NV, NR>(pv, sg.part, lb, sg.nblocks);
-}
-
-// RUN lanes: s = r - alpha v ; z = P^-1 s (fly: z is formed where it is read).
-// RESCALE lanes (mixed): r32 = r64 scale ; r0 = r32 ; p = v = 0.
-template <typename T, int NR>
-__global__ __launch_bounds__(kBlock) void k_supdate(const Seg<T>* __restrict__ segs, const int* __restrict__ bseg, T* r, T* v, T* s, T* z,
-                                                    T* r0, T* p, MixVec mv, int fly) {
-    int lb;
-    int64_t row;
-    const Seg<T>& sg = seg_of<kXcdRun>(segs, bseg, lb, row);
-    const auto L = lane_stat<NR>(sg);
-    if (row >= sg.op.D || !seg_any(L, M_STAGE2)) return;
-    const size_t i = (size_t)(sg.off + row * NR);
-    const uint8_t f = ldg(&sg.op.flag[row]);
-    auto rv = vload<T, NR>(r + i);
-    auto vv = vload<T, NR>(v + i);
-    if (seg_any(L, M_RUN)) {
-        typename VT<T, NR>::type sv;
-#pragma unroll
-        for (int k = 0; k < NR; ++k) {   // a group owns kMaxNR states: every lane's load is valid
-            const T a = (T)ldg(&sg.st[k].alpha);
-            setlane(sv, k, -a * lane(vv, k) + lane(rv, k));   // s.Copy(-alpha, v, r)
-        }
-        vstore<T, NR>(s + i, sv);
-        if (!fly) vstore<T, NR>(z + i, prow_apply<T, NR>(prow_of(sg, row, f), prow_div(sg), sv));
-    }
-    if (std::is_same<T, float>::value && seg_any(L, M_RESCALE)) {
-        auto r0v = vload<T, NR>(r0 + i);
-        auto pv = vload<T, NR>(p + i);
-#pragma unroll
-        for (int k = 0; k < NR; ++k)
-            if (lane_in(L, k, M_RESCALE)) {
-                const T rk = (T)(ldg(&mv.r64[lm_at(sg, k, row)]) * ldg(&sg.st[k].scale));
-                setlane(rv, k, rk);
-                setlane(r0v, k, rk);
-                setlane(pv, k, (T)0);
-                setlane(vv, k, (T)0);
-            }
-        vstore<T, NR>(r + i, rv);
-        vstore<T, NR>(r0 + i, r0v);
-        vstore<T, NR>(p + i, pv);
-        vstore<T, NR>(v + i, vv);
-    }
-}
-
-// Jacobi sweep `sweep` (>= 1) of RUN lanes: y += omega D^-1 (x - A y) on the
-// rows below dofs, with A y already in ay (GeneralizedBiCGStabSystem.h:366-378).
-template <typename T, int NR>
-__global__ __launch_bounds__(kBlock) void k_jacobi(const Seg<T>* __restrict__ segs, const int* __restrict__ bseg,
-                                                   const T* x, const T* ay, T* y, int sweep) {
-    int lb;
-    int64_t row;
-    const Seg<T>& sg = seg_of<kXcdRun>(segs, bseg, lb, row);
-    const auto L = lane_stat<NR>(sg);
-    if (sg.precond != 2 || sweep >= sg.precond_iters) return;
-    if (row >= sg.op.D - sg.op.nD || !seg_any(L, M_RUN)) return;
-    const size_t i = (size_t)(sg.off + row * NR);
-    const uint8_t f = ldg(&sg.op.flag[row]);
-    auto xv = vload<T, NR>(x + i);
-    auto av = vload<T, NR>(ay + i);
-    auto yv = vload<T, NR>(y + i);
-#pragma unroll
-    for (int k = 0; k < NR; ++k)
-        if (lane_in(L, k, M_RUN))
-            setlane(yv, k, lane(yv, k) + (T)kJacobiOmega * diag_inverse(sg, row, f, (T)(lane(xv, k) - lane(av, k))));
-    vstore<T, NR>(y + i, yv);
-}
-
-template <typename T, int NR>
-__global__ __launch_bounds__(kBlock) void k_xrupdate(const Seg<T>* __restrict__ segs, const int* __restrict__ bseg, T* x, const T* y,
-                                                     const T* z, T* r, const T* s, const T* t, const T* r0, int fly) {
-    int lb;
-    int64_t row;
-    const Seg<T>& sg = seg_of<kXcdRun>(segs, bseg, lb, row);
-    const auto L = lane_stat<NR>(sg);
-    if (!seg_any(L, M_RUN)) return;
-    double pv[2][NR];
-#pragma unroll
-    for (int k = 0; k < NR; ++k) { pv[0][k] = 0.0; pv[1][k] = 0.0; }
-    if (row < sg.op.D) {
-        const size_t i = (size_t)(sg.off + row * NR);
-        auto xv = vload<T, NR>(x + i);
-        auto yv = vload<T, NR>(y + i);   // fly: p
-        auto sv = vload<T, NR>(s + i);
-        auto tv = vload<T, NR>(t + i);
-        auto r0v = vload<T, NR>(r0 + i);
-        const uint8_t f = ldg(&sg.op.flag[row]);
-        // r is rewritten on every RUN lane: read only to keep the others
-        const unsigned run = L.of(M_RUN);
-        const bool all_run = run == (1u << NR) - 1u;
-        typename VT<T, NR>::type rv = all_run ? (typename VT<T, NR>::type)(T)0 : vload<T, NR>(r + i);
-        typename VT<T, NR>::type zv;
-        if (fly) {   // y = P^-1 p, z = P^-1 s
-            const PRow<T> pr = prow_of(sg, row, f);
-            const bool div = prow_div(sg);
-            yv = prow_apply<T, NR>(pr, div, yv);
-            zv = prow_apply<T, NR>(pr, div, sv);
-        } else {
-            zv = vload<T, NR>(z + i);
-        }
-#pragma unroll
-        for (int k = 0; k < NR; ++k) {   // a group owns kMaxNR states: every lane's load is valid
-            if (!((run >> k) & 1u)) continue;
-            const T a = (T)ldg(&sg.st[k].alpha), w = (T)ldg(&sg.st[k].omega);
-            T xk = a * lane(yv, k) + lane(xv, k);   // x.Copy(alpha, y, x)
-            xk = w * lane(zv, k) + xk;               // x.Copy(w, z, x)
-            T rk = -w * lane(tv, k) + lane(sv, k);   // r.Copy(-w, t, s)
-            setlane(xv, k, xk);
-            setlane(rv, k, rk);
-            pv[0][k] = (double)rk * (double)rk;
-            pv[1][k] = (double)lane(r0v, k) * (double)rk;
-        }
-        vstore<T, NR>(x + i, xv);
-        vstore<T, NR>(r + i, rv);
-    }
-    block_partials<2, NR>(pv, sg.part, lb, sg.nblocks);
-}
-
-// FP64 restart, BiCGStab.h:62-71: r = b - A x (A x already in ax), r0 = r; partial (r, r).
-template <typename T, int NR>
-__global__ __launch_bounds__(kBlock) void k_restart(const Seg<T>* __restrict__ segs, const int* __restrict__ bseg, const T* b,
-                                                    const T* ax, T* r, T* r0) {
-    int lb;
-    int64_t row;
-    const Seg<T>& sg = seg_of<kXcdRun>(segs, bseg, lb, row);
-    const auto L = lane_stat<NR>(sg);
-    if (!seg_any(L, M_RESTART)) return;
-    double pv[1][NR];
-#pragma unroll
-    for (int k = 0; k < NR; ++k) pv[0][k] = 0.0;
-    if (row < sg.op.D) {
-        const size_t i = (size_t)(sg.off + row * NR);
-        auto bv = vload<T, NR>(b + i);
-        auto av = vload<T, NR>(ax + i);
-        auto rv = vload<T, NR>(r + i);
-        auto r0v = vload<T, NR>(r0 + i);
-#pragma unroll
-        for (int k = 0; k < NR; ++k) {
-            if (!lane_in(L, k, M_RESTART)) continue;
-            T rk = lane(bv, k) - lane(av, k);
-            setlane(rv, k, rk);
-            setlane(r0v, k, rk);
-            pv[0][k] = (double)rk * (double)rk;
-        }
-        vstore<T, NR>(r + i, rv);
-        vstore<T, NR>(r0 + i, r0v);
-    }
-    block_partials<1, NR>(pv, sg.part, lb, sg.nblocks);
-}
-
-// ---------------------------------------------------------------- mixed precision start
-// x64 = 0, r64 = b ; partial (b, b)
-template <int NR>
-__global__ __launch_bounds__(kBlock) void k_mx_start(const Seg<double>* __restrict__ segs, const int* __restrict__ bseg, const double* b,
-                                                     double* x, double* r) {
-    int lb;
-    int64_t row;
-    const Seg<double>& sg = seg_of<kXcdRun>(segs, bseg, lb, row);
-    double pv[1][NR];
-#pragma unroll
-    for (int k = 0; k < NR; ++k) pv[0][k] = 0.0;
-    if (row < sg.op.D) {
-#pragma unroll
-        for (int k = 0; k < NR; ++k) {
-            const size_t j = lm_at(sg, k, row);
-            const double bk = b[j];
-            r[j] = bk;
-            x[j] = 0.0;
-            pv[0][k] = bk * bk;
-        }
-    }
-    block_partials<1, NR>(pv, sg.part, lb, sg.nblocks);
-}
-
-// FP32 start of the lanes in ST_RESCALE: r32 = r64 * scale, r0 = r32,
-// p = v = x32 = 0 ; partial (r32, r32).
-template <int NR>
-__global__ __launch_bounds__(kBlock) void k_mx_down(const Seg<double>* __restrict__ segs, const int* __restrict__ bseg, const double* r64,
-                                                    float* r, float* r0, float* p, float* v, float* x) {
-    int lb;
-    int64_t row;
-    const Seg<double>& sg = seg_of<kXcdRun>(segs, bseg, lb, row);
-    const auto L = lane_stat<NR>(sg);
-    if (!seg_any(L, M_RESCALE)) return;
-    double pv[1][NR];
-#pragma unroll
-    for (int k = 0; k < NR; ++k) pv[0][k] = 0.0;
-    if (row < sg.op.D) {
-        const size_t i = (size_t)(sg.off + row * NR);
-        auto ro = vload<float, NR>(r + i);
-        auto r0o = vload<float, NR>(r0 + i);
-        auto po = vload<float, NR>(p + i);
-        auto vo = vload<float, NR>(v + i);
-        auto xo = vload<float, NR>(x + i);
-#pragma unroll
-        for (int k = 0; k < NR; ++k) {
-            if (!lane_in(L, k, M_RESCALE)) continue;
-            const float rk = (float)(r64[lm_at(sg, k, row)] * ldg(&sg.st[k].scale));
-            setlane(ro, k, rk);
-            setlane(r0o, k, rk);
-            setlane(po, k, 0.0f);
-            setlane(vo, k, 0.0f);
-            setlane(xo, k, 0.0f);
-            pv[0][k] = (double)rk * (double)rk;
-        }
-        vstore<float, NR>(r + i, ro);
-        vstore<float, NR>(r0 + i, r0o);
-        vstore<float, NR>(p + i, po);
-        vstore<float, NR>(v + i, vo);
-        vstore<float, NR>(x + i, xo);
-    }
-    block_partials<1, NR>(pv, sg.part, lb, sg.nblocks);
-}
-
 // ---------------------------------------------------------------- finalisers
 enum FinKind : int {
     FIN_INIT = 0, FIN_ALPHA, FIN_OMEGA, FIN_ITER64, FIN_RESTART64, FIN_MX_START, FIN_MX_INIT, FIN_ITER_MX
@@ -1379,21 +992,15 @@ __device__ void fin_scalar(KState& s, const double* tot) {
     }
 }
 
-// One workgroup per segment: fixed-order sum of the producing kernel's
-// block partials, then the scalar recurrence for each active lane.
-template <typename T, int NR, int KIND>
-__global__ __launch_bounds__(kBlock) void k_fin(const Seg<T>* __restrict__ segs, int nseg) {
-    constexpr int NV = FinTraits<KIND>::NV;
-    constexpr unsigned M = FinTraits<KIND>::M;
-    // One workgroup per (segment, rhs lane): the lane's NV components over all
-    // block partials, U blocks per thread in flight at once (the partials were
-    // just written by another kernel, so every round costs a full memory
-    // latency), then a workgroup sum and the lane's scalar update.
-    const Seg<T>& sg = segs[blockIdx.x / NR];
-    const int k = (int)(blockIdx.x % NR);
-    if (k >= sg.nr || !lane_in(sg, k, M)) return;   // same test the producer used
+// ---------------------------------------------------------------- folded finalisers
+// A lane's components over all block partials of its segment, U blocks per
+// thread in flight at once (the partials were just written by another
+// kernel, so every round costs a full memory latency), then a workgroup sum
+// in a fixed order: thread 0 holds the totals.
+template <int NV, int NR, typename T>
+__device__ __forceinline__ void part_totals(const Seg<T>& sg, const double* part, int k, double (*red)[kBlock / 64],
+                                            double (&tot)[NV]) {
     constexpr int U = 8;
-    __shared__ double red[NV][kBlock / 64];
     const int lanei = threadIdx.x & 63, wave = threadIdx.x >> 6;
     double acc[NV];
 #pragma unroll
@@ -1405,7 +1012,7 @@ __global__ __launch_bounds__(kBlock) void k_fin(const Seg<T>* __restrict__ segs,
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const int b = b0 + kBlock * u;
-                v[a][u] = b < sg.nblocks ? ldg(&sg.part[(size_t)(a * NR + k) * sg.nblocks + b]) : 0.0;
+                v[a][u] = b < sg.nblocks ? ldg(&part[(size_t)(a * NR + k) * sg.nblocks + b]) : 0.0;
             }
 #pragma unroll
         for (int a = 0; a < NV; ++a)
@@ -1418,14 +1025,853 @@ __global__ __launch_bounds__(kBlock) void k_fin(const Seg<T>* __restrict__ segs,
         if (lanei == 0) red[a][wave] = t;
     }
     __syncthreads();
-    if (threadIdx.x != 0) return;
-    double tot[NV];
-    for (int a = 0; a < NV; ++a) {
-        double t = 0.0;
-        for (int w = 0; w < kBlock / 64; ++w) t += red[a][w];
-        tot[a] = t;
+    if (threadIdx.x == 0)
+        for (int a = 0; a < NV; ++a) {
+            double t = 0.0;
+            for (int w = 0; w < kBlock / 64; ++w) t += red[a][w];
+            tot[a] = t;
+        }
+}
+
+// Partials of the kernel that leads to copy `in` of the states: xrupdate
+// (copy 2) writes its own while workgroups still sum lfinish's.
+template <int NR, typename T>
+__device__ __forceinline__ double* part_of(const Seg<T>& sg, int copy) {
+    return sg.part + (copy == 2 ? (size_t)2 * NR * sg.nblocks : 0);
+}
+
+// The finaliser KIND folded into the kernel that first needs its result: every
+// workgroup of a segment sums the same partials in the same order and runs
+// the same scalar update on its own copy of the lanes' states (in LDS), and
+// the segment's first workgroup stores it for the kernels after it.  A
+// finaliser of its own costs a launch (2.3-4 us with its gap, three an
+// iteration); the sums cost each workgroup one round of loads that mostly
+// hit the L2.  States live in three copies (Seg::sst apart): copy `in` is
+// only read here while copy `out` is written, so no workgroup meets a state
+// that another has already advanced.
+template <int KIND, int NR>
+struct LaneState {
+    static constexpr int NV = FinTraits<KIND>::NV;
+    KState s[NR];
+    double tot[NV * NR];
+};
+// The loads of a fold, issued before the caller's own so that they overlap:
+// the states' words and the first kBlock partials of the wave's first component.
+struct FoldLoads {
+    double v[kBlock / 64];
+    int w0, w1;
+};
+template <int KIND, int NR, typename T>
+__device__ __forceinline__ void fold_begin(const Seg<T>& sg, int in, FoldLoads& f) {
+    constexpr int C = FinTraits<KIND>::NV * NR;
+    constexpr int W = (int)(sizeof(KState) / 4) * NR;   // a group owns kMaxNR states: every load is valid
+    static_assert(W <= 2 * kBlock, "a thread copies at most two words");
+    const int t = (int)threadIdx.x, lanei = t & 63, wave = t >> 6;
+    const int* src = reinterpret_cast<const int*>(sg.st + (int64_t)in * sg.sst);
+    f.w0 = t < W ? ldg(&src[t]) : 0;
+    f.w1 = W > kBlock && t + kBlock < W ? ldg(&src[t + kBlock]) : 0;
+    const double* p = part_of<NR>(sg, in) + (size_t)(wave < C ? wave : 0) * sg.nblocks;
+#pragma unroll
+    for (int w = 0; w < kBlock / 64; ++w) f.v[w] = lanei + 64 * w < sg.nblocks ? ldg(&p[lanei + 64 * w]) : 0.0;
+}
+template <int KIND, int NR, typename T>
+__device__ __forceinline__ LaneStat<NR> fold_end(const Seg<T>& sg, int in, int out, bool writer, const FoldLoads& f,
+                                                 LaneState<KIND, NR>& sh) {
+    constexpr int NV = FinTraits<KIND>::NV, C = NV * NR, NW = kBlock / 64, U = 2;
+    constexpr int W = (int)(sizeof(KState) / 4) * NR;
+    const int t = (int)threadIdx.x, lanei = t & 63, wave = t >> 6;
+    int* lds = reinterpret_cast<int*>(sh.s);
+    if (t < W) lds[t] = f.w0;
+    if (W > kBlock && t + kBlock < W) lds[t + kBlock] = f.w1;
+    // a wave sums whole components, in part_totals' order: its lane l adds
+    // what threads l, 64 + l, .. of that sum add, each in an accumulator of
+    // its own (the sums of lanes that are not in the finaliser's mask are
+    // formed and not used)
+    for (int c = wave; c < C; c += NW) {
+        const double* p = part_of<NR>(sg, in) + (size_t)c * sg.nblocks;
+        double acc[NW];
+        int b0 = lanei;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) acc[w] = 0.0;
+        if (c == wave) {
+#pragma unroll
+            for (int w = 0; w < NW; ++w) acc[w] += f.v[w];
+            b0 += kBlock;
+        }
+        for (; b0 < sg.nblocks; b0 += kBlock * U) {
+            double v[U][NW];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int w = 0; w < NW; ++w) {
+                    const int b = b0 + kBlock * u + 64 * w;
+                    v[u][w] = b < sg.nblocks ? ldg(&p[b]) : 0.0;
+                }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int w = 0; w < NW; ++w) acc[w] += v[u][w];
+        }
+        double sum = 0.0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) sum += wave_sum(acc[w]);
+        if (lanei == 0) sh.tot[c] = sum;
     }
-    fin_scalar<KIND>(sg.st[k], tot);
+    __syncthreads();
+    if (t < NR && t < sg.nr && ((FinTraits<KIND>::M >> sh.s[t].status) & 1u)) {
+        double tot[NV];
+#pragma unroll
+        for (int a = 0; a < NV; ++a) tot[a] = sh.tot[a * NR + t];
+        fin_scalar<KIND>(sh.s[t], tot);
+    }
+    __syncthreads();
+    if (writer) {
+        int* dst = reinterpret_cast<int*>(sg.st + (int64_t)out * sg.sst);
+        for (int k = t; k < W; k += kBlock) stg(&dst[k], lds[k]);
+    }
+    LaneStat<NR> L;
+#pragma unroll
+    for (int k = 0; k < NR; ++k) L.s[k] = sh.s[k].status;
+    L.nr = sg.nr;
+    return L;
+}
+template <int KIND, int NR, typename T>
+__device__ __forceinline__ LaneStat<NR> fold_states(const Seg<T>& sg, int in, int out, bool writer, LaneState<KIND, NR>& sh) {
+    FoldLoads f;
+    fold_begin<KIND, NR>(sg, in, f);
+    return fold_end<KIND, NR>(sg, in, out, writer, f, sh);
+}
+
+// The states of a kernel that folds finaliser FOLD (copy IN to copy OUT), or
+// of copy 0 where FOLD < 0: L their statuses, ST(k, f) field f of lane k.
+#define FOLDED_STATES(FOLD, IN, OUT)                                                                      \
+    __shared__ LaneState<(FOLD >= 0 ? FOLD : 0), (FOLD >= 0 ? NR : 1)> lst;                               \
+    LaneStat<NR> L;                                                                                       \
+    if constexpr (FOLD >= 0) L = fold_states<FOLD, NR>(sg, IN, OUT, lb == 0, lst);                        \
+    else L = lane_stat<NR>(sg)
+#define ST(k, f) (FOLD >= 0 ? lst.s[FOLD >= 0 ? (k) : 0].f : ldg(&sg.st[k].f))
+
+template <typename T, int NR>
+__global__ __launch_bounds__(kBlock) void k_init(const Seg<T>* __restrict__ segs, const int* __restrict__ bseg, const T* b, T* x, T* r,
+                                                 T* r0, T* p, T* v) {
+    int lb;
+    int64_t row;
+    const Seg<T>& sg = seg_of(segs, bseg, lb, row);
+    double pv[1][NR];
+#pragma unroll
+    for (int k = 0; k < NR; ++k) pv[0][k] = 0.0;
+    if (row < sg.op.D) {
+        const size_t i = (size_t)(sg.off + row * NR);
+        auto bv = vload<T, NR>(b + i);
+        typename VT<T, NR>::type zero = (typename VT<T, NR>::type)(T)0;
+        vstore<T, NR>(r + i, bv);
+        vstore<T, NR>(r0 + i, bv);
+        vstore<T, NR>(x + i, zero);
+        vstore<T, NR>(p + i, zero);
+        vstore<T, NR>(v + i, zero);
+#pragma unroll
+        for (int k = 0; k < NR; ++k) pv[0][k] = (double)lane(bv, k) * (double)lane(bv, k);
+    }
+    block_partials<1, NR>(pv, sg.part, lb, sg.nblocks);
+}
+
+// RUN lanes: p = (p - w v) beta + r ; y = P^-1 p (fly: y is formed where it is read).
+// UPDATE lanes (mixed): x64 += x32 / scale ; x32 = 0.
+template <typename T, int NR, int FOLD>
+__global__ __launch_bounds__(kBlock) void k_pupdate(const Seg<T>* __restrict__ segs, const int* __restrict__ bseg, T* p, const T* v,
+                                                    const T* r, T* y, T* x, MixVec mv, int fly) {
+    int lb;
+    int64_t row;
+    const Seg<T>& sg = seg_of(segs, bseg, lb, row);
+    FOLDED_STATES(FOLD, 2, 0);   // the loop test of the last iteration
+    if (row >= sg.op.D || !seg_any(L, M_STAGE1)) return;
+    const size_t i = (size_t)(sg.off + row * NR);
+    if (seg_any(L, M_RUN)) {
+        const uint8_t f = ldg(&sg.op.flag[row]);
+        auto pv = vload<T, NR>(p + i);
+        auto vv = vload<T, NR>(v + i);
+        auto rv = vload<T, NR>(r + i);
+        const unsigned run = L.of(M_RUN);
+#pragma unroll
+        for (int k = 0; k < NR; ++k) {   // a group owns kMaxNR states: every lane's load is valid
+            const T beta = (T)ST(k, beta), w = (T)ST(k, omega);
+            const T pk = (-w * lane(vv, k) + lane(pv, k)) * beta + lane(rv, k);   // p.Copy(-w,v,p); p*=beta; p+=r
+            if ((run >> k) & 1u) setlane(pv, k, pk);
+        }
+        vstore<T, NR>(p + i, pv);
+        if (!fly) vstore<T, NR>(y + i, prow_apply<T, NR>(prow_of(sg, row, f), prow_div(sg), pv));
+    }
+    if (std::is_same<T, float>::value && seg_any(L, M_UPDATE)) {
+        auto xv = vload<T, NR>(x + i);
+#pragma unroll
+        for (int k = 0; k < NR; ++k)
+            if (lane_in(L, k, M_UPDATE)) {
+                double* xd = mv.x64 + lm_at(sg, k, row);
+                stg(xd, ldg(xd) + (double)lane(xv, k) / ST(k, scale));
+                setlane(xv, k, (T)0);
+            }
+        vstore<T, NR>(x + i, xv);
+    }
+}
+
+// tmp = E x.  Rows are independent; a thread owns one row and all NR rhs.
+// UPDATE lanes (mixed, first gather of the iteration): tmp64 = E64 x64.
+// E x for the instance segments.  Tiles with an LDS list copy their x rows
+// into LDS once and gather every stencil line from there; the other tiles
+// (lists longer than the LDS, or operators without tiles) read x directly.
+template <typename T, int NR>
+__global__ __launch_bounds__(kBlock) void k_egather(const Seg<T>* __restrict__ segs, const int* __restrict__ bseg, const T* x, T* out,
+                                                    unsigned lanes, MixVec mv, int copy) {
+    typedef typename VT<T, NR>::type V;
+    constexpr int LR = LdsTile<T, NR>::kRows;
+    __shared__ V lx[LR > 0 ? LR : 1];
+    const LdsRows<V> lrows{lx, LR > 0 ? LR : 1};
+    int lb;
+    int64_t row;
+    const Seg<T>& sg = seg_of(segs, bseg, lb, row);
+    if (lb >= sg.nblocks) return;   // a launch with more tiles (k_egather_upd's) than row blocks
+    const auto L = lane_stat<NR>(sg, lanes != 0, copy);
+    if (lanes && !seg_any(L, lanes)) return;               // uniform per workgroup
+    const bool main = !lanes || seg_any(L, lanes & ~M_UPDATE);
+    const size_t i = (size_t)(sg.off + row * NR);
+    const T* xb = x + sg.off;
+    const int nu = (LR > 0 && main && sg.op.fmt == OP_TP && sg.op.tln) ? ldg(&sg.op.tln[lb]) : -1;
+    if (nu >= 0 && nu <= LR) {
+        // Loads in two rounds, each issued as soon as the previous one's
+        // values are in: the tile's list entries with the row's flag,
+        // exception record and weights (rows past the end read the last
+        // row's, unused), all unconditional; then the listed x rows with the
+        // row's LDS positions (a plain row's 16 line positions, or a moved
+        // row's exception record and extra value, in one register array) or
+        // an identity row's own x.  Then the LDS copy, the barrier and every
+        // stencil line from LDS.
+        FillIdx<LR> f;
+        lds_fill_index<LR>(sg.op.tlr + ldg(&sg.op.tlo[lb]), nu, f);
+        const bool act = row < sg.op.D;
+        const int64_t rr = act ? row : sg.op.D - 1;
+        const int64_t D = sg.op.D;
+        const int e = ldg(&sg.op.exc[rr]);
+        const uint8_t fl = ldg(&sg.op.flag[rr]);
+        TpRow<T> m;
+#pragma unroll
+        for (int q = 0; q < 12; ++q) m.w[q] = ldg(&sg.op.tpw[q * D + rr]);
+        const int kind = act ? ((fl & ROW_IDENTITY) ? 2 : (e < 0 ? 0 : 1)) : 3;
+        ExcRow mx;   // kind 0: words 0..15 are the line positions; kind 1: the exception record
+        T xval = (T)0;
+        V xi = (V)(T)0;
+        if (kind == 0) {
+#pragma unroll
+            for (int l = 0; l < 16; ++l) mx.pk[l] = ldg(&sg.op.tpl[l * D + row]);
+        } else if (kind == 1) {   // rows an interior boundary moved
+            exc_row_load(sg.op.tlx, e, mx);
+            xval = ldg(&sg.op.xval[e]);
+        } else if (kind == 2) {
+            xi = vload<T, NR>(xb + (size_t)row * NR);
+        }
+        lds_fill_rows<T, NR, LR>(f, xb, lrows, [](const V& v, int) { return v; });
+        if (act) {
+            V acc = (V)(T)0;
+#pragma unroll
+            for (int l = 0; l < 16; ++l) m.p[l] = mx.pk[l];
+            if (kind == 2) acc = xi;
+            else if (kind == 0) egather_tp_lds<T, V, NR>(m, lrows, acc);
+            else egather_grp_exc<T, V>(m.w, xval, mx, lrows, acc);
+            vstore<T, NR>(out + i, acc);
+        }
+    } else if (main && row < sg.op.D) {
+        vstore<T, NR>(out + i, erow<T, NR>(sg.op, row, xb, NR));
+    }
+}
+
+// FP64 gathers of the refinement lanes of FP32 segments: tmp64 = E64 x64 for
+// every lane in an UPDATE status (a launch of its own beside the FP32
+// gather, which then carries only FP32 work).  A lane's FP64 vectors are a
+// run of D values, the one-right-hand-side layout, so block lb gathers tile
+// lb of the operator's shared-stencil tiles for each such lane in turn;
+// operators without tiles read x64 directly, a row per thread.
+// x32: the solutions' FP32 parts are still to be added (fused iterations),
+// null: pupdate has added them.
+template <int NR>
+__global__ __launch_bounds__(kBlock) void k_egather_upd(const Seg<float>* __restrict__ segs, const int* __restrict__ bseg,
+                                                        MixVec mv, const float* x32) {
+    constexpr int LR = GrpTile<double, 1>::kRows;
+    static_assert(LR > 0, "FP64 shared-stencil tiles fit the LDS");
+    __shared__ double lx[LR];
+    const LdsRows<double> lrows{lx, LR};
+    int lb;
+    int64_t row;
+    const Seg<float>& sg = seg_of(segs, bseg, lb, row);
+    const auto L = lane_stat<NR>(sg);
+    if (!seg_any(L, M_UPDATE)) return;   // uniform per workgroup
+    if (sg.op64.ngt > 0) {
+        if (lb >= sg.op64.ngt) return;
+        bool first = true;
+        for (int k = 0; k < sg.nr; ++k)
+            if (lane_in(L, k, M_UPDATE)) {
+                if (!first) __syncthreads();   // the previous lane's LDS reads are done
+                first = false;
+                double* ob = mv.tmp64 + lm_at(sg, k, 0);
+                if (x32) {
+                    SrcX64<NR> src{mv.x64 + lm_at(sg, k, 0), x32 + sg.off + k, ldg(&sg.st[k].scale)};
+                    egather_grp_tile<double, 1, LR>(sg.op64, lb, src, ob, lrows, [](auto&) { return true; });
+                } else {
+                    SrcPlain<double, 1, false> src{nullptr, mv.x64 + lm_at(sg, k, 0)};
+                    egather_grp_tile<double, 1, LR>(sg.op64, lb, src, ob, lrows, [](auto&) { return true; });
+                }
+            }
+        return;
+    }
+    if (row >= sg.op.D) return;
+    for (int k = 0; k < sg.nr; ++k)
+        if (lane_in(L, k, M_UPDATE))
+            stg(&mv.tmp64[lm_at(sg, k, row)], erow<double, 1>(sg.op64, row, mv.x64 + lm_at(sg, k, 0), 1));
+}
+
+// E x for launches whose every segment has shared-stencil tiles: block lb of
+// a segment takes its tile lb.  32 KB of LDS and at most 128 VGPRs, so four
+// workgroups share a CU (a direct-read path for other segments, even out of
+// line, made the FP32 x 8 kernel spill).
+// FLY: x is p (or s) and the launch gathers y = P^-1 p (z = P^-1 s).
+template <typename T, int NR, int WPE, bool FLY>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) void k_egather_grp(
+    const Seg<T>* __restrict__ segs, const int* __restrict__ bseg, const T* x, T* out, unsigned lanes, MixVec mv,
+    int copy) {
+    typedef typename VT<T, NR>::type V;
+    constexpr int LR = GrpTile<T, NR>::kRows;
+    static_assert(LR > 0, "shared-stencil tiles do not fit this value size");
+    __shared__ V lx[LR];
+    const LdsRows<V> lrows{lx, LR};
+    int lb;
+    int64_t row;
+    const Seg<T>& sg = seg_of(segs, bseg, lb, row);
+    const auto L = lane_stat<NR>(sg, lanes != 0, copy);
+    if (lanes && !seg_any(L, lanes)) return;               // uniform per workgroup
+    const bool main = !lanes || seg_any(L, lanes & ~M_UPDATE);
+    if (!main || lb >= sg.op.ngt) return;
+    SrcPlain<T, NR, FLY> src{&sg, x + sg.off};
+    egather_grp_tile<T, NR, LR>(sg.op, lb, src, out + sg.off, lrows, [](auto&) { return true; });
+}
+
+// out = A x from tmp = E x.  RED = 0: no reduction; 1: partial (other, out);
+// 2: partials (out, out), (out, other).
+// Mixed, RED = 1: UPDATE lanes r64 = b - A64 x64, partial (r64, r64).
+// Mixed, RED = 2: RESCALE lanes partial (r32, r32) (rv32 = r32).
+template <typename T, int NR, int RED>
+__global__ __launch_bounds__(kBlock) void k_lfinish(const Seg<T>* __restrict__ segs, const int* __restrict__ bseg, const T* x,
+                                                    const T* tmp, T* out, const T* other, const T* rv32,
+                                                    unsigned lanes, MixVec mv, int fly, int copy) {
+    int lb;
+    int64_t row;
+    const Seg<T>& sg = seg_of(segs, bseg, lb, row);
+    const auto L = lane_stat<NR>(sg, lanes != 0, copy);
+    if (lanes && !seg_any(L, lanes)) return;   // uniform per segment
+    constexpr int NV = RED == 2 ? 2 : 1;
+    double pv[NV][NR];
+#pragma unroll
+    for (int a = 0; a < NV; ++a)
+#pragma unroll
+        for (int k = 0; k < NR; ++k) pv[a][k] = 0.0;
+    if (row < sg.op.D) {
+        const size_t i = (size_t)(sg.off + row * NR);
+        if (!lanes || seg_any(L, lanes & ~(M_UPDATE | M_RESCALE))) {
+            typename VT<T, NR>::type res, ov;
+            if (sg.op.fmt == OP_TP) {   // every load that waits on no other in one round
+                TpLRow<T, NR> a;
+                arow_tp_load<T, NR>(sg.op, row, x + i, a);
+                if (RED > 0) ov = vload<T, NR>(other + i);
+                res = arow_tp<T, NR>(sg, row, a, tmp + sg.off, NR, fly);   // fly: x is p or s
+            } else {
+                auto xv = vload<T, NR>(x + i);
+                if (RED > 0) ov = vload<T, NR>(other + i);
+                if (fly) xv = precond_row<T, NR>(sg, row, ldg(&sg.op.flag[row]), xv);
+                res = arow<T, NR>(sg.op, sg.m, sg.n, row, xv, tmp + sg.off, NR);
+            }
+            vstore<T, NR>(out + i, res);
+            if (RED > 0) {
+#pragma unroll
+                for (int k = 0; k < NR; ++k) {
+                    const double rk = (double)lane(res, k);
+                    if (RED == 1) {
+                        pv[0][k] = (double)lane(ov, k) * rk;
+                    } else {
+                        pv[0][k] = rk * rk;
+                        pv[NV - 1][k] = rk * (double)lane(ov, k);
+                    }
+                }
+            }
+        }
+        if (std::is_same<T, float>::value && RED == 1 && seg_any(L, M_UPDATE)) {
+#pragma unroll
+            for (int k = 0; k < NR; ++k)   // constant indices keep pv in registers
+                if (k < sg.nr && lane_in(L, k, M_UPDATE)) {
+                    const size_t j = lm_at(sg, k, row);
+                    const double ax =
+                        arow<double, 1>(sg.op64, sg.m, sg.n, row, ldg(&mv.x64[j]), mv.tmp64 + lm_at(sg, k, 0), 1);
+                    const double rk = ldg(&mv.b64[j]) - ax;
+                    stg(&mv.r64[j], rk);
+                    pv[0][k] = rk * rk;
+                }
+        }
+        if (std::is_same<T, float>::value && RED == 2 && seg_any(L, M_RESCALE)) {
+            auto rr = vload<T, NR>(rv32 + i);
+#pragma unroll
+            for (int k = 0; k < NR; ++k)
+                if (lane_in(L, k, M_RESCALE)) {
+                    const double rk = (double)lane(rr, k);
+                    pv[0][k] = rk * rk;
+                    pv[NV - 1][k] = 0.0;
+                }
+        }
+    }
+    if (RED > 0) block_partials<NV, NR>(pv, sg.part, lb, sg.nblocks);
+}
+
+// RUN lanes: s = r - alpha v ; z = P^-1 s (fly: z is formed where it is read).
+// RESCALE lanes (mixed): r32 = r64 scale ; r0 = r32 ; p = v = 0.
+template <typename T, int NR, int FOLD>
+__global__ __launch_bounds__(kBlock) void k_supdate(const Seg<T>* __restrict__ segs, const int* __restrict__ bseg, T* r, T* v, T* s, T* z,
+                                                    T* r0, T* p, MixVec mv, int fly) {
+    int lb;
+    int64_t row;
+    const Seg<T>& sg = seg_of(segs, bseg, lb, row);
+    FOLDED_STATES(FOLD, 0, 1);   // alpha
+    if (row >= sg.op.D || !seg_any(L, M_STAGE2)) return;
+    const size_t i = (size_t)(sg.off + row * NR);
+    const uint8_t f = ldg(&sg.op.flag[row]);
+    auto rv = vload<T, NR>(r + i);
+    auto vv = vload<T, NR>(v + i);
+    if (seg_any(L, M_RUN)) {
+        typename VT<T, NR>::type sv;
+#pragma unroll
+        for (int k = 0; k < NR; ++k) {   // a group owns kMaxNR states: every lane's load is valid
+            const T a = (T)ST(k, alpha);
+            setlane(sv, k, -a * lane(vv, k) + lane(rv, k));   // s.Copy(-alpha, v, r)
+        }
+        vstore<T, NR>(s + i, sv);
+        if (!fly) vstore<T, NR>(z + i, prow_apply<T, NR>(prow_of(sg, row, f), prow_div(sg), sv));
+    }
+    if (std::is_same<T, float>::value && seg_any(L, M_RESCALE)) {
+        auto r0v = vload<T, NR>(r0 + i);
+        auto pv = vload<T, NR>(p + i);
+#pragma unroll
+        for (int k = 0; k < NR; ++k)
+            if (lane_in(L, k, M_RESCALE)) {
+                const T rk = (T)(ldg(&mv.r64[lm_at(sg, k, row)]) * ST(k, scale));
+                setlane(rv, k, rk);
+                setlane(r0v, k, rk);
+                setlane(pv, k, (T)0);
+                setlane(vv, k, (T)0);
+            }
+        vstore<T, NR>(r + i, rv);
+        vstore<T, NR>(r0 + i, r0v);
+        vstore<T, NR>(p + i, pv);
+        vstore<T, NR>(v + i, vv);
+    }
+}
+
+// Jacobi sweep `sweep` (>= 1) of RUN lanes: y += omega D^-1 (x - A y) on the
+// rows below dofs, A y from tmp = E y (GeneralizedBiCGStabSystem.h:366-378).
+// A y is formed here rather than stored by a launch of lfinish: a sweep is
+// launch-bound on the geodesic problems that use it (10,906 rows, 2,000
+// sweeps an application).
+template <typename T, int NR>
+__global__ __launch_bounds__(kBlock) void k_jacobi(const Seg<T>* __restrict__ segs, const int* __restrict__ bseg,
+                                                   const T* x, const T* tmp, T* y, int sweep, int copy) {
+    int lb;
+    int64_t row;
+    const Seg<T>& sg = seg_of(segs, bseg, lb, row);
+    const auto L = lane_stat<NR>(sg, true, copy);
+    if (sg.precond != 2 || sweep >= sg.precond_iters) return;
+    if (row >= sg.op.D - sg.op.nD || !seg_any(L, M_RUN)) return;
+    const size_t i = (size_t)(sg.off + row * NR);
+    const uint8_t f = ldg(&sg.op.flag[row]);
+    auto xv = vload<T, NR>(x + i);
+    typename VT<T, NR>::type yv, av;
+    if (sg.op.fmt == OP_TP) {
+        TpLRow<T, NR> a;
+        arow_tp_load<T, NR>(sg.op, row, y + i, a);
+        yv = a.xv;
+        av = arow_tp<T, NR>(sg, row, a, tmp + sg.off, NR, false);
+    } else {
+        yv = vload<T, NR>(y + i);
+        av = arow<T, NR>(sg.op, sg.m, sg.n, row, yv, tmp + sg.off, NR);
+    }
+#pragma unroll
+    for (int k = 0; k < NR; ++k)
+        if (lane_in(L, k, M_RUN))
+            setlane(yv, k, lane(yv, k) + (T)kJacobiOmega * diag_inverse(sg, row, f, (T)(lane(xv, k) - lane(av, k))));
+    vstore<T, NR>(y + i, yv);
+}
+
+template <typename T, int NR, int FOLD>
+__global__ __launch_bounds__(kBlock) void k_xrupdate(const Seg<T>* __restrict__ segs, const int* __restrict__ bseg, T* x, const T* y,
+                                                     const T* z, T* r, const T* s, const T* t, const T* r0, int fly) {
+    int lb;
+    int64_t row;
+    const Seg<T>& sg = seg_of(segs, bseg, lb, row);
+    FOLDED_STATES(FOLD, 1, 2);   // omega
+    if (!seg_any(L, M_RUN)) return;
+    double pv[2][NR];
+#pragma unroll
+    for (int k = 0; k < NR; ++k) { pv[0][k] = 0.0; pv[1][k] = 0.0; }
+    if (row < sg.op.D) {
+        const size_t i = (size_t)(sg.off + row * NR);
+        auto xv = vload<T, NR>(x + i);
+        auto yv = vload<T, NR>(y + i);   // fly: p
+        auto sv = vload<T, NR>(s + i);
+        auto tv = vload<T, NR>(t + i);
+        auto r0v = vload<T, NR>(r0 + i);
+        const uint8_t f = ldg(&sg.op.flag[row]);
+        // r is rewritten on every RUN lane: read only to keep the others
+        const unsigned run = L.of(M_RUN);
+        const bool all_run = run == (1u << NR) - 1u;
+        typename VT<T, NR>::type rv = all_run ? (typename VT<T, NR>::type)(T)0 : vload<T, NR>(r + i);
+        typename VT<T, NR>::type zv;
+        if (fly) {   // y = P^-1 p, z = P^-1 s
+            const PRow<T> pr = prow_of(sg, row, f);
+            const bool div = prow_div(sg);
+            yv = prow_apply<T, NR>(pr, div, yv);
+            zv = prow_apply<T, NR>(pr, div, sv);
+        } else {
+            zv = vload<T, NR>(z + i);
+        }
+#pragma unroll
+        for (int k = 0; k < NR; ++k) {   // a group owns kMaxNR states: every lane's load is valid
+            if (!((run >> k) & 1u)) continue;
+            const T a = (T)ST(k, alpha), w = (T)ST(k, omega);
+            T xk = a * lane(yv, k) + lane(xv, k);   // x.Copy(alpha, y, x)
+            xk = w * lane(zv, k) + xk;               // x.Copy(w, z, x)
+            T rk = -w * lane(tv, k) + lane(sv, k);   // r.Copy(-w, t, s)
+            setlane(xv, k, xk);
+            setlane(rv, k, rk);
+            pv[0][k] = (double)rk * (double)rk;
+            pv[1][k] = (double)lane(r0v, k) * (double)rk;
+        }
+        vstore<T, NR>(x + i, xv);
+        vstore<T, NR>(r + i, rv);
+    }
+    block_partials<2, NR>(pv, part_of<NR>(sg, FOLD >= 0 ? 2 : 0), lb, sg.nblocks);
+}
+
+// ---------------------------------------------------------------- fused iterations
+// Iterations of launches whose gathers fill LDS from shared-stencil tiles and
+// whose preconditioner is pointwise, with folded finalisers, in five launches
+// instead of ten: pupdate and supdate have no launch of their own.
+//
+//   fgather<1>   (loop test) p formed in the LDS fill ; tmp = E P^-1 p
+//   flfinish<1>  p formed again and stored ; v = A P^-1 p from tmp ; (r0, v)
+//   fgather<2>   (alpha) s formed in the LDS fill ; tmp = E P^-1 s
+//   flfinish<2>  s formed again ; t = A P^-1 s ; (t, t), (t, s)
+//   fxrupdate    (omega) s formed again ; x, r ; (r, r), (r0, r)
+//
+// s is never stored.  A row's values are formed by the same operations
+// wherever they are needed, so the results are the separate kernels' to the
+// bit.  Every tile lists a row's neighbours too, so the fills read p, v and r
+// (1.5 rows each per row) where the separate kernels read one vector: more
+// bytes, fewer launches, which pays while an iteration is bound by its
+// launches and their dependent loads rather than by its bytes (fuse_limit,
+// capi.hip).  Refinement (mixed) lanes: x64 += x32 / scale is formed in
+// k_egather_upd's fill and stored by flfinish<1>, the rescaled residual is
+// stored by flfinish<2>.
+
+// PH 1: tmp = E P^-1 p, after the loop test (FOLD) ; PH 2: tmp = E P^-1 s, after alpha.
+template <typename T, int NR, bool ONE, int WPE, int PH, int FOLD>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) void k_fgather(
+    const SegArg<T> segs, Vecs<T> w) {
+    typedef typename VT<T, NR>::type V;
+    constexpr int LR = GrpTile<T, NR>::kRows;
+    __shared__ V lx[LR];
+    __shared__ LaneState<(FOLD >= 0 ? FOLD : 0), (FOLD >= 0 ? NR : 1)> lst;
+    const LdsRows<V> lrows{lx, LR};
+    int lb;
+    int64_t row;
+    const Seg<T>& sg = seg_of<ONE>(segs, lb, row);
+    if (lb >= sg.op.ngt) return;
+    constexpr int in = PH == 1 ? 2 : 0, out = PH == 1 ? 0 : 1;
+    FoldLoads f;
+    if constexpr (FOLD >= 0) fold_begin<(FOLD >= 0 ? FOLD : 0), NR>(sg, in, f);
+    typename std::conditional<PH == 1, SrcP<T, NR>, SrcS<T, NR>>::type src;
+    src.sg = &sg;
+    src.v = w.v + sg.off;
+    src.r = w.r + sg.off;
+    if constexpr (PH == 1) src.p = w.p + sg.off;
+    egather_grp_tile<T, NR, LR>(sg.op, lb, src, w.tmp + sg.off, lrows, [&](auto& q) {
+        LaneStat<NR> L;
+        if constexpr (FOLD >= 0) L = fold_end<(FOLD >= 0 ? FOLD : 0), NR>(sg, in, out, lb == 0, f, lst);
+        else L = lane_stat<NR>(sg);
+        if (!seg_any(L, M_RUN)) return false;
+#pragma unroll
+        for (int k = 0; k < NR; ++k) {
+            if constexpr (PH == 1) {
+                q.beta[k] = (T)ST(k, beta);
+                q.w[k] = (T)ST(k, omega);
+            } else {
+                q.alpha[k] = (T)ST(k, alpha);
+            }
+        }
+        if constexpr (PH == 1) q.run = L.of(M_RUN);
+        return true;
+    });
+}
+
+template <typename T, int NR, bool ONE, int PH>
+__global__ __launch_bounds__(kBlock) void k_flfinish(const SegArg<T> segs, Vecs<T> w,
+                                                     MixVec mv) {
+    int lb;
+    int64_t row;
+    const Seg<T>& sg = seg_of<ONE>(segs, lb, row);
+    const KState* st = sg.st + (PH == 1 ? 0 : sg.sst);
+    const auto L = lane_stat<NR>(sg, true, PH == 1 ? 0 : 1);
+    if (!seg_any(L, PH == 1 ? M_STAGE1 : M_STAGE2)) return;   // uniform per segment
+    constexpr int NV = PH;
+    double pv[NV][NR];
+#pragma unroll
+    for (int a = 0; a < NV; ++a)
+#pragma unroll
+        for (int k = 0; k < NR; ++k) pv[a][k] = 0.0;
+    if (row < sg.op.D) {
+        const size_t i = (size_t)(sg.off + row * NR);
+        if (seg_any(L, M_RUN)) {
+            TpLRow<T, NR> a;
+            typename VT<T, NR>::type ov;   // r0 ; s
+            if constexpr (PH == 1) {
+                SrcP<T, NR> src;
+                src.p = w.p;
+                src.v = w.v;
+                src.r = w.r;
+                src.run = L.of(M_RUN);
+#pragma unroll
+                for (int k = 0; k < NR; ++k) {
+                    src.beta[k] = (T)ldg(&st[k].beta);
+                    src.w[k] = (T)ldg(&st[k].omega);
+                }
+                arow_tp_load<T, NR>(sg.op, row, w.r0 + i, a);
+                const typename SrcP<T, NR>::Raw q{vload<T, NR>(w.p + i), vload<T, NR>(w.v + i), vload<T, NR>(w.r + i)};
+                ov = a.xv;
+                a.xv = src.direction(q);
+                vstore<T, NR>(w.p + i, a.xv);
+            } else {
+                SrcS<T, NR> src;
+#pragma unroll
+                for (int k = 0; k < NR; ++k) src.alpha[k] = (T)ldg(&st[k].alpha);
+                arow_tp_load<T, NR>(sg.op, row, w.r + i, a);
+                const typename SrcS<T, NR>::Raw q{a.xv, vload<T, NR>(w.v + i)};
+                ov = a.xv = src.residual(q);
+            }
+            const typename VT<T, NR>::type res = arow_tp<T, NR>(sg, row, a, w.tmp + sg.off, NR, true);
+            vstore<T, NR>((PH == 1 ? w.v : w.t) + i, res);
+#pragma unroll
+            for (int k = 0; k < NR; ++k) {
+                const double rk = (double)lane(res, k);
+                if (PH == 1) {
+                    pv[0][k] = (double)lane(ov, k) * rk;
+                } else {
+                    pv[0][k] = rk * rk;
+                    pv[NV - 1][k] = rk * (double)lane(ov, k);
+                }
+            }
+        }
+        if (std::is_same<T, float>::value && PH == 1 && seg_any(L, M_UPDATE)) {
+            auto xv = vload<T, NR>(w.x + i);
+#pragma unroll
+            for (int k = 0; k < NR; ++k)
+                if (lane_in(L, k, M_UPDATE)) {
+                    const size_t j = lm_at(sg, k, row);
+                    const double xd = ldg(&mv.x64[j]) + (double)lane(xv, k) / ldg(&st[k].scale);
+                    stg(&mv.x64[j], xd);
+                    setlane(xv, k, (T)0);
+                    const double ax = arow<double, 1>(sg.op64, sg.m, sg.n, row, xd, mv.tmp64 + lm_at(sg, k, 0), 1);
+                    const double rk = ldg(&mv.b64[j]) - ax;
+                    stg(&mv.r64[j], rk);
+                    pv[0][k] = rk * rk;
+                }
+            vstore<T, NR>(w.x + i, xv);
+        }
+        if (std::is_same<T, float>::value && PH == 2 && seg_any(L, M_RESCALE)) {
+            auto rv = vload<T, NR>(w.r + i), r0v = vload<T, NR>(w.r0 + i), p = vload<T, NR>(w.p + i), v = vload<T, NR>(w.v + i);
+#pragma unroll
+            for (int k = 0; k < NR; ++k)
+                if (lane_in(L, k, M_RESCALE)) {
+                    const T rk = (T)(ldg(&mv.r64[lm_at(sg, k, row)]) * ldg(&st[k].scale));
+                    setlane(rv, k, rk);
+                    setlane(r0v, k, rk);
+                    setlane(p, k, (T)0);
+                    setlane(v, k, (T)0);
+                    pv[0][k] = (double)rk * (double)rk;
+                    pv[NV - 1][k] = 0.0;
+                }
+            vstore<T, NR>(w.r + i, rv);
+            vstore<T, NR>(w.r0 + i, r0v);
+            vstore<T, NR>(w.p + i, p);
+            vstore<T, NR>(w.v + i, v);
+        }
+    }
+    block_partials<NV, NR>(pv, sg.part, lb, sg.nblocks);
+}
+
+template <typename T, int NR, bool ONE>
+__global__ __launch_bounds__(kBlock) void k_fxrupdate(const SegArg<T> segs, Vecs<T> w) {
+    int lb;
+    int64_t row;
+    const Seg<T>& sg = seg_of<ONE>(segs, lb, row);
+    __shared__ LaneState<FIN_OMEGA, NR> lst;
+    FoldLoads f;
+    fold_begin<FIN_OMEGA, NR>(sg, 1, f);
+    typedef typename VT<T, NR>::type V;
+    const bool in = row < sg.op.D;
+    const size_t i = (size_t)(sg.off + (in ? row : 0) * NR);
+    V xv = vload<T, NR>(w.x + i);
+    const V pp = vload<T, NR>(w.p + i), vv = vload<T, NR>(w.v + i), tv = vload<T, NR>(w.t + i), r0v = vload<T, NR>(w.r0 + i);
+    V rv = vload<T, NR>(w.r + i);
+    const uint8_t fl = ldg(&sg.op.flag[in ? row : 0]);
+    const auto L = fold_end<FIN_OMEGA, NR>(sg, 1, 2, lb == 0, f, lst);
+    if (!seg_any(L, M_RUN)) return;
+    double pv[2][NR];
+#pragma unroll
+    for (int k = 0; k < NR; ++k) { pv[0][k] = 0.0; pv[1][k] = 0.0; }
+    if (in) {
+        const unsigned run = L.of(M_RUN);
+        const PRow<T> pr = prow_of(sg, row, fl);
+        const bool div = prow_div(sg);
+        V sv;
+#pragma unroll
+        for (int k = 0; k < NR; ++k) setlane(sv, k, -(T)lst.s[k].alpha * lane(vv, k) + lane(rv, k));
+        const V yv = prow_apply<T, NR>(pr, div, pp), zv = prow_apply<T, NR>(pr, div, sv);   // y = P^-1 p, z = P^-1 s
+#pragma unroll
+        for (int k = 0; k < NR; ++k) {
+            if (!((run >> k) & 1u)) continue;
+            const T a = (T)lst.s[k].alpha, om = (T)lst.s[k].omega;
+            T xk = a * lane(yv, k) + lane(xv, k);
+            xk = om * lane(zv, k) + xk;
+            const T rk = -om * lane(tv, k) + lane(sv, k);
+            setlane(xv, k, xk);
+            setlane(rv, k, rk);
+            pv[0][k] = (double)rk * (double)rk;
+            pv[1][k] = (double)lane(r0v, k) * (double)rk;
+        }
+        vstore<T, NR>(w.x + i, xv);
+        vstore<T, NR>(w.r + i, rv);
+    }
+    block_partials<2, NR>(pv, part_of<NR>(sg, 2), lb, sg.nblocks);
+}
+
+// FP64 restart, BiCGStab.h:62-71: r = b - A x (A x already in ax), r0 = r; partial (r, r).
+template <typename T, int NR>
+__global__ __launch_bounds__(kBlock) void k_restart(const Seg<T>* __restrict__ segs, const int* __restrict__ bseg, const T* b,
+                                                    const T* ax, T* r, T* r0) {
+    int lb;
+    int64_t row;
+    const Seg<T>& sg = seg_of(segs, bseg, lb, row);
+    const auto L = lane_stat<NR>(sg);
+    if (!seg_any(L, M_RESTART)) return;
+    double pv[1][NR];
+#pragma unroll
+    for (int k = 0; k < NR; ++k) pv[0][k] = 0.0;
+    if (row < sg.op.D) {
+        const size_t i = (size_t)(sg.off + row * NR);
+        auto bv = vload<T, NR>(b + i);
+        auto av = vload<T, NR>(ax + i);
+        auto rv = vload<T, NR>(r + i);
+        auto r0v = vload<T, NR>(r0 + i);
+#pragma unroll
+        for (int k = 0; k < NR; ++k) {
+            if (!lane_in(L, k, M_RESTART)) continue;
+            T rk = lane(bv, k) - lane(av, k);
+            setlane(rv, k, rk);
+            setlane(r0v, k, rk);
+            pv[0][k] = (double)rk * (double)rk;
+        }
+        vstore<T, NR>(r + i, rv);
+        vstore<T, NR>(r0 + i, r0v);
+    }
+    block_partials<1, NR>(pv, sg.part, lb, sg.nblocks);
+}
+
+// ---------------------------------------------------------------- mixed precision start
+// x64 = 0, r64 = b ; partial (b, b)
+template <int NR>
+__global__ __launch_bounds__(kBlock) void k_mx_start(const Seg<double>* __restrict__ segs, const int* __restrict__ bseg, const double* b,
+                                                     double* x, double* r) {
+    int lb;
+    int64_t row;
+    const Seg<double>& sg = seg_of(segs, bseg, lb, row);
+    double pv[1][NR];
+#pragma unroll
+    for (int k = 0; k < NR; ++k) pv[0][k] = 0.0;
+    if (row < sg.op.D) {
+#pragma unroll
+        for (int k = 0; k < NR; ++k) {
+            const size_t j = lm_at(sg, k, row);
+            const double bk = b[j];
+            r[j] = bk;
+            x[j] = 0.0;
+            pv[0][k] = bk * bk;
+        }
+    }
+    block_partials<1, NR>(pv, sg.part, lb, sg.nblocks);
+}
+
+// FP32 start of the lanes in ST_RESCALE: r32 = r64 * scale, r0 = r32,
+// p = v = x32 = 0 ; partial (r32, r32).
+template <int NR>
+__global__ __launch_bounds__(kBlock) void k_mx_down(const Seg<double>* __restrict__ segs, const int* __restrict__ bseg, const double* r64,
+                                                    float* r, float* r0, float* p, float* v, float* x) {
+    int lb;
+    int64_t row;
+    const Seg<double>& sg = seg_of(segs, bseg, lb, row);
+    const auto L = lane_stat<NR>(sg);
+    if (!seg_any(L, M_RESCALE)) return;
+    double pv[1][NR];
+#pragma unroll
+    for (int k = 0; k < NR; ++k) pv[0][k] = 0.0;
+    if (row < sg.op.D) {
+        const size_t i = (size_t)(sg.off + row * NR);
+        auto ro = vload<float, NR>(r + i);
+        auto r0o = vload<float, NR>(r0 + i);
+        auto po = vload<float, NR>(p + i);
+        auto vo = vload<float, NR>(v + i);
+        auto xo = vload<float, NR>(x + i);
+#pragma unroll
+        for (int k = 0; k < NR; ++k) {
+            if (!lane_in(L, k, M_RESCALE)) continue;
+            const float rk = (float)(r64[lm_at(sg, k, row)] * ldg(&sg.st[k].scale));
+            setlane(ro, k, rk);
+            setlane(r0o, k, rk);
+            setlane(po, k, 0.0f);
+            setlane(vo, k, 0.0f);
+            setlane(xo, k, 0.0f);
+            pv[0][k] = (double)rk * (double)rk;
+        }
+        vstore<float, NR>(r + i, ro);
+        vstore<float, NR>(r0 + i, r0o);
+        vstore<float, NR>(p + i, po);
+        vstore<float, NR>(v + i, vo);
+        vstore<float, NR>(x + i, xo);
+    }
+    block_partials<1, NR>(pv, sg.part, lb, sg.nblocks);
+}
+
+// One workgroup per (segment, rhs lane): the sums of the producing kernel's
+// partials, then the lane's scalar update; copy `in` of the states to copy
+// `out` (the same where they are kept once).
+template <typename T, int NR, int KIND>
+__global__ __launch_bounds__(kBlock) void k_fin(const Seg<T>* __restrict__ segs, int in, int out) {
+    constexpr int NV = FinTraits<KIND>::NV;
+    constexpr unsigned M = FinTraits<KIND>::M;
+    const Seg<T>& sg = segs[blockIdx.x / NR];
+    const int k = (int)(blockIdx.x % NR);
+    if (k >= sg.nr) return;
+    const KState* src = sg.st + (int64_t)in * sg.sst + k;
+    KState* dst = sg.st + (int64_t)out * sg.sst + k;
+    __shared__ double red[NV][kBlock / 64];
+    double tot[NV];
+    const bool act = (M >> ldg(&src->status)) & 1u;   // same test the producer used
+    if (!act && src == dst) return;
+    if (act) part_totals<NV, NR>(sg, part_of<NR>(sg, in), k, red, tot);
+    if (threadIdx.x != 0) return;
+    KState s = *src;
+    if (act) fin_scalar<KIND>(s, tot);
+    *dst = s;
 }
 
 __global__ void k_reset_states(KState* st, int n, double tol2, int max_it, double delta2) {
@@ -1450,6 +1896,10 @@ void launch_reset_states(KState* st, int n, double tol2, int max_it, double delt
 #define LAUNCH_GATHER(kern, ...)                                                                         \
     hipLaunchKernelGGL(kern, dim3(c.gblocks), dim3(kBlock), 0, c.stream, c.segs,                        \
                        c.nseg == 1 ? nullptr : c.bseg + c.nblocks, __VA_ARGS__)
+// The refinement lanes' gathers run the same workgroups segment by segment.
+#define LAUNCH_UPD(kern, ...)                                                                            \
+    hipLaunchKernelGGL(kern, dim3(c.gblocks), dim3(kBlock), 0, c.stream, c.segs,                        \
+                       c.nseg == 1 ? nullptr : c.bseg + c.nblocks + c.gblocks, __VA_ARGS__)
 // E gather of launch c; FL: form P^-1 of the gathered vector (only with
 // shared-stencil tiles, grp_launch).
 #define EGATHER(FL, ...)                                                     \
@@ -1463,7 +1913,9 @@ void launch_reset_states(KState* st, int n, double tol2, int max_it, double delt
         }                                                                    \
         LAUNCH_GATHER((k_egather<T, NR>), __VA_ARGS__);                      \
     } while (0)
-#define FIN(T, NR, KIND) hipLaunchKernelGGL((k_fin<T, NR, KIND>), dim3(c.nseg * NR), dim3(kBlock), 0, c.stream, c.segs, c.nseg)
+#define FIN_COPY(T, NR, KIND, IN, OUT) \
+    hipLaunchKernelGGL((k_fin<T, NR, KIND>), dim3(c.nseg * NR), dim3(kBlock), 0, c.stream, c.segs, IN, OUT)
+#define FIN(T, NR, KIND) FIN_COPY(T, NR, KIND, 0, 0)
 
 // Waves per SIMD the shared-stencil gather is compiled for: four (128 VGPRs)
 // where that does not spill, two (256 VGPRs) for FP32 x 4 and the FP64 shapes.
@@ -1508,7 +1960,8 @@ void Launch<T, NR>::init(const LaunchCfg<T>& c, const T* b, T* x, T* r, T* r0, T
     FIN(T, NR, FIN_INIT);
 }
 template <typename T, int NR>
-void Launch<T, NR>::iteration(const LaunchCfg<T>& c, Vecs<T>& w, bool mixed, const MixVec& mv) {
+template <bool FOLD>
+void Launch<T, NR>::iteration(const LaunchCfg<T>& c, Vecs<T>& w, bool mixed, const MixVec& mv, bool first) {
     // fly: y = P^-1 p and z = P^-1 s are formed where they are read (the
     // gathers' LDS fills, lfinish, xrupdate) rather than stored: launches
     // whose gathers fill LDS from shared-stencil tiles and whose
@@ -1517,54 +1970,95 @@ void Launch<T, NR>::iteration(const LaunchCfg<T>& c, Vecs<T>& w, bool mixed, con
     const int fl = fly ? 1 : 0;
     const T* yp = fly ? w.p : w.y;   // the vector the first gather and lfinish read
     const T* zs = fly ? w.s : w.z;   // ... the second
-    LAUNCH((k_pupdate<T, NR>), w.p, w.v, w.r, w.y, w.x, mv, fl);
+    constexpr int kIter = std::is_same<T, float>::value ? FIN_ITER_MX : FIN_ITER64;
+    constexpr int A = FOLD ? FIN_ALPHA : -1, O = FOLD ? FIN_OMEGA : -1, I = FOLD ? kIter : -1;
+    const int s1 = FOLD ? 1 : 0;   // copy of the states after alpha
+    if (FOLD && !first) LAUNCH((k_pupdate<T, NR, I>), w.p, w.v, w.r, w.y, w.x, mv, fl);
+    else LAUNCH((k_pupdate<T, NR, -1>), w.p, w.v, w.r, w.y, w.x, mv, fl);
     for (int sw = 1; sw < c.jacobi_sweeps; ++sw) {   // y = P^-1 p, Jacobi sweeps after the first
-        apply(c, w.y, w.tmp, w.t, M_RUN);
-        LAUNCH((k_jacobi<T, NR>), w.p, w.t, w.y, sw);
+        EGATHER(false, w.y, w.tmp, M_RUN, MixVec{}, 0);
+        LAUNCH((k_jacobi<T, NR>), w.p, w.tmp, w.y, sw, 0);
     }
     if constexpr (std::is_same<T, float>::value) {
         if (mixed) {   // FP32 lanes in the gather, refinement lanes' FP64 gathers in a launch of their own
-            EGATHER(fly, yp, w.tmp, M_RUN, mv);
-            LAUNCH_GATHER((k_egather_upd<NR>), mv);
+            EGATHER(fly, yp, w.tmp, M_RUN, mv, 0);
+            LAUNCH_UPD((k_egather_upd<NR>), mv, (const float*)nullptr);
         } else {
-            EGATHER(fly, yp, w.tmp, M_STAGE1, mv);
+            EGATHER(fly, yp, w.tmp, M_STAGE1, mv, 0);
         }
     } else {
-        EGATHER(fly, yp, w.tmp, M_STAGE1, mv);
+        EGATHER(fly, yp, w.tmp, M_STAGE1, mv, 0);
     }
-    LAUNCH((k_lfinish<T, NR, 1>), yp, w.tmp, w.v, w.r0, (const T*)nullptr, M_STAGE1, mv, fl);
-    FIN(T, NR, FIN_ALPHA);
-    LAUNCH((k_supdate<T, NR>), w.r, w.v, w.s, w.z, w.r0, w.p, mv, fl);
+    LAUNCH((k_lfinish<T, NR, 1>), yp, w.tmp, w.v, w.r0, (const T*)nullptr, M_STAGE1, mv, fl, 0);
+    if (!FOLD) FIN(T, NR, FIN_ALPHA);
+    LAUNCH((k_supdate<T, NR, A>), w.r, w.v, w.s, w.z, w.r0, w.p, mv, fl);
     for (int sw = 1; sw < c.jacobi_sweeps; ++sw) {   // z = P^-1 s
-        apply(c, w.z, w.tmp, w.t, M_RUN);
-        LAUNCH((k_jacobi<T, NR>), w.s, w.t, w.z, sw);
+        EGATHER(false, w.z, w.tmp, M_RUN, MixVec{}, s1);
+        LAUNCH((k_jacobi<T, NR>), w.s, w.tmp, w.z, sw, s1);
     }
-    EGATHER(fly, zs, w.tmp, M_RUN, mv);
-    LAUNCH((k_lfinish<T, NR, 2>), zs, w.tmp, w.t, w.s, (const T*)w.r, M_STAGE2, mv, fl);
-    FIN(T, NR, FIN_OMEGA);
-    LAUNCH((k_xrupdate<T, NR>), w.x, yp, w.z, w.r, w.s, w.t, w.r0, fl);
-    if (mixed) FIN(T, NR, FIN_ITER_MX);
-    else FIN(T, NR, FIN_ITER64);
+    EGATHER(fly, zs, w.tmp, M_RUN, mv, s1);
+    LAUNCH((k_lfinish<T, NR, 2>), zs, w.tmp, w.t, w.s, (const T*)w.r, M_STAGE2, mv, fl, s1);
+    if (!FOLD) FIN(T, NR, FIN_OMEGA);
+    LAUNCH((k_xrupdate<T, NR, O>), w.x, yp, w.z, w.r, w.s, w.t, w.r0, fl);
+    if (!FOLD) {
+        if (mixed) FIN(T, NR, FIN_ITER_MX);
+        else FIN(T, NR, FIN_ITER64);
+    }
+}
+template <typename T, int NR>
+void Launch<T, NR>::iterations(const LaunchCfg<T>& c, Vecs<T>& w, bool mixed, const MixVec& mv, int n) {
+    if (!c.fold) {
+        for (int i = 0; i < n; ++i) iteration<false>(c, w, mixed, mv, false);
+        return;
+    }
+    bool fused = false;
+    if constexpr (NR == 1) {
+        fused = c.fuse && grp_launch<T, NR>(c) && c.jacobi_sweeps <= 1 && precond_fly();
+        constexpr int kIter = std::is_same<T, float>::value ? FIN_ITER_MX : FIN_ITER64;
+        // waves per SIMD that the fused gathers are compiled for: as many as do not spill
+        constexpr int WPE = sizeof(T) == 4 ? 4 : 2;
+        auto run = [&](auto one) {
+            constexpr bool ONE = decltype(one)::value;
+            const SegArg<T> rows{c.segs, c.bseg, *c.first}, tiles{c.segs, c.bseg + c.nblocks, *c.first};
+            const dim3 gb(c.gblocks), nb(c.nblocks), tb(kBlock);
+            for (int i = 0; i < n; ++i) {
+                if (i == 0) hipLaunchKernelGGL((k_fgather<T, NR, ONE, WPE, 1, -1>), gb, tb, 0, c.stream, tiles, w);
+                else hipLaunchKernelGGL((k_fgather<T, NR, ONE, WPE, 1, kIter>), gb, tb, 0, c.stream, tiles, w);
+                if constexpr (std::is_same<T, float>::value)
+                    if (mixed) LAUNCH_UPD((k_egather_upd<NR>), mv, (const float*)w.x);
+                hipLaunchKernelGGL((k_flfinish<T, NR, ONE, 1>), nb, tb, 0, c.stream, rows, w, mv);
+                hipLaunchKernelGGL((k_fgather<T, NR, ONE, WPE, 2, FIN_ALPHA>), gb, tb, 0, c.stream, tiles, w);
+                hipLaunchKernelGGL((k_flfinish<T, NR, ONE, 2>), nb, tb, 0, c.stream, rows, w, mv);
+                hipLaunchKernelGGL((k_fxrupdate<T, NR, ONE>), nb, tb, 0, c.stream, rows, w);
+            }
+        };
+        if (fused && c.nseg == 1) run(std::true_type{});
+        else if (fused) run(std::false_type{});
+    }
+    for (int i = 0; !fused && i < n; ++i) iteration<true>(c, w, mixed, mv, i == 0);
+    // the loop test of the last iteration, so that copy 0 is current
+    if (mixed) FIN_COPY(T, NR, FIN_ITER_MX, 2, 0);
+    else FIN_COPY(T, NR, FIN_ITER64, 2, 0);
 }
 template <typename T, int NR>
 void Launch<T, NR>::restart(const LaunchCfg<T>& c, Vecs<T>& w) {
     const MixVec none{};
-    EGATHER(false, w.x, w.tmp, M_RESTART, none);
-    LAUNCH((k_lfinish<T, NR, 0>), w.x, w.tmp, w.t, (const T*)nullptr, (const T*)nullptr, M_RESTART, none, 0);
+    EGATHER(false, w.x, w.tmp, M_RESTART, none, 0);
+    LAUNCH((k_lfinish<T, NR, 0>), w.x, w.tmp, w.t, (const T*)nullptr, (const T*)nullptr, M_RESTART, none, 0, 0);
     LAUNCH((k_restart<T, NR>), w.b, w.t, w.r, w.r0);
     FIN(T, NR, FIN_RESTART64);
 }
 template <typename T, int NR>
 void Launch<T, NR>::apply(const LaunchCfg<T>& c, const T* x, T* tmp, T* y, unsigned lanes) {
     const MixVec none{};
-    EGATHER(false, x, tmp, lanes, none);
-    LAUNCH((k_lfinish<T, NR, 0>), x, tmp, y, (const T*)nullptr, (const T*)nullptr, lanes, none, 0);
+    EGATHER(false, x, tmp, lanes, none, 0);
+    LAUNCH((k_lfinish<T, NR, 0>), x, tmp, y, (const T*)nullptr, (const T*)nullptr, lanes, none, 0, 0);
 }
 
 template <typename T>
 void launch_lfinish_plain(const LaunchCfg<T>& c, const T* x, const T* tmp, T* out) {
     const MixVec none{};
-    LAUNCH((k_lfinish<T, 1, 0>), x, tmp, out, (const T*)nullptr, (const T*)nullptr, 0u, none, 0);
+    LAUNCH((k_lfinish<T, 1, 0>), x, tmp, out, (const T*)nullptr, (const T*)nullptr, 0u, none, 0, 0);
 }
 template void launch_lfinish_plain<double>(const LaunchCfg<double>&, const double*, const double*, double*);
 
@@ -1572,7 +2066,7 @@ template <typename T, int NR>
 void launch_egather(const LaunchCfg<T>& c, const T* x, T* out, bool fly) {
     const MixVec none{};
     const bool fl = fly && grp_launch<T, NR>(c) && precond_fly();
-    EGATHER(fl, x, out, 0u, none);
+    EGATHER(fl, x, out, 0u, none, 0);
 }
 
 template <int NR>

@@ -32,12 +32,6 @@
 #ifndef CPMGPU_XCD_RUN
 #define CPMGPU_XCD_RUN 16
 #endif
-#ifndef CPMGPU_GATHER_RUN
-#define CPMGPU_GATHER_RUN 16
-#endif
-#ifndef CPMGPU_LFINISH_RUN
-#define CPMGPU_LFINISH_RUN 16
-#endif
 #ifndef CPMGPU_LDS_ROWS
 #define CPMGPU_LDS_ROWS 2560
 #endif

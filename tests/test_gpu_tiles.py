@@ -19,8 +19,8 @@ def _circle():
     ("Sphere", 0.5, None),          # a few hundred rows: one partly filled run
     ("Sphere", 0.31, None),         # an odd spacing, a last tile that is nearly empty
     ("Sphere", 0.12, "circle"),     # moved columns, ghost rows, identity rows
-    ("Sphere", 0.045, "circle"),    # several runs of 64 items
-    ("Torus", 0.05, None),          # 128 items a tile
+    ("Sphere", 0.045, "circle"),    # full tiles of 256 items
+    ("Torus", 0.05, None),          # 256 items a tile, another shape
     ("Sphere", 0.15, "point"),      # a point's ghost rows (lists of few, scattered rows)
 ])
 def test_tiles_equal_direct_gather(gpu_ctx, monkeypatch, surface, dx, ibc):
