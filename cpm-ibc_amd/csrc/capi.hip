@@ -125,13 +125,15 @@ void* Arena::take(size_t bytes, const char* what) {
 Ctx::Ctx(int dev) : device(dev) {
     HIPCHK(hipSetDevice(dev));
     HIPCHK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-    HIPCHK(hipHostMalloc(&host_states, sizeof(KState) * kHostStates));
+    HIPCHK(hipHostMalloc(&host_states, 2 * sizeof(KState) * kHostStates));
+    for (auto& e : polled) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     scratch_setup(dev);
 }
 Ctx::~Ctx() {
     (void)hipStreamSynchronize(stream);
     ws.clear();
     (void)hipHostFree(host_states);
+    for (auto& e : polled) (void)hipEventDestroy(e);
     (void)hipStreamDestroy(stream);
 }
 
@@ -472,6 +474,20 @@ static void reserve_batch_workspaces(Ctx* ctx, const Op* op, int NR, bool refine
     ctx->workspace("pack", b.pack);
 }
 
+// Iterations a running lane is expected to need until its residual meets the
+// tolerance, at its mean rate so far (a large number while that says
+// nothing; scheduling only).
+static double iterations_left(const KState& s, bool refine) {
+    const double most = 1e6;
+    double rr = s.rr;
+    if (refine) {
+        rr = s.scale > 0 ? s.rr / (s.scale * s.scale) : s.rr_true;
+        if (!(rr < s.rr_true)) rr = s.rr_true;
+    }
+    if (!(s.iters > 0 && s.bsq > 0 && rr > 0 && rr < s.bsq && s.tol2 > 0)) return most;
+    return std::max(0.0, s.iters * (std::log(s.tol2 / rr) / std::log(rr / s.bsq)));
+}
+
 template <int NR>
 static void run_batch(Ctx* ctx, const std::vector<Group>& groups, const std::vector<const double*>& rhs,
                       const std::vector<double*>& xs, const cpm_solve_opts& o, std::vector<cpm_solve_info>& infos) {
@@ -591,33 +607,35 @@ static void run_batch(Ctx* ctx, const std::vector<Group>& groups, const std::vec
     const double delta = o.update_delta > 0 ? std::min(o.update_delta, 0.999) : kDefaultUpdateDelta;
     launch_reset_states(sts, nstate, o.tol * o.tol, o.max_iters, delta * delta, st);
 
-    // Iterations are queued in growing chunks; every kernel skips instances
-    // that have stopped, so the host only looks at the states between chunks.
-    KState* hs = ctx->host_states;
-    auto poll = [&](bool& run, bool& restart) {
-        HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(hs, sts, sizeof(KState) * nstate, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipStreamSynchronize(st));
-        run = restart = false;
-        for (int g = 0; g < G; ++g)
-            for (size_t k = 0; k < groups[g].inst.size(); ++k) {
-                const int s = hs[g * kMaxNR + k].status;
-                run |= s == ST_RUN || (s >= ST_UPDATE && s <= ST_READY);
-                restart |= s == ST_RESTART;
-            }
-    };
-    int chunk = 4;
-    bool run = false, restart = false;
+    // Iterations are queued in chunks, each followed by a copy of the states;
+    // every kernel skips instances that have stopped.  The next chunk is
+    // queued before the host looks at the last one's states, so the GPU never
+    // waits for the host, and its length follows the iterations the slowest
+    // instance is expected to need still (its residual's mean rate so far),
+    // so few are queued in vain: with chunks that doubled to 64, 188
+    // iterations were launched for a solve of 130.
+    // Iterations of many Jacobi sweeps (thousands of launches each) are queued
+    // one at a time, none ahead.
     // graph replays (use_graph): the launches of 4 iterations captured once
     // into a HIP graph and replayed chunk / 4 times per chunk (chunks are
     // multiples of 4)
     // (never inside the allocation-free entry point: instantiating a graph allocates)
-    const bool graph = !ctx->arena && use_graph(refine && G == 1);
+    const bool single = sweeps > 16;
+    const bool graph = !ctx->arena && !single && use_graph(refine && G == 1);
     IterGraph ig;
     const MixVec mv{V64.x, V64.r, V64.b, V64.tmp};
     auto iterations = [&](int n) {
         if (refine) Launch<float, NR>::iterations(c32, V32, true, mv, n);
         else Launch<double, NR>::iterations(c64, V64, false, MixVec{}, n);
+    };
+    auto queue = [&](int chunk, int slot) {
+        if (graph)
+            for (int c = 0; c < chunk; c += 4) ig.run(st, [&] { iterations(4); });
+        else iterations(chunk);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(ctx->host_states + (size_t)slot * Ctx::kHostStates, sts, sizeof(KState) * nstate,
+                              hipMemcpyDeviceToHost, st));
+        HIPCHK(hipEventRecord(ctx->polled[slot], st));
     };
     if (refine) {
         MixedLaunch<NR>::start(c64, V64.b, V64.x, V64.r);
@@ -625,17 +643,28 @@ static void run_batch(Ctx* ctx, const std::vector<Group>& groups, const std::vec
     } else {
         Launch<double, NR>::init(c64, V64.b, V64.x, V64.r, V64.r0, V64.p, V64.v);
     }
-    for (;;) {
-        if (graph)
-            for (int c = 0; c < chunk; c += 4) ig.run(st, [&] { iterations(4); });
-        else iterations(chunk);
-        poll(run, restart);
-        if (restart) {   // rare: handled between chunks, the other instances wait
-            Launch<double, NR>::restart(c64, V64);
-            continue;
-        }
-        if (!run) break;
-        chunk = std::min(chunk * 2, 64);
+    KState* hs = ctx->host_states;
+    int slot = 0, ahead = 4;
+    if (!single) queue(ahead, 0);
+    for (;; slot ^= 1) {
+        if (single) queue(1, slot);
+        else queue(ahead, slot ^ 1);
+        HIPCHK(hipEventSynchronize(ctx->polled[slot]));
+        hs = ctx->host_states + (size_t)slot * Ctx::kHostStates;
+        bool run = false, restart = false;
+        double left = 0.0;   // iterations still expected
+        for (int g = 0; g < G; ++g)
+            for (size_t k = 0; k < groups[g].inst.size(); ++k) {
+                const KState& s = hs[g * kMaxNR + k];
+                restart |= s.status == ST_RESTART;
+                if (!(s.status == ST_RUN || (s.status >= ST_UPDATE && s.status <= ST_READY))) continue;
+                run = true;
+                left = std::max(left, iterations_left(s, refine));
+            }
+        if (!run && !restart) break;   // the chunk in flight finds nothing to do
+        if (restart) Launch<double, NR>::restart(c64, V64);   // rare: handled between chunks, the other instances wait
+        // a third of what is left after the chunk in flight
+        ahead = std::max(4, std::min(32, (int)((left - ahead) / 3.0) & ~3));
     }
     hipLaunchKernelGGL(k_pack, dim3((unsigned)pb.size()), dim3(256), 0, st, dpe, dpb, V64.x, (float*)nullptr, 0);
     HIPCHK(hipGetLastError());

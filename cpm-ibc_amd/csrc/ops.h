@@ -31,7 +31,8 @@ struct Ctx {
     static constexpr int kHostStates = 8192;
     int device = 0;
     hipStream_t stream = nullptr;
-    KState* host_states = nullptr;                            // pinned mirror of device states
+    KState* host_states = nullptr;                            // pinned mirrors of device states, two of kHostStates
+    hipEvent_t polled[2] = {nullptr, nullptr};                // when a solve's copies into them are done
     std::map<std::string, std::unique_ptr<Buffer>> ws;        // grow-only named workspaces
     std::map<void*, int64_t> user_bytes;
     int64_t op_bytes = 0;
