@@ -159,63 +159,140 @@ __global__ void k_tube_normals(int64_t N, const int* ecol, const double* eval, i
 // Breadth-first traversal over tube nodes (IBCSubset.cpp:39-109), level
 // synchronous with the FIFO position reproduced by (parent rank, neighbour
 // slot) claims.  The start node is not pre-marked, as in the reference.
-__global__ void k_tbfs_expand(const int32_t* frontier, int64_t nf, const int32_t* nbr, int32_t* vis, int32_t* cand,
-                              int* ncand) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nf * 6) return;
-    const int64_t fi = t / 6;
-    const int slot = (int)(t - fi * 6);
-    const int32_t nb = nbr[6 * (int64_t)frontier[fi] + slot];
-    if (nb < 0) return;
-    const int32_t v = __hip_atomic_load(vis + nb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (v < kCand || v == kOutside) return;
-    const int32_t old = atomicMin(vis + nb, kCand + (int32_t)t);
-    if (old == kUnvisited) cand[atomicAdd(ncand, 1)] = nb;
-}
+//
+// One workgroup walks one curve, all its levels in one launch, the curves of
+// a problem side by side.  A level's frontier is the band's cross-section
+// (about 300 nodes, whatever the grid spacing) and its candidates' closest
+// points are chains of dependent loads, so a level is bound by latency, not
+// by the one CU it runs on: seven launches and two host waits a level took
+// about 90 us (357 levels of three curves: 30 of the 38 ms of a problem).
+// Polylines whose hierarchy fits are copied to LDS first, which the
+// traversals then read.
+constexpr int kBfsThreads = 512;
+constexpr int kBfsLds = 120 * 1024;   // one workgroup per CU
 
-__global__ void k_tbfs_eval(const int32_t* cand, const int* ncand, const int64_t* rec, int64_t N1d, double xs, double dx,
-                            SurfDev sd, double radius, int32_t* vis, int32_t* slot, double* ccp, double* cdist,
-                            int32_t* cbdy) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= *ncand) return;
-    const int32_t nb = cand[i];
-    double x[3], c[3], d;
-    int b;
-    node_coords(rec[nb], N1d, xs, dx, x);
-    cp_surface(sd, x, c, d, b);
-    if (d < radius) {
-        slot[vis[nb] - kCand] = (int32_t)i;
-        for (int k = 0; k < 3; ++k) ccp[3 * i + k] = c[k];
-        cdist[i] = d;
-        cbdy[i] = b;
-    } else {
-        vis[nb] = kOutside;
+struct BfsCurve {
+    SurfDev sd;
+    int nnodes, nverts, nprim;   // polyline hierarchy (0: none)
+    int32_t start;
+    int32_t* vis;                // [N] kUnvisited; members end with their position, others above kCand
+    int32_t* cand;               // [N]
+    int32_t* slot;               // [6 fcap], as the four below
+    double* ccp;
+    double* cdist;
+    int32_t* cbdy;
+    int64_t cap;                 // room of t_set .. t_bdy
+    int fcap;                    // longest frontier
+    int32_t* t_set;
+    double* t_cpc;
+    double* t_dist;
+    int32_t* t_bdy;
+    int32_t* result;             // [2]: members; 1 the outputs, 2 the frontier did not fit
+};
+
+__global__ __launch_bounds__(kBfsThreads) void k_tagging_bfs(const BfsCurve* curves, const int32_t* nbr, const int64_t* rec,
+                                                             int64_t N1d, double xs, double dx, double radius) {
+    __shared__ __align__(16) char lds[kBfsLds];
+    __shared__ int ncand, wsum[kBfsThreads / 64];
+    const BfsCurve& q = curves[blockIdx.x];
+    const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6;
+    SurfDev sd = q.sd;
+    const size_t bn = sizeof(BvhNode) * (size_t)q.nnodes, bv = sizeof(double) * 3 * (size_t)q.nverts,
+                 bp = sizeof(int) * (size_t)q.nprim;
+    if (q.nnodes > 0 && bn + bv + bp <= kBfsLds) {   // multiples of 4 bytes
+        int* dst = reinterpret_cast<int*>(lds);
+        const int* src[3] = {reinterpret_cast<const int*>(sd.mesh.nodes), reinterpret_cast<const int*>(sd.mesh.v), sd.mesh.prim};
+        const size_t words[3] = {bn / 4, bv / 4, bp / 4};
+        size_t at = 0;
+        for (int a = 0; a < 3; ++a) {
+            for (size_t k = t; k < words[a]; k += kBfsThreads) dst[at + k] = src[a][k];
+            at += words[a];
+        }
+        sd.mesh.nodes = reinterpret_cast<const BvhNode*>(lds);
+        sd.mesh.v = reinterpret_cast<const double*>(lds + bn);
+        sd.mesh.prim = reinterpret_cast<const int*>(lds + bn + bv);
+    }
+    int64_t f0 = 0, nt = 0;
+    int nf = 1;
+    bool seed = true;
+    while (nf > 0) {   // nf, nt, f0 are the same on every thread
+        const int ns = nf * 6;
+        if (t == 0) ncand = 0;
+        for (int k = t; k < ns; k += kBfsThreads) q.slot[k] = -1;
+        __syncthreads();
+        // claim the neighbours: the lowest (parent rank, neighbour slot) wins
+        for (int k = t; k < ns; k += kBfsThreads) {
+            const int fi = k / 6;
+            const int32_t node = seed ? q.start : q.t_set[f0 + fi];
+            const int32_t nb = nbr[6 * (int64_t)node + (k - 6 * fi)];
+            if (nb < 0) continue;
+            const int32_t v = __hip_atomic_load(q.vis + nb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (v < kCand || v == kOutside) continue;
+            if (atomicMin(q.vis + nb, kCand + k) == kUnvisited) q.cand[atomicAdd(&ncand, 1)] = nb;
+        }
+        __syncthreads();
+        const int nc = ncand;
+        for (int i = t; i < nc; i += kBfsThreads) {
+            const int32_t nb = q.cand[i];
+            double x[3], c[3], d;
+            int b;
+            node_coords(rec[nb], N1d, xs, dx, x);
+            cp_surface(sd, x, c, d, b);
+            if (d < radius) {
+                q.slot[__hip_atomic_load(q.vis + nb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - kCand] = i;
+                for (int k = 0; k < 3; ++k) q.ccp[3 * i + k] = c[k];
+                q.cdist[i] = d;
+                q.cbdy[i] = b;
+            } else {
+                __hip_atomic_store(q.vis + nb, kOutside, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        __syncthreads();
+        // the occupied slots in order are the next level
+        int64_t at = nt;
+        for (int k0 = 0; k0 < ns; k0 += kBfsThreads) {
+            const int k = k0 + t;
+            const int ci = k < ns ? q.slot[k] : -1;
+            const unsigned long long m = __ballot(ci >= 0);
+            if (lane == 0) wsum[wave] = __popcll(m);
+            __syncthreads();
+            int64_t p = at + __popcll(m & ((1ull << lane) - 1ull));
+            for (int w = 0; w < kBfsThreads / 64; ++w) {
+                if (w < wave) p += wsum[w];
+                at += wsum[w];
+            }
+            if (ci >= 0 && p < q.cap) {
+                const int32_t nb = q.cand[ci];
+                __hip_atomic_store(q.vis + nb, (int32_t)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                q.t_set[p] = nb;
+                for (int d = 0; d < 3; ++d) q.t_cpc[3 * p + d] = q.ccp[3 * ci + d];
+                q.t_dist[p] = q.cdist[ci];
+                q.t_bdy[p] = q.cbdy[ci];
+            }
+            __syncthreads();
+        }
+        const int64_t found = at - nt;
+        if (at > q.cap || found > q.fcap) {
+            if (t == 0) q.result[1] = at > q.cap ? 1 : 2;
+            return;
+        }
+        f0 = nt;
+        nf = (int)found;
+        nt = at;
+        seed = false;
+    }
+    if (t == 0) {
+        q.result[0] = (int32_t)nt;
+        q.result[1] = 0;
     }
 }
 
-__global__ void k_tbfs_emit(const int32_t* slot, int64_t ns, const int* boff, const int32_t* cand, const double* ccp,
-                            const double* cdist, const int32_t* cbdy, int64_t base, int32_t* vis, int32_t* t_set,
-                            double* t_cpc, double* t_dist, int32_t* t_bdy, int32_t* next) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int32_t ci = i < ns ? slot[i] : -1;
-    const int occ = ci >= 0;
-    const unsigned long long m = __ballot(occ);
-    __shared__ int ws[4];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    if (lane == 0) ws[w] = __popcll(m);
-    __syncthreads();
-    if (!occ) return;
-    int before = boff[blockIdx.x];
-    for (int k = 0; k < w; ++k) before += ws[k];
-    before += __popcll(m & ((1ull << lane) - 1ull));
-    const int64_t t = base + before;
-    const int32_t nb = cand[ci];
-    vis[nb] = (int32_t)t;
-    t_set[t] = nb;
-    for (int k = 0; k < 3; ++k) t_cpc[3 * t + k] = ccp[3 * ci + k];
-    t_dist[t] = cdist[ci];
-    t_bdy[t] = cbdy[ci];
-    next[before] = nb;   // the frontier holds tube indices
+// Subset index of every tube node: a member's position, -1 elsewhere.
+__global__ void k_sub_index(int64_t N, const int32_t* vis, int32_t* sub) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= N) return;
+    const int32_t v = vis[i];
+    sub[i] = v >= kCand || v < 0 ? -1 : v;
 }
 
 // ---------------------------------------------------------------- ordered selection
@@ -613,12 +690,10 @@ static int64_t select_flags(Ctx* ctx, const uint8_t* flag, int64_t n, int32_t* o
     return h;
 }
 
-// Tagging subset of one curve (IBCSubset::ComputeSubset, IBCSubset.cpp:12-36).
-static void tagging_subset(Tube* t, Ctx* ctx, IbcData& I, const double* tube_normals) {
-    const hipStream_t st = ctx->stream;
-    const int64_t N = t->N;
-    const double radius = 2.0 * t->r_t;
-    // FindStartingPoint (IBCSubset.cpp:112-116): nearest tube node of the curve's first parameterisation point
+// Tube node the tagging subset of one curve starts from: FindStartingPoint
+// (IBCSubset.cpp:112-116), the nearest tube node of the curve's first
+// parameterisation point.
+static int32_t tagging_start(const Tube* t, const IbcData& I) {
     const double* p0 = I.spec.surf.type == "Polyline" ? I.spec.surf.verts.data() : nullptr;
     double x0[3];
     if (p0) { x0[0] = p0[0]; x0[1] = p0[1]; x0[2] = p0[2]; }
@@ -650,74 +725,126 @@ static void tagging_subset(Tube* t, Ctx* ctx, IbcData& I, const double* tube_nor
     HIPCHK(hipMemcpy(&start, t->gidx.as<int32_t>() + l0, 4, hipMemcpyDeviceToHost));
     if (start < 0 || start >= kCand) throw GeomError("IBC start point is not in the tube");
 
-    int32_t* vis = reinterpret_cast<int32_t*>(ctx->workspace("ibc_vis", N * 4));
-    hipLaunchKernelGGL(k_fill_i32, dim3(std::min<unsigned>(nblk(N), 4096)), dim3(256), 0, st, vis, N, kUnvisited);
-    int64_t cap = 1 << 14;
-    realloc<int32_t>(I.t_set, cap);
-    realloc<double>(I.t_cpc, cap * 3);
-    realloc<double>(I.t_dist, cap);
-    realloc<int32_t>(I.t_bdy, cap);
-    std::unique_ptr<Buffer> fr(new Buffer(cap * 4)), fr2(new Buffer(cap * 4));
-    HIPCHK(hipMemcpyAsync(fr->p, &start, 4, hipMemcpyHostToDevice, st));
-    int* dint = reinterpret_cast<int*>(ctx->workspace("ibc_int", 64));
-    int* hbuf = reinterpret_cast<int*>(ctx->host_states);
-    int64_t nt = 0, nf = 1;
-    while (nf > 0) {
-        HIPCHK(hipStreamSynchronize(st));
-        const int64_t ns = nf * 6, nb = (ns + 255) / 256;
-        int32_t* cand = reinterpret_cast<int32_t*>(ctx->workspace("ibc_cand", ns * 4));
-        int32_t* slot = reinterpret_cast<int32_t*>(ctx->workspace("ibc_slot", ns * 4));
-        double* ccp = ctx->workspace("ibc_ccp", ns * 24);
-        double* cdist = ctx->workspace("ibc_cdist", ns * 8);
-        int32_t* cbdy = reinterpret_cast<int32_t*>(ctx->workspace("ibc_cbdy", ns * 4));
-        int* bcount = reinterpret_cast<int*>(ctx->workspace("ibc_bcount", nb * 4));
-        HIPCHK(hipMemsetAsync(dint, 0, 16, st));
-        hipLaunchKernelGGL(k_fill_i32, dim3(std::min<unsigned>((unsigned)nb, 4096)), dim3(256), 0, st, slot, ns, -1);
-        hipLaunchKernelGGL(k_tbfs_expand, dim3((unsigned)nb), dim3(256), 0, st, fr->as<int32_t>(), nf,
-                           t->nbr.as<int32_t>(), vis, cand, dint);
-        hipLaunchKernelGGL(k_tbfs_eval, dim3((unsigned)nb), dim3(256), 0, st, cand, dint, t->rec.as<int64_t>(), t->N1d,
-                           t->xstart, t->dx, I.sd, radius, vis, slot, ccp, cdist, cbdy);
-        hipLaunchKernelGGL(k_count, dim3((unsigned)nb), dim3(256), 0, st, slot, ns, bcount);
-        hipLaunchKernelGGL(k_scan, dim3(1), dim3(256), 0, st, bcount, nb, dint + 1);
-        HIPCHK(hipMemcpyAsync(hbuf, dint, 8, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipStreamSynchronize(st));
-        const int64_t cnt = hbuf[1];
-        if (nt + cnt > cap || cnt > cap) {
-            int64_t nc = cap;
-            while (nc < nt + cnt || nc < cnt) nc *= 2;
-            auto grow = [&](Buffer& b, size_t esz) {
-                Buffer nbuf(nc * esz);
-                if (nt) HIPCHK(hipMemcpy(nbuf.p, b.p, nt * esz, hipMemcpyDeviceToDevice));
-                std::swap(b.p, nbuf.p);
-                std::swap(b.bytes, nbuf.bytes);
-            };
-            grow(I.t_set, 4);
-            grow(I.t_cpc, 24);
-            grow(I.t_dist, 8);
-            grow(I.t_bdy, 4);
-            std::unique_ptr<Buffer> a(new Buffer(nc * 4)), b(new Buffer(nc * 4));
-            HIPCHK(hipMemcpy(a->p, fr->p, nf * 4, hipMemcpyDeviceToDevice));
-            fr.swap(a);
-            fr2.swap(b);
-            cap = nc;
+    return start;
+}
+
+// Length of a curve (0: a point).
+static double curve_length(const IbcSpec& c) {
+    const auto& P = c.surf.params;
+    if (c.surf.type == "Circle3D") return 2 * M_PI * P[0];
+    if (c.surf.type == "Arc") return P[0] * (P[2] - P[1]);
+    double len = 0.0;
+    const std::vector<double>& v = c.surf.verts;
+    for (size_t k = 3; k + 2 < v.size(); k += 3)
+        len += std::sqrt((v[k] - v[k - 3]) * (v[k] - v[k - 3]) + (v[k + 1] - v[k - 2]) * (v[k + 1] - v[k - 2]) +
+                         (v[k + 2] - v[k - 1]) * (v[k + 2] - v[k - 1]));
+    return len;
+}
+
+// Members of the curves' tagging subsets (IBCSubset::ComputeSubset,
+// IBCSubset.cpp:12-109), the curves in one launch as far as their node arrays
+// stay within 512 MB.
+static void tagging_members(Tube* t, Ctx* ctx, std::vector<IbcData>& ibc) {
+    const hipStream_t st = ctx->stream;
+    const int64_t N = t->N;
+    const double radius = 2.0 * t->r_t;
+    const size_t most = std::max<size_t>(1, (size_t(512) << 20) / ((size_t)N * 8));
+    auto r256 = [](size_t n) { return (n + 255) & ~size_t(255); };
+    for (size_t c0 = 0; c0 < ibc.size(); c0 += most) {
+        const size_t n = std::min(most, ibc.size() - c0);
+        // outputs hold the band around the curve (about 16.5 x 8.25 nodes a grid spacing of its
+        // length, and its two ends) and half as much again; too small a guess is doubled
+        std::vector<int64_t> cap(n);
+        std::vector<int32_t> start(n);
+        std::vector<bool> todo(n, true);
+        for (size_t k = 0; k < n; ++k) {
+            const IbcData& I = ibc[c0 + k];
+            start[k] = tagging_start(t, I);
+            cap[k] = std::min<int64_t>(N, (int64_t)(1.5 * 136.0 * (curve_length(I.spec) / t->dx + 16.0)));
         }
-        hipLaunchKernelGGL(k_tbfs_emit, dim3((unsigned)nb), dim3(256), 0, st, slot, ns, bcount, cand, ccp, cdist, cbdy, nt,
-                           vis, I.t_set.as<int32_t>(), I.t_cpc.as<double>(), I.t_dist.as<double>(),
-                           I.t_bdy.as<int32_t>(), fr2->as<int32_t>());
-        fr.swap(fr2);
-        nt += cnt;
-        nf = cnt;
+        int fcap = 4096;
+        for (bool again = true; again;) {
+            again = false;
+            std::vector<BfsCurve> h;
+            std::vector<size_t> who;
+            const size_t slots = 6 * (size_t)fcap;
+            const size_t one = r256((size_t)N * 4) * 2 + r256(slots * 4) * 2 + r256(slots * 24) + r256(slots * 8);
+            for (size_t k = 0; k < n; ++k)
+                if (todo[k]) who.push_back(k);
+            char* w = reinterpret_cast<char*>(ctx->workspace("ibc_bfs", one * who.size()));
+            char* tab = reinterpret_cast<char*>(ctx->workspace("ibc_bfs_tab", r256(sizeof(BfsCurve) * who.size()) + 8 * who.size()));
+            int32_t* res = reinterpret_cast<int32_t*>(tab + r256(sizeof(BfsCurve) * who.size()));
+            for (size_t j = 0; j < who.size(); ++j) {
+                IbcData& I = ibc[c0 + who[j]];
+                const int64_t cp = cap[who[j]];
+                if (I.t_set.bytes < (size_t)cp * 4) {
+                    realloc<int32_t>(I.t_set, cp);
+                    realloc<double>(I.t_cpc, cp * 3);
+                    realloc<double>(I.t_dist, cp);
+                    realloc<int32_t>(I.t_bdy, cp);
+                }
+                char* p = w + one * j;
+                auto carve = [&](size_t bytes) {
+                    char* a = p;
+                    p += r256(bytes);
+                    return a;
+                };
+                BfsCurve q{};
+                q.sd = I.sd;
+                q.nnodes = I.bvh.nnodes;
+                q.nprim = I.bvh.ntri;
+                q.nverts = I.bvh.nnodes > 0 ? (int)(I.spec.surf.verts.size() / 3) : 0;
+                q.start = start[who[j]];
+                q.vis = reinterpret_cast<int32_t*>(carve((size_t)N * 4));
+                q.cand = reinterpret_cast<int32_t*>(carve((size_t)N * 4));
+                q.slot = reinterpret_cast<int32_t*>(carve(slots * 4));
+                q.cbdy = reinterpret_cast<int32_t*>(carve(slots * 4));
+                q.ccp = reinterpret_cast<double*>(carve(slots * 24));
+                q.cdist = reinterpret_cast<double*>(carve(slots * 8));
+                q.cap = cp;
+                q.fcap = fcap;
+                q.t_set = I.t_set.as<int32_t>();
+                q.t_cpc = I.t_cpc.as<double>();
+                q.t_dist = I.t_dist.as<double>();
+                q.t_bdy = I.t_bdy.as<int32_t>();
+                q.result = res + 2 * j;
+                h.push_back(q);
+                hipLaunchKernelGGL(k_fill_i32, dim3(std::min<unsigned>(nblk(N), 4096)), dim3(256), 0, st, q.vis, N, kUnvisited);
+            }
+            HIPCHK(hipMemcpyAsync(tab, h.data(), sizeof(BfsCurve) * h.size(), hipMemcpyHostToDevice, st));
+            hipLaunchKernelGGL(k_tagging_bfs, dim3((unsigned)h.size()), dim3(kBfsThreads), 0, st,
+                               reinterpret_cast<const BfsCurve*>(tab), t->nbr.as<int32_t>(), t->rec.as<int64_t>(), t->N1d,
+                               t->xstart, t->dx, radius);
+            for (size_t j = 0; j < who.size(); ++j) {
+                IbcData& I = ibc[c0 + who[j]];
+                if (I.t_sub.bytes != (size_t)N * 4) realloc<int32_t>(I.t_sub, N);
+                hipLaunchKernelGGL(k_sub_index, dim3(nblk(N)), dim3(256), 0, st, N, h[j].vis, I.t_sub.as<int32_t>());
+            }
+            HIPCHK(hipGetLastError());
+            std::vector<int32_t> r(2 * who.size());
+            HIPCHK(hipMemcpyAsync(r.data(), res, 4 * r.size(), hipMemcpyDeviceToHost, st));
+            HIPCHK(hipStreamSynchronize(st));
+            bool wider = false;
+            for (size_t j = 0; j < who.size(); ++j) {
+                const size_t k = who[j];
+                if (r[2 * j + 1] == 0) {
+                    ibc[c0 + k].nt = r[2 * j];
+                    todo[k] = false;
+                    continue;
+                }
+                again = true;
+                if (r[2 * j + 1] == 1) cap[k] = std::min<int64_t>(N, 2 * cap[k]);
+                else wider = true;
+            }
+            if (wider) fcap *= 2;
+        }
     }
-    HIPCHK(hipStreamSynchronize(st));
-    I.nt = nt;
-    // subset index of every tube node: vis holds it for members, sentinels elsewhere
-    realloc<int32_t>(I.t_sub, N);
-    {
-        std::vector<int32_t> h(N);
-        HIPCHK(hipMemcpy(h.data(), vis, N * 4, hipMemcpyDeviceToHost));
-        for (auto& v : h) if (v >= kCand || v < 0) v = -1;
-        HIPCHK(hipMemcpy(I.t_sub.p, h.data(), N * 4, hipMemcpyHostToDevice));
-    }
+}
+
+// Stencil directions of one curve's tagging subset (IBCSubset.cpp:120-268).
+static void tagging_directions(Tube* t, Ctx* ctx, IbcData& I, const double* tube_normals) {
+    const hipStream_t st = ctx->stream;
+    const int64_t nt = I.nt;
     if (nt == 0) throw GeomError("IBC tagging subset is empty");
     // cp_diff and its on-curve fix-up
     realloc<double>(I.t_cpdiff, nt * 3);
@@ -805,8 +932,9 @@ Problem* problem_build(Tube* t, const std::vector<IbcSpec>& specs, Ctx* bctx) {
             }
             I.sd = make_surfdev(I.spec.surf, I.verts.as<double>());
         }
-        tagging_subset(t, ctx, I, P->normals.as<double>());
     }
+    tagging_members(t, ctx, P->ibc);
+    for (auto& I : P->ibc) tagging_directions(t, ctx, I, P->normals.as<double>());
     for (auto& I : P->ibc) dof_subset(t, ctx, I);
     // IBCSubsets::IBCStartingColumns / TotalDOFs (IBCSubsets.cpp:74-116)
     int64_t G_ = 0, K_ = 0, ident_start = 0;

@@ -1864,14 +1864,20 @@ __global__ __launch_bounds__(kBlock) void k_fin(const Seg<T>* __restrict__ segs,
     const KState* src = sg.st + (int64_t)in * sg.sst + k;
     KState* dst = sg.st + (int64_t)out * sg.sst + k;
     __shared__ double red[NV][kBlock / 64];
+    __shared__ KState s;
     double tot[NV];
+    // the state's words, loaded with its status and the partials (loaded
+    // after the sums they cost the launch another memory latency)
+    constexpr int W = (int)(sizeof(KState) / 4);
+    const int t = (int)threadIdx.x;
+    const int word = t < W ? ldg(reinterpret_cast<const int*>(src) + t) : 0;
     const bool act = (M >> ldg(&src->status)) & 1u;   // same test the producer used
     if (!act && src == dst) return;
+    if (t < W) reinterpret_cast<int*>(&s)[t] = word;
     if (act) part_totals<NV, NR>(sg, part_of<NR>(sg, in), k, red, tot);
-    if (threadIdx.x != 0) return;
-    KState s = *src;
-    if (act) fin_scalar<KIND>(s, tot);
-    *dst = s;
+    if (act && t == 0) fin_scalar<KIND>(s, tot);
+    __syncthreads();
+    if (t < W) stg(reinterpret_cast<int*>(dst) + t, reinterpret_cast<const int*>(&s)[t]);
 }
 
 __global__ void k_reset_states(KState* st, int n, double tol2, int max_it, double delta2) {
