@@ -995,9 +995,38 @@ static void solve_stream(Op* op, const std::vector<const double*>& rhs, const st
     record_fp32(op->ctx, ops, infos);
 }
 
+// Whether applies and steps run on the callers' vectors in place (krylov.h).
+static bool in_place(const Op* op) {
+    grp_refresh_override();
+    return op->perm.p && op->nD == 0 && grp_gather<double, 1>(op->ngt);
+}
+
+// Whether two vectors of the operator's rows share no element (steps in
+// place write one while other threads still read the other).
+static bool apart(const Op* op, const double* a, const double* b) { return a + op->D <= b || b + op->D <= a; }
+
+// The operator as the only segment of a launch, with (m, n).
+static Seg<double> whole_seg(const Op* op, double m, double n) {
+    Seg<double> h{};
+    fill_seg(h, op, 0, row_blocks(op), 1, nullptr, nullptr);
+    h.m = m;
+    h.n = n;
+    return h;
+}
+
+static HeldRows held_rows(const Op* op) {
+    return HeldRows{op->nh, op->hw, op->hrow.as<int>(), op->hcol.as<int>(), op->hval.as<double>()};
+}
+
 void multiply(Op* op, const double* dx, double* dy, double m, double n) {
     Ctx* ctx = op->ctx;
     const hipStream_t st = ctx->stream;
+    if (in_place(op) && apart(op, dx, dy)) {
+        double* tmp = ctx->workspace("mul_tmp", sizeof(double) * op->D * 3);
+        launch_apply_caller(whole_seg(op, m, n), op->perm.as<int>(), dx, tmp, dy, st);
+        HIPCHK(hipGetLastError());
+        return;
+    }
     const int nblocks = (int)((op->D + kBlock - 1) / kBlock);
     char* tb = reinterpret_cast<char*>(ctx->workspace("mul_tables", 8192 + sizeof(int) * nblocks));
     Seg<double> h{};
@@ -1198,6 +1227,11 @@ static void extension(Op* op, const StepTables& t, const double* z, double* y) {
 
 void apply_E(Op* op, const double* x, double* y) {
     const hipStream_t st = op->ctx->stream;
+    if (in_place(op)) {
+        launch_extend_caller(whole_seg(op, 1.0, 0.0), op->perm.as<int>(), x, y, st);
+        HIPCHK(hipGetLastError());
+        return;
+    }
     const StepTables t = step_tables(op, "applyE_tables", {0.0}, {pack_in(x), pack_out(y)});
     double* w = op->ctx->workspace("applyE_vecs", sizeof(double) * op->D * 2);
     hipLaunchKernelGGL(k_pack, dim3(t.nblocks), dim3(256), 0, st, t.pe, t.bseg, w, (float*)nullptr, 1);
@@ -1218,6 +1252,14 @@ static void heat_step(Op* op, int method, double dt, const double* d_g, double* 
     Ctx* ctx = op->ctx;
     const hipStream_t st = ctx->stream;
     const int64_t D = op->D;
+    if (method == 0 && in_place(op) && apart(op, d_u, d_g)) {
+        double* z = ctx->workspace("heat_vecs", sizeof(double) * D * 3);
+        launch_step_caller<1>(whole_seg(op, 1.0, dt), held_rows(op), op->perm.as<int>(), &d_u, &d_g, &dt, 0.0, 0.0, 0.0, z, st);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipStreamSynchronize(st));
+        if (info) *info = cpm_solve_info{CPM_SOLVE_CONVERGED, 0, 0, 0, 0.0};
+        return;
+    }
     if (method == 0) {
         // internal order: x = P u ; z = x + dt Lfull x ; y = E z ; u = P^T y ; Dirichlet rows
         const StepTables t = step_tables(op, "heat_tables", {dt}, {pack_in(d_u), pack_out(d_u)});
@@ -1275,6 +1317,24 @@ static void rd_step(Op* op, const cpm_rd_params& p, int nf, double* const* d_u, 
     const unsigned nb = (unsigned)((D + 255) / 256);
     if (p.method == 0) {
         double* w = ctx->workspace("rd_vecs", sizeof(double) * D * 4);
+        bool free = in_place(op);
+        for (int f = 0; f < nf; ++f)
+            for (const double* o : {(const double*)d_u[f], (const double*)d_v[f]})
+                free = free && apart(op, o, d_gu) && apart(op, o, d_gv) && apart(op, d_u[f], d_v[f]);
+        if (free) {
+            const double coef[2] = {p.nu_u * p.dt, p.nu_v * p.dt};
+            const double* g[2] = {d_gu, d_gv};
+            for (int f = 0; f < nf; ++f) {
+                double* uv[2] = {d_u[f], d_v[f]};
+                launch_step_caller<2>(whole_seg(op, 1.0, 0.0), held_rows(op), op->perm.as<int>(), uv, g, coef, p.dt, p.F, p.k, w,
+                                      st);
+            }
+            HIPCHK(hipGetLastError());
+            HIPCHK(hipStreamSynchronize(st));
+            if (infos)
+                for (int i = 0; i < 2 * nf; ++i) infos[i] = cpm_solve_info{CPM_SOLVE_CONVERGED, 0, 0, 0, 0.0};
+            return;
+        }
         double *xu = w, *xv = w + D, *zu = w + 2 * D, *zv = w + 3 * D;
         for (int f = 0; f < nf; ++f) {
             const StepTables t = step_tables(op, "rd_tables", {p.nu_u * p.dt, p.nu_v * p.dt},

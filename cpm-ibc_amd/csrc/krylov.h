@@ -85,6 +85,24 @@ struct MixedLaunch {
 template <typename T>
 void launch_lfinish_plain(const LaunchCfg<T>& c, const T* x, const T* tmp, T* out);
 
+// Operators with shared-stencil tiles on callers' vectors (perm: the
+// operator's row -> the caller's): y = A x (tmp: D doubles); y = E x
+// (identity rows copy); an explicit step u <- E (u + coef Lfull u), identity
+// rows <- g, of one field (heat) or of two with the Gray-Scott reaction (z:
+// NR D doubles).  sg: the operator's segment, only D, op, m, n and nblocks
+// are read.
+void launch_apply_caller(const Seg<double>& sg, const int* perm, const double* x, double* tmp, double* y, hipStream_t st);
+void launch_extend_caller(const Seg<double>& sg, const int* perm, const double* x, double* y, hipStream_t st);
+struct HeldRows {   // Lfull rows of identity rows (Op::hrow ..)
+    int64_t nh;
+    int hw;
+    const int *row, *col;
+    const double* val;
+};
+template <int NR>
+void launch_step_caller(const Seg<double>& sg, const HeldRows& h, const int* perm, double* const* u, const double* const* g,
+                        const double* coef, double dt, double F, double k, double* z, hipStream_t st);
+
 // E-gather alone (identity rows copy), for measurement; fly: of P^-1 x, as
 // the iterations gather (where the launch uses shared-stencil tiles).
 template <typename T, int NR>

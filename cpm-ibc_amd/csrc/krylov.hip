@@ -719,12 +719,51 @@ struct SrcX64 {
     __device__ __forceinline__ V value(const Raw& q, int64_t, bool) const { return q.x + (double)q.d / scale; }
 };
 
-// One shared-stencil tile of E x, ob[row] = (E x)_row with x from src: thread
+// x of a caller's vector, whose row perm[r] the operator's row r is.
+struct SrcPerm {
+    typedef double V;
+    typedef double Raw;
+    const double* x;
+    const int* perm;
+    __device__ __forceinline__ Raw load(int64_t row) const { return ldg(x + ldg(perm + row)); }
+    __device__ __forceinline__ V value(const Raw& v, int64_t, bool) const { return v; }
+};
+
+// Where a tile's rows go: to out, interleaved like x; or, DstPerm, to NR
+// caller's vectors, identity rows taking the values of g (null: as gathered).
+template <typename T, int NR>
+struct DstPlain {
+    static constexpr bool kSkipIdentity = false;
+    T* out;
+    __device__ __forceinline__ void store(int64_t row, const typename VT<T, NR>::type& v) const {
+        vstore<T, NR>(out + (size_t)row * NR, v);
+    }
+    __device__ __forceinline__ void identity(int64_t) const {}
+};
+template <int NR, bool HELD>
+struct DstPerm {
+    static constexpr bool kSkipIdentity = HELD;
+    double* out[NR];
+    const double* g[NR];
+    const int* perm;
+    __device__ __forceinline__ void store(int64_t row, const typename VT<double, NR>::type& v) const {
+        const int c = ldg(perm + row);
+#pragma unroll
+        for (int k = 0; k < NR; ++k) stg(out[k] + c, (double)lane(v, k));
+    }
+    __device__ __forceinline__ void identity(int64_t row) const {
+        const int c = ldg(perm + row);
+#pragma unroll
+        for (int k = 0; k < NR; ++k) stg(out[k] + c, ldg(g[k] + c));
+    }
+};
+
+// One shared-stencil tile of E x, (E x)_row to dst with x from src: thread
 // t takes the item at place tile kBlock + t.  mid(src), called once the loads
 // are under way, completes src (the scalars its values need) and says whether
 // to go on (the same on every thread).
-template <typename T, int NR, int LR, typename V, typename Src, typename Mid>
-__device__ __forceinline__ void egather_grp_tile(const OpView<T>& op, int tile, Src& src, T* ob, const LdsRows<V>& lrows,
+template <typename T, int NR, int LR, typename V, typename Src, typename Dst, typename Mid>
+__device__ __forceinline__ void egather_grp_tile(const OpView<T>& op, int tile, Src& src, const Dst& dst, const LdsRows<V>& lrows,
                                                  Mid&& mid) {
     // Loads in two rounds, each issued as soon as the previous one's values
     // are in: the list entries (first: the x rows wait on them), the item's
@@ -779,18 +818,18 @@ __device__ __forceinline__ void egather_grp_tile(const OpView<T>& op, int tile, 
         egather_grp_lds<T, V, NR>(m, n, lrows, acc);
 #pragma unroll
         for (int g = 0; g < kGrpRows; ++g)
-            if (g < n) vstore<T, NR>(ob + (size_t)m.row[g] * NR, acc[g]);
+            if (g < n) dst.store(m.row[g], acc[g]);
     } else if (kind == 1) {
         V acc = (V)(T)0;
         egather_grp_exc<T, V>(m.w[0], xval, mx, lrows, acc);
-        vstore<T, NR>(ob + (size_t)m.row[0] * NR, acc);
+        dst.store(m.row[0], acc);
     } else if (kind == 2) {
 #pragma unroll
         for (int g = 0; g < kGrpRows; ++g)
             if (g < n) {
                 const int64_t r = m.pp[g];
-                vstore<T, NR>(ob + (size_t)r * NR,
-                              src.value(src.load(r), r, ldg(&op.flag[r]) & (ROW_IDENTITY | ROW_NODIAG)));
+                if (Dst::kSkipIdentity) dst.identity(r);
+                else dst.store(r, src.value(src.load(r), r, ldg(&op.flag[r]) & (ROW_IDENTITY | ROW_NODIAG)));
             }
     }
 }
@@ -1310,7 +1349,7 @@ __global__ __launch_bounds__(kBlock) void k_egather_upd(const Seg<float>* __rest
             if (lane_in(L, k, M_UPDATE)) {
                 if (!first) __syncthreads();   // the previous lane's LDS reads are done
                 first = false;
-                double* ob = mv.tmp64 + lm_at(sg, k, 0);
+                const DstPlain<double, 1> ob{mv.tmp64 + lm_at(sg, k, 0)};
                 if (x32) {
                     SrcX64<NR> src{mv.x64 + lm_at(sg, k, 0), x32 + sg.off + k, ldg(&sg.st[k].scale)};
                     egather_grp_tile<double, 1, LR>(sg.op64, lb, src, ob, lrows, [](auto&) { return true; });
@@ -1349,7 +1388,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
     const bool main = !lanes || seg_any(L, lanes & ~M_UPDATE);
     if (!main || lb >= sg.op.ngt) return;
     SrcPlain<T, NR, FLY> src{&sg, x + sg.off};
-    egather_grp_tile<T, NR, LR>(sg.op, lb, src, out + sg.off, lrows, [](auto&) { return true; });
+    egather_grp_tile<T, NR, LR>(sg.op, lb, src, DstPlain<T, NR>{out + sg.off}, lrows, [](auto&) { return true; });
 }
 
 // out = A x from tmp = E x.  RED = 0: no reduction; 1: partial (other, out);
@@ -1595,7 +1634,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
     src.v = w.v + sg.off;
     src.r = w.r + sg.off;
     if constexpr (PH == 1) src.p = w.p + sg.off;
-    egather_grp_tile<T, NR, LR>(sg.op, lb, src, w.tmp + sg.off, lrows, [&](auto& q) {
+    egather_grp_tile<T, NR, LR>(sg.op, lb, src, DstPlain<T, NR>{w.tmp + sg.off}, lrows, [&](auto& q) {
         LaneStat<NR> L;
         if constexpr (FOLD >= 0) L = fold_end<(FOLD >= 0 ? FOLD : 0), NR>(sg, in, out, lb == 0, f, lst);
         else L = lane_stat<NR>(sg);
@@ -1753,6 +1792,113 @@ __global__ __launch_bounds__(kBlock) void k_fxrupdate(const SegArg<T> segs, Vecs
         vstore<T, NR>(w.r + i, rv);
     }
     block_partials<2, NR>(pv, part_of<NR>(sg, 2), lb, sg.nblocks);
+}
+
+// ---------------------------------------------------------------- applies on callers' vectors
+// An apply or an explicit step of a shared-stencil operator reads and writes
+// the caller's vectors in place through the row permutation, its segment an
+// argument of the launch: no packing launches before and after, no tables to
+// copy.  (An apply of 1.05 M rows: two packs of 10 us beside a gather of 29
+// and an lfinish of 11; of 10,906 rows: launches and copies.)
+
+// Gather through a permutation: x and y in the caller's order, or tmp in the operator's.
+template <int NR, typename Src, typename Dst>
+__global__ __launch_bounds__(kBlock) void k_gather_caller(const SegArg<double> a, Src src, const Dst dst) {
+    typedef typename VT<double, NR>::type V;
+    constexpr int LR = GrpTile<double, NR>::kRows;
+    __shared__ V lx[LR];
+    const LdsRows<V> lrows{lx, LR};
+    int lb;
+    int64_t row;
+    const Seg<double>& sg = seg_of<true>(a, lb, row);
+    if (lb >= sg.op.ngt) return;
+    egather_grp_tile<double, NR, LR>(sg.op, lb, src, dst, lrows, [](auto&) { return true; });
+}
+
+// y = m x + n (L_ii x + L_off tmp), x and y in the caller's order.
+__global__ __launch_bounds__(kBlock) void k_lfinish_caller(const SegArg<double> a, const int* perm, const double* x,
+                                                           const double* tmp, double* y) {
+    int lb;
+    int64_t row;
+    const Seg<double>& sg = seg_of<true>(a, lb, row);
+    if (row >= sg.op.D) return;
+    const int c = ldg(perm + row);
+    TpLRow<double, 1> r;
+    arow_tp_load<double, 1>(sg.op, row, x + c, r);
+    stg(y + c, arow_tp<double, 1>(sg, row, r, tmp, 1, false));
+}
+
+// Explicit diffusion of NR fields, z = x + c (Lfull x) (m = 1, n = c[k]), and
+// for two fields the Gray-Scott reaction (ReactionDiffusionWithIBC.cpp:89-93)
+// of their old values: fields in the caller's order, z interleaved in the
+// operator's.  Identity rows take their Lfull rows from k_diffuse_held.
+struct StepArg {
+    const int* perm;
+    const double* x[2];
+    double c[2];
+    double dt, F, k;
+    double* z;
+};
+template <int NR>
+__device__ __forceinline__ void diffuse_store(const StepArg& s, int64_t row, const double (&x)[NR], const double (&d)[NR]) {
+    double z[NR];
+#pragma unroll
+    for (int f = 0; f < NR; ++f) z[f] = x[f] + s.c[f] * d[f];
+    if constexpr (NR == 2) {
+        z[0] += s.dt * (-x[0] * x[1] * x[1] + s.F * (1.0 - x[0]));
+        z[1] += s.dt * (x[0] * x[1] * x[1] - (s.F + s.k) * x[1]);
+    }
+    typename VT<double, NR>::type v;
+#pragma unroll
+    for (int f = 0; f < NR; ++f) setlane(v, f, z[f]);
+    vstore<double, NR>(s.z + (size_t)row * NR, v);
+}
+template <int NR>
+__global__ __launch_bounds__(kBlock) void k_diffuse(const SegArg<double> a, const StepArg s) {
+    int lb;
+    int64_t row;
+    const Seg<double>& sg = seg_of<true>(a, lb, row);
+    const OpView<double>& op = sg.op;
+    if (row >= op.D || (ldg(&op.flag[row]) & ROW_IDENTITY)) return;
+    int c[7];
+#pragma unroll
+    for (int q = 0; q < 6; ++q) c[q] = ldg(&op.lcol[(int64_t)q * op.D + row]);
+    c[6] = ldg(s.perm + row);
+    double x[NR], d[NR];
+#pragma unroll
+    for (int f = 0; f < NR; ++f) x[f] = ldg(s.x[f] + c[6]);
+#pragma unroll
+    for (int q = 0; q < 6; ++q) c[q] = c[q] >= 0 ? ldg(s.perm + c[q]) : -1;
+#pragma unroll
+    for (int f = 0; f < NR; ++f) {
+        double lo = 0.0;
+#pragma unroll
+        for (int q = 0; q < 6; ++q) lo += (c[q] >= 0 ? op.loff : 0.0) * ldg(s.x[f] + (c[q] >= 0 ? c[q] : c[6]));
+        d[f] = op.ldu * x[f] + lo;
+    }
+    diffuse_store<NR>(s, row, x, d);
+}
+template <int NR>
+__global__ void k_diffuse_held(int64_t nh, int hw, const int* hrow, const int* hcol, const double* hval, const uint8_t* flag,
+                               const StepArg s) {
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= nh) return;
+    const int r = hrow[k];
+    if (!(flag[r] & ROW_IDENTITY)) return;
+    double x[NR], d[NR];
+    const int c = s.perm[r];
+#pragma unroll
+    for (int f = 0; f < NR; ++f) {
+        x[f] = s.x[f][c];
+        d[f] = 0.0;
+    }
+    for (int q = 0; q < hw; ++q) {
+        const double v = hval[(int64_t)q * nh + k];
+        const int h = s.perm[hcol[(int64_t)q * nh + k]];
+#pragma unroll
+        for (int f = 0; f < NR; ++f) d[f] += v * s.x[f][h];
+    }
+    diffuse_store<NR>(s, r, x, d);
 }
 
 // FP64 restart, BiCGStab.h:62-71: r = b - A x (A x already in ax), r0 = r; partial (r, r).
@@ -2067,6 +2213,43 @@ void launch_lfinish_plain(const LaunchCfg<T>& c, const T* x, const T* tmp, T* ou
     LAUNCH((k_lfinish<T, 1, 0>), x, tmp, out, (const T*)nullptr, (const T*)nullptr, 0u, none, 0, 0);
 }
 template void launch_lfinish_plain<double>(const LaunchCfg<double>&, const double*, const double*, double*);
+
+static SegArg<double> caller_arg(const Seg<double>& sg) { return SegArg<double>{nullptr, nullptr, sg}; }
+
+void launch_apply_caller(const Seg<double>& sg, const int* perm, const double* x, double* tmp, double* y, hipStream_t st) {
+    const SegArg<double> a = caller_arg(sg);
+    hipLaunchKernelGGL((k_gather_caller<1, SrcPerm, DstPlain<double, 1>>), dim3(sg.op.ngt), dim3(kBlock), 0, st, a,
+                       SrcPerm{x, perm}, DstPlain<double, 1>{tmp});
+    hipLaunchKernelGGL(k_lfinish_caller, dim3(sg.nblocks), dim3(kBlock), 0, st, a, perm, x, tmp, y);
+}
+
+void launch_extend_caller(const Seg<double>& sg, const int* perm, const double* x, double* y, hipStream_t st) {
+    hipLaunchKernelGGL((k_gather_caller<1, SrcPerm, DstPerm<1, false>>), dim3(sg.op.ngt), dim3(kBlock), 0, st, caller_arg(sg),
+                       SrcPerm{x, perm}, DstPerm<1, false>{{y}, {nullptr}, perm});
+}
+
+template <int NR>
+void launch_step_caller(const Seg<double>& sg, const HeldRows& h, const int* perm, double* const* u, const double* const* g,
+                        const double* coef, double dt, double F, double k, double* z, hipStream_t st) {
+    const SegArg<double> a = caller_arg(sg);
+    StepArg s{perm, {u[0], NR > 1 ? u[NR - 1] : nullptr}, {coef[0], coef[NR - 1]}, dt, F, k, z};
+    hipLaunchKernelGGL(k_diffuse<NR>, dim3(sg.nblocks), dim3(kBlock), 0, st, a, s);
+    if (h.nh > 0)
+        hipLaunchKernelGGL(k_diffuse_held<NR>, dim3((unsigned)((h.nh + 255) / 256)), dim3(256), 0, st, h.nh, h.hw, h.row, h.col,
+                           h.val, sg.op.flag, s);
+    DstPerm<NR, true> dst;
+    for (int f = 0; f < NR; ++f) {
+        dst.out[f] = u[f];
+        dst.g[f] = g[f];
+    }
+    dst.perm = perm;
+    hipLaunchKernelGGL((k_gather_caller<NR, SrcPlain<double, NR, false>, DstPerm<NR, true>>), dim3(sg.op.ngt), dim3(kBlock), 0, st,
+                       a, (SrcPlain<double, NR, false>{nullptr, z}), dst);
+}
+template void launch_step_caller<1>(const Seg<double>&, const HeldRows&, const int*, double* const*, const double* const*,
+                                    const double*, double, double, double, double*, hipStream_t);
+template void launch_step_caller<2>(const Seg<double>&, const HeldRows&, const int*, double* const*, const double* const*,
+                                    const double*, double, double, double, double*, hipStream_t);
 
 template <typename T, int NR>
 void launch_egather(const LaunchCfg<T>& c, const T* x, T* out, bool fly) {
