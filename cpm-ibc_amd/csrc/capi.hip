@@ -503,6 +503,7 @@ static void run_batch(Ctx* ctx, const std::vector<Group>& groups, const std::vec
     grp_refresh_override();
     const int grp = fewest_tiles(groups.begin(), groups.end(), [](const Group& g) { return g.op; });
     const bool by_tile = refine ? grp_gather<float, NR>(grp) : grp_gather<double, NR>(grp);
+    const bool ell = std::all_of(groups.begin(), groups.end(), [](const Group& g) { return g.op->fmt == OP_ELL; });
     // layout
     std::vector<int64_t> off(G);
     std::vector<int> b0(G), nb(G), ng(G);
@@ -602,8 +603,8 @@ static void run_batch(Ctx* ctx, const std::vector<Group>& groups, const std::vec
     int sweeps = 0;
     for (auto& g : groups)
         if (g.op->precond == CPM_PRECOND_JACOBI) sweeps = std::max(sweeps, g.op->precond_iters);
-    const LaunchCfg<double> c64{segs64, h64.data(), bseg, blocks, gblocks, G, st, sweeps, fold, fuse, grp};
-    const LaunchCfg<float> c32{segs32, h32.data(), bseg, blocks, gblocks, G, st, sweeps, fold, fuse, grp};
+    const LaunchCfg<double> c64{segs64, h64.data(), bseg, blocks, gblocks, G, st, sweeps, fold, fuse, grp, ell};
+    const LaunchCfg<float> c32{segs32, h32.data(), bseg, blocks, gblocks, G, st, sweeps, fold, fuse, grp, ell};
     const double delta = o.update_delta > 0 ? std::min(o.update_delta, 0.999) : kDefaultUpdateDelta;
     launch_reset_states(sts, nstate, o.tol * o.tol, o.max_iters, delta * delta, st);
 
@@ -789,7 +790,7 @@ static void run_stream(Ctx* ctx, Op* op, const std::vector<const double*>& rhs, 
         }
     HIPCHK(hipMemcpyAsync(sts, hst.data(), sizeof(KState) * nstate, hipMemcpyHostToDevice, st));
     int sweeps = op->precond == CPM_PRECOND_JACOBI ? op->precond_iters : 0;
-    const LaunchCfg<float> c32{seg32, h32.data(), bseg, blocks, gblocks, G, st, sweeps, fold, fuse, op->ngt};
+    const LaunchCfg<float> c32{seg32, h32.data(), bseg, blocks, gblocks, G, st, sweeps, fold, fuse, op->ngt, op->fmt == OP_ELL};
     const MixVec mv{V64.x, V64.r, V64.b, V64.tmp};
     KState* hs = ctx->host_states;
     int done = 0;
@@ -1051,7 +1052,8 @@ void multiply(Op* op, const double* dx, double* dy, double m, double n) {
     double* w = ctx->workspace("mul_tmp", sizeof(double) * op->D * 3);
     double *xi = w, *yi = w + op->D, *tmp = w + 2 * op->D;
     grp_refresh_override();
-    LaunchCfg<double> c{dseg, &h, dbseg, nblocks, grp_blocks(grp_gather<double, 1>(op->ngt), op->ngt, nblocks), 1, st, 0, false, false, op->ngt};
+    LaunchCfg<double> c{dseg, &h, dbseg, nblocks, grp_blocks(grp_gather<double, 1>(op->ngt), op->ngt, nblocks), 1, st, 0, false, false, op->ngt,
+                        op->fmt == OP_ELL};
     if (op->perm.p) {   // caller order -> internal order and back
         hipLaunchKernelGGL(k_pack, dim3(nblocks), dim3(256), 0, st, dpe, dbseg, xi, (float*)nullptr, 1);
         Launch<double, 1>::apply(c, xi, tmp, yi);

@@ -28,6 +28,7 @@ struct LaunchCfg {
     bool fold = false;     // the finalisers run inside the kernels that need them (Seg::sst set)
     bool fuse = false;     // ... and pupdate and supdate inside the gathers and lfinish, where those allow it
     int grp = 0;           // fewest shared-stencil tiles of the segments' operators (0: some have none)
+    bool ell = false;      // every operator is in the ELL format
 };
 
 // Whether the E gathers of a launch use shared-stencil tiles: values whose

@@ -834,21 +834,28 @@ __device__ __forceinline__ void egather_grp_tile(const OpView<T>& op, int tile, 
     }
 }
 
-// E row of the ELL format (eight slots in flight).
+// E row of the ELL format, U slots in flight: a slot's x waits for its column,
+// so a row is 2 ew / U memory latencies long, and a small operator has too few
+// rows to hide them (18,855 rows of 64 slots are 74 workgroups).  32 slots for
+// one value per row, 8 where a slot's x takes more registers.
 template <typename T, typename V, int W>
 __device__ __forceinline__ void egather_ell(const OpView<T>& op, int64_t row, const T* xb, int stride, V& acc) {
+    constexpr int U = W == 1 ? 32 : 8;
     const int64_t D = op.D;
     const int* col = op.ecol + row;
     const T* val = op.eval + row;
     const int ew = op.ew;
     int s = 0;
-    for (; s + 8 <= ew; s += 8) {
-        int c[8];
-        T w[8];
+    for (; s + U <= ew; s += U) {
+        int c[U];
+        T w[U];
+        V x[U];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) { c[u] = ldg(&col[(int64_t)(s + u) * D]); w[u] = ldg(&val[(int64_t)(s + u) * D]); }
+        for (int u = 0; u < U; ++u) { c[u] = ldg(&col[(int64_t)(s + u) * D]); w[u] = ldg(&val[(int64_t)(s + u) * D]); }
 #pragma unroll
-        for (int u = 0; u < 8; ++u) acc += w[u] * vload<T, W>(xb + (size_t)c[u] * stride);
+        for (int u = 0; u < U; ++u) x[u] = vload<T, W>(xb + (size_t)c[u] * stride);
+#pragma unroll
+        for (int u = 0; u < U; ++u) acc += w[u] * x[u];
     }
     for (; s < ew; ++s) acc += ldg(&val[(int64_t)s * D]) * vload<T, W>(xb + (size_t)ldg(&col[(int64_t)s * D]) * stride);
 }
@@ -886,11 +893,23 @@ __device__ __forceinline__ typename VT<T, W>::type arow(const OpView<T>& op, dou
         }
         ld = op.ldu;
     } else {
-        for (int s = 0; s < op.lw; ++s) {
+        ld = ldg(&op.ldiag[row]);
+        int s = 0;
+        for (; s + 6 <= op.lw; s += 6) {   // six slots in flight (the Laplacian's neighbours)
+            int c[6];
+            T w[6];
+#pragma unroll
+            for (int u = 0; u < 6; ++u) {
+                c[u] = ldg(&op.lcol[(int64_t)(s + u) * D + row]);
+                w[u] = ldg(&op.lval[(int64_t)(s + u) * D + row]);
+            }
+#pragma unroll
+            for (int u = 0; u < 6; ++u) lo += w[u] * vload<T, W>(tb + (size_t)c[u] * stride);
+        }
+        for (; s < op.lw; ++s) {
             const int c = ldg(&op.lcol[(int64_t)s * D + row]);
             lo += ldg(&op.lval[(int64_t)s * D + row]) * vload<T, W>(tb + (size_t)c * stride);
         }
-        ld = ldg(&op.ldiag[row]);
     }
     return (T)m * xv + (T)n * (ld * xv + lo);
 }
@@ -1320,6 +1339,24 @@ __global__ __launch_bounds__(kBlock) void k_egather(const Seg<T>* __restrict__ s
     } else if (main && row < sg.op.D) {
         vstore<T, NR>(out + i, erow<T, NR>(sg.op, row, xb, NR));
     }
+}
+
+// E x for launches whose every segment is in the ELL format: no LDS, and only
+// this loop's registers.
+template <typename T, int NR>
+__global__ __launch_bounds__(kBlock) void k_egather_ell(const Seg<T>* __restrict__ segs, const int* __restrict__ bseg, const T* x,
+                                                        T* out, unsigned lanes, MixVec, int copy) {
+    typedef typename VT<T, NR>::type V;
+    int lb;
+    int64_t row;
+    const Seg<T>& sg = seg_of(segs, bseg, lb, row);
+    const auto L = lane_stat<NR>(sg, lanes != 0, copy);
+    if (row >= sg.op.D || (lanes && !seg_any(L, lanes & ~M_UPDATE))) return;
+    const T* xb = x + sg.off;
+    V acc = (V)(T)0;
+    if (ldg(&sg.op.flag[row]) & ROW_IDENTITY) acc = vload<T, NR>(xb + (size_t)row * NR);
+    else egather_ell<T, V, NR>(sg.op, row, xb, NR, acc);
+    vstore<T, NR>(out + (size_t)(sg.off + row * NR), acc);
 }
 
 // FP64 gathers of the refinement lanes of FP32 segments: tmp64 = E64 x64 for
@@ -2063,7 +2100,8 @@ void launch_reset_states(KState* st, int n, double tol2, int max_it, double delt
                 break;                                                       \
             }                                                                \
         }                                                                    \
-        LAUNCH_GATHER((k_egather<T, NR>), __VA_ARGS__);                      \
+        if (c.ell) LAUNCH_GATHER((k_egather_ell<T, NR>), __VA_ARGS__);       \
+        else LAUNCH_GATHER((k_egather<T, NR>), __VA_ARGS__);                 \
     } while (0)
 #define FIN_COPY(T, NR, KIND, IN, OUT) \
     hipLaunchKernelGGL((k_fin<T, NR, KIND>), dim3(c.nseg * NR), dim3(kBlock), 0, c.stream, c.segs, IN, OUT)
