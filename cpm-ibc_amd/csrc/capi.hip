@@ -438,8 +438,14 @@ struct BatchBytes {
 };
 // Whether a launch folds its finalisers into the kernels that need them
 // (krylov.hip): every workgroup then sums its segment's partials, most a
-// segment's row blocks.
-static bool fold_fins(int most, int NR) { return most * NR <= 1024; }
+// segment's row blocks. One lane's launches, which then also run fused, gain
+// until those sums cost what the launches did: FP64 solves of 181k, 273k,
+// 406k, 607k and 776k rows 14.9 -> 13.6, 20.6 -> 18.5, 28.4 -> 27.2,
+// 42.6 -> 42.2 and 65.8 -> 67.6 ms, mixed ones of 406k and 607k rows 27.8 ->
+// 25.8 and 42.7 -> 41.1 ms. Several lanes are not fused and sum as many times
+// the partials: 4 lanes of 293k rows would take 2.70 ms against 2.16, 18 lanes
+// of 6 surfaces of 36k rows 17.5 against 16.5.
+static bool fold_fins(int most, int NR) { return NR == 1 ? most <= 2560 : most * NR <= 1024; }
 // Whether its iterations run fused as well (krylov.hip).
 static bool fuse_iterations(bool fold, int NR) { return fold && NR == 1; }
 

@@ -1111,75 +1111,121 @@ template <int KIND, int NR>
 struct LaneState {
     static constexpr int NV = FinTraits<KIND>::NV;
     KState s[NR];
-    double tot[NV * NR];
+    static constexpr int R = NV * NR <= 2 ? kBlock / 64 : 1;
+    double red[NV * NR][R];   // the components' sums, of each wave or whole (FoldLoads::kAll)
 };
 // The loads of a fold, issued before the caller's own so that they overlap:
-// the states' words and the first kBlock partials of the wave's first component.
+// the states' words and the first partials. With one lane every thread takes
+// kFoldU partials of each component at a time (kAll): 4 x 256 loads a
+// component in flight, which is what a sum over 2,000 partials waits for
+// (before, a wave summed a component alone: plain solve of 42k / 117k / 181k
+// rows 4.50 / 7.66 / 14.9 -> 4.30 / 7.12 / 13.7 ms). With more lanes a wave
+// sums whole components, as all of them in turn cost more than they gain
+// (6 surfaces x 3 right-hand sides of 8k rows: 5.35 against 5.85 ms).
+constexpr int kFoldU = 4;
+template <int C>
 struct FoldLoads {
-    double v[kBlock / 64];
+    static constexpr bool kAll = C <= 2;
+    static constexpr int P = kAll ? C : 1;
+    double v[P][kFoldU];
     int w0, w1;
 };
+// kFoldU partials at b0, b0 + STEP, .. of the P components from part on
+template <int P, int STEP>
+__device__ __forceinline__ void fold_load(const double* part, int nblocks, int b0, double (&v)[P][kFoldU]) {
+#pragma unroll
+    for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int u = 0; u < kFoldU; ++u) {
+            const int b = b0 + STEP * u;
+            v[p][u] = b < nblocks ? ldg(&part[(size_t)p * nblocks + b]) : 0.0;
+        }
+}
 template <int KIND, int NR, typename T>
-__device__ __forceinline__ void fold_begin(const Seg<T>& sg, int in, FoldLoads& f) {
+__device__ __forceinline__ void fold_begin(const Seg<T>& sg, int in, FoldLoads<FinTraits<KIND>::NV * NR>& f) {
     constexpr int C = FinTraits<KIND>::NV * NR;
     constexpr int W = (int)(sizeof(KState) / 4) * NR;   // a group owns kMaxNR states: every load is valid
     static_assert(W <= 2 * kBlock, "a thread copies at most two words");
-    const int t = (int)threadIdx.x, lanei = t & 63, wave = t >> 6;
+    const int t = (int)threadIdx.x, wave = t >> 6;
     const int* src = reinterpret_cast<const int*>(sg.st + (int64_t)in * sg.sst);
     f.w0 = t < W ? ldg(&src[t]) : 0;
     f.w1 = W > kBlock && t + kBlock < W ? ldg(&src[t + kBlock]) : 0;
-    const double* p = part_of<NR>(sg, in) + (size_t)(wave < C ? wave : 0) * sg.nblocks;
-#pragma unroll
-    for (int w = 0; w < kBlock / 64; ++w) f.v[w] = lanei + 64 * w < sg.nblocks ? ldg(&p[lanei + 64 * w]) : 0.0;
+    const double* part = part_of<NR>(sg, in);
+    if constexpr (FoldLoads<C>::kAll)
+        fold_load<FoldLoads<C>::P, kBlock>(part, sg.nblocks, t, f.v);
+    else
+        fold_load<1, 64>(part + (size_t)(wave < C ? wave : 0) * sg.nblocks, sg.nblocks, t & 63, f.v);
 }
+// Each component's sum in part_totals' order: its lane l of wave w adds
+// partials 64 w + l, 64 w + l + kBlock, .., and the waves' sums are added in
+// order (the sums of lanes that are not in the finaliser's mask are formed and
+// not used).
 template <int KIND, int NR, typename T>
-__device__ __forceinline__ LaneStat<NR> fold_end(const Seg<T>& sg, int in, int out, bool writer, const FoldLoads& f,
-                                                 LaneState<KIND, NR>& sh) {
-    constexpr int NV = FinTraits<KIND>::NV, C = NV * NR, NW = kBlock / 64, U = 2;
+__device__ __forceinline__ LaneStat<NR> fold_end(const Seg<T>& sg, int in, int out, bool writer,
+                                                 const FoldLoads<FinTraits<KIND>::NV * NR>& f, LaneState<KIND, NR>& sh) {
+    constexpr int NV = FinTraits<KIND>::NV, C = NV * NR, NW = kBlock / 64;
     constexpr int W = (int)(sizeof(KState) / 4) * NR;
     const int t = (int)threadIdx.x, lanei = t & 63, wave = t >> 6;
     int* lds = reinterpret_cast<int*>(sh.s);
     if (t < W) lds[t] = f.w0;
     if (W > kBlock && t + kBlock < W) lds[t + kBlock] = f.w1;
-    // a wave sums whole components, in part_totals' order: its lane l adds
-    // what threads l, 64 + l, .. of that sum add, each in an accumulator of
-    // its own (the sums of lanes that are not in the finaliser's mask are
-    // formed and not used)
-    for (int c = wave; c < C; c += NW) {
-        const double* p = part_of<NR>(sg, in) + (size_t)c * sg.nblocks;
-        double acc[NW];
-        int b0 = lanei;
+    const double* part = part_of<NR>(sg, in);
+    if constexpr (FoldLoads<C>::kAll) {
+        double acc[C], v[C][kFoldU];
 #pragma unroll
-        for (int w = 0; w < NW; ++w) acc[w] = 0.0;
-        if (c == wave) {
+        for (int c = 0; c < C; ++c) {
+            acc[c] = 0.0;
 #pragma unroll
-            for (int w = 0; w < NW; ++w) acc[w] += f.v[w];
-            b0 += kBlock;
+            for (int u = 0; u < kFoldU; ++u) acc[c] += f.v[c][u];
         }
-        for (; b0 < sg.nblocks; b0 += kBlock * U) {
-            double v[U][NW];
+        for (int b0 = kBlock * kFoldU; b0 < sg.nblocks; b0 += kBlock * kFoldU) {
+            fold_load<C, kBlock>(part, sg.nblocks, b0 + t, v);
 #pragma unroll
-            for (int u = 0; u < U; ++u)
+            for (int c = 0; c < C; ++c)
 #pragma unroll
-                for (int w = 0; w < NW; ++w) {
-                    const int b = b0 + kBlock * u + 64 * w;
-                    v[u][w] = b < sg.nblocks ? ldg(&p[b]) : 0.0;
-                }
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-                for (int w = 0; w < NW; ++w) acc[w] += v[u][w];
+                for (int u = 0; u < kFoldU; ++u) acc[c] += v[c][u];
         }
-        double sum = 0.0;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) sum += wave_sum(acc[w]);
-        if (lanei == 0) sh.tot[c] = sum;
+        for (int c = 0; c < C; ++c) {
+            const double sum = wave_sum(acc[c]);
+            if (lanei == 0) sh.red[c][wave] = sum;
+        }
+    } else {
+        static_assert(kFoldU == NW, "a wave's load is one partial of every wave of part_totals");
+        for (int c = wave; c < C; c += NW) {
+            const double* pc = part + (size_t)c * sg.nblocks;
+            double acc[NW], v[2][1][kFoldU];
+            int b0 = 0;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) acc[w] = 0.0;
+            if (c == wave) {
+#pragma unroll
+                for (int w = 0; w < NW; ++w) acc[w] += f.v[0][w];
+                b0 = kBlock;
+            }
+            for (; b0 < sg.nblocks; b0 += 2 * kBlock) {
+                fold_load<1, 64>(pc, sg.nblocks, b0 + lanei, v[0]);
+                fold_load<1, 64>(pc, sg.nblocks, b0 + kBlock + lanei, v[1]);
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+#pragma unroll
+                    for (int w = 0; w < NW; ++w) acc[w] += v[u][0][w];
+            }
+            double sum = 0.0;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) sum += wave_sum(acc[w]);
+            if (lanei == 0) sh.red[c][0] = sum;
+        }
     }
     __syncthreads();
     if (t < NR && t < sg.nr && ((FinTraits<KIND>::M >> sh.s[t].status) & 1u)) {
         double tot[NV];
 #pragma unroll
-        for (int a = 0; a < NV; ++a) tot[a] = sh.tot[a * NR + t];
+        for (int a = 0; a < NV; ++a) {
+            double sum = 0.0;
+            for (int w = 0; w < LaneState<KIND, NR>::R; ++w) sum += sh.red[a * NR + t][w];
+            tot[a] = sum;
+        }
         fin_scalar<KIND>(sh.s[t], tot);
     }
     __syncthreads();
@@ -1195,7 +1241,7 @@ __device__ __forceinline__ LaneStat<NR> fold_end(const Seg<T>& sg, int in, int o
 }
 template <int KIND, int NR, typename T>
 __device__ __forceinline__ LaneStat<NR> fold_states(const Seg<T>& sg, int in, int out, bool writer, LaneState<KIND, NR>& sh) {
-    FoldLoads f;
+    FoldLoads<FinTraits<KIND>::NV * NR> f;
     fold_begin<KIND, NR>(sg, in, f);
     return fold_end<KIND, NR>(sg, in, out, writer, f, sh);
 }
@@ -1664,7 +1710,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
     const Seg<T>& sg = seg_of<ONE>(segs, lb, row);
     if (lb >= sg.op.ngt) return;
     constexpr int in = PH == 1 ? 2 : 0, out = PH == 1 ? 0 : 1;
-    FoldLoads f;
+    FoldLoads<FinTraits<(FOLD >= 0 ? FOLD : 0)>::NV * NR> f;
     if constexpr (FOLD >= 0) fold_begin<(FOLD >= 0 ? FOLD : 0), NR>(sg, in, f);
     typename std::conditional<PH == 1, SrcP<T, NR>, SrcS<T, NR>>::type src;
     src.sg = &sg;
@@ -1791,7 +1837,7 @@ __global__ __launch_bounds__(kBlock) void k_fxrupdate(const SegArg<T> segs, Vecs
     int64_t row;
     const Seg<T>& sg = seg_of<ONE>(segs, lb, row);
     __shared__ LaneState<FIN_OMEGA, NR> lst;
-    FoldLoads f;
+    FoldLoads<FinTraits<FIN_OMEGA>::NV * NR> f;
     fold_begin<FIN_OMEGA, NR>(sg, 1, f);
     typedef typename VT<T, NR>::type V;
     const bool in = row < sg.op.D;

@@ -1,6 +1,6 @@
 """Iterations with finalisers folded into their kernels, and fused ones, end
 bit for bit where the separate kernels end: batch and streamed solves of one
-right-hand side (folded up to 1,024 row blocks, fused on tensor-product
+right-hand side (folded up to 2,560 row blocks, fused on tensor-product
 operators) against request servers of one lane, which run the separate
 kernels."""
 import numpy as np
@@ -37,8 +37,10 @@ def _serve(ctx, op, d_b, d_x, o):
     ("Sphere", 0.5, False, "tp"),        # fewer rows than one wave has partials
     ("Sphere", 0.1, True, "tp"),         # moved columns and identity rows, 43 blocks
     ("Sphere", 0.05, False, "tp"),       # 164 blocks
-    ("Sphere", 0.0201, False, "tp"),     # the most blocks that fold
-    ("Sphere", 0.0199, False, "tp"),     # too many
+    ("Sphere", 0.0201, False, "tp"),     # a full first load of partials
+    ("Sphere", 0.0199, False, "tp"),     # and a second one
+    ("Sphere", 0.0126, False, "tp"),     # the most blocks that fold
+    ("Sphere", 0.0125, False, "tp"),     # too many
     ("Sphere", 0.1, True, "ell"),        # folded, not fused
 ])
 @pytest.mark.parametrize("precision", [cpmgpu.CPM_FP64, cpmgpu.CPM_FP32_REFINE])
