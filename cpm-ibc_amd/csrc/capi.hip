@@ -449,9 +449,11 @@ static bool fold_fins(int most, int NR) { return NR == 1 ? most <= 2560 : most *
 // Whether its iterations run fused as well (krylov.hip).
 static bool fuse_iterations(bool fold, int NR) { return fold && NR == 1; }
 
-// Bytes of a launch's block maps (block_map); a launch of one segment has none.
+// Bytes of a launch's block maps (block_map).  A launch of one segment has
+// none and leaves its place empty: what the no-alloc scratch holds, and the
+// operators that it refuses, do not depend on it.
 static size_t map_bytes(int G, int blocks, int gblocks) {
-    return G == 1 ? 0 : sizeof(int) * ((size_t)blocks + 2 * (size_t)gblocks);
+    return sizeof(int) * ((size_t)blocks + (G == 1 ? (size_t)blocks : 2 * (size_t)gblocks));
 }
 
 static BatchBytes batch_bytes(int G, int blocks, int gblocks, int64_t total, int NR, bool refine, bool fold) {

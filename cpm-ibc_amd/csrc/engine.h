@@ -64,8 +64,8 @@ struct OpView {
     const int* tlr;      // lists of x rows
     const int16_t* tpl;  // [16][D] position of line (i, j)'s first row in the tile's list
     const int16_t* tlx;  // [nexc][kExcPos] positions of an exception row's 64 columns and extra entry
-    // Shared-stencil tiles (built beside the row tiles; gln, glr, glx are
-    // their tln, tlr, tlx).  Rows whose E stencils are the same 4x4x4 block
+    // Shared-stencil tiles (built with the operator; gln, glr, glx are what
+    // tln, tlr, tlx are to row tiles).  Rows whose E stencils are the same 4x4x4 block
     // of nodes are handled by one thread, which reads each x row of the block
     // from LDS once for all of them.  Tile t owns the item places t kBlock ..
     // (t + 1) kBlock - 1, one per thread (places past its items hold empty

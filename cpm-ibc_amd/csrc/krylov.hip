@@ -19,7 +19,12 @@
 // Reductions: every workgroup writes its partial sums; a one-workgroup-per-
 // instance "fin" kernel adds them in a fixed order and runs the scalar part
 // of the recurrence on the device, so iterations need no host round trip and
-// results are reproducible run to run.  (No device-scope fences: on the
+// results are reproducible run to run.  Where a segment has few row blocks
+// the fins are folded: every workgroup of the kernel that needs the scalars
+// sums the partials itself, in the same order (fold_states), and workgroup 0
+// of the segment writes the new states; one right-hand side's iterations then
+// run as five kernels (k_fgather with pupdate or supdate formed where x is
+// read, k_flfinish, k_fxrupdate).  (No device-scope fences: on the
 // multi-XCD MI355X a release/acquire at agent scope writes back / invalidates
 // L2 and costs more than the whole kernel.)
 //

@@ -21,6 +21,11 @@
 //         64      2560         2     1024        37.7        355.0
 //         64      2560         2     1536        30.8        318.5
 //
+// These were tiles in plain order of their stencils, which fill lists of 1,280
+// rows.  Tiles of 256 items along a Hilbert curve share more of their rows
+// (1.53 list rows per row; 2.2 before) and fit lists of 1,024: 32 KB of LDS,
+// five workgroups of a CU instead of four; grp_lds 1024 chosen.
+//
 // Measured again once the E gathers took a launch's segments round-robin
 // (bench.py's default run: 128 right-hand sides streamed through 64 lanes,
 // FP64 batches and one-right-hand-side solves), xcd_run 64 -> 16: streamed

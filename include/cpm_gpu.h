@@ -116,7 +116,8 @@ int cpm_op_format(const cpm_op* op);
 /* LDS tiles of a tensor-product operator's E gather, into out[6]:
  * shared-stencil tiles (0: none), their items (one per thread), their items
  * of plain rows sharing a stencil block, rows in their lists; row tiles with
- * a list, rows in the row tiles' lists.  No counterpart in the reference. */
+ * a list, rows in the row tiles' lists (built for this report where the
+ * operator's launches use shared-stencil tiles).  No counterpart in the reference. */
 int cpm_op_tile_stats(const cpm_op* op, int64_t* out);
 /* Which E gather single-operator launches of `precision` (CPM_FP64 or
  * CPM_FP32_REFINE) with nrhs (1, 2, 4, 8) interleaved right-hand sides use:
@@ -151,9 +152,7 @@ int cpm_solve_device(cpm_op* op, const double* d_rhs, double* d_x, const cpm_sol
  * array of CPM_NOALLOC_SCRATCH_BYTES that the library holds on each GPU it
  * runs on until the process ends; nothing is allocated or freed.  An operator
  * needs about 88 B per row (up to ~760,000 rows); larger ones are rejected
- * with CPM_ERR_ARG before anything is launched.  Shared-stencil tiles are
- * used only if an earlier solve of the operator built them (results are the
- * same either way).  Every call on one GPU shares that GPU's array and leaves
+ * with CPM_ERR_ARG before anything is launched.  Every call on one GPU shares that GPU's array and leaves
  * its contents behind: calls that overlap on one GPU (other threads, other
  * contexts) race, and the caller must serialise them. */
 #define CPM_NOALLOC_SCRATCH_BYTES (64ll << 20)
