@@ -508,7 +508,6 @@ static void run_batch(Ctx* ctx, const std::vector<Group>& groups, const std::vec
         // first attempt, has already written its results out)
         ctx->arena->used = 0;
     }
-    grp_refresh_override();
     const int grp = fewest_tiles(groups.begin(), groups.end(), [](const Group& g) { return g.op; });
     const bool by_tile = refine ? grp_gather<float, NR>(grp) : grp_gather<double, NR>(grp);
     const bool ell = std::all_of(groups.begin(), groups.end(), [](const Group& g) { return g.op->fmt == OP_ELL; });
@@ -611,8 +610,9 @@ static void run_batch(Ctx* ctx, const std::vector<Group>& groups, const std::vec
     int sweeps = 0;
     for (auto& g : groups)
         if (g.op->precond == CPM_PRECOND_JACOBI) sweeps = std::max(sweeps, g.op->precond_iters);
-    const LaunchCfg<double> c64{segs64, h64.data(), bseg, blocks, gblocks, G, st, sweeps, fold, fuse, grp, ell};
-    const LaunchCfg<float> c32{segs32, h32.data(), bseg, blocks, gblocks, G, st, sweeps, fold, fuse, grp, ell};
+    const bool fly = by_tile && precond_fly();
+    const LaunchCfg<double> c64{segs64, h64.data(), bseg, blocks, gblocks, G, st, sweeps, fold, fuse, by_tile, ell, fly};
+    const LaunchCfg<float> c32{segs32, h32.data(), bseg, blocks, gblocks, G, st, sweeps, fold, fuse, by_tile, ell, fly};
     const double delta = o.update_delta > 0 ? std::min(o.update_delta, 0.999) : kDefaultUpdateDelta;
     launch_reset_states(sts, nstate, o.tol * o.tol, o.max_iters, delta * delta, st);
 
@@ -711,8 +711,8 @@ static void run_stream(Ctx* ctx, Op* op, const std::vector<const double*>& rhs, 
     if (nstate > Ctx::kHostStates) throw ArgError("too many lanes");
     const bool fold = fold_fins(nb, NR), fuse = fuse_iterations(fold, NR);
     const int64_t sst = fold ? nstate : 0;
-    grp_refresh_override();
-    const int ng = grp_blocks(grp_gather<float, NR>(op->ngt), op->ngt, nb);
+    const bool by_tile = grp_gather<float, NR>(op->ngt);
+    const int ng = grp_blocks(by_tile, op->ngt, nb);
     const int gblocks = G * ng;
     const int64_t seg_total = (D * NR + 63) & ~int64_t(63);   // vector entries of one segment
     const int64_t total = seg_total * G;
@@ -798,7 +798,8 @@ static void run_stream(Ctx* ctx, Op* op, const std::vector<const double*>& rhs, 
         }
     HIPCHK(hipMemcpyAsync(sts, hst.data(), sizeof(KState) * nstate, hipMemcpyHostToDevice, st));
     int sweeps = op->precond == CPM_PRECOND_JACOBI ? op->precond_iters : 0;
-    const LaunchCfg<float> c32{seg32, h32.data(), bseg, blocks, gblocks, G, st, sweeps, fold, fuse, op->ngt, op->fmt == OP_ELL};
+    const LaunchCfg<float> c32{seg32, h32.data(), bseg, blocks, gblocks, G, st, sweeps, fold, fuse,
+                               by_tile, op->fmt == OP_ELL, by_tile && precond_fly()};
     const MixVec mv{V64.x, V64.r, V64.b, V64.tmp};
     KState* hs = ctx->host_states;
     int done = 0;
@@ -1006,7 +1007,6 @@ static void solve_stream(Op* op, const std::vector<const double*>& rhs, const st
 
 // Whether applies and steps run on the callers' vectors in place (krylov.h).
 static bool in_place(const Op* op) {
-    grp_refresh_override();
     return op->perm.p && op->nD == 0 && grp_gather<double, 1>(op->ngt);
 }
 
@@ -1059,8 +1059,8 @@ void multiply(Op* op, const double* dx, double* dy, double m, double n) {
     HIPCHK(hipMemcpyAsync(dbseg, hb.data(), sizeof(int) * nblocks, hipMemcpyHostToDevice, st));
     double* w = ctx->workspace("mul_tmp", sizeof(double) * op->D * 3);
     double *xi = w, *yi = w + op->D, *tmp = w + 2 * op->D;
-    grp_refresh_override();
-    LaunchCfg<double> c{dseg, &h, dbseg, nblocks, grp_blocks(grp_gather<double, 1>(op->ngt), op->ngt, nblocks), 1, st, 0, false, false, op->ngt,
+    const bool by_tile = grp_gather<double, 1>(op->ngt);
+    LaunchCfg<double> c{dseg, &h, dbseg, nblocks, grp_blocks(by_tile, op->ngt, nblocks), 1, st, 0, false, false, by_tile,
                         op->fmt == OP_ELL};
     if (op->perm.p) {   // caller order -> internal order and back
         hipLaunchKernelGGL(k_pack, dim3(nblocks), dim3(256), 0, st, dpe, dbseg, xi, (float*)nullptr, 1);
@@ -1074,13 +1074,13 @@ void multiply(Op* op, const double* dx, double* dy, double m, double n) {
 
 template <typename T, int NR>
 static void profile_egather_t(Op* op, int G, int reps, double* avg_ms, double* bytes) {
-    grp_refresh_override();
     Ctx* ctx = op->ctx;
     const hipStream_t st = ctx->stream;
     const int nblocks = (int)((op->D + kBlock - 1) / kBlock);
     const int64_t seg_total = (op->D * NR + 63) & ~int64_t(63);
     std::vector<Seg<T>> h(G);
-    const int ng = grp_blocks(grp_gather<T, NR>(op->ngt), op->ngt, nblocks);
+    const bool by_tile = grp_gather<T, NR>(op->ngt);
+    const int ng = grp_blocks(by_tile, op->ngt, nblocks);
     for (int g = 0; g < G; ++g) {   // G copies of the operator in one launch, as streamed solves of 16, 32 lanes
         fill_seg(h[g], op, g * seg_total, nblocks, NR, nullptr, nullptr);
     }
@@ -1099,7 +1099,7 @@ static void profile_egather_t(Op* op, int G, int reps, double* avg_ms, double* b
     T* xs = reinterpret_cast<T*>(ctx->workspace("prof_x", vec_bytes * nbuf));
     T* ys = reinterpret_cast<T*>(ctx->workspace("prof_y", vec_bytes * nbuf));
     HIPCHK(hipMemsetAsync(xs, 0, vec_bytes * nbuf, st));
-    LaunchCfg<T> c{dseg, h.data(), dbseg, nblocks * G, ng * G, G, st, 0, false, false, op->ngt};
+    LaunchCfg<T> c{dseg, h.data(), dbseg, nblocks * G, ng * G, G, st, 0, false, false, by_tile, false, by_tile && precond_fly()};
     auto buf = [&](T* b, int r) { return b + (size_t)(r % nbuf) * seg_total * G; };
     // the gather the iterations launch: of P^-1 x unless Jacobi sweeps follow the first
     const bool fly = !(op->precond == CPM_PRECOND_JACOBI && op->precond_iters > 1);
@@ -1127,7 +1127,7 @@ static void profile_egather_t(Op* op, int G, int reps, double* avg_ms, double* b
     // extra entry; LDS tiles also read their lists, 4 bytes per row)
     double opb;
     const double sT = sizeof(T);
-    if (grp_gather<T, NR>(op->ngt)) {
+    if (by_tile) {
         // shared-stencil tiles: per plain item 16 int16 positions and its
         // slot offset, per plain row 12 weights and its row index; exception
         // rows as in the row tiles plus slot offset and row index; identity
@@ -1230,8 +1230,9 @@ static void explicit_diffusion(Op* op, const StepTables& t, int k, double c, con
 }
 
 static void extension(Op* op, const StepTables& t, const double* z, double* y) {
-    LaunchCfg<double> cfg{t.seg, nullptr, t.bseg, t.nblocks, grp_blocks(grp_gather<double, 1>(op->ngt), op->ngt, t.nblocks), 1,
-                          op->ctx->stream, 0, false, false, op->ngt};
+    const bool by_tile = grp_gather<double, 1>(op->ngt);
+    LaunchCfg<double> cfg{t.seg, nullptr, t.bseg, t.nblocks, grp_blocks(by_tile, op->ngt, t.nblocks), 1, op->ctx->stream, 0,
+                          false, false, by_tile};
     launch_egather<double, 1>(cfg, z, y);
 }
 
@@ -1460,7 +1461,8 @@ struct Server : ServerBase {
     RangePool ranges;   // vector ranges of the pools
     std::vector<Req> reqs;
     bool dirty = true;
-    int nblocks = 0, gblocks = 0, grp = 0;
+    int nblocks = 0, gblocks = 0;
+    bool by_tile = false, fly = false;   // the gather that rebuild laid the block maps out for
     Seg<float>* d_segs = nullptr;
     int* d_bseg = nullptr;
     double* d_part = nullptr;
@@ -1602,9 +1604,8 @@ struct Server : ServerBase {
 
     void rebuild() {
         ensure_tables();
-        grp_refresh_override();
-        grp = fewest_tiles(reqs.begin(), reqs.end(), [](const Req& q) { return q.op; });
-        const bool by_tile = grp_gather<float, NR>(grp);
+        by_tile = grp_gather<float, NR>(fewest_tiles(reqs.begin(), reqs.end(), [](const Req& q) { return q.op; }));
+        fly = by_tile && precond_fly();
         std::vector<Seg<float>> h(reqs.size());
         std::vector<int> nbs, ngs;
         int b0 = 0;
@@ -1634,7 +1635,7 @@ struct Server : ServerBase {
         const hipStream_t st = ctx->stream;
         const Vecs<float> V32{nullptr, v32(0), v32(1), v32(2), v32(3), v32(4), v32(5), v32(6), v32(7), v32(8), v32(9)};
         const MixVec mv{v64(1), v64(2), v64(0), v64(4)};
-        const LaunchCfg<float> c{d_segs, nullptr, d_bseg, nblocks, gblocks, (int)reqs.size(), st, 0, false, false, grp};
+        const LaunchCfg<float> c{d_segs, nullptr, d_bseg, nblocks, gblocks, (int)reqs.size(), st, 0, false, false, by_tile, false, fly};
         Vecs<float> w = V32;
         Launch<float, NR>::iterations(c, w, true, mv, iters);
         HIPCHK(hipGetLastError());
@@ -1712,7 +1713,8 @@ struct Server64 : ServerBase {
     RangePool ranges;
     std::vector<Req> reqs;
     bool dirty = true;
-    int nblocks = 0, gblocks = 0, grp = 0;
+    int nblocks = 0, gblocks = 0;
+    bool by_tile = false, fly = false;   // the gather that rebuild laid the block maps out for
     Seg<double>* d_segs = nullptr;
     int* d_bseg = nullptr;
     double* d_part = nullptr;
@@ -1814,7 +1816,7 @@ struct Server64 : ServerBase {
         Seg<double> h{};
         fill_seg(h, op, off, nb, nrhs, sts, i_part());
         HIPCHK(hipMemcpyAsync(i_seg(), &h, sizeof(h), hipMemcpyHostToDevice, st));
-        const LaunchCfg<double> c1{i_seg(), &h, nullptr, nb, nb, 1, st, 0, false, false, 0};   // no gather
+        const LaunchCfg<double> c1{i_seg(), &h, nullptr, nb, nb, 1, st, 0};   // no gather
         Launch<double, NR>::init(c1, v64(0), v64(1), v64(2), v64(3), v64(4), v64(5));
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(st));
@@ -1825,9 +1827,8 @@ struct Server64 : ServerBase {
 
     void rebuild() {
         ensure_tables();
-        grp_refresh_override();
-        grp = fewest_tiles(reqs.begin(), reqs.end(), [](const Req& q) { return q.op; });
-        const bool by_tile = grp_gather<double, NR>(grp);
+        by_tile = grp_gather<double, NR>(fewest_tiles(reqs.begin(), reqs.end(), [](const Req& q) { return q.op; }));
+        fly = by_tile && precond_fly();
         std::vector<Seg<double>> h(reqs.size());
         std::vector<int> nbs, ngs;
         int b0 = 0;
@@ -1856,7 +1857,7 @@ struct Server64 : ServerBase {
         if (dirty) rebuild();
         const hipStream_t st = ctx->stream;
         Vecs<double> V{v64(0), v64(1), v64(2), v64(3), v64(4), v64(5), v64(6), v64(7), v64(8), v64(9), v64(10)};
-        const LaunchCfg<double> c{d_segs, nullptr, d_bseg, nblocks, gblocks, (int)reqs.size(), st, 0, false, false, grp};
+        const LaunchCfg<double> c{d_segs, nullptr, d_bseg, nblocks, gblocks, (int)reqs.size(), st, 0, false, false, by_tile, false, fly};
         Launch<double, NR>::iterations(c, V, false, MixVec{}, iters);
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(ctx->host_states, states.template as<KState>(), sizeof(KState) * (size_t)slots * kMaxNR,
@@ -2036,7 +2037,6 @@ int cpm_op_gather_kind(const cpm_op* op, int precision, int nrhs) {
     if (!op || (nrhs != 1 && nrhs != 2 && nrhs != 4 && nrhs != 8)) return -1;
     const Op* o = O(op);
     const bool f32 = precision == CPM_FP32_REFINE;
-    grp_refresh_override();
     const bool grp = f32 ? (nrhs == 1 ? grp_gather<float, 1>(o->ngt) : nrhs == 2 ? grp_gather<float, 2>(o->ngt)
                             : nrhs == 4 ? grp_gather<float, 4>(o->ngt) : grp_gather<float, 8>(o->ngt))
                          : (nrhs == 1 ? grp_gather<double, 1>(o->ngt) : nrhs == 2 ? grp_gather<double, 2>(o->ngt)
@@ -2205,7 +2205,6 @@ int cpm_solve_device_noalloc(cpm_op* op, const double* d_rhs, double* d_x, const
             Use(Ctx* c_, Arena* ar) : c(c_) { c->arena = ar; }
             ~Use() { c->arena = nullptr; }
         } use(cx, &a);
-        grp_refresh_override();
         std::vector<cpm_solve_info> inf;
         solve_batch(cx, std::vector<Op*>{o}, std::vector<const double*>{d_rhs}, std::vector<double*>{d_x}, so, inf);
         if (info) *info = inf[0];

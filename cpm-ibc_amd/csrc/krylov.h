@@ -27,22 +27,28 @@ struct LaunchCfg {
     int jacobi_sweeps;     // largest precond_iters over Jacobi-preconditioned segments (0: none)
     bool fold = false;     // the finalisers run inside the kernels that need them (Seg::sst set)
     bool fuse = false;     // ... and pupdate and supdate inside the gathers and lfinish, where those allow it
-    int grp = 0;           // fewest shared-stencil tiles of the segments' operators (0: some have none)
+    // Which gather kernel runs is decided once, where gblocks and the block
+    // maps are laid out for it, and kept here: a choice made again at a launch
+    // could meet a grid that was laid out for the other kernel.
+    bool tiles = false;    // the E gathers run by shared-stencil tiles (grp_gather)
     bool ell = false;      // every operator is in the ELL format
+    bool fly = false;      // iterations form P^-1 where it is read (precond_fly; with tiles)
 };
 
 // Whether the E gathers of a launch use shared-stencil tiles: values whose
-// rows fit the tiles' LDS, every operator with tiles (ntiles: the fewest).
+// rows fit the tiles' LDS, every operator with tiles (ntiles: the fewest), and
+// the environment does not say CPMGPU_GROUP_GATHER=none.
 template <typename T, int NR>
 bool grp_gather(int ntiles);
+// Whether iterations that gather by tiles form y = P^-1 p and z = P^-1 s where
+// they are read (CPMGPU_PRECOND_FLY=0 stores them instead).
+bool precond_fly();
 // Workgroups that the E gathers of such a launch (grp) take for an operator
 // of ntiles tiles and nblocks row blocks; other launches gather by row blocks
 // (the refinement lanes' FP64 gathers by tiles in both).
 inline int grp_blocks(bool grp, int ntiles, int nblocks) {
     return grp ? ntiles : ntiles > nblocks ? ntiles : nblocks;
 }
-// Re-read the CPMGPU_GROUP_GATHER override (once per launch sequence).
-void grp_refresh_override();
 
 // Workspace vectors of one precision; every vector spans all segments
 // (segment g occupies [off_g, off_g + D_g * NR)).

@@ -57,8 +57,6 @@
 // rounding: the FP32 and FP64 operators differ in the last bits.)
 #include <hip/hip_runtime.h>
 
-#include <atomic>
-
 #include <cmath>
 #include <cstdlib>
 #include <string>
@@ -2141,11 +2139,11 @@ void launch_reset_states(KState* st, int n, double tol2, int max_it, double delt
     hipLaunchKernelGGL(kern, dim3(c.gblocks), dim3(kBlock), 0, c.stream, c.segs,                        \
                        c.nseg == 1 ? nullptr : c.bseg + c.nblocks + c.gblocks, __VA_ARGS__)
 // E gather of launch c; FL: form P^-1 of the gathered vector (only with
-// shared-stencil tiles, grp_launch).
+// shared-stencil tiles).
 #define EGATHER(FL, ...)                                                     \
     do {                                                                     \
         if constexpr (GrpTile<T, NR>::kRows > 0) {                           \
-            if (grp_launch<T, NR>(c)) {                                      \
+            if (c.tiles) {                                                   \
                 if (FL) LAUNCH_GATHER((k_egather_grp<T, NR, GrpWaves<T, NR>::kWaves, true>), __VA_ARGS__); \
                 else LAUNCH_GATHER((k_egather_grp<T, NR, GrpWaves<T, NR>::kWaves, false>), __VA_ARGS__); \
                 break;                                                       \
@@ -2165,34 +2163,16 @@ struct GrpWaves {
     static constexpr int kWaves = (sizeof(T) == 4 && NR != 4) ? 4 : CPMGPU_GROUP_WAVES_WIDE;
 };
 
-// CPMGPU_GROUP_GATHER=none: no launch gathers through shared-stencil tiles.
-// The override is read from the environment once per solve, tile build or
-// query (grp_refresh_override, called where a launch sequence starts), not
-// per launch: a solve makes thousands of launches.
-static std::atomic<int> g_grp_override{-2};   // -2 unread, -1 no override, 0 "none"
-// y = P^-1 p and z = P^-1 s formed where they are read (launches that allow
-// it, Launch::iteration); CPMGPU_PRECOND_FLY=0 stores them instead.
-static std::atomic<int> g_fly_override{-1};   // -1 none, 0 off
-static bool precond_fly() { return g_fly_override.load(std::memory_order_relaxed) != 0; }
-
-void grp_refresh_override() {
-    const char* e = std::getenv("CPMGPU_GROUP_GATHER");
-    const std::string v = e ? e : "";
-    g_grp_override.store(v == "none" ? 0 : -1, std::memory_order_relaxed);
-    const char* fe = std::getenv("CPMGPU_PRECOND_FLY");
-    g_fly_override.store(fe && std::string(fe) == "0" ? 0 : -1, std::memory_order_relaxed);
+bool precond_fly() {
+    const char* e = std::getenv("CPMGPU_PRECOND_FLY");
+    return !(e && std::string(e) == "0");
 }
 
 template <typename T, int NR>
 bool grp_gather(int ntiles) {
-    if (g_grp_override.load(std::memory_order_relaxed) == -2) grp_refresh_override();
-    return GrpTile<T, NR>::kRows > 0 && ntiles > 0 && g_grp_override.load(std::memory_order_relaxed) != 0;
-}
-
-// Whether the E gathers of launch c use shared-stencil tiles (EGATHER's choice).
-template <typename T, int NR>
-static bool grp_launch(const LaunchCfg<T>& c) {
-    return grp_gather<T, NR>(c.grp);
+    if (GrpTile<T, NR>::kRows == 0 || ntiles <= 0) return false;
+    const char* e = std::getenv("CPMGPU_GROUP_GATHER");
+    return !(e && std::string(e) == "none");
 }
 
 template <typename T, int NR>
@@ -2207,7 +2187,7 @@ void Launch<T, NR>::iteration(const LaunchCfg<T>& c, Vecs<T>& w, bool mixed, con
     // gathers' LDS fills, lfinish, xrupdate) rather than stored: launches
     // whose gathers fill LDS from shared-stencil tiles and whose
     // preconditioner is pointwise (no Jacobi sweeps after the first)
-    const bool fly = grp_launch<T, NR>(c) && c.jacobi_sweeps <= 1 && precond_fly();
+    const bool fly = c.fly && c.jacobi_sweeps <= 1;
     const int fl = fly ? 1 : 0;
     const T* yp = fly ? w.p : w.y;   // the vector the first gather and lfinish read
     const T* zs = fly ? w.s : w.z;   // ... the second
@@ -2254,7 +2234,7 @@ void Launch<T, NR>::iterations(const LaunchCfg<T>& c, Vecs<T>& w, bool mixed, co
     }
     bool fused = false;
     if constexpr (NR == 1) {
-        fused = c.fuse && grp_launch<T, NR>(c) && c.jacobi_sweeps <= 1 && precond_fly();
+        fused = c.fuse && c.fly && c.jacobi_sweeps <= 1;
         constexpr int kIter = std::is_same<T, float>::value ? FIN_ITER_MX : FIN_ITER64;
         // waves per SIMD that the fused gathers are compiled for: as many as do not spill
         constexpr int WPE = sizeof(T) == 4 ? 4 : 2;
@@ -2343,7 +2323,7 @@ template void launch_step_caller<2>(const Seg<double>&, const HeldRows&, const i
 template <typename T, int NR>
 void launch_egather(const LaunchCfg<T>& c, const T* x, T* out, bool fly) {
     const MixVec none{};
-    const bool fl = fly && grp_launch<T, NR>(c) && precond_fly();
+    const bool fl = fly && c.fly;
     EGATHER(fl, x, out, 0u, none, 0);
 }
 

@@ -179,3 +179,38 @@ def test_problem_built_on_second_context(gpu_ctx):
         op1.close(), op2.close(), P1.close(), P2.close()
     finally:
         bctx.close()
+
+
+@pytest.mark.parametrize("precision", [cpmgpu.CPM_FP64, cpmgpu.CPM_FP32_REFINE])
+@pytest.mark.parametrize("lanes", [1, 4])
+def test_gather_choice_holds_between_runs(gpu_ctx, monkeypatch, precision, lanes):
+    """A server's launches keep the gather that its block maps were laid out for: the environment's
+    choice changes, and another call reads it, between two runs of the same requests."""
+    print(f"case gather choice precision={precision} lanes={lanes}", flush=True)
+    monkeypatch.setenv("CPMGPU_FP64_ROUTING", "0")
+    op = cpmgpu.Tube(gpu_ctx, "Sphere", 0.05).operator(1.0, -1.0)
+    D = op.D
+    assert op.tile_info()["shared_stencil_tiles"] < (D + 255) // 256   # fewer gather workgroups than row blocks
+    rng = np.random.default_rng(8)
+    b = rng.standard_normal(D)
+    d = [gpu_ctx.alloc(8 * D) for _ in range(2)]
+    gpu_ctx.h2d(d[0], b)
+    o = cpmgpu.opts(tol=1e-9, precision=precision, max_iters=400)
+    res = []
+    for change in (False, True):
+        monkeypatch.delenv("CPMGPU_GROUP_GATHER", raising=False)
+        srv = cpmgpu.Server(gpu_ctx, 90 * lanes * (D + 64) + 4096, lanes=lanes, o=o)
+        assert srv.submit(op, d[:1], d[1:], 1)
+        done, active = srv.run(8)
+        assert not done and active == 1
+        if change:
+            monkeypatch.setenv("CPMGPU_GROUP_GATHER", "none")
+            op.multiply(b, 1.0, -1.0)
+        while not done:
+            done, _ = srv.run(16)
+        srv.close()
+        res.append((done[0][1], gpu_ctx.d2h(np.zeros(D), d[1])))
+    assert res[0][0][0]["status"] == "converged" and res[0][0] == res[1][0]
+    assert np.array_equal(res[0][1], res[1][1])
+    for p in d:
+        gpu_ctx.free(p)
