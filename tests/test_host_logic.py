@@ -56,3 +56,20 @@ def test_fp64_routing_rule(tmp_path):
     out = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert out.returncode == 0, out.stderr
     assert "route ok" in out.stdout
+
+
+def test_chunks_of_a_batch_solve(tmp_path):
+    """Iterations that a batch solve queues between two looks at its states (cpm-ibc_amd/csrc/schedule.h):
+    hardly more than the system or its iteration limit takes, and within 4..32 whatever the residual says."""
+    if shutil.which("g++") is None:
+        pytest.skip("g++ not available")
+    exe = str(tmp_path / "schedule_test")
+    src = os.path.join(REPO, "tests", "cpp", "schedule_test.cpp")
+    inc = os.path.join(REPO, "cpm-ibc_amd", "csrc")
+    build = subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-fsanitize=undefined",
+                            "-fsanitize=float-cast-overflow", "-fno-sanitize-recover=all", "-I", inc, src, "-o", exe],
+                           capture_output=True, text=True, timeout=180)
+    assert build.returncode == 0, build.stderr
+    out = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert out.returncode == 0, out.stderr
+    assert "schedule ok" in out.stdout
