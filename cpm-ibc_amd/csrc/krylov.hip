@@ -837,19 +837,14 @@ __device__ __forceinline__ void egather_grp_tile(const OpView<T>& op, int tile, 
     }
 }
 
-// E row of the ELL format, U slots in flight: a slot's x waits for its column,
-// so a row is 2 ew / U memory latencies long, and a small operator has too few
-// rows to hide them (18,855 rows of 64 slots are 74 workgroups).  32 slots for
-// one value per row, 8 where a slot's x takes more registers.
-template <typename T, typename V, int W>
-__device__ __forceinline__ void egather_ell(const OpView<T>& op, int64_t row, const T* xb, int stride, V& acc) {
-    constexpr int U = W == 1 ? 32 : 8;
+// Slots s, s + 1, .. of an E row of the ELL format in rounds of U as long as
+// whole ones are left, each round's columns, values and x loaded together.
+template <int U, typename T, typename V, int W>
+__device__ __forceinline__ int ell_rounds(const OpView<T>& op, int64_t row, const T* xb, int stride, int s, V& acc) {
     const int64_t D = op.D;
     const int* col = op.ecol + row;
     const T* val = op.eval + row;
-    const int ew = op.ew;
-    int s = 0;
-    for (; s + U <= ew; s += U) {
+    for (; s + U <= op.ew; s += U) {
         int c[U];
         T w[U];
         V x[U];
@@ -860,7 +855,20 @@ __device__ __forceinline__ void egather_ell(const OpView<T>& op, int64_t row, co
 #pragma unroll
         for (int u = 0; u < U; ++u) acc += w[u] * x[u];
     }
-    for (; s < ew; ++s) acc += ldg(&val[(int64_t)s * D]) * vload<T, W>(xb + (size_t)ldg(&col[(int64_t)s * D]) * stride);
+    return s;
+}
+
+// E row of the ELL format: a slot's x waits for its column, so a row's time is
+// memory latencies, two for each round of slots, and a small operator has too
+// few rows to hide them (18,855 rows of 64 slots are 74 workgroups). Rounds of
+// U slots, then of 8, and what 8 does not divide slot by slot. 60 FP64 iterations with
+// the remainder of 32 slot by slot and in rounds of 8: 27 slots a row, 91,741
+// rows 4.1 and 2.9 ms; 125 slots, 50,970 rows 5.5 and 4.2 ms.
+template <int U, typename T, typename V, int W>
+__device__ __forceinline__ void egather_ell(const OpView<T>& op, int64_t row, const T* xb, int stride, V& acc) {
+    int s = ell_rounds<U, T, V, W>(op, row, xb, stride, 0, acc);
+    if constexpr (U > 8) s = ell_rounds<8, T, V, W>(op, row, xb, stride, s, acc);
+    ell_rounds<1, T, V, W>(op, row, xb, stride, s, acc);
 }
 
 // (E x)_row for W consecutive values per row of xb.
@@ -870,7 +878,7 @@ __device__ __forceinline__ typename VT<T, W>::type erow(const OpView<T>& op, int
     V acc = (V)(T)0;
     if (ldg(&op.flag[row]) & ROW_IDENTITY) return vload<T, W>(xb + (size_t)row * stride);
     if (op.fmt == OP_TP) egather_tp<T, V, W>(op, row, xb, stride, acc);
-    else egather_ell<T, V, W>(op, row, xb, stride, acc);
+    else egather_ell<8, T, V, W>(op, row, xb, stride, acc);
     return acc;
 }
 
@@ -1391,9 +1399,16 @@ __global__ __launch_bounds__(kBlock) void k_egather(const Seg<T>* __restrict__ s
 }
 
 // E x for launches whose every segment is in the ELL format: no LDS, and only
-// this loop's registers.
+// this loop's registers. amdgpu_waves_per_eu(1, 2) lets the compiler keep a
+// round's slots in registers (144 for one FP64 value, 107 for one FP32 value,
+// 98 and 168 for four and eight FP64 values); left alone it schedules for eight
+// waves a SIMD (68, 61, 60, 64 registers) and waits inside the rounds. 60
+// iterations, milliseconds, with it and without: 64 slots a row, 41,870 rows,
+// mixed x 1 2.63 and 3.17, FP64 x 8 6.15 and 7.31; 260,062 rows FP64 x 4 14.4
+// and 15.9, x 8 24.2 and 34.2 (14.5 and 27.4 in k_egather); FP64 x 1 the same
+// with both. 16 slots a round for two values: within 3% either way.
 template <typename T, int NR>
-__global__ __launch_bounds__(kBlock) void k_egather_ell(const Seg<T>* __restrict__ segs, const int* __restrict__ bseg, const T* x,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(1, 2))) void k_egather_ell(const Seg<T>* __restrict__ segs, const int* __restrict__ bseg, const T* x,
                                                         T* out, unsigned lanes, MixVec, int copy) {
     typedef typename VT<T, NR>::type V;
     int lb;
@@ -1404,7 +1419,7 @@ __global__ __launch_bounds__(kBlock) void k_egather_ell(const Seg<T>* __restrict
     const T* xb = x + sg.off;
     V acc = (V)(T)0;
     if (ldg(&sg.op.flag[row]) & ROW_IDENTITY) acc = vload<T, NR>(xb + (size_t)row * NR);
-    else egather_ell<T, V, NR>(sg.op, row, xb, NR, acc);
+    else egather_ell<NR == 1 ? 32 : 8, T, V, NR>(sg.op, row, xb, NR, acc);
     vstore<T, NR>(out + (size_t)(sg.off + row * NR), acc);
 }
 
