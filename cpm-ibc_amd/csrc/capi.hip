@@ -438,17 +438,37 @@ struct BatchBytes {
     }
 };
 // Whether a launch folds its finalisers into the kernels that need them
-// (krylov.hip): every workgroup then sums its segment's partials, most a
-// segment's row blocks. One lane's launches, which then also run fused, gain
-// until those sums cost what the launches did: FP64 solves of 181k, 273k,
-// 406k, 607k and 776k rows 14.9 -> 13.6, 20.6 -> 18.5, 28.4 -> 27.2,
-// 42.6 -> 42.2 and 65.8 -> 67.6 ms, mixed ones of 406k and 607k rows 27.8 ->
-// 25.8 and 42.7 -> 41.1 ms. Several lanes are not fused and sum as many times
-// the partials: 4 lanes of 293k rows would take 2.70 ms against 2.16, 18 lanes
-// of 6 surfaces of 36k rows 17.5 against 16.5.
-static bool fold_fins(int most, int NR) { return NR == 1 ? most <= 2560 : most * NR <= 1024; }
-// Whether its iterations run fused as well (krylov.hip).
-static bool fuse_iterations(bool fold, int NR) { return fold && NR == 1; }
+// (krylov.hip), and whether its iterations run fused as well: `most` row blocks
+// in its largest segment, `total` in all of them, NR lanes; fusable: gathers by
+// tiles with a pointwise preconditioner.
+//
+// Folded, every workgroup sums its segment's partials; fused, the fills read
+// p, v and r at 1.53 rows a row. Both save launches and pay in work, so they
+// end where the launch is large enough for the work to count. Milliseconds,
+// separate / folded / fused:
+//  - one segment, one lane: FP64 solves of 607k rows (2,371 row blocks) 42.6
+//    separate and 42.2 fused, of 776k 65.8 and 67.6; mixed ones of 607k 42.7
+//    and 41.1. Line 2,560.
+//  - several segments, one lane, 60 iterations: FP64, 2 of 398 row blocks
+//    3.28 / 2.93 / 2.81, 4 of 398 4.15 / 4.00 / 4.31, 8 of 398 6.19 / 6.29 /
+//    7.03; mixed 3.14 / 2.86 / 2.58, 3.85 / 3.65 / 3.40, 5.16 / 5.36 / 5.58.
+//    Fused up to 1,024 in all in FP64 and 2,560 mixed, folded up to 2,560.
+//  - not fusable (ELL, Jacobi sweeps), one lane, separate / folded: FP64 ELL of
+//    1,016 row blocks 7.02 / 6.83, of 1,585 12.65 / 12.71, of 2,399 18.9 / 19.3;
+//    two Jacobi sweeps of 2,399 4.18 / 4.36. Line 1,280.
+//  - several lanes sum as many times the partials and are not fused: 4 FP64
+//    lanes of 4 x 164 row blocks 4.31 / 4.26, of 650 4.24 / 4.43; 8 mixed
+//    lanes of 4 x 75 4.13 / 4.26. Line 1,024 lanes x row blocks a segment, and
+//    2,560 in all.
+struct Folding {
+    bool fold, fuse;
+};
+static Folding folding(int64_t most, int64_t total, int segments, int NR, bool f32, bool fusable) {
+    if (NR == 1 && fusable && total <= (segments == 1 || f32 ? 2560 : 1024)) return {true, true};
+    return {most * NR <= (NR == 1 ? 1280 : 1024) && total * NR <= 2560, false};
+}
+// Whether it can fold at all: what workspaces are sized for.
+static bool may_fold(int64_t total, int NR) { return total * NR <= 2560; }
 
 // Bytes of a launch's block maps (block_map).  A launch of one segment has
 // none and leaves its place empty: what the no-alloc scratch holds, and the
@@ -470,7 +490,7 @@ static BatchBytes batch_bytes(int G, int blocks, int gblocks, int64_t total, int
 // One operator with NR right-hand sides.
 static BatchBytes batch_bytes1(const Op* op, int NR, bool refine) {
     const int nb = row_blocks(op);
-    return batch_bytes(1, nb, std::max(nb, op->ngt), (op->D * NR + 63) & ~int64_t(63), NR, refine, fold_fins(nb, NR));
+    return batch_bytes(1, nb, std::max(nb, op->ngt), (op->D * NR + 63) & ~int64_t(63), NR, refine, may_fold(nb, NR));
 }
 
 // Grow the context's workspaces to what a batch of one operator with NR
@@ -514,7 +534,11 @@ static void run_batch(Ctx* ctx, const std::vector<Group>& groups, const std::vec
         gblocks += ng[g];
         most = std::max(most, nb[g]);
     }
-    const bool fold = fold_fins(most, NR), fuse = fuse_iterations(fold, NR);
+    int sweeps = 0;
+    for (auto& g : groups)
+        if (g.op->precond == CPM_PRECOND_JACOBI) sweeps = std::max(sweeps, g.op->precond_iters);
+    const bool fly = by_tile && precond_fly();
+    const auto [fold, fuse] = folding(most, blocks, G, NR, refine, fly && sweeps <= 1);
     // device tables: segments (one per precision), block map, states, partials.
     // The FP64 and FP32 segments of a group share one state record per rhs.
     const int nstate = G * kMaxNR;
@@ -594,10 +618,6 @@ static void run_batch(Ctx* ctx, const std::vector<Group>& groups, const std::vec
     HIPCHK(hipMemcpyAsync(dpb, pb.data(), sizeof(int) * pb.size(), hipMemcpyHostToDevice, st));
     hipLaunchKernelGGL(k_pack, dim3((unsigned)pb.size()), dim3(256), 0, st, dpe, dpb, V64.b, (float*)nullptr, 1);
 
-    int sweeps = 0;
-    for (auto& g : groups)
-        if (g.op->precond == CPM_PRECOND_JACOBI) sweeps = std::max(sweeps, g.op->precond_iters);
-    const bool fly = by_tile && precond_fly();
     const LaunchCfg<double> c64{segs64, h64.data(), bseg, blocks, gblocks, G, st, sweeps, fold, fuse, by_tile, ell, fly};
     const LaunchCfg<float> c32{segs32, h32.data(), bseg, blocks, gblocks, G, st, sweeps, fold, fuse, by_tile, ell, fly};
     const double delta = o.update_delta > 0 ? std::min(o.update_delta, 0.999) : kDefaultUpdateDelta;
@@ -714,9 +734,10 @@ static void run_stream(Ctx* ctx, Op* op, const std::vector<const double*>& rhs, 
     const int blocks = G * nb;
     const int nstate = G * kMaxNR;
     if (nstate > Ctx::kHostStates) throw ArgError("too many lanes");
-    const bool fold = fold_fins(nb, NR), fuse = fuse_iterations(fold, NR);
+    const int sweeps = op->precond == CPM_PRECOND_JACOBI ? op->precond_iters : 0;
+    const bool by_tile = grp_gather<float, NR>(op->ngt), fly = by_tile && precond_fly();
+    const auto [fold, fuse] = folding(nb, blocks, G, NR, true, fly && sweeps <= 1);
     const int64_t sst = fold ? nstate : 0;
-    const bool by_tile = grp_gather<float, NR>(op->ngt);
     const int ng = grp_blocks(by_tile, op->ngt, nb);
     const int gblocks = G * ng;
     const int64_t seg_total = (D * NR + 63) & ~int64_t(63);   // vector entries of one segment
@@ -802,9 +823,8 @@ static void run_stream(Ctx* ctx, Op* op, const std::vector<const double*>& rhs, 
             cur[g * kMaxNR + k] = next++;
         }
     HIPCHK(hipMemcpyAsync(sts, hst.data(), sizeof(KState) * nstate, hipMemcpyHostToDevice, st));
-    int sweeps = op->precond == CPM_PRECOND_JACOBI ? op->precond_iters : 0;
     const LaunchCfg<float> c32{seg32, h32.data(), bseg, blocks, gblocks, G, st, sweeps, fold, fuse,
-                               by_tile, op->fmt == OP_ELL, by_tile && precond_fly()};
+                               by_tile, op->fmt == OP_ELL, fly};
     const MixVec mv{V64.x, V64.r, V64.b, V64.tmp};
     KState* hs = ctx->host_states;
     int done = 0;

@@ -1709,10 +1709,25 @@ __global__ __launch_bounds__(kBlock) void k_xrupdate(const Seg<T>* __restrict__ 
 // bit.  Every tile lists a row's neighbours too, so the fills read p, v and r
 // (1.5 rows each per row) where the separate kernels read one vector: more
 // bytes, fewer launches, which pays while an iteration is bound by its
-// launches and their dependent loads rather than by its bytes (fuse_limit,
+// launches and their dependent loads rather than by its bytes (folding,
 // capi.hip).  Refinement (mixed) lanes: x64 += x32 / scale is formed in
 // k_egather_upd's fill and stored by flfinish<1>, the rescaled residual is
 // stored by flfinish<2>.
+
+// A finished segment of a launch over several: whether no lane's status in
+// copy `in` is in mask, read before the kernel's own loads are issued. Its
+// first workgroup still runs the finaliser and hands the states on. (Without
+// it a finished system streams its vectors until the last one ends: eight FP64
+// systems of 260,062 rows that end after 8 to 340 iterations took 75.0 ms.)
+// The only segment of a launch is not looked at: its status would cost a
+// memory latency before the first load.
+template <int FOLD, int NR, typename T, typename LST>
+__device__ __forceinline__ bool segment_done(const Seg<T>& sg, int in, int out, int lb, unsigned mask, LST& lst) {
+    if (seg_any(lane_stat<NR>(sg, true, in), mask)) return false;
+    if constexpr (FOLD >= 0)
+        if (lb == 0) fold_states<FOLD, NR>(sg, in, out, true, lst);
+    return true;
+}
 
 // PH 1: tmp = E P^-1 p, after the loop test (FOLD) ; PH 2: tmp = E P^-1 s, after alpha.
 template <typename T, int NR, bool ONE, int WPE, int PH, int FOLD>
@@ -1727,7 +1742,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
     int64_t row;
     const Seg<T>& sg = seg_of<ONE>(segs, lb, row);
     if (lb >= sg.op.ngt) return;
-    constexpr int in = PH == 1 ? 2 : 0, out = PH == 1 ? 0 : 1;
+    constexpr int in = PH == 1 && FOLD >= 0 ? 2 : 0, out = PH == 1 ? 0 : 1;
+    if (!ONE && segment_done<FOLD, NR>(sg, in, out, lb, M_STAGE3, lst)) return;   // before the loop test: RUN or READY
     FoldLoads<FinTraits<(FOLD >= 0 ? FOLD : 0)>::NV * NR> f;
     if constexpr (FOLD >= 0) fold_begin<(FOLD >= 0 ? FOLD : 0), NR>(sg, in, f);
     typename std::conditional<PH == 1, SrcP<T, NR>, SrcS<T, NR>>::type src;
@@ -1855,6 +1871,7 @@ __global__ __launch_bounds__(kBlock) void k_fxrupdate(const SegArg<T> segs, Vecs
     int64_t row;
     const Seg<T>& sg = seg_of<ONE>(segs, lb, row);
     __shared__ LaneState<FIN_OMEGA, NR> lst;
+    if (!ONE && segment_done<FIN_OMEGA, NR>(sg, 1, 2, lb, M_RUN, lst)) return;
     FoldLoads<FinTraits<FIN_OMEGA>::NV * NR> f;
     fold_begin<FIN_OMEGA, NR>(sg, 1, f);
     typedef typename VT<T, NR>::type V;

@@ -66,3 +66,83 @@ def test_folded_iterations_equal_separate_kernels(gpu_ctx, monkeypatch, surface,
     assert np.array_equal(x1, x2)
     gpu_ctx.free(d_b)
     gpu_ctx.free(d_x)
+
+
+def _dev(ctx, n, D, seed):
+    d = []
+    for k in range(n):
+        d.append((ctx.alloc(8 * D), ctx.alloc(8 * D)))
+        ctx.h2d(d[-1][0], np.random.default_rng([seed, k]).standard_normal(D))
+    return d
+
+
+def _serve_all(ctx, reqs, lanes, o):
+    """reqs: (operator, [(d_b, d_x) ..]) each; the infos of every right-hand side in order."""
+    s = cpmgpu.Server(ctx, sum(90 * lanes * (op.D + 64) for op, _ in reqs) + 4096, lanes=lanes, o=o)
+    for tag, (op, d) in enumerate(reqs):
+        assert s.submit(op, [b for b, _ in d], [x for _, x in d], tag)
+    out = {}
+    while len(out) < len(reqs):
+        out.update(dict(s.run(16)[0]))
+    s.close()
+    return [i for tag in range(len(reqs)) for i in out[tag]]
+
+
+@pytest.mark.parametrize("hs", [
+    (0.1, 0.08, 0.13),       # three small segments, fused in both precisions
+    (0.03, 0.0325),          # 833 row blocks in all: fused in both
+    (0.0275, 0.028),         # 1,052: FP64 folded, mixed fused
+    (0.0175, 0.018),         # 2,573: separate in both
+])
+@pytest.mark.parametrize("precision", [cpmgpu.CPM_FP64, cpmgpu.CPM_FP32_REFINE])
+def test_several_operators_end_apart(gpu_ctx, monkeypatch, hs, precision):
+    """One right-hand side on each of several operators whose systems end at different times: FP64
+    against a server (separate kernels), mixed against iterations that are not fused."""
+    print(f"case several operators {hs} {precision}", flush=True)
+    monkeypatch.setenv("CPMGPU_FP64_ROUTING", "0")
+    ops = [cpmgpu.Tube(gpu_ctx, "Sphere", h).operator(1.0, -c) for h, c in zip(hs, (1.0, 1e-4, 1e-2))]
+    o = cpmgpu.opts(tol=1e-9, precision=precision)
+    dev = [_dev(gpu_ctx, 1, op.D, k) for k, op in enumerate(ops)]
+    read = lambda: [gpu_ctx.d2h(np.zeros(op.D), d[0][1]) for op, d in zip(ops, dev)]   # noqa: E731
+    batch = lambda: gpu_ctx.solve_batch_device(ops, [d[0][0] for d in dev], [d[0][1] for d in dev], o)   # noqa: E731
+    i1, x1 = batch(), read()
+    if precision == cpmgpu.CPM_FP64:
+        i2 = _serve_all(gpu_ctx, list(zip(ops, dev)), 1, o)
+    else:
+        monkeypatch.setenv("CPMGPU_PRECOND_FLY", "0")
+        i2 = batch()
+    x2 = read()
+    print([i["iters"] for i in i1], flush=True)
+    assert all(i["status"] == "converged" for i in i1) and len({i["iters"] for i in i1}) == len(ops)
+    assert [(i["iters"], i["updates"], i["fallback_iters"]) for i in i1] == [(i["iters"], i["updates"], i["fallback_iters"]) for i in i2]
+    assert all(np.array_equal(p, q) for p, q in zip(x1, x2))
+    for d in dev:
+        for p in d[0]:
+            gpu_ctx.free(p)
+
+
+@pytest.mark.parametrize("n,h", [
+    (2, 0.0283), (2, 0.0279),     # 506 and 520 row blocks x 2 lanes
+    (3, 0.0405), (3, 0.0395),     # 247 and 260 x 4
+    (8, 0.057), (8, 0.0555),      # 125 and 132 x 8
+])
+@pytest.mark.parametrize("precision", [cpmgpu.CPM_FP64, cpmgpu.CPM_FP32_REFINE])
+def test_folded_lanes_equal_separate_kernels(gpu_ctx, monkeypatch, n, h, precision):
+    """Several right-hand sides of one operator on both sides of 1,024 lanes x row blocks, in batches
+    (FP64; eight in the general format, which takes them in one group) and streams (mixed)."""
+    print(f"case lanes {n} {h} {precision}", flush=True)
+    monkeypatch.setenv("CPMGPU_FP64_ROUTING", "0")
+    fp64 = precision == cpmgpu.CPM_FP64
+    op = _operator(gpu_ctx, monkeypatch, "Sphere", h, False, "ell" if fp64 and n == 8 else "tp")
+    lanes = 4 if n == 3 else n
+    o = cpmgpu.opts(tol=1e-9, precision=precision)
+    d = _dev(gpu_ctx, n, op.D, 5)
+    bs, xs = [b for b, _ in d], [x for _, x in d]
+    i1 = gpu_ctx.solve_batch_device([op] * n, bs, xs, o) if fp64 else gpu_ctx.solve_stream_device(op, bs, xs, lanes=lanes, o=o)
+    x1 = [gpu_ctx.d2h(np.zeros(op.D), x) for x in xs]
+    i2 = _serve_all(gpu_ctx, [(op, d)], lanes, o)
+    x2 = [gpu_ctx.d2h(np.zeros(op.D), x) for x in xs]
+    assert [(i["status"], i["iters"], i["updates"]) for i in i1] == [(i["status"], i["iters"], i["updates"]) for i in i2]
+    assert all(np.array_equal(p, q) for p, q in zip(x1, x2))
+    for p in bs + xs:
+        gpu_ctx.free(p)
