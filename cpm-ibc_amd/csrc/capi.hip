@@ -344,16 +344,39 @@ static void fill_seg(Seg<T>& s, const Op* op, int64_t off, int nblocks, int nr, 
     s.part = part;
 }
 
+static int row_blocks(const Op* op) { return (int)((op->D + kBlock - 1) / kBlock); }
+
+// The E gathers of a launch: each segment's workgroups and the kernel of all.
+// Gathers by rows take the larger of an operator's row blocks and tiles, as the
+// refinement lanes' gathers take the same workgroups and go by tiles in any case.
+struct GatherPlan {
+    std::vector<int> ng;
+    int total = 0, tiles = 0, ell = 0;   // workgroups; segments gathered by tiles, in the ELL format
+    template <typename T, int NR>
+    void add(const Op* op) {
+        const bool by_tile = grp_gather<T, NR>(op->ngt);
+        tiles += by_tile;
+        ell += op->fmt == OP_ELL;
+        ng.push_back(by_tile ? op->ngt : std::max(op->ngt, row_blocks(op)));
+        total += ng.back();
+    }
+    GatherKind kind() const {
+        const int n = (int)ng.size();
+        return n > 0 && tiles == n ? GATHER_TILES : ell == n ? GATHER_ELL : tiles > 0 ? GATHER_MIXED : GATHER_ROWS;
+    }
+};
+
 // Block maps of a launch over segments of nb[g] row blocks and ng[g] gather
 // workgroups each (entries: segment | block within it << kSegBits), one after
-// the other: segment by segment over the row blocks, which the vector kernels run (a workgroup's rows stream from one region of
-// each vector), then round-robin (block b of every segment, then block b +
-// 1), which the E gathers run: segments that share an operator (the groups of
-// a streamed solve) gather through each tile together, its metadata read
-// into an L2 once for all of them rather than once per segment.  The
-// refinement lanes' FP64 gathers take the gather workgroups segment by
-// segment: few segments refine at once, and their workgroups belong together
-// (round-robin 43 us against 29 us a launch, 8 groups of 405,928 rows).
+// the other: segment by segment over the row blocks, which the vector kernels
+// run (a workgroup's rows stream from one region of each vector), then
+// round-robin (block b of every segment, then block b + 1), which the E gathers
+// run: segments that share an operator (the groups of a streamed solve) gather
+// through each tile together, its metadata read into an L2 once for all of
+// them rather than once per segment.  The refinement lanes' FP64 gathers take
+// the gather workgroups segment by segment: few segments refine at once, and
+// their workgroups belong together (round-robin 43 us against 29 us a launch,
+// 8 groups of 405,928 rows).
 static std::vector<int> block_map(const std::vector<int>& nb, const std::vector<int>& ng) {
     if (nb.size() > (size_t)kMaxSegs) throw ArgError("too many segments in one launch");
     int most = 0;
@@ -374,16 +397,6 @@ static std::vector<int> block_map(const std::vector<int>& nb, const std::vector<
         for (int b = 0; b < ng[g]; ++b) m.push_back((int)g | (b << kSegBits));
     return m;
 }
-
-// Fewest shared-stencil tiles of the operators of a launch (0: some have none).
-template <typename It, typename F>
-static int fewest_tiles(It b, It e, F&& op_of) {
-    int grp = b == e ? 0 : INT_MAX;
-    for (; b != e; ++b) grp = std::min(grp, op_of(*b)->ngt);
-    return grp;
-}
-
-static int row_blocks(const Op* op) { return (int)((op->D + kBlock - 1) / kBlock); }
 
 // The launches of a run of iterations between two host checks (16 of a
 // streamed solve, 4 at a time of a batch solve's chunks) captured once into a
@@ -515,29 +528,28 @@ static void run_batch(Ctx* ctx, const std::vector<Group>& groups, const std::vec
         // first attempt, has already written its results out)
         ctx->arena->used = 0;
     }
-    const int grp = fewest_tiles(groups.begin(), groups.end(), [](const Group& g) { return g.op; });
-    const bool by_tile = refine ? grp_gather<float, NR>(grp) : grp_gather<double, NR>(grp);
-    const bool ell = std::all_of(groups.begin(), groups.end(), [](const Group& g) { return g.op->fmt == OP_ELL; });
     // layout
     std::vector<int64_t> off(G);
-    std::vector<int> b0(G), nb(G), ng(G);
+    std::vector<int> b0(G), nb(G);
+    GatherPlan gp;
     int64_t total = 0;
-    int blocks = 0, gblocks = 0, most = 0;
+    int blocks = 0, most = 0;
     for (int g = 0; g < G; ++g) {
         off[g] = total;
         total += groups[g].op->D * NR;
         total = (total + 63) & ~int64_t(63);
         b0[g] = blocks;
         nb[g] = row_blocks(groups[g].op);
-        ng[g] = grp_blocks(by_tile, groups[g].op->ngt, nb[g]);
+        if (refine) gp.add<float, NR>(groups[g].op);
+        else gp.add<double, NR>(groups[g].op);
         blocks += nb[g];
-        gblocks += ng[g];
         most = std::max(most, nb[g]);
     }
     int sweeps = 0;
     for (auto& g : groups)
         if (g.op->precond == CPM_PRECOND_JACOBI) sweeps = std::max(sweeps, g.op->precond_iters);
-    const bool fly = by_tile && precond_fly();
+    const int gblocks = gp.total;
+    const bool fly = gp.kind() == GATHER_TILES && precond_fly();
     const auto [fold, fuse] = folding(most, blocks, G, NR, refine, fly && sweeps <= 1);
     // device tables: segments (one per precision), block map, states, partials.
     // The FP64 and FP32 segments of a group share one state record per rhs.
@@ -571,7 +583,7 @@ static void run_batch(Ctx* ctx, const std::vector<Group>& groups, const std::vec
         h64[g].m = h32[g].m = groups[g].m;
         h64[g].n = h32[g].n = groups[g].n;
     }
-    const std::vector<int> hb = G > 1 ? block_map(nb, ng) : std::vector<int>();
+    const std::vector<int> hb = G > 1 ? block_map(nb, gp.ng) : std::vector<int>();
     HIPCHK(hipMemcpyAsync(segs64, h64.data(), sizeof(Seg<double>) * G, hipMemcpyHostToDevice, st));
     if (refine) HIPCHK(hipMemcpyAsync(segs32, h32.data(), sizeof(Seg<float>) * G, hipMemcpyHostToDevice, st));
     if (G > 1) HIPCHK(hipMemcpyAsync(bseg, hb.data(), sizeof(int) * hb.size(), hipMemcpyHostToDevice, st));
@@ -618,8 +630,8 @@ static void run_batch(Ctx* ctx, const std::vector<Group>& groups, const std::vec
     HIPCHK(hipMemcpyAsync(dpb, pb.data(), sizeof(int) * pb.size(), hipMemcpyHostToDevice, st));
     hipLaunchKernelGGL(k_pack, dim3((unsigned)pb.size()), dim3(256), 0, st, dpe, dpb, V64.b, (float*)nullptr, 1);
 
-    const LaunchCfg<double> c64{segs64, h64.data(), bseg, blocks, gblocks, G, st, sweeps, fold, fuse, by_tile, ell, fly};
-    const LaunchCfg<float> c32{segs32, h32.data(), bseg, blocks, gblocks, G, st, sweeps, fold, fuse, by_tile, ell, fly};
+    const LaunchCfg<double> c64{segs64, h64.data(), bseg, blocks, gblocks, gp.kind(), G, st, sweeps, fold, fuse, fly};
+    const LaunchCfg<float> c32{segs32, h32.data(), bseg, blocks, gblocks, gp.kind(), G, st, sweeps, fold, fuse, fly};
     const double delta = o.update_delta > 0 ? std::min(o.update_delta, 0.999) : kDefaultUpdateDelta;
     launch_reset_states(sts, nstate, o.tol * o.tol, o.max_iters, delta * delta, st);
 
@@ -735,11 +747,12 @@ static void run_stream(Ctx* ctx, Op* op, const std::vector<const double*>& rhs, 
     const int nstate = G * kMaxNR;
     if (nstate > Ctx::kHostStates) throw ArgError("too many lanes");
     const int sweeps = op->precond == CPM_PRECOND_JACOBI ? op->precond_iters : 0;
-    const bool by_tile = grp_gather<float, NR>(op->ngt), fly = by_tile && precond_fly();
+    GatherPlan gp;
+    for (int g = 0; g < G; ++g) gp.add<float, NR>(op);
+    const int gblocks = gp.total;
+    const bool fly = gp.kind() == GATHER_TILES && precond_fly();
     const auto [fold, fuse] = folding(nb, blocks, G, NR, true, fly && sweeps <= 1);
     const int64_t sst = fold ? nstate : 0;
-    const int ng = grp_blocks(by_tile, op->ngt, nb);
-    const int gblocks = G * ng;
     const int64_t seg_total = (D * NR + 63) & ~int64_t(63);   // vector entries of one segment
     const int64_t total = seg_total * G;
     auto r256 = [](size_t k) { return (k + 255) & ~size_t(255); };
@@ -765,8 +778,7 @@ static void run_stream(Ctx* ctx, Op* op, const std::vector<const double*>& rhs, 
         fill_seg(h64[g], op, g * seg_total, nb, nr0[g], sts + g * kMaxNR, part + part_stride * g * nb, sst);
         fill_seg(h32[g], op, g * seg_total, nb, nr0[g], sts + g * kMaxNR, part + part_stride * g * nb, sst);
     }
-    const std::vector<int> hb =
-        G > 1 ? block_map(std::vector<int>((size_t)G, nb), std::vector<int>((size_t)G, ng)) : std::vector<int>();
+    const std::vector<int> hb = G > 1 ? block_map(std::vector<int>((size_t)G, nb), gp.ng) : std::vector<int>();
     HIPCHK(hipMemcpyAsync(seg64, h64.data(), sizeof(Seg<double>) * G, hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(seg32, h32.data(), sizeof(Seg<float>) * G, hipMemcpyHostToDevice, st));
     if (G > 1) HIPCHK(hipMemcpyAsync(bseg, hb.data(), sizeof(int) * hb.size(), hipMemcpyHostToDevice, st));
@@ -823,8 +835,7 @@ static void run_stream(Ctx* ctx, Op* op, const std::vector<const double*>& rhs, 
             cur[g * kMaxNR + k] = next++;
         }
     HIPCHK(hipMemcpyAsync(sts, hst.data(), sizeof(KState) * nstate, hipMemcpyHostToDevice, st));
-    const LaunchCfg<float> c32{seg32, h32.data(), bseg, blocks, gblocks, G, st, sweeps, fold, fuse,
-                               by_tile, op->fmt == OP_ELL, fly};
+    const LaunchCfg<float> c32{seg32, h32.data(), bseg, blocks, gblocks, gp.kind(), G, st, sweeps, fold, fuse, fly};
     const MixVec mv{V64.x, V64.r, V64.b, V64.tmp};
     KState* hs = ctx->host_states;
     int done = 0;
@@ -1083,9 +1094,9 @@ void multiply(Op* op, const double* dx, double* dy, double m, double n) {
     HIPCHK(hipMemcpyAsync(dbseg, hb.data(), sizeof(int) * nblocks, hipMemcpyHostToDevice, st));
     double* w = ctx->workspace("mul_tmp", sizeof(double) * op->D * 3);
     double *xi = w, *yi = w + op->D, *tmp = w + 2 * op->D;
-    const bool by_tile = grp_gather<double, 1>(op->ngt);
-    LaunchCfg<double> c{dseg, &h, dbseg, nblocks, grp_blocks(by_tile, op->ngt, nblocks), 1, st, 0, false, false, by_tile,
-                        op->fmt == OP_ELL};
+    GatherPlan gp;
+    gp.add<double, 1>(op);
+    LaunchCfg<double> c{dseg, &h, dbseg, nblocks, gp.total, gp.kind(), 1, st, 0};
     if (op->perm.p) {   // caller order -> internal order and back
         hipLaunchKernelGGL(k_pack, dim3(nblocks), dim3(256), 0, st, dpe, dbseg, xi, (float*)nullptr, 1);
         Launch<double, 1>::apply(c, xi, tmp, yi);
@@ -1103,13 +1114,14 @@ static void profile_egather_t(Op* op, int G, int reps, double* avg_ms, double* b
     const int nblocks = (int)((op->D + kBlock - 1) / kBlock);
     const int64_t seg_total = (op->D * NR + 63) & ~int64_t(63);
     std::vector<Seg<T>> h(G);
-    const bool by_tile = grp_gather<T, NR>(op->ngt);
-    const int ng = grp_blocks(by_tile, op->ngt, nblocks);
+    GatherPlan gp;
     for (int g = 0; g < G; ++g) {   // G copies of the operator in one launch, as streamed solves of 16, 32 lanes
         fill_seg(h[g], op, g * seg_total, nblocks, NR, nullptr, nullptr);
+        gp.add<T, NR>(op);
     }
+    const bool by_tile = gp.kind() == GATHER_TILES;
     const std::vector<int> hb =   // both maps (the gather runs the second)
-        block_map(std::vector<int>((size_t)G, nblocks), std::vector<int>((size_t)G, ng));
+        block_map(std::vector<int>((size_t)G, nblocks), gp.ng);
     const size_t seg_bytes = (sizeof(Seg<T>) * G + 255) & ~size_t(255);
     char* tb = reinterpret_cast<char*>(ctx->workspace("prof_tables", seg_bytes + sizeof(int) * hb.size()));
     auto* dseg = reinterpret_cast<Seg<T>*>(tb);
@@ -1123,7 +1135,7 @@ static void profile_egather_t(Op* op, int G, int reps, double* avg_ms, double* b
     T* xs = reinterpret_cast<T*>(ctx->workspace("prof_x", vec_bytes * nbuf));
     T* ys = reinterpret_cast<T*>(ctx->workspace("prof_y", vec_bytes * nbuf));
     HIPCHK(hipMemsetAsync(xs, 0, vec_bytes * nbuf, st));
-    LaunchCfg<T> c{dseg, h.data(), dbseg, nblocks * G, ng * G, G, st, 0, false, false, by_tile, false, by_tile && precond_fly()};
+    LaunchCfg<T> c{dseg, h.data(), dbseg, nblocks * G, gp.total, gp.kind(), G, st, 0, false, false, by_tile && precond_fly()};
     auto buf = [&](T* b, int r) { return b + (size_t)(r % nbuf) * seg_total * G; };
     // the gather the iterations launch: of P^-1 x unless Jacobi sweeps follow the first
     const bool fly = !(op->precond == CPM_PRECOND_JACOBI && op->precond_iters > 1);
@@ -1245,7 +1257,7 @@ static PackEntry pack_out(double* dst) { PackEntry e{}; e.dst = dst; return e; }
 // apply kernel with tmp = x, the identity rows from the held Lfull rows.
 static void explicit_diffusion(Op* op, const StepTables& t, int k, double c, const double* x, double* z) {
     const hipStream_t st = op->ctx->stream;
-    LaunchCfg<double> cfg{t.seg + k, nullptr, t.bseg, t.nblocks, t.nblocks, 1, st, 0};
+    LaunchCfg<double> cfg{t.seg + k, nullptr, t.bseg, t.nblocks, 0, GATHER_ROWS, 1, st, 0};
     launch_lfinish_plain<double>(cfg, x, x, z);
     if (op->nh > 0)
         hipLaunchKernelGGL(k_held_apply, dim3((unsigned)((op->nh + 255) / 256)), dim3(256), 0, st, op->nh, op->hw,
@@ -1254,9 +1266,9 @@ static void explicit_diffusion(Op* op, const StepTables& t, int k, double c, con
 }
 
 static void extension(Op* op, const StepTables& t, const double* z, double* y) {
-    const bool by_tile = grp_gather<double, 1>(op->ngt);
-    LaunchCfg<double> cfg{t.seg, nullptr, t.bseg, t.nblocks, grp_blocks(by_tile, op->ngt, t.nblocks), 1, op->ctx->stream, 0,
-                          false, false, by_tile};
+    GatherPlan gp;
+    gp.add<double, 1>(op);
+    LaunchCfg<double> cfg{t.seg, nullptr, t.bseg, t.nblocks, gp.total, gp.kind(), 1, op->ctx->stream, 0};
     launch_egather<double, 1>(cfg, z, y);
 }
 
@@ -1485,8 +1497,10 @@ struct Server : ServerBase {
     RangePool ranges;   // vector ranges of the pools
     std::vector<Req> reqs;
     bool dirty = true;
-    int nblocks = 0, gblocks = 0;
-    bool by_tile = false, fly = false;   // the gather that rebuild laid the block maps out for
+    int nblocks = 0;
+    int gblocks = 0;
+    GatherKind gather = GATHER_ROWS;   // that rebuild laid the block maps out for
+    bool fly = false;
     Seg<float>* d_segs = nullptr;
     int* d_bseg = nullptr;
     double* d_part = nullptr;
@@ -1628,24 +1642,24 @@ struct Server : ServerBase {
 
     void rebuild() {
         ensure_tables();
-        by_tile = grp_gather<float, NR>(fewest_tiles(reqs.begin(), reqs.end(), [](const Req& q) { return q.op; }));
-        fly = by_tile && precond_fly();
         std::vector<Seg<float>> h(reqs.size());
-        std::vector<int> nbs, ngs;
+        std::vector<int> nbs;
+        GatherPlan gp;
         int b0 = 0;
-        gblocks = 0;
         for (size_t g = 0; g < reqs.size(); ++g) {
             const Req& q = reqs[g];
             const int nb = (int)((q.op->D + kBlock - 1) / kBlock);
             fill_seg(h[g], q.op, q.off, nb, q.nr, states.template as<KState>() + (size_t)q.slot * kMaxNR,
                      d_part + (size_t)2 * NR * b0);
             nbs.push_back(nb);
-            ngs.push_back(grp_blocks(by_tile, q.op->ngt, nb));
+            gp.template add<float, NR>(q.op);
             b0 += nb;
-            gblocks += ngs.back();
         }
-        const std::vector<int> map = block_map(nbs, ngs);
+        const std::vector<int> map = block_map(nbs, gp.ng);
         nblocks = b0;
+        gblocks = gp.total;
+        gather = gp.kind();
+        fly = gather == GATHER_TILES && precond_fly();
         const hipStream_t st = ctx->stream;
         HIPCHK(hipMemcpyAsync(d_segs, h.data(), sizeof(Seg<float>) * h.size(), hipMemcpyHostToDevice, st));
         HIPCHK(hipMemcpyAsync(d_bseg, map.data(), sizeof(int) * map.size(), hipMemcpyHostToDevice, st));
@@ -1659,7 +1673,7 @@ struct Server : ServerBase {
         const hipStream_t st = ctx->stream;
         const Vecs<float> V32{nullptr, v32(0), v32(1), v32(2), v32(3), v32(4), v32(5), v32(6), v32(7), v32(8), v32(9)};
         const MixVec mv{v64(1), v64(2), v64(0), v64(4)};
-        const LaunchCfg<float> c{d_segs, nullptr, d_bseg, nblocks, gblocks, (int)reqs.size(), st, 0, false, false, by_tile, false, fly};
+        const LaunchCfg<float> c{d_segs, nullptr, d_bseg, nblocks, gblocks, gather, (int)reqs.size(), st, 0, false, false, fly};
         Vecs<float> w = V32;
         Launch<float, NR>::iterations(c, w, true, mv, iters);
         HIPCHK(hipGetLastError());
@@ -1737,8 +1751,10 @@ struct Server64 : ServerBase {
     RangePool ranges;
     std::vector<Req> reqs;
     bool dirty = true;
-    int nblocks = 0, gblocks = 0;
-    bool by_tile = false, fly = false;   // the gather that rebuild laid the block maps out for
+    int nblocks = 0;
+    int gblocks = 0;
+    GatherKind gather = GATHER_ROWS;   // that rebuild laid the block maps out for
+    bool fly = false;
     Seg<double>* d_segs = nullptr;
     int* d_bseg = nullptr;
     double* d_part = nullptr;
@@ -1840,7 +1856,7 @@ struct Server64 : ServerBase {
         Seg<double> h{};
         fill_seg(h, op, off, nb, nrhs, sts, i_part());
         HIPCHK(hipMemcpyAsync(i_seg(), &h, sizeof(h), hipMemcpyHostToDevice, st));
-        const LaunchCfg<double> c1{i_seg(), &h, nullptr, nb, nb, 1, st, 0};   // no gather
+        const LaunchCfg<double> c1{i_seg(), &h, nullptr, nb, 0, GATHER_ROWS, 1, st, 0};   // no gather
         Launch<double, NR>::init(c1, v64(0), v64(1), v64(2), v64(3), v64(4), v64(5));
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(st));
@@ -1851,24 +1867,24 @@ struct Server64 : ServerBase {
 
     void rebuild() {
         ensure_tables();
-        by_tile = grp_gather<double, NR>(fewest_tiles(reqs.begin(), reqs.end(), [](const Req& q) { return q.op; }));
-        fly = by_tile && precond_fly();
         std::vector<Seg<double>> h(reqs.size());
-        std::vector<int> nbs, ngs;
+        std::vector<int> nbs;
+        GatherPlan gp;
         int b0 = 0;
-        gblocks = 0;
         for (size_t g = 0; g < reqs.size(); ++g) {
             const Req& q = reqs[g];
             const int nb = (int)((q.op->D + kBlock - 1) / kBlock);
             fill_seg(h[g], q.op, q.off, nb, q.nr, states.template as<KState>() + (size_t)q.slot * kMaxNR,
                      d_part + (size_t)2 * NR * b0);
             nbs.push_back(nb);
-            ngs.push_back(grp_blocks(by_tile, q.op->ngt, nb));
+            gp.template add<double, NR>(q.op);
             b0 += nb;
-            gblocks += ngs.back();
         }
-        const std::vector<int> map = block_map(nbs, ngs);
+        const std::vector<int> map = block_map(nbs, gp.ng);
         nblocks = b0;
+        gblocks = gp.total;
+        gather = gp.kind();
+        fly = gather == GATHER_TILES && precond_fly();
         const hipStream_t st = ctx->stream;
         HIPCHK(hipMemcpyAsync(d_segs, h.data(), sizeof(Seg<double>) * h.size(), hipMemcpyHostToDevice, st));
         HIPCHK(hipMemcpyAsync(d_bseg, map.data(), sizeof(int) * map.size(), hipMemcpyHostToDevice, st));
@@ -1881,7 +1897,7 @@ struct Server64 : ServerBase {
         if (dirty) rebuild();
         const hipStream_t st = ctx->stream;
         Vecs<double> V{v64(0), v64(1), v64(2), v64(3), v64(4), v64(5), v64(6), v64(7), v64(8), v64(9), v64(10)};
-        const LaunchCfg<double> c{d_segs, nullptr, d_bseg, nblocks, gblocks, (int)reqs.size(), st, 0, false, false, by_tile, false, fly};
+        const LaunchCfg<double> c{d_segs, nullptr, d_bseg, nblocks, gblocks, gather, (int)reqs.size(), st, 0, false, false, fly};
         Launch<double, NR>::iterations(c, V, false, MixVec{}, iters);
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(ctx->host_states, states.template as<KState>(), sizeof(KState) * (size_t)slots * kMaxNR,

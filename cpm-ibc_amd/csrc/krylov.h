@@ -13,6 +13,11 @@ struct SegArg {
     Seg<T> one;
 };
 
+// The kernel of a launch's E gathers: every operator by shared-stencil tiles,
+// every operator in the ELL format, some by tiles and the others by rows, or
+// none by tiles (none built, or values too wide for their LDS).
+enum GatherKind : int { GATHER_TILES, GATHER_ELL, GATHER_MIXED, GATHER_ROWS };
+
 template <typename T>
 struct LaunchCfg {
     const Seg<T>* segs;    // device segment table
@@ -21,34 +26,25 @@ struct LaunchCfg {
                            // segment, gblocks round-robin over the segments (the E gathers'), gblocks
                            // segment by segment (the refinement lanes' gathers'); not read where nseg = 1
     int nblocks;
-    int gblocks;           // workgroups of an E gather (grp_blocks)
+    int gblocks;           // workgroups of an E gather
+    GatherKind gather;     // decided once, where gblocks and the block maps are laid out for it: a choice
+                           // made again at a launch could meet a grid that was laid out for another kernel
     int nseg;
     hipStream_t stream;
     int jacobi_sweeps;     // largest precond_iters over Jacobi-preconditioned segments (0: none)
     bool fold = false;     // the finalisers run inside the kernels that need them (Seg::sst set)
     bool fuse = false;     // ... and pupdate and supdate inside the gathers and lfinish, where those allow it
-    // Which gather kernel runs is decided once, where gblocks and the block
-    // maps are laid out for it, and kept here: a choice made again at a launch
-    // could meet a grid that was laid out for the other kernel.
-    bool tiles = false;    // the E gathers run by shared-stencil tiles (grp_gather)
-    bool ell = false;      // every operator is in the ELL format
-    bool fly = false;      // iterations form P^-1 where it is read (precond_fly; with tiles)
+    bool fly = false;      // iterations form P^-1 where it is read (precond_fly; every gather by tiles)
 };
 
-// Whether the E gathers of a launch use shared-stencil tiles: values whose
-// rows fit the tiles' LDS, every operator with tiles (ntiles: the fewest), and
-// the environment does not say CPMGPU_GROUP_GATHER=none.
+// Whether the E gathers of an operator with ntiles shared-stencil tiles use
+// them: there are some, the values' rows fit the tiles' LDS, and the
+// environment does not say CPMGPU_GROUP_GATHER=none.
 template <typename T, int NR>
 bool grp_gather(int ntiles);
 // Whether iterations that gather by tiles form y = P^-1 p and z = P^-1 s where
 // they are read (CPMGPU_PRECOND_FLY=0 stores them instead).
 bool precond_fly();
-// Workgroups that the E gathers of such a launch (grp) take for an operator
-// of ntiles tiles and nblocks row blocks; other launches gather by row blocks
-// (the refinement lanes' FP64 gathers by tiles in both).
-inline int grp_blocks(bool grp, int ntiles, int nblocks) {
-    return grp ? ntiles : ntiles > nblocks ? ntiles : nblocks;
-}
 
 // Workspace vectors of one precision; every vector spans all segments
 // (segment g occupies [off_g, off_g + D_g * NR)).

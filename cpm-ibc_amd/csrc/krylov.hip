@@ -1492,6 +1492,33 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WPE))) v
     egather_grp_tile<T, NR, LR>(sg.op, lb, src, DstPlain<T, NR>{out + sg.off}, lrows, [](auto&) { return true; });
 }
 
+// E x for launches over operators of which some have shared-stencil tiles:
+// those by their tiles, a row a thread of the others. 60 FP64 iterations of 3
+// right-hand sides of an ELL operator of 19,021 rows and two others of 41,870
+// and 41,185 / of 51,765, 115,734 and 113,404 rows: 4.6 / 7.2 ms; in a kernel
+// each, which run one after the other, 5.5 / 7.9; every operator's rows read
+// directly 5.5 / 9.7, tensor-product ones through row tiles 5.0 / 8.6.
+template <typename T, int NR>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(CPMGPU_GROUP_WAVES_WIDE))) void k_egather_mixed(
+    const Seg<T>* __restrict__ segs, const int* __restrict__ bseg, const T* x, T* out, unsigned lanes, MixVec, int copy) {
+    typedef typename VT<T, NR>::type V;
+    constexpr int LR = GrpTile<T, NR>::kRows;
+    __shared__ V lx[LR];
+    const LdsRows<V> lrows{lx, LR};
+    int lb;
+    int64_t row;
+    const Seg<T>& sg = seg_of(segs, bseg, lb, row);
+    const auto L = lane_stat<NR>(sg, lanes != 0, copy);
+    if (lanes && !seg_any(L, lanes & ~M_UPDATE)) return;   // uniform per workgroup
+    if (sg.op.ngt > 0) {
+        if (lb >= sg.op.ngt) return;
+        SrcPlain<T, NR, false> src{&sg, x + sg.off};
+        egather_grp_tile<T, NR, LR>(sg.op, lb, src, DstPlain<T, NR>{out + sg.off}, lrows, [](auto&) { return true; });
+    } else if (row < sg.op.D) {
+        vstore<T, NR>(out + (size_t)(sg.off + row * NR), erow<T, NR>(sg.op, row, x + sg.off, NR));
+    }
+}
+
 // out = A x from tmp = E x.  RED = 0: no reduction; 1: partial (other, out);
 // 2: partials (out, out), (out, other).
 // Mixed, RED = 1: UPDATE lanes r64 = b - A64 x64, partial (r64, r64).
@@ -2162,28 +2189,10 @@ void launch_reset_states(KState* st, int n, double tol2, int max_it, double delt
 // ---------------------------------------------------------------- launchers
 #define LAUNCH(kern, ...) \
     hipLaunchKernelGGL(kern, dim3(c.nblocks), dim3(kBlock), 0, c.stream, c.segs, c.nseg == 1 ? nullptr : c.bseg, __VA_ARGS__)
-// The E gathers run the round-robin block map.
-#define LAUNCH_GATHER(kern, ...)                                                                         \
-    hipLaunchKernelGGL(kern, dim3(c.gblocks), dim3(kBlock), 0, c.stream, c.segs,                        \
-                       c.nseg == 1 ? nullptr : c.bseg + c.nblocks, __VA_ARGS__)
 // The refinement lanes' gathers run the same workgroups segment by segment.
 #define LAUNCH_UPD(kern, ...)                                                                            \
     hipLaunchKernelGGL(kern, dim3(c.gblocks), dim3(kBlock), 0, c.stream, c.segs,                        \
                        c.nseg == 1 ? nullptr : c.bseg + c.nblocks + c.gblocks, __VA_ARGS__)
-// E gather of launch c; FL: form P^-1 of the gathered vector (only with
-// shared-stencil tiles).
-#define EGATHER(FL, ...)                                                     \
-    do {                                                                     \
-        if constexpr (GrpTile<T, NR>::kRows > 0) {                           \
-            if (c.tiles) {                                                   \
-                if (FL) LAUNCH_GATHER((k_egather_grp<T, NR, GrpWaves<T, NR>::kWaves, true>), __VA_ARGS__); \
-                else LAUNCH_GATHER((k_egather_grp<T, NR, GrpWaves<T, NR>::kWaves, false>), __VA_ARGS__); \
-                break;                                                       \
-            }                                                                \
-        }                                                                    \
-        if (c.ell) LAUNCH_GATHER((k_egather_ell<T, NR>), __VA_ARGS__);       \
-        else LAUNCH_GATHER((k_egather<T, NR>), __VA_ARGS__);                 \
-    } while (0)
 #define FIN_COPY(T, NR, KIND, IN, OUT) \
     hipLaunchKernelGGL((k_fin<T, NR, KIND>), dim3(c.nseg * NR), dim3(kBlock), 0, c.stream, c.segs, IN, OUT)
 #define FIN(T, NR, KIND) FIN_COPY(T, NR, KIND, 0, 0)
@@ -2194,6 +2203,20 @@ template <typename T, int NR>
 struct GrpWaves {
     static constexpr int kWaves = (sizeof(T) == 4 && NR != 4) ? 4 : CPMGPU_GROUP_WAVES_WIDE;
 };
+
+// E gathers of launch c; fly: of P^-1 x (only by tiles).
+template <typename T, int NR>
+static void egather(const LaunchCfg<T>& c, bool fly, const T* x, T* out, unsigned lanes, const MixVec& mv, int copy) {
+    const int* map = c.nseg == 1 ? nullptr : c.bseg + c.nblocks;   // the round-robin block map
+    auto run = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(c.gblocks), dim3(kBlock), 0, c.stream, c.segs, map, x, out, lanes, mv, copy); };
+    if constexpr (GrpTile<T, NR>::kRows > 0) {
+        constexpr int W = GrpWaves<T, NR>::kWaves;
+        if (c.gather == GATHER_TILES) return fly ? run(k_egather_grp<T, NR, W, true>) : run(k_egather_grp<T, NR, W, false>);
+        if (c.gather == GATHER_MIXED) return run(k_egather_mixed<T, NR>);
+    }
+    if (c.gather == GATHER_ELL) return run(k_egather_ell<T, NR>);
+    run(k_egather<T, NR>);
+}
 
 bool precond_fly() {
     const char* e = std::getenv("CPMGPU_PRECOND_FLY");
@@ -2229,27 +2252,27 @@ void Launch<T, NR>::iteration(const LaunchCfg<T>& c, Vecs<T>& w, bool mixed, con
     if (FOLD && !first) LAUNCH((k_pupdate<T, NR, I>), w.p, w.v, w.r, w.y, w.x, mv, fl);
     else LAUNCH((k_pupdate<T, NR, -1>), w.p, w.v, w.r, w.y, w.x, mv, fl);
     for (int sw = 1; sw < c.jacobi_sweeps; ++sw) {   // y = P^-1 p, Jacobi sweeps after the first
-        EGATHER(false, w.y, w.tmp, M_RUN, MixVec{}, 0);
+        egather<T, NR>(c, false, w.y, w.tmp, M_RUN, MixVec{}, 0);
         LAUNCH((k_jacobi<T, NR>), w.p, w.tmp, w.y, sw, 0);
     }
     if constexpr (std::is_same<T, float>::value) {
         if (mixed) {   // FP32 lanes in the gather, refinement lanes' FP64 gathers in a launch of their own
-            EGATHER(fly, yp, w.tmp, M_RUN, mv, 0);
+            egather<T, NR>(c, fly, yp, w.tmp, M_RUN, mv, 0);
             LAUNCH_UPD((k_egather_upd<NR>), mv, (const float*)nullptr);
         } else {
-            EGATHER(fly, yp, w.tmp, M_STAGE1, mv, 0);
+            egather<T, NR>(c, fly, yp, w.tmp, M_STAGE1, mv, 0);
         }
     } else {
-        EGATHER(fly, yp, w.tmp, M_STAGE1, mv, 0);
+        egather<T, NR>(c, fly, yp, w.tmp, M_STAGE1, mv, 0);
     }
     LAUNCH((k_lfinish<T, NR, 1>), yp, w.tmp, w.v, w.r0, (const T*)nullptr, M_STAGE1, mv, fl, 0);
     if (!FOLD) FIN(T, NR, FIN_ALPHA);
     LAUNCH((k_supdate<T, NR, A>), w.r, w.v, w.s, w.z, w.r0, w.p, mv, fl);
     for (int sw = 1; sw < c.jacobi_sweeps; ++sw) {   // z = P^-1 s
-        EGATHER(false, w.z, w.tmp, M_RUN, MixVec{}, s1);
+        egather<T, NR>(c, false, w.z, w.tmp, M_RUN, MixVec{}, s1);
         LAUNCH((k_jacobi<T, NR>), w.s, w.tmp, w.z, sw, s1);
     }
-    EGATHER(fly, zs, w.tmp, M_RUN, mv, s1);
+    egather<T, NR>(c, fly, zs, w.tmp, M_RUN, mv, s1);
     LAUNCH((k_lfinish<T, NR, 2>), zs, w.tmp, w.t, w.s, (const T*)w.r, M_STAGE2, mv, fl, s1);
     if (!FOLD) FIN(T, NR, FIN_OMEGA);
     LAUNCH((k_xrupdate<T, NR, O>), w.x, yp, w.z, w.r, w.s, w.t, w.r0, fl);
@@ -2296,7 +2319,7 @@ void Launch<T, NR>::iterations(const LaunchCfg<T>& c, Vecs<T>& w, bool mixed, co
 template <typename T, int NR>
 void Launch<T, NR>::restart(const LaunchCfg<T>& c, Vecs<T>& w) {
     const MixVec none{};
-    EGATHER(false, w.x, w.tmp, M_RESTART, none, 0);
+    egather<T, NR>(c, false, w.x, w.tmp, M_RESTART, none, 0);
     LAUNCH((k_lfinish<T, NR, 0>), w.x, w.tmp, w.t, (const T*)nullptr, (const T*)nullptr, M_RESTART, none, 0, 0);
     LAUNCH((k_restart<T, NR>), w.b, w.t, w.r, w.r0);
     FIN(T, NR, FIN_RESTART64);
@@ -2304,7 +2327,7 @@ void Launch<T, NR>::restart(const LaunchCfg<T>& c, Vecs<T>& w) {
 template <typename T, int NR>
 void Launch<T, NR>::apply(const LaunchCfg<T>& c, const T* x, T* tmp, T* y, unsigned lanes) {
     const MixVec none{};
-    EGATHER(false, x, tmp, lanes, none, 0);
+    egather<T, NR>(c, false, x, tmp, lanes, none, 0);
     LAUNCH((k_lfinish<T, NR, 0>), x, tmp, y, (const T*)nullptr, (const T*)nullptr, lanes, none, 0, 0);
 }
 
@@ -2356,7 +2379,7 @@ template <typename T, int NR>
 void launch_egather(const LaunchCfg<T>& c, const T* x, T* out, bool fly) {
     const MixVec none{};
     const bool fl = fly && c.fly;
-    EGATHER(fl, x, out, 0u, none, 0);
+    egather<T, NR>(c, fl, x, out, 0u, none, 0);
 }
 
 template <int NR>
