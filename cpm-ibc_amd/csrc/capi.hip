@@ -477,6 +477,8 @@ struct Folding {
     bool fold, fuse;
 };
 static Folding folding(int64_t most, int64_t total, int segments, int NR, bool f32, bool fusable) {
+    const char* e = std::getenv("CPMGPU_FOLD");   // 0: separate kernels, for comparison (read per launch sequence)
+    if (e && std::string(e) == "0") return {false, false};
     if (NR == 1 && fusable && total <= (segments == 1 || f32 ? 2560 : 1024)) return {true, true};
     return {most * NR <= (NR == 1 ? 1280 : 1024) && total * NR <= 2560, false};
 }
@@ -1501,6 +1503,8 @@ struct Server : ServerBase {
     int gblocks = 0;
     GatherKind gather = GATHER_ROWS;   // that rebuild laid the block maps out for
     bool fly = false;
+    Folding fd{false, false};
+    std::vector<Seg<float>> h_segs;
     Seg<float>* d_segs = nullptr;
     int* d_bseg = nullptr;
     double* d_part = nullptr;
@@ -1516,7 +1520,7 @@ struct Server : ServerBase {
         p32 = Buffer(sizeof(float) * (size_t)cap * 10);
         p64 = Buffer(sizeof(double) * (size_t)cap * 5);
         slots = Ctx::kHostStates / kMaxNR;
-        states = Buffer(sizeof(KState) * (size_t)slots * kMaxNR);
+        states = Buffer(sizeof(KState) * 3 * (size_t)slots * kMaxNR);   // three copies: folded finalisers
         for (int i = slots - 1; i >= 0; --i) free_slots.push_back(i);
         ranges.reset(cap);
     }
@@ -1556,7 +1560,7 @@ struct Server : ServerBase {
         auto r256 = [](size_t k) { return (k + 255) & ~size_t(255); };
         const size_t sseg = r256(sizeof(Seg<float>) * std::max<size_t>(reqs.size(), 1));
         const size_t smap = r256(sizeof(int) * (size_t)std::max(blocks + 2 * gblocks, 1));   // block maps
-        const size_t spart = r256(sizeof(double) * 2 * NR * std::max(blocks, 1));
+        const size_t spart = r256(sizeof(double) * 4 * NR * std::max(blocks, 1));
         const size_t spack = r256(sizeof(PackEntry));
         const size_t szero = r256(sizeof(int) * zn);
         const size_t need = sseg + smap + spart + spack + szero;
@@ -1642,26 +1646,29 @@ struct Server : ServerBase {
 
     void rebuild() {
         ensure_tables();
-        std::vector<Seg<float>> h(reqs.size());
         std::vector<int> nbs;
         GatherPlan gp;
-        int b0 = 0;
-        for (size_t g = 0; g < reqs.size(); ++g) {
-            const Req& q = reqs[g];
-            const int nb = (int)((q.op->D + kBlock - 1) / kBlock);
-            fill_seg(h[g], q.op, q.off, nb, q.nr, states.template as<KState>() + (size_t)q.slot * kMaxNR,
-                     d_part + (size_t)2 * NR * b0);
-            nbs.push_back(nb);
+        int most = 0, total = 0;
+        for (const Req& q : reqs) {
+            nbs.push_back(row_blocks(q.op));
+            most = std::max(most, nbs.back());
+            total += nbs.back();
             gp.template add<float, NR>(q.op);
-            b0 += nb;
         }
-        const std::vector<int> map = block_map(nbs, gp.ng);
-        nblocks = b0;
+        nblocks = total;
         gblocks = gp.total;
         gather = gp.kind();
         fly = gather == GATHER_TILES && precond_fly();
+        // between runs the current states are copy 0 and no iteration is half done, so requests may be
+        // folded or fused in one run and not in the next (the same bits either way)
+        fd = folding(most, total, (int)reqs.size(), NR, true, fly);
+        h_segs.resize(reqs.size());
+        for (size_t g = 0, b0 = 0; g < reqs.size(); b0 += (size_t)nbs[g++])
+            fill_seg(h_segs[g], reqs[g].op, reqs[g].off, nbs[g], reqs[g].nr, states.template as<KState>() + (size_t)reqs[g].slot * kMaxNR,
+                     d_part + (size_t)(fd.fold ? 4 : 2) * NR * b0, fd.fold ? (int64_t)slots * kMaxNR : 0);
+        const std::vector<int> map = block_map(nbs, gp.ng);
         const hipStream_t st = ctx->stream;
-        HIPCHK(hipMemcpyAsync(d_segs, h.data(), sizeof(Seg<float>) * h.size(), hipMemcpyHostToDevice, st));
+        HIPCHK(hipMemcpyAsync(d_segs, h_segs.data(), sizeof(Seg<float>) * h_segs.size(), hipMemcpyHostToDevice, st));
         HIPCHK(hipMemcpyAsync(d_bseg, map.data(), sizeof(int) * map.size(), hipMemcpyHostToDevice, st));
         HIPCHK(hipStreamSynchronize(st));
         dirty = false;
@@ -1673,7 +1680,7 @@ struct Server : ServerBase {
         const hipStream_t st = ctx->stream;
         const Vecs<float> V32{nullptr, v32(0), v32(1), v32(2), v32(3), v32(4), v32(5), v32(6), v32(7), v32(8), v32(9)};
         const MixVec mv{v64(1), v64(2), v64(0), v64(4)};
-        const LaunchCfg<float> c{d_segs, nullptr, d_bseg, nblocks, gblocks, gather, (int)reqs.size(), st, 0, false, false, fly};
+        const LaunchCfg<float> c{d_segs, h_segs.data(), d_bseg, nblocks, gblocks, gather, (int)reqs.size(), st, 0, fd.fold, fd.fuse, fly};
         Vecs<float> w = V32;
         Launch<float, NR>::iterations(c, w, true, mv, iters);
         HIPCHK(hipGetLastError());
@@ -1755,6 +1762,8 @@ struct Server64 : ServerBase {
     int gblocks = 0;
     GatherKind gather = GATHER_ROWS;   // that rebuild laid the block maps out for
     bool fly = false;
+    Folding fd{false, false};
+    std::vector<Seg<double>> h_segs;
     Seg<double>* d_segs = nullptr;
     int* d_bseg = nullptr;
     double* d_part = nullptr;
@@ -1768,7 +1777,7 @@ struct Server64 : ServerBase {
         if (cap < 64) throw ArgError("server pool too small");
         p64 = Buffer(sizeof(double) * (size_t)cap * 11);
         slots = Ctx::kHostStates / kMaxNR;
-        states = Buffer(sizeof(KState) * (size_t)slots * kMaxNR);
+        states = Buffer(sizeof(KState) * 3 * (size_t)slots * kMaxNR);   // three copies: folded finalisers
         for (int i = slots - 1; i >= 0; --i) free_slots.push_back(i);
         ranges.reset(cap);
         const int zn = (int)((cap + kBlock - 1) / kBlock);
@@ -1813,7 +1822,7 @@ struct Server64 : ServerBase {
         auto r256 = [](size_t k) { return (k + 255) & ~size_t(255); };
         const size_t sseg = r256(sizeof(Seg<double>) * std::max<size_t>(reqs.size(), 1));
         const size_t smap = r256(sizeof(int) * (size_t)std::max(blocks + 2 * gblocks, 1));   // block maps
-        const size_t spart = r256(sizeof(double) * 2 * NR * std::max(blocks, 1));
+        const size_t spart = r256(sizeof(double) * 4 * NR * std::max(blocks, 1));
         const size_t need = sseg + smap + spart;
         if (need > tables_bytes) {
             HIPCHK(hipStreamSynchronize(ctx->stream));
@@ -1867,26 +1876,29 @@ struct Server64 : ServerBase {
 
     void rebuild() {
         ensure_tables();
-        std::vector<Seg<double>> h(reqs.size());
         std::vector<int> nbs;
         GatherPlan gp;
-        int b0 = 0;
-        for (size_t g = 0; g < reqs.size(); ++g) {
-            const Req& q = reqs[g];
-            const int nb = (int)((q.op->D + kBlock - 1) / kBlock);
-            fill_seg(h[g], q.op, q.off, nb, q.nr, states.template as<KState>() + (size_t)q.slot * kMaxNR,
-                     d_part + (size_t)2 * NR * b0);
-            nbs.push_back(nb);
+        int most = 0, total = 0;
+        for (const Req& q : reqs) {
+            nbs.push_back(row_blocks(q.op));
+            most = std::max(most, nbs.back());
+            total += nbs.back();
             gp.template add<double, NR>(q.op);
-            b0 += nb;
         }
-        const std::vector<int> map = block_map(nbs, gp.ng);
-        nblocks = b0;
+        nblocks = total;
         gblocks = gp.total;
         gather = gp.kind();
         fly = gather == GATHER_TILES && precond_fly();
+        // between runs the current states are copy 0 and no iteration is half done, so requests may be
+        // folded or fused in one run and not in the next (the same bits either way)
+        fd = folding(most, total, (int)reqs.size(), NR, false, fly);
+        h_segs.resize(reqs.size());
+        for (size_t g = 0, b0 = 0; g < reqs.size(); b0 += (size_t)nbs[g++])
+            fill_seg(h_segs[g], reqs[g].op, reqs[g].off, nbs[g], reqs[g].nr, states.template as<KState>() + (size_t)reqs[g].slot * kMaxNR,
+                     d_part + (size_t)(fd.fold ? 4 : 2) * NR * b0, fd.fold ? (int64_t)slots * kMaxNR : 0);
+        const std::vector<int> map = block_map(nbs, gp.ng);
         const hipStream_t st = ctx->stream;
-        HIPCHK(hipMemcpyAsync(d_segs, h.data(), sizeof(Seg<double>) * h.size(), hipMemcpyHostToDevice, st));
+        HIPCHK(hipMemcpyAsync(d_segs, h_segs.data(), sizeof(Seg<double>) * h_segs.size(), hipMemcpyHostToDevice, st));
         HIPCHK(hipMemcpyAsync(d_bseg, map.data(), sizeof(int) * map.size(), hipMemcpyHostToDevice, st));
         HIPCHK(hipStreamSynchronize(st));
         dirty = false;
@@ -1897,7 +1909,7 @@ struct Server64 : ServerBase {
         if (dirty) rebuild();
         const hipStream_t st = ctx->stream;
         Vecs<double> V{v64(0), v64(1), v64(2), v64(3), v64(4), v64(5), v64(6), v64(7), v64(8), v64(9), v64(10)};
-        const LaunchCfg<double> c{d_segs, nullptr, d_bseg, nblocks, gblocks, gather, (int)reqs.size(), st, 0, false, false, fly};
+        const LaunchCfg<double> c{d_segs, h_segs.data(), d_bseg, nblocks, gblocks, gather, (int)reqs.size(), st, 0, fd.fold, fd.fuse, fly};
         Launch<double, NR>::iterations(c, V, false, MixVec{}, iters);
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(ctx->host_states, states.template as<KState>(), sizeof(KState) * (size_t)slots * kMaxNR,

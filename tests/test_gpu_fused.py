@@ -1,8 +1,8 @@
 """Iterations with finalisers folded into their kernels, and fused ones, end
 bit for bit where the separate kernels end: batch and streamed solves of one
 right-hand side (folded up to 2,560 row blocks, fused on tensor-product
-operators) against request servers of one lane, which run the separate
-kernels."""
+operators) against request servers of one lane that run the separate kernels
+(CPMGPU_FOLD=0)."""
 import numpy as np
 import pytest
 
@@ -24,13 +24,7 @@ def _operator(ctx, monkeypatch, surface, dx, ibc, fmt):
 
 
 def _serve(ctx, op, d_b, d_x, o):
-    s = cpmgpu.Server(ctx, 256 * op.D, lanes=1, o=o)
-    assert s.submit(op, [d_b], [d_x], 7)
-    while True:
-        done, _ = s.run(16)
-        if done:
-            s.close()
-            return done[0][1][0]
+    return _serve_all(ctx, [(op, [(d_b, d_x)])], 1, o)[0]
 
 
 @pytest.mark.parametrize("surface,dx,ibc,fmt", [
@@ -76,15 +70,20 @@ def _dev(ctx, n, D, seed):
     return d
 
 
-def _serve_all(ctx, reqs, lanes, o):
+def _serve_all(ctx, reqs, lanes, o, fold="0", chunks=(16,)):
     """reqs: (operator, [(d_b, d_x) ..]) each; the infos of every right-hand side in order."""
-    s = cpmgpu.Server(ctx, sum(90 * lanes * (op.D + 64) for op, _ in reqs) + 4096, lanes=lanes, o=o)
-    for tag, (op, d) in enumerate(reqs):
-        assert s.submit(op, [b for b, _ in d], [x for _, x in d], tag)
-    out = {}
-    while len(out) < len(reqs):
-        out.update(dict(s.run(16)[0]))
-    s.close()
+    with pytest.MonkeyPatch.context() as m:
+        m.setenv("CPMGPU_FOLD", fold)
+        s = cpmgpu.Server(ctx, sum(90 * lanes * (op.D + 64) for op, _ in reqs) + 4096, lanes=lanes, o=o)
+        out, waiting, k = {}, list(enumerate(reqs)), 0
+        while len(out) < len(reqs):
+            for _ in range(len(reqs) if len(chunks) == 1 else 1):   # all at once, or one before each run
+                if waiting:
+                    tag, (op, d) = waiting.pop(0)
+                    assert s.submit(op, [b for b, _ in d], [x for _, x in d], tag)
+            out.update(dict(s.run(chunks[k % len(chunks)])[0]))
+            k += 1
+        s.close()
     return [i for tag in range(len(reqs)) for i in out[tag]]
 
 
@@ -146,3 +145,33 @@ def test_folded_lanes_equal_separate_kernels(gpu_ctx, monkeypatch, n, h, precisi
     assert all(np.array_equal(p, q) for p, q in zip(x1, x2))
     for p in bs + xs:
         gpu_ctx.free(p)
+
+
+@pytest.mark.parametrize("hs,lanes,n", [
+    ((0.1,), 1, 1),                     # one request: fused
+    ((0.03, 0.0325, 0.2), 1, 1),        # fused while few are in, then folded (FP64)
+    ((0.0175, 0.018, 0.1), 1, 1),       # past both lines while all are in
+    ((0.1, 0.08, 0.13, 0.2), 4, 3),     # folded
+    ((0.0405, 0.08), 4, 3),             # folded until both are in
+])
+@pytest.mark.parametrize("precision", [cpmgpu.CPM_FP64, cpmgpu.CPM_FP32_REFINE])
+def test_servers_fold(gpu_ctx, monkeypatch, hs, lanes, n, precision):
+    """Requests joining and leaving a server that folds or fuses where it may, with runs of odd
+    lengths, against one that never does."""
+    print(f"case servers fold {hs} {lanes} {precision}", flush=True)
+    monkeypatch.setenv("CPMGPU_FP64_ROUTING", "0")
+    reqs = []
+    for k, h in enumerate(hs):
+        op = cpmgpu.Tube(gpu_ctx, "Sphere", h).operator(1.0, -(0.1 ** (k % 3)))
+        reqs.append((op, _dev(gpu_ctx, n, op.D, k)))
+    o = cpmgpu.opts(tol=1e-9, precision=precision)
+    res = []
+    for fold in ("1", "0"):
+        infos = _serve_all(gpu_ctx, reqs, lanes, o, fold, (3, 1, 16, 7))
+        res.append((infos, [gpu_ctx.d2h(np.zeros(op.D), x) for op, d in reqs for _, x in d]))
+    assert all(i["status"] == "converged" for i in res[0][0]) and res[0][0] == res[1][0]
+    assert all(np.array_equal(p, q) for p, q in zip(res[0][1], res[1][1]))
+    for _, d in reqs:
+        for b, x in d:
+            gpu_ctx.free(b)
+            gpu_ctx.free(x)
