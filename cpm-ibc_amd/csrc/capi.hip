@@ -508,14 +508,27 @@ static BatchBytes batch_bytes1(const Op* op, int NR, bool refine) {
     return batch_bytes(1, nb, std::max(nb, op->ngt), (op->D * NR + 63) & ~int64_t(63), NR, refine, may_fold(nb, NR));
 }
 
-// Grow the context's workspaces to what a batch of one operator with NR
-// right-hand sides needs, so that such a batch allocates nothing.
-static void reserve_batch_workspaces(Ctx* ctx, const Op* op, int NR, bool refine) {
-    const BatchBytes b = batch_bytes1(op, NR, refine);
-    ctx->workspace("tables", b.tables);
-    ctx->workspace("vec64", b.vec64);
-    if (refine) ctx->workspace("vec32", b.vec32);
-    ctx->workspace("pack", b.pack);
+// Right-hand sides of one operator in a group: at most kMaxNR, at most 4 in
+// FP64 where the operator has LDS tiles for FP64 x 4 (FP64 x 8 rows do not fit
+// them).
+static int group_cap(const Op* op, bool refine) {
+    return !refine && op->fmt == OP_TP && (op->ngt > 0 || op->tln.p) ? 4 : kMaxNR;
+}
+// Lanes of a launch whose largest group has n right-hand sides.
+static int group_lanes(int n) { return n <= 1 ? 1 : n == 2 ? 2 : n <= 4 ? 4 : kMaxNR; }
+
+// Grow the context's workspaces to what an FP64 batch of any 1 .. nrhs
+// right-hand sides of one operator needs, grouped as solve_batch groups them,
+// so that such a batch allocates nothing.
+static void reserve_fp64_batches(Ctx* ctx, const Op* op, int nrhs) {
+    const int cap = group_cap(op, false), nb = row_blocks(op), ng = std::max(nb, op->ngt);
+    for (int n = 1; n <= nrhs; ++n) {
+        const int G = (n + cap - 1) / cap, NR = group_lanes(std::min(n, cap));
+        const BatchBytes b = batch_bytes(G, G * nb, G * ng, G * ((op->D * NR + 63) & ~int64_t(63)), NR, false, may_fold((int64_t)G * nb, NR));
+        ctx->workspace("tables", b.tables);
+        ctx->workspace("vec64", b.vec64);
+        ctx->workspace("pack", b.pack);
+    }
 }
 
 template <int NR>
@@ -991,8 +1004,7 @@ void solve_batch(Ctx* ctx, const std::vector<Op*>& ops, const std::vector<const 
             return;
         }
     }
-    // group instances that share an operator and its (m, n): at most kMaxNR per group, at most 4
-    // in FP64 where the operator has LDS tiles for FP64 x 4 (FP64 x 8 rows do not fit them)
+    // group instances that share an operator and its (m, n)
     std::vector<Group> groups;
     std::map<std::tuple<Op*, double, double>, int> open;
     for (int i = 0; i < n; ++i) {
@@ -1000,8 +1012,7 @@ void solve_batch(Ctx* ctx, const std::vector<Op*>& ops, const std::vector<const 
         const double nn = mn ? (*mn)[(size_t)i].second : ops[i]->n;
         const auto key = std::make_tuple(ops[i], m, nn);
         auto it = open.find(key);
-        const size_t cap = (o.precision == CPM_FP64 && ops[i]->fmt == OP_TP && (ops[i]->ngt > 0 || ops[i]->tln.p))
-                               ? 4 : (size_t)kMaxNR;
+        const size_t cap = (size_t)group_cap(ops[i], o.precision != CPM_FP64);
         if (it == open.end() || groups[it->second].inst.size() == cap) {
             groups.push_back(Group{ops[i], m, nn, {}});
             open[key] = (int)groups.size() - 1;
@@ -1011,10 +1022,12 @@ void solve_batch(Ctx* ctx, const std::vector<Op*>& ops, const std::vector<const 
     }
     size_t nr = 1;
     for (auto& g : groups) nr = std::max(nr, g.inst.size());
-    if (nr == 1) run_batch<1>(ctx, groups, rhs, xs, o, infos);
-    else if (nr == 2) run_batch<2>(ctx, groups, rhs, xs, o, infos);
-    else if (nr <= 4) run_batch<4>(ctx, groups, rhs, xs, o, infos);
-    else run_batch<8>(ctx, groups, rhs, xs, o, infos);
+    switch (group_lanes((int)nr)) {
+    case 1: run_batch<1>(ctx, groups, rhs, xs, o, infos); break;
+    case 2: run_batch<2>(ctx, groups, rhs, xs, o, infos); break;
+    case 4: run_batch<4>(ctx, groups, rhs, xs, o, infos); break;
+    default: run_batch<8>(ctx, groups, rhs, xs, o, infos);
+    }
     if (o.precision == CPM_FP32_REFINE) {
         fp64_fallback(ctx, ops, rhs, xs, o, infos, mn);
         record_fp32(ctx, ops, infos);
@@ -1596,7 +1609,7 @@ struct Server : ServerBase {
         if (len > cap) throw ArgError("request larger than the server pool");
         // the FP64 re-solve of this request's lanes (when their refinement stalls) runs in the
         // context's workspaces: grow them now, so that retiring the request allocates nothing
-        reserve_batch_workspaces(ctx, op, NR, false);
+        reserve_fp64_batches(ctx, op, nrhs);
         if (fp64_routing() && prefer_fp64(ctx, op)) {
             // the operator (or its family) stalled in FP32 before: the request is solved in FP64
             // from zero now, as the re-solve of a stalled request is, without FP32 iterations

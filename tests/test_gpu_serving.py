@@ -214,3 +214,38 @@ def test_gather_choice_holds_between_runs(gpu_ctx, monkeypatch, precision, lanes
     assert np.array_equal(res[0][1], res[1][1])
     for p in d:
         gpu_ctx.free(p)
+
+
+@pytest.mark.parametrize("h,lanes,nrhs", [
+    (0.055, 8, 3), (0.055, 8, 4), (0.055, 8, 5), (0.055, 8, 8),   # 133 row blocks
+    (0.0405, 8, 4), (0.0405, 8, 7),                               # 247
+    (0.0365, 4, 2), (0.0365, 4, 3), (0.029, 4, 2),                # 306, 483
+    (0.0275, 2, 1), (0.0275, 2, 2), (0.02, 2, 1),                 # 538, 1,016
+    (0.03, 1, 1),
+])
+def test_retiring_allocates_nothing(monkeypatch, h, lanes, nrhs):
+    """A request whose refinement stalls (a tolerance below what FP64 resolves) is solved again in FP64
+    in the workspaces that its submission reserved, whichever lanes and folding that solve takes."""
+    print(f"case retiring h={h} lanes={lanes} nrhs={nrhs}", flush=True)
+    monkeypatch.setenv("CPMGPU_FP64_ROUTING", "0")
+    ctx = cpmgpu.Context(0)   # no workspaces of earlier solves
+    op = cpmgpu.Tube(ctx, "Sphere", h).operator(1.0, -1e-4)
+    D = op.D
+    d = [ctx.alloc(8 * D) for _ in range(2 * nrhs)]
+    for k in range(nrhs):
+        ctx.h2d(d[k], np.random.default_rng(k).standard_normal(D))
+    srv = cpmgpu.Server(ctx, 90 * lanes * (D + 64) + 4096, lanes=lanes,
+                        o=cpmgpu.opts(tol=1e-18, max_iters=3000, precision=cpmgpu.CPM_FP32_REFINE))
+    assert srv.submit(op, d[:nrhs], d[nrhs:], 1)
+    held = ctx.device_bytes()
+    done = []
+    while not done:
+        done, _ = srv.run(16)
+    print([(i["status"], i["iters"], i["fallback_iters"]) for i in done[0][1]], flush=True)
+    assert any(i["fallback_iters"] for i in done[0][1])
+    assert ctx.device_bytes() == held
+    srv.close()
+    for p in d:
+        ctx.free(p)
+    op.close()
+    ctx.close()
