@@ -167,9 +167,17 @@ __global__ void k_tube_normals(int64_t N, const int* ecol, const double* eval, i
 // by the one CU it runs on: seven launches and two host waits a level took
 // about 90 us (357 levels of three curves: 30 of the 38 ms of a problem).
 // Polylines whose hierarchy fits are copied to LDS first, which the
-// traversals then read.
+// traversals then read.  A curve that winds close to itself joins into a wide
+// frontier, up to the tube's own cross-section, which one CU is too few for:
+// past kBfsWide nodes its levels run over the whole GPU, a few launches each
+// (k_tbfs_*), until half of that are left.  Problems whose curve is a spiral
+// over the unit sphere, h = 0.04 (5 turns, a frontier of about 1,700) and 0.01
+// (20 turns, 5,000): every level on one CU 34.9 and 259 ms, all levels over the
+// GPU 23.4 and 61.7, lines of 512 / 1,024 / 2,048 nodes 23.5 / 27.9 / 34.4 and
+// 53.6 / 56.9 / 67.9.
 constexpr int kBfsThreads = 512;
 constexpr int kBfsLds = 120 * 1024;   // one workgroup per CU
+constexpr int kBfsWide = 512;
 
 struct BfsCurve {
     SurfDev sd;
@@ -177,17 +185,17 @@ struct BfsCurve {
     int32_t start;
     int32_t* vis;                // [N] kUnvisited; members end with their position, others above kCand
     int32_t* cand;               // [N]
-    int32_t* slot;               // [6 fcap], as the four below
+    int32_t* slot;               // [6 kBfsWide], as the four below
     double* ccp;
     double* cdist;
     int32_t* cbdy;
     int64_t cap;                 // room of t_set .. t_bdy
-    int fcap;                    // longest frontier
     int32_t* t_set;
     double* t_cpc;
     double* t_dist;
     int32_t* t_bdy;
-    int32_t* result;             // [2]: members; 1 the outputs, 2 the frontier did not fit
+    int32_t f0, nf, nt;          // where to go on: frontier nf members from f0 on, nt members (0: at the start node)
+    int32_t* result;             // [4]: 0 done, 1 the outputs did not fit, 2 the frontier is wide; nt, f0, nf
 };
 
 __global__ __launch_bounds__(kBfsThreads) void k_tagging_bfs(const BfsCurve* curves, const int32_t* nbr, const int64_t* rec,
@@ -212,9 +220,10 @@ __global__ __launch_bounds__(kBfsThreads) void k_tagging_bfs(const BfsCurve* cur
         sd.mesh.v = reinterpret_cast<const double*>(lds + bn);
         sd.mesh.prim = reinterpret_cast<const int*>(lds + bn + bv);
     }
-    int64_t f0 = 0, nt = 0;
-    int nf = 1;
-    bool seed = true;
+    int64_t f0 = q.f0, nt = q.nt;
+    int nf = nt > 0 ? q.nf : 1;
+    bool seed = nt == 0;
+    int status = 0;
     while (nf > 0) {   // nf, nt, f0 are the same on every thread
         const int ns = nf * 6;
         if (t == 0) ncand = 0;
@@ -271,20 +280,80 @@ __global__ __launch_bounds__(kBfsThreads) void k_tagging_bfs(const BfsCurve* cur
             }
             __syncthreads();
         }
-        const int64_t found = at - nt;
-        if (at > q.cap || found > q.fcap) {
-            if (t == 0) q.result[1] = at > q.cap ? 1 : 2;
-            return;
+        if (at > q.cap) {
+            status = 1;
+            break;
         }
         f0 = nt;
-        nf = (int)found;
+        nf = (int)(at - nt);
         nt = at;
         seed = false;
+        if (nf > kBfsWide) {
+            status = 2;
+            break;
+        }
     }
     if (t == 0) {
-        q.result[0] = (int32_t)nt;
-        q.result[1] = 0;
+        q.result[0] = status;
+        q.result[1] = (int32_t)nt;
+        q.result[2] = (int32_t)f0;
+        q.result[3] = nf;
     }
+}
+
+// A wide level's claims, closest points and members, as above.
+__global__ void k_tbfs_expand(const int32_t* frontier, int64_t nf, const int32_t* nbr, int32_t* vis, int32_t* cand,
+                              int* ncand) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= nf * 6) return;
+    const int64_t fi = t / 6;
+    const int32_t nb = nbr[6 * (int64_t)frontier[fi] + (t - fi * 6)];
+    if (nb < 0) return;
+    const int32_t v = __hip_atomic_load(vis + nb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (v < kCand || v == kOutside) return;
+    if (atomicMin(vis + nb, kCand + (int32_t)t) == kUnvisited) cand[atomicAdd(ncand, 1)] = nb;
+}
+
+__global__ void k_tbfs_eval(const int32_t* cand, const int* ncand, const int64_t* rec, int64_t N1d, double xs, double dx,
+                            SurfDev sd, double radius, int32_t* vis, int32_t* slot, double* ccp, double* cdist,
+                            int32_t* cbdy) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= *ncand) return;
+    const int32_t nb = cand[i];
+    double x[3], c[3], d;
+    int b;
+    node_coords(rec[nb], N1d, xs, dx, x);
+    cp_surface(sd, x, c, d, b);
+    if (!(d < radius)) {
+        vis[nb] = kOutside;
+        return;
+    }
+    slot[vis[nb] - kCand] = (int32_t)i;
+    for (int k = 0; k < 3; ++k) ccp[3 * i + k] = c[k];
+    cdist[i] = d;
+    cbdy[i] = b;
+}
+
+// boff: exclusive sums of the blocks' occupied slots.
+__global__ void k_tbfs_emit(const int32_t* slot, int64_t ns, const int* boff, const int32_t* cand, const double* ccp,
+                            const double* cdist, const int32_t* cbdy, int64_t base, int32_t* vis, int32_t* t_set,
+                            double* t_cpc, double* t_dist, int32_t* t_bdy) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int32_t ci = i < ns ? slot[i] : -1;
+    const unsigned long long m = __ballot(ci >= 0);
+    __shared__ int ws[4];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (lane == 0) ws[w] = __popcll(m);
+    __syncthreads();
+    if (ci < 0) return;
+    int64_t p = base + boff[blockIdx.x] + __popcll(m & ((1ull << lane) - 1ull));
+    for (int k = 0; k < w; ++k) p += ws[k];
+    const int32_t nb = cand[ci];
+    vis[nb] = (int32_t)p;
+    t_set[p] = nb;
+    for (int k = 0; k < 3; ++k) t_cpc[3 * p + k] = ccp[3 * ci + k];
+    t_dist[p] = cdist[ci];
+    t_bdy[p] = cbdy[ci];
 }
 
 // Subset index of every tube node: a member's position, -1 elsewhere.
@@ -724,7 +793,6 @@ static int32_t tagging_start(const Tube* t, const IbcData& I) {
     int32_t start = -1;
     HIPCHK(hipMemcpy(&start, t->gidx.as<int32_t>() + l0, 4, hipMemcpyDeviceToHost));
     if (start < 0 || start >= kCand) throw GeomError("IBC start point is not in the tube");
-
     return start;
 }
 
@@ -741,6 +809,65 @@ static double curve_length(const IbcSpec& c) {
     return len;
 }
 
+// Room for `cap` members of a tagging subset, the first `keep` of them kept.
+static void tagging_room(IbcData& I, int64_t cap, int64_t keep) {
+    if (I.t_set.bytes >= (size_t)cap * 4) return;
+    auto grow = [&](Buffer& b, size_t size) {
+        Buffer n((size_t)cap * size);
+        if (keep) HIPCHK(hipMemcpy(n.p, b.p, (size_t)keep * size, hipMemcpyDeviceToDevice));
+        b = std::move(n);
+    };
+    grow(I.t_set, 4);
+    grow(I.t_cpc, 24);
+    grow(I.t_dist, 8);
+    grow(I.t_bdy, 4);
+}
+
+// Levels of one curve while its frontier is wide; q.f0, q.nf and q.nt move on.
+static void tagging_wide(Tube* t, Ctx* ctx, IbcData& I, BfsCurve& q, double radius) {
+    const hipStream_t st = ctx->stream;
+    auto r256 = [](size_t n) { return (n + 255) & ~size_t(255); };
+    int* found = reinterpret_cast<int*>(ctx->host_states);
+    while (q.nf > kBfsWide / 2) {
+        const int64_t ns = 6 * (int64_t)q.nf, nb = (ns + 255) / 256;
+        char* w = reinterpret_cast<char*>(ctx->workspace("ibc_wide", 256 + r256(ns * 4) * 2 + r256(ns * 24) + r256(ns * 8) + r256(nb * 4)));
+        auto carve = [&](size_t bytes) {
+            char* a = w;
+            w += r256(bytes);
+            return a;
+        };
+        int* count = reinterpret_cast<int*>(carve(256));   // candidates, members
+        int32_t* slot = reinterpret_cast<int32_t*>(carve(ns * 4));
+        int32_t* cbdy = reinterpret_cast<int32_t*>(carve(ns * 4));
+        double* ccp = reinterpret_cast<double*>(carve(ns * 24));
+        double* cdist = reinterpret_cast<double*>(carve(ns * 8));
+        int* bcount = reinterpret_cast<int*>(carve(nb * 4));
+        HIPCHK(hipMemsetAsync(count, 0, 8, st));
+        hipLaunchKernelGGL(k_fill_i32, dim3(std::min<unsigned>((unsigned)nb, 4096)), dim3(256), 0, st, slot, ns, -1);
+        hipLaunchKernelGGL(k_tbfs_expand, dim3((unsigned)nb), dim3(256), 0, st, I.t_set.as<int32_t>() + q.f0, (int64_t)q.nf,
+                           t->nbr.as<int32_t>(), q.vis, q.cand, count);
+        hipLaunchKernelGGL(k_tbfs_eval, dim3((unsigned)nb), dim3(256), 0, st, q.cand, count, t->rec.as<int64_t>(), t->N1d,
+                           t->xstart, t->dx, I.sd, radius, q.vis, slot, ccp, cdist, cbdy);
+        hipLaunchKernelGGL(k_count, dim3((unsigned)nb), dim3(256), 0, st, slot, ns, bcount);
+        hipLaunchKernelGGL(k_scan, dim3(1), dim3(256), 0, st, bcount, nb, count + 1);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(found, count + 1, 4, hipMemcpyDeviceToHost, st));
+        HIPCHK(hipStreamSynchronize(st));
+        const int64_t cnt = *found;
+        if (q.nt + cnt > q.cap) {
+            q.cap = std::min<int64_t>(t->N, std::max<int64_t>(2 * q.cap, q.nt + cnt));
+            tagging_room(I, q.cap, q.nt);
+        }
+        hipLaunchKernelGGL(k_tbfs_emit, dim3((unsigned)nb), dim3(256), 0, st, slot, ns, bcount, q.cand, ccp, cdist, cbdy,
+                           (int64_t)q.nt, q.vis, I.t_set.as<int32_t>(), I.t_cpc.as<double>(), I.t_dist.as<double>(),
+                           I.t_bdy.as<int32_t>());
+        HIPCHK(hipGetLastError());
+        q.f0 = q.nt;
+        q.nf = (int32_t)cnt;
+        q.nt += (int32_t)cnt;
+    }
+}
+
 // Members of the curves' tagging subsets (IBCSubset::ComputeSubset,
 // IBCSubset.cpp:12-109), the curves in one launch as far as their node arrays
 // stay within 512 MB.
@@ -752,91 +879,89 @@ static void tagging_members(Tube* t, Ctx* ctx, std::vector<IbcData>& ibc) {
     auto r256 = [](size_t n) { return (n + 255) & ~size_t(255); };
     for (size_t c0 = 0; c0 < ibc.size(); c0 += most) {
         const size_t n = std::min(most, ibc.size() - c0);
-        // outputs hold the band around the curve (about 16.5 x 8.25 nodes a grid spacing of its
-        // length, and its two ends) and half as much again; too small a guess is doubled
-        std::vector<int64_t> cap(n);
-        std::vector<int32_t> start(n);
-        std::vector<bool> todo(n, true);
+        constexpr size_t kSlots = 6 * (size_t)kBfsWide;
+        const size_t one = r256((size_t)N * 4) * 2 + r256(kSlots * 4) * 2 + r256(kSlots * 24) + r256(kSlots * 8);
+        const size_t stab = r256(sizeof(BfsCurve) * n);
+        char* w = reinterpret_cast<char*>(ctx->workspace("ibc_bfs", one * n));
+        char* tab = reinterpret_cast<char*>(ctx->workspace("ibc_bfs_tab", stab + 16 * n));
+        int32_t* res = reinterpret_cast<int32_t*>(tab + stab);
+        std::vector<BfsCurve> h(n);
+        std::vector<size_t> who(n);   // curves still on their way
         for (size_t k = 0; k < n; ++k) {
-            const IbcData& I = ibc[c0 + k];
-            start[k] = tagging_start(t, I);
-            cap[k] = std::min<int64_t>(N, (int64_t)(1.5 * 136.0 * (curve_length(I.spec) / t->dx + 16.0)));
+            IbcData& I = ibc[c0 + k];
+            BfsCurve& q = h[k];
+            q.sd = I.sd;
+            q.nnodes = I.bvh.nnodes;
+            q.nprim = I.bvh.ntri;
+            q.nverts = I.bvh.nnodes > 0 ? (int)(I.spec.surf.verts.size() / 3) : 0;
+            q.start = tagging_start(t, I);
+            auto carve = [&](size_t bytes) {
+                char* a = w;
+                w += r256(bytes);
+                return a;
+            };
+            q.vis = reinterpret_cast<int32_t*>(carve((size_t)N * 4));
+            q.cand = reinterpret_cast<int32_t*>(carve((size_t)N * 4));
+            q.slot = reinterpret_cast<int32_t*>(carve(kSlots * 4));
+            q.cbdy = reinterpret_cast<int32_t*>(carve(kSlots * 4));
+            q.ccp = reinterpret_cast<double*>(carve(kSlots * 24));
+            q.cdist = reinterpret_cast<double*>(carve(kSlots * 8));
+            // outputs hold the band around the curve (about 16.5 x 8.25 nodes a grid spacing of its length
+            // in degree 3, 19 x 10 in degree 4, and its two ends) and half as much again (in degree 4,
+            // 7%); too small a guess is doubled
+            q.cap = std::min<int64_t>(N, (int64_t)(1.5 * 136.0 * (curve_length(I.spec) / t->dx + 16.0)));
+            who[k] = k;
         }
-        int fcap = 4096;
-        for (bool again = true; again;) {
-            again = false;
-            std::vector<BfsCurve> h;
-            std::vector<size_t> who;
-            const size_t slots = 6 * (size_t)fcap;
-            const size_t one = r256((size_t)N * 4) * 2 + r256(slots * 4) * 2 + r256(slots * 24) + r256(slots * 8);
-            for (size_t k = 0; k < n; ++k)
-                if (todo[k]) who.push_back(k);
-            char* w = reinterpret_cast<char*>(ctx->workspace("ibc_bfs", one * who.size()));
-            char* tab = reinterpret_cast<char*>(ctx->workspace("ibc_bfs_tab", r256(sizeof(BfsCurve) * who.size()) + 8 * who.size()));
-            int32_t* res = reinterpret_cast<int32_t*>(tab + r256(sizeof(BfsCurve) * who.size()));
+        while (!who.empty()) {
+            std::vector<BfsCurve> run;
             for (size_t j = 0; j < who.size(); ++j) {
                 IbcData& I = ibc[c0 + who[j]];
-                const int64_t cp = cap[who[j]];
-                if (I.t_set.bytes < (size_t)cp * 4) {
-                    realloc<int32_t>(I.t_set, cp);
-                    realloc<double>(I.t_cpc, cp * 3);
-                    realloc<double>(I.t_dist, cp);
-                    realloc<int32_t>(I.t_bdy, cp);
-                }
-                char* p = w + one * j;
-                auto carve = [&](size_t bytes) {
-                    char* a = p;
-                    p += r256(bytes);
-                    return a;
-                };
-                BfsCurve q{};
-                q.sd = I.sd;
-                q.nnodes = I.bvh.nnodes;
-                q.nprim = I.bvh.ntri;
-                q.nverts = I.bvh.nnodes > 0 ? (int)(I.spec.surf.verts.size() / 3) : 0;
-                q.start = start[who[j]];
-                q.vis = reinterpret_cast<int32_t*>(carve((size_t)N * 4));
-                q.cand = reinterpret_cast<int32_t*>(carve((size_t)N * 4));
-                q.slot = reinterpret_cast<int32_t*>(carve(slots * 4));
-                q.cbdy = reinterpret_cast<int32_t*>(carve(slots * 4));
-                q.ccp = reinterpret_cast<double*>(carve(slots * 24));
-                q.cdist = reinterpret_cast<double*>(carve(slots * 8));
-                q.cap = cp;
-                q.fcap = fcap;
+                BfsCurve& q = h[who[j]];
+                tagging_room(I, q.cap, q.nt);
                 q.t_set = I.t_set.as<int32_t>();
                 q.t_cpc = I.t_cpc.as<double>();
                 q.t_dist = I.t_dist.as<double>();
                 q.t_bdy = I.t_bdy.as<int32_t>();
-                q.result = res + 2 * j;
-                h.push_back(q);
-                hipLaunchKernelGGL(k_fill_i32, dim3(std::min<unsigned>(nblk(N), 4096)), dim3(256), 0, st, q.vis, N, kUnvisited);
+                q.result = res + 4 * j;
+                run.push_back(q);
+                if (q.nt == 0)
+                    hipLaunchKernelGGL(k_fill_i32, dim3(std::min<unsigned>(nblk(N), 4096)), dim3(256), 0, st, q.vis, N, kUnvisited);
             }
-            HIPCHK(hipMemcpyAsync(tab, h.data(), sizeof(BfsCurve) * h.size(), hipMemcpyHostToDevice, st));
-            hipLaunchKernelGGL(k_tagging_bfs, dim3((unsigned)h.size()), dim3(kBfsThreads), 0, st,
+            HIPCHK(hipMemcpyAsync(tab, run.data(), sizeof(BfsCurve) * run.size(), hipMemcpyHostToDevice, st));
+            hipLaunchKernelGGL(k_tagging_bfs, dim3((unsigned)run.size()), dim3(kBfsThreads), 0, st,
                                reinterpret_cast<const BfsCurve*>(tab), t->nbr.as<int32_t>(), t->rec.as<int64_t>(), t->N1d,
                                t->xstart, t->dx, radius);
-            for (size_t j = 0; j < who.size(); ++j) {
-                IbcData& I = ibc[c0 + who[j]];
-                if (I.t_sub.bytes != (size_t)N * 4) realloc<int32_t>(I.t_sub, N);
-                hipLaunchKernelGGL(k_sub_index, dim3(nblk(N)), dim3(256), 0, st, N, h[j].vis, I.t_sub.as<int32_t>());
-            }
             HIPCHK(hipGetLastError());
-            std::vector<int32_t> r(2 * who.size());
+            std::vector<int32_t> r(4 * who.size());
             HIPCHK(hipMemcpyAsync(r.data(), res, 4 * r.size(), hipMemcpyDeviceToHost, st));
             HIPCHK(hipStreamSynchronize(st));
-            bool wider = false;
+            std::vector<size_t> rest;
             for (size_t j = 0; j < who.size(); ++j) {
-                const size_t k = who[j];
-                if (r[2 * j + 1] == 0) {
-                    ibc[c0 + k].nt = r[2 * j];
-                    todo[k] = false;
+                IbcData& I = ibc[c0 + who[j]];
+                BfsCurve& q = h[who[j]];
+                const int32_t* s = &r[4 * j];
+                if (s[0] == 1) {   // again from the start
+                    q.cap = std::min<int64_t>(N, 2 * q.cap);
+                    q.nt = 0;
+                    rest.push_back(who[j]);
                     continue;
                 }
-                again = true;
-                if (r[2 * j + 1] == 1) cap[k] = std::min<int64_t>(N, 2 * cap[k]);
-                else wider = true;
+                q.nt = s[1];
+                q.f0 = s[2];
+                q.nf = s[3];
+                if (s[0] == 2) {
+                    tagging_wide(t, ctx, I, q, radius);
+                    if (q.nf > 0) {
+                        rest.push_back(who[j]);
+                        continue;
+                    }
+                }
+                I.nt = q.nt;
+                if (I.t_sub.bytes != (size_t)N * 4) realloc<int32_t>(I.t_sub, N);
+                hipLaunchKernelGGL(k_sub_index, dim3(nblk(N)), dim3(256), 0, st, N, q.vis, I.t_sub.as<int32_t>());
             }
-            if (wider) fcap *= 2;
+            HIPCHK(hipGetLastError());
+            who.swap(rest);
         }
     }
 }
