@@ -799,8 +799,8 @@ static int32_t tagging_start(const Tube* t, const IbcData& I) {
 // Length of a curve (0: a point).
 static double curve_length(const IbcSpec& c) {
     const auto& P = c.surf.params;
-    if (c.surf.type == "Circle3D") return 2 * M_PI * P[0];
-    if (c.surf.type == "Arc") return P[0] * (P[2] - P[1]);
+    if (c.surf.type == "Circle3D") return 2 * M_PI * std::fabs(P[0]);
+    if (c.surf.type == "Arc") return std::fabs(P[0]) * (P[2] - P[1]);
     double len = 0.0;
     const std::vector<double>& v = c.surf.verts;
     for (size_t k = 3; k + 2 < v.size(); k += 3)
@@ -909,7 +909,8 @@ static void tagging_members(Tube* t, Ctx* ctx, std::vector<IbcData>& ibc) {
             // outputs hold the band around the curve (about 16.5 x 8.25 nodes a grid spacing of its length
             // in degree 3, 19 x 10 in degree 4, and its two ends) and half as much again (in degree 4,
             // 7%); too small a guess is doubled
-            q.cap = std::min<int64_t>(N, (int64_t)(1.5 * 136.0 * (curve_length(I.spec) / t->dx + 16.0)));
+            const double guess = 1.5 * 136.0 * (curve_length(I.spec) / t->dx + 16.0);
+            q.cap = guess < (double)N ? (int64_t)guess : N;
             who[k] = k;
         }
         while (!who.empty()) {

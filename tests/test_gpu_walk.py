@@ -60,3 +60,14 @@ def test_members_past_the_first_room(gpu_ctx):
     s, cp, _ = Q.subset(0, 0)
     assert len(order) > 204 * 16
     assert np.array_equal(s, order) and np.array_equal(cp, np.broadcast_to(p, cp.shape))
+
+
+def test_room_of_a_circle_with_negative_radius(gpu_ctx):
+    """The first room is guessed from the curve's length, which a signed radius must not turn into a
+    failing allocation: such a circle's closest points lie opposite, and its subset is empty."""
+    print("case walk negative radius", flush=True)
+    n = np.array([1.1, 1.234, 1.321])
+    n /= np.linalg.norm(n)
+    tube = cpmgpu.Tube(gpu_ctx, "Sphere", 0.05)
+    with pytest.raises(cpmgpu.CpmError, match="tagging subset is empty"):
+        cpmgpu.Problem(tube, [cpmgpu.IBC("Circle3D", params=[-np.sqrt(1 - 0.31 ** 2), *(0.31 * n), *n], on_ibc_tolerance=0.1 * 0.05 ** 2)])
