@@ -30,7 +30,7 @@ TUNE = os.path.join(HERE, "_tune")
 DEFAULT = dict(xcd_run=16, lds_rows=2560, grp_rows=2, grp_lds=1024)
 TIE = 0.005
 VARIANTS = [DEFAULT] + [dict(DEFAULT, **{k: v}) for k, vs in (
-    ("xcd_run", (8, 32, 64)), ("lds_rows", (3072,)), ("grp_rows", (1, 3)), ("grp_lds", (1280, 1536))) for v in vs]
+    ("xcd_run", (8, 32, 64)), ("lds_rows", (3072,)), ("grp_rows", (1, 3)), ("grp_lds", (2048,))) for v in vs]
 DEFINES = dict(xcd_run="CPMGPU_XCD_RUN", lds_rows="CPMGPU_LDS_ROWS", grp_rows="CPMGPU_GROUP_ROWS",
                grp_lds="CPMGPU_GROUP_LDS_ROWS")
 
