@@ -267,7 +267,7 @@ __global__ void k_slot_weights(const T* tpw, int64_t D, const int* grow, int64_t
     for (int q = 0; q < 12; ++q) gw[s * 12 + q] = tpw[q * D + r];
 }
 
-// Tensor-product rows on the host, for the tile builders.
+// Tensor-product rows on the host, for the row tiles' builder.
 struct HostTp {
     int64_t D = 0, ne = 0;
     std::vector<uint8_t> flag;
@@ -284,37 +284,7 @@ struct HostTp {
             HIPCHK(hipMemcpy(xcol.data(), xcol_.p, (size_t)ne * 4, hipMemcpyDeviceToHost));
         }
     }
-    // the x rows row r's E row reads (kind 0: 16 lines of 4; exception rows:
-    // the 64 slot columns and the extra column)
-    template <typename F>
-    void columns(int64_t r, F&& f) const {
-        const int e = exc[(size_t)r];
-        if (e >= 0) {
-            for (int s = 0; s < 64; ++s) f(ecx[(size_t)e * 64 + s]);
-            if (xcol[(size_t)e] >= 0) f(xcol[(size_t)e]);
-            return;
-        }
-        for (int l = 0; l < 16; ++l)
-            for (int k = 0; k < 4; ++k) f(tpc[(size_t)l * D + r] + k);
-    }
 };
-
-static void upload(Buffer& b, const void* p, size_t bytes) {
-    b = Buffer(bytes);
-    HIPCHK(hipMemcpy(b.p, p, bytes, hipMemcpyHostToDevice));
-}
-
-template <typename Body>
-static void parallel_for(int64_t n, Body&& body) {
-    const int nth = (int)std::max<int64_t>(
-        1, std::min<int64_t>({16, n, (int64_t)std::max(1u, std::thread::hardware_concurrency())}));
-    std::vector<std::thread> th;
-    for (int w = 0; w < nth; ++w)
-        th.emplace_back([&, w] {
-            for (int64_t i = n * w / nth; i < n * (w + 1) / nth; ++i) body(i);
-        });
-    for (auto& x : th) x.join();
-}
 
 // ---------------------------------------------------------------- shared-stencil tiles
 // Built on the device.  Rows are sorted by the place of their stencil block
