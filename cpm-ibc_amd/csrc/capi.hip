@@ -1289,7 +1289,7 @@ static void extension(Op* op, const StepTables& t, const double* z, double* y) {
 
 void apply_E(Op* op, const double* x, double* y) {
     const hipStream_t st = op->ctx->stream;
-    if (in_place(op)) {
+    if (in_place(op) && apart(op, x, y)) {
         launch_extend_caller(whole_seg(op, 1.0, 0.0), op->perm.as<int>(), x, y, st);
         HIPCHK(hipGetLastError());
         return;
