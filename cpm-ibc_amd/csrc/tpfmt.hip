@@ -632,10 +632,14 @@ __global__ void k_grp_first(const int* parts, int n, int* first, int* total) {
 
 // Items per tile: 256, one per thread of a gather workgroup (the most x rows
 // shared: 1.53 list rows per row, 1.90 with 128, 2.48 with 64), also where
-// that leaves fewer workgroups than the GPU has CUs; fewer for operators of
-// less than 64 such tiles.  Measured with 256 / 128 / 64 items: FP64 solve of
+// that leaves fewer workgroups than the GPU has CUs; 128 for operators of less
+// than 64 such tiles.  Measured with 256 / 128 / 64 items: FP64 solve of
 // 260,000 rows 20.5 / 23.2 / 26.2 ms, of 41,870 rows 4.38 / 4.33 / 4.39 ms,
-// batch of six tubes of 57,000 rows in all 5.20 / 5.01 / 4.99 ms.
+// batch of six tubes of 57,000 rows in all 5.20 / 5.01 / 4.99 ms.  Small
+// operators alone would take 64 (an apply of 10,906 rows 7.67 / 7.32 / 7.14 us,
+// their solves the same), but their workgroups are three quarters empty, and
+// many together pay for it: 60 iterations of 128 FP64 systems of 10,906 rows
+// 10.1 / 11.1 / 13.7 ms (row tiles 11.5), of 240 of 3,190 6.2 / 7.0 / 7.9 (7.1).
 static int group_tile_items(int nitem) {
     // CPMGPU_GROUP_ITEMS: items per tile, rounded down to a power of two (measurements); read once per process
     static const int forced = [] {
@@ -645,9 +649,7 @@ static int group_tile_items(int nitem) {
         return e ? m : 0;
     }();
     if (forced) return forced;
-    int m = kBlock;
-    while (m > 64 && nitem < m * 64) m >>= 1;
-    return m;
+    return nitem < kBlock * 64 ? kBlock / 2 : kBlock;
 }
 
 // Returns false (nothing built) for operators whose slots exceed gofs's bits.
