@@ -23,8 +23,9 @@
 //
 // These were tiles in plain order of their stencils, which fill lists of 1,280
 // rows.  Tiles of 256 items along a Hilbert curve share more of their rows
-// (1.53 list rows per row; 2.2 before) and fit lists of 1,024: 32 KB of LDS,
-// five workgroups of a CU instead of four; grp_lds 1024 chosen.
+// (1.53 list rows per row; 2.2 before) and fit lists of 1,024, 32 KB of LDS
+// (the FP32 x 8 gather's 113 registers hold it at four workgroups a CU with
+// either length); grp_lds 1024 chosen.
 //
 // Measured again once the E gathers took a launch's segments round-robin
 // (bench.py's default run: 128 right-hand sides streamed through 64 lanes,

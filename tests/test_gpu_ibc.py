@@ -251,17 +251,19 @@ def test_plot_matrix_matches_oracle(gpu_ctx, kw):
     _operator_parity(Ag, Ao, x, what="plot rows")
 
 
-@pytest.mark.parametrize("shapes", ["default", "all"])
+@pytest.mark.parametrize("shapes", ["default", "none"])
 def test_lds_tiles_bitwise(gpu_ctx, monkeypatch, shapes):
     """The LDS-tiled E gathers (row tiles, CPMGPU_LDS_TILES=rows, and
-    shared-stencil tiles, built beside them by default and used for FP32 x 8
-    or, with CPMGPU_GROUP_GATHER=all, for every value shape) form the same
+    shared-stencil tiles, built by default and used for every value shape but
+    FP64 x 8, or, with CPMGPU_GROUP_GATHER=none, for none: row tiles where the
+    tile report has built them) form the same
     products in the same order as the direct gather (CPMGPU_LDS_TILES=0): an
     FP64 apply, FP32+refine batch solves of 8 and 3 right-hand sides and an
     FP64 batch solve of 3 agree to the bit, on the torus-knot system (tube
     rows, ghost rows with moved columns, identity rows)."""
-    if shapes == "all":
-        monkeypatch.setenv("CPMGPU_GROUP_GATHER", "all")
+    if shapes == "none":
+        monkeypatch.setenv("CPMGPU_GROUP_GATHER", "none")
+    kernel = "k_egather" if shapes == "none" else "k_egather_grp"
     print("case lds tiles bitwise", flush=True)
     dx = 0.02
     tube = cpmgpu.Tube(gpu_ctx, "Torus", dx, params=[1.0, 0.4], bbox=(-1.4, 1.4))
@@ -288,8 +290,8 @@ def test_lds_tiles_bitwise(gpu_ctx, monkeypatch, shapes):
         for mode in ("1", "rows"):
             assert [i["iters"] for i in xs[mode][1]] == [i["iters"] for i in xs["0"][1]], (mode, nb)
             assert all(np.array_equal(p, q) for p, q in zip(xs[mode][0], xs["0"][0])), (mode, nb)
-    assert ops["1"].gather_kernel(cpmgpu.CPM_FP64, 4) == "k_egather_grp<double,4>"
-    assert ops["1"].gather_kernel(cpmgpu.CPM_FP32_REFINE, 8) == "k_egather_grp<float,8>"
+    assert ops["1"].gather_kernel(cpmgpu.CPM_FP64, 4) == f"{kernel}<double,4>"
+    assert ops["1"].gather_kernel(cpmgpu.CPM_FP32_REFINE, 8) == f"{kernel}<float,8>"
     assert ops["rows"].gather_kernel(cpmgpu.CPM_FP32_REFINE, 8) == "k_egather<float,8>"
 
 
